@@ -113,12 +113,11 @@ __device__ inline uint4 slot_mbr(const PairSlot &e, const float2 *posf, uint32_t
     return make_uint4(f2o(fminf(o.x, e.px)), f2o(fminf(o.y, e.py)), f2o(fmaxf(o.x, e.px)), f2o(fmaxf(o.y, e.py)));
 }
 
+struct MeetCounts { unsigned long long live, expired, fresh, cont; };
+
 struct Counters {             /* device-side counters, copied back once per sync point */
     unsigned long long units;
-    unsigned long long new_keys;
-    unsigned long long continuing;
     unsigned long long ambiguous_nodes;
-    unsigned long long live, expired;
     unsigned long long kv_count;
     uint32_t nodes, leaves;
     uint32_t frontier[NLEVELS + 1];
@@ -128,6 +127,7 @@ struct Counters {             /* device-side counters, copied back once per sync
     uint32_t table_fail;
     uint32_t lookup_overflow;          /* border lookups whose node stack was full */
     uint32_t border_part[64];          /* border points, by partition workgroup mod 64 */
+    MeetCounts meet_part[64];          /* the merge's totals, by workgroup mod 64 */
     /* the collect pass's counters, from candidates to pk_over: cleared together before each pass */
     unsigned long long candidates;
     unsigned long long pairs;          /* slots reserved by the collect pass (pairs and band combinations) */
@@ -1895,29 +1895,44 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
         else join(mold + o0);
         __builtin_amdgcn_wave_barrier(); /* the wave's LDS is reused by its next tile */
     }
-    if (staged) {
-        __builtin_amdgcn_wave_barrier();
-        flush_stage(stage, staged, ma, mt, cnt, lane);
-    }
-    /* one update of each counter per workgroup: updates of one address serialise */
-    __shared__ unsigned long long bsum[256 / STC_WAVE][4];
+    /* the waves' last staged meetings with one reservation, and one update of each counter, per
+     * workgroup; the counters by workgroup mod 64, added up on the host: updates of one address
+     * serialise at about 4 ns each (1M objects, 10.5M slots: 618 us with a reservation per wave, one tile
+     * a wave and one counter of each kind, 168 us = 4.3 TB/s so) */
+    __shared__ MeetCounts bsum[256 / STC_WAVE];
+    __shared__ uint32_t bstaged[256 / STC_WAVE];
+    __shared__ unsigned long long bkb;
     n_live = wave_sum_u64(n_live);
     n_exp = wave_sum_u64(n_exp);
     n_fresh = wave_sum_u64(n_fresh);
     n_cont = wave_sum_u64(n_cont);
     if (lane == 0) {
-        bsum[wv][0] = n_live;
-        bsum[wv][1] = n_exp;
-        bsum[wv][2] = n_fresh;
-        bsum[wv][3] = n_cont;
+        bsum[wv] = MeetCounts{n_live, n_exp, n_fresh, n_cont};
+        bstaged[wv] = staged;
     }
     __syncthreads();
-    if (threadIdx.x < 4) {
-        unsigned long long v = 0;
-        for (int k = 0; k < 256 / STC_WAVE; k++) v += bsum[k][threadIdx.x];
-        unsigned long long *dst[4] = {&cnt->live, &cnt->expired, &cnt->new_keys, &cnt->continuing};
-        if (v) atomicAdd(dst[threadIdx.x], v);
+    if (threadIdx.x == 0) {
+        uint32_t ts = 0;
+        MeetCounts v{0, 0, 0, 0};
+        for (int k = 0; k < 256 / STC_WAVE; k++) {
+            ts += bstaged[k];
+            v.live += bsum[k].live;
+            v.expired += bsum[k].expired;
+            v.fresh += bsum[k].fresh;
+            v.cont += bsum[k].cont;
+        }
+        bkb = ts ? atomicAdd(&cnt->kv_count, 2ull * ts) : 0ull;
+        MeetCounts *part = &cnt->meet_part[blockIdx.x % 64];
+        if (v.live) atomicAdd(&part->live, v.live);
+        if (v.expired) atomicAdd(&part->expired, v.expired);
+        if (v.fresh) atomicAdd(&part->fresh, v.fresh);
+        if (v.cont) atomicAdd(&part->cont, v.cont);
     }
+    __syncthreads();
+    unsigned long long kb = bkb;
+    for (int k = 0; k < wv; k++) kb += 2ull * bstaged[k];
+    for (uint32_t e = lane; e < staged; e += STC_WAVE)
+        write_meeting_records(stage[e], ma.prev, kb + 2ull * e, ma.end_time_min, mt);
 }
 
 #define SEG_CAP 4096u  /* LDS sort keys of the four-wave segment sort */
@@ -3025,14 +3040,17 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
                            (const uint32_t *)c->towner.p, c->tbounds.p);
     }
     CK(hipGetLastError());
-    const uint32_t mgrid = std::max<uint32_t>(std::min<uint32_t>((n_tiles + 3) / 4, 65536), 1);
+    /* ten tiles a wave, but at least 2k workgroups (fewer would leave CUs idle) and at most 64k: each
+     * workgroup reserves its last records on one counter (82k tiles: 245 us with a tile per wave, 187 with
+     * 8k workgroups, 168 with 2k; 2M tiles: 3.61 ms with 64k, 3.59 with 16k, 3.73 with 2k) */
+    const uint32_t mgrid = std::max<uint32_t>(
+        std::min<uint32_t>((n_tiles + 3) / 4, std::min<uint32_t>(std::max<uint32_t>(n_tiles / 40, 2048), 65536)), 1);
     /* the merge writes meet[nx] and, after a flush emptied the memtable, records from index 0 */
     wait_readers(c, nx, kv_before == 0);
     for (int attempt = 0;; attempt++) {
         /* the merge rewrites the same buckets, so a re-run with more record room is exact */
         *c->hinit = before;
-        c->hinit->new_keys = c->hinit->continuing = 0;
-        c->hinit->live = c->hinit->expired = 0;
+        memset(c->hinit->meet_part, 0, sizeof(c->hinit->meet_part));
         c->hinit->kv_count = kv_before;
         CK(hipMemcpyAsync(cnt, c->hinit, sizeof(Counters), hipMemcpyHostToDevice, s));
         const MemtableDev mt{c->rec_keys, c->rec_boxes, c->rec_cap, c->same_pid_count, c->o_boxs, c->sids};
@@ -3068,11 +3086,18 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     }
     c->kv_count = h.kv_count;
     c->oversize_oid_count = h.oversize_oid_count;
-    c->last_live = h.live;
-    c->last_expired = h.expired;
+    MeetCounts met{0, 0, 0, 0};
+    for (const MeetCounts &p : h.meet_part) {
+        met.live += p.live;
+        met.expired += p.expired;
+        met.fresh += p.fresh;
+        met.cont += p.cont;
+    }
+    c->last_live = met.live;
+    c->last_expired = met.expired;
     c->cur = nx;
     c->mlen = c->plen;
-    g.pairs = h.live;
+    g.pairs = met.live;
     CK(hipEventRecord(c->ev[4], s));
 
     /* 10: flush */
@@ -3172,14 +3197,14 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         out->cross_units = g.units;
         out->candidates = g.candidates;
         out->pairs = g.pairs;
-        out->active_meetings = h.live;
-        out->expired = h.expired;
+        out->active_meetings = met.live;
+        out->expired = met.expired;
         out->kv_count = h.kv_count;
         out->overflow_points = h.overflow;
         out->ambiguous_pairs = g.ambiguous;
         out->ambiguous_nodes = h.ambiguous_nodes;
         out->table_buckets = c->mlen;
-        out->table_occupied = h.live + h.expired;
+        out->table_occupied = met.live + met.expired;
         out->flushed = flushed;
         out->rebuilt = 0;
         hipEventElapsedTime(&out->ms_partition, c->ev[0], c->ev[1]);
@@ -3190,8 +3215,8 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         hipEventElapsedTime(&out->ms_total, c->ev[0], c->ev[5]);
         hipEventElapsedTime(&out->ms_refine_kernel, c->ev[6], c->ev[7]);
         hipEventElapsedTime(&out->ms_identify_kernel, c->ev[8], c->ev[9]);
-        out->continuing = h.continuing;
-        out->new_keys = h.new_keys;
+        out->continuing = met.cont;
+        out->new_keys = met.fresh;
         if (g.units || g.nodes) hipEventElapsedTime(&out->ms_count_kernel, c->ev[10], c->ev[11]);
         if (schema_step) hipEventElapsedTime(&out->ms_schema, c->ev[12], c->ev[13]);
         if (flushed && !c->cfg.async_flush) {
