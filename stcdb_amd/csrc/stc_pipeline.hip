@@ -135,6 +135,7 @@ struct Counters {             /* device-side counters, copied back once per sync
     unsigned long long pk_used[64];    /* psrc slots reserved in each slice by the collecting waves */
     unsigned long long cand_part[64], pairs_part[64]; /* the collect pass's totals, by workgroup mod 64 */
     uint32_t big, huge, giant;         /* segments left to the wave sort, the block sort, the global-scratch sort */
+    uint32_t many;                     /* owners with more sources than the collect pass lists */
     uint32_t pk_over;                  /* a collecting wave's reservation exceeded its slice of psrc */
 };
 
@@ -556,9 +557,8 @@ __device__ inline float4 pair_mbr(float ax, float ay, float bx, float by) {
 
 /* Every (unit, member) combination of the step whose pair is owned by a,
  * visited by the 64 lanes of a wave, at most one per lane per call of
- * f(valid, other, decision, probe, mbr, source) (source: the other point's
- * index in the leaf-ordered arrays, or SRC_REV | its index in the reverse
- * lists):
+ * f(valid, decision, source) (source: the other point's index in the
+ * leaf-ordered arrays, or SRC_REV | its index in the reverse lists):
  *   (i)   a against the later (larger-id) kept members of its own leaf (the
  *         inside unit of geometry.cu:258; probe a);
  *   (ii)  a against the kept members above a of the leaves of a's cross units
@@ -566,7 +566,8 @@ __device__ inline float4 pair_mbr(float ax, float ay, float bx, float by) {
  *   (iii) the border points above a that have a cross unit to a's leaf, when a
  *         is a kept member of it (probe: the border point).
  * Each combination of the reference's refinement (geometry.cu:424-497) is
- * visited exactly once, by the owner of its pair. Wave-uniform. */
+ * visited exactly once, by the owner of its pair. Wave-uniform. The collect
+ * pass takes this form only for an owner with more sources than it lists. */
 /* first index i in [0, n) with arr[i] > v (n when none) for ascending arr: the
  * wave's lanes probe 64 evenly spaced entries per round, so a search takes one
  * or two dependent loads where a binary search takes log2(n). Wave-uniform. */
@@ -592,7 +593,7 @@ __device__ inline uint32_t wave_upper_bound(const uint32_t *arr, uint32_t n, uin
     return lo;
 }
 
-template <bool OTHER, class F>
+template <class F>
 __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const PairGeo &g, int lane, F &f) {
     const uint32_t L = g.lleaf[w];
     uint32_t s = g.leaf_count[L];
@@ -600,22 +601,16 @@ __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const Pair
     const uint32_t st = g.leaf_start[L], rank = w - st;
     const double2 pa = g.lxy[w];
     const double pda = g.ld[w], pia = 1.0 / pda; /* dlon[a] (k_prep) and its reciprocal */
-    const float afx = (float)pa.x, afy = (float)pa.y;
     /* (i) */
     for (uint32_t m0 = rank + 1; m0 < s; m0 += STC_WAVE) {
         const uint32_t m = m0 + lane;
         const bool v = m < s;
         int dec = 0;
-        uint32_t q = 0;
-        float4 mb = make_float4(0.f, 0.f, 0.f, 0.f);
         if (v) {
             const double2 qq = g.lxy[st + m];
-            const double qx = qq.x, qy = qq.y;
-            dec = pair_decide(pa, &g.ld[w], pia, qx, qy, g);
-            if (OTHER) q = g.lp[st + m];
-            mb = pair_mbr(afx, afy, (float)qx, (float)qy);
+            dec = pair_decide(pa, &g.ld[w], pia, qq.x, qq.y, g);
         }
-        f(v, q, dec, a, mb, st + m);
+        f(v, dec, st + m);
     }
     /* (ii) */
     const uint2 un = g.lunits[w];
@@ -629,131 +624,26 @@ __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const Pair
             const uint32_t m = m0 + lane;
             const bool v = m < s2;
             int dec = 0;
-            uint32_t q = 0;
-            float4 mb = make_float4(0.f, 0.f, 0.f, 0.f);
             if (v) {
                 const double2 qq = g.lxy[st2 + m];
-                const double qx = qq.x, qy = qq.y;
-                dec = pair_decide(pa, &g.ld[w], pia, qx, qy, g);
-                if (OTHER) q = g.lp[st2 + m];
-                mb = pair_mbr(afx, afy, (float)qx, (float)qy);
+                dec = pair_decide(pa, &g.ld[w], pia, qq.x, qq.y, g);
             }
-            f(v, q, dec, a, mb, st2 + m);
+            f(v, dec, st2 + m);
         }
     }
     /* (iii) */
     if (rank < s) {
         const uint32_t r0 = g.rev_start[L], r1 = g.rev_start[L + 1];
-        const double qx = g.lxy[st + rank].x, qy = g.lxy[st + rank].y;
-        const float qfx = (float)qx, qfy = (float)qy;
         for (uint32_t i0 = r0 + wave_upper_bound(g.rev_pid + r0, r1 - r0, a, lane); i0 < r1; i0 += STC_WAVE) {
             const uint32_t i = i0 + lane;
             const bool v = i < r1;
             int dec = 0;
-            uint32_t p = 0;
-            float4 mb = make_float4(0.f, 0.f, 0.f, 0.f);
             if (v) {
-                if (OTHER) p = g.rev[i].pid;
                 const RevPt rp = g.rev[i];
-                const double2 pp = make_double2(rp.x, rp.y);
-                dec = pair_decide(pp, &g.rev_dl[i], rp.il, qx, qy, g);
-                mb = pair_mbr((float)pp.x, (float)pp.y, qfx, qfy);
+                dec = pair_decide(make_double2(rp.x, rp.y), &g.rev_dl[i], rp.il, pa.x, pa.y, g);
             }
-            f(v, p, dec, p, mb, SRC_REV | i);
+            f(v, dec, SRC_REV | i);
         }
-    }
-}
-
-/* the number of combinations owner_combos visits for the owner at leaf-order
- * place w: its later leaf members, the members above it of its cross units'
- * leaves, the border points above it with a unit to its leaf. Wave-uniform. */
-__device__ inline uint32_t owner_candidates(uint32_t w, const PairGeo &g, int lane) {
-    const uint4 pr = g.prange[w];
-    const uint2 un = g.lunits[w];
-    unsigned long long t = 0;
-    for (uint32_t k = (uint32_t)lane; k < un.y; k += STC_WAVE) t += g.urange[un.x + k].y;
-    t = wave_sum_u64(t);
-    return pr.y + pr.w + (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)t);
-}
-
-/* The same combinations as owner_combos_by_source, with the owner's sources
- * laid end to end so that every call of f but the last fills all 64 lanes
- * (OTHER false: the other point's id and the probe are left out of the call,
- * for a caller that rebuilds them from the source index when it needs them):
- * lane j describes source j (j = 0: (i); 1 .. nu: the cross units; nu + 1:
- * (iii)) by its first index and length, and each lane finds the source of its
- * combination from the prefix of the lengths. Owners with more than 62 cross
- * units take the per-source loops. on_total receives the number of
- * combinations before the first call of f. Wave-uniform. */
-template <bool OTHER, class F, class T>
-__device__ inline void owner_combos(uint32_t w, uint32_t a, const PairGeo &g, int lane, F &f, T &&on_total) {
-    const uint2 un = g.lunits[w];
-    const uint32_t u0 = un.x, nu = un.y;
-    if (nu + 2 > STC_WAVE) {
-        on_total(owner_candidates(w, g, lane));
-        owner_combos_by_source<OTHER>(w, a, g, lane, f);
-        return;
-    }
-    const uint4 pr = g.prange[w];
-    const double2 pa = g.lxy[w];
-    const double pda = g.ld[w], pia = 1.0 / pda; /* dlon[a] (k_prep) and its reciprocal */
-    const float afx = (float)pa.x, afy = (float)pa.y;
-    /* source table: first index (into the leaf-ordered arrays, or rev_pid for
-     * the last source) and length, held by lane j for source j */
-    uint32_t sbase = 0, slen = 0;
-    if (lane == 0) {
-        sbase = pr.x;
-        slen = pr.y;
-    } else if ((uint32_t)lane <= nu) {
-        const uint2 ur = g.urange[u0 + lane - 1];
-        sbase = ur.x;
-        slen = ur.y;
-    } else if ((uint32_t)lane == nu + 1) {
-        sbase = pr.z;
-        slen = pr.w;
-    }
-    /* exclusive prefix of the lengths */
-    uint32_t scum = slen;
-    for (int o = 1; o < STC_WAVE; o <<= 1) {
-        const uint32_t y = __shfl_up(scum, o, STC_WAVE);
-        if (lane >= o) scum += y;
-    }
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)scum, STC_WAVE - 1);
-    on_total(total);
-    scum -= slen;
-    const uint32_t nseg = nu + 2;
-    const double qax = pa.x, qay = pa.y; /* a's position as a member of its leaf */
-    for (uint32_t c0 = 0; c0 < total; c0 += STC_WAVE) {
-        const uint32_t c = c0 + lane;
-        const bool v = c < total;
-        uint32_t j = 0;
-        for (uint32_t k = 1; k < nseg; k++) /* k is wave-uniform: a lane read, no exchange */
-            if ((uint32_t)__builtin_amdgcn_readlane((int)scum, (int)k) <= c) j = k;
-        const uint32_t jb = __shfl(sbase, (int)j, STC_WAVE), jc = __shfl(scum, (int)j, STC_WAVE);
-        int dec = 0;
-        uint32_t q = 0, probe = a, src = 0;
-        float4 mb = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (v) {
-            const uint32_t idx = jb + (c - jc);
-            src = idx;
-            if (j + 1 < nseg) { /* a member of the owner's leaf or of a cross unit's leaf; probe a */
-                if (OTHER) q = g.lp[idx]; /* read with the position, not after the decision */
-                const double2 qq = g.lxy[idx];
-                const double qx = qq.x, qy = qq.y;
-                dec = pair_decide(pa, &g.ld[w], pia, qx, qy, g);
-                mb = pair_mbr(afx, afy, (float)qx, (float)qy);
-            } else { /* a border point with a cross unit to a's leaf; probe the border point */
-                const RevPt rp = g.rev[idx];
-                const uint32_t p = rp.pid;
-                const double2 pp = make_double2(rp.x, rp.y);
-                dec = pair_decide(pp, &g.rev_dl[idx], rp.il, qax, qay, g);
-                q = p;
-                probe = p;
-                src = SRC_REV | idx;
-                mb = pair_mbr((float)pp.x, (float)pp.y, (float)qax, (float)qay);
-            }
-        }
-        f(v, q, dec, probe, mb, src);
     }
 }
 
@@ -843,90 +733,215 @@ __device__ inline uint64_t lanemask_lt(int lane) { return lane == 0 ? 0ull : (~0
 #define PK_SLICES 64u        /* psrc slices, each with its own reservation counter */
 static_assert(sizeof(((Counters *)nullptr)->pk_used) == PK_SLICES * sizeof(unsigned long long), "one counter per slice");
 
-/* The pair pass: per owner (one wave, owners in leaf order), every
- * combination is decided once; those that are pairs or lie in the guard band
- * take a slot of the owner's segment and their sources (the other point's
- * index in the leaf-ordered arrays or SRC_REV | its reverse-list index, with
- * SRC_AMB on band combinations) are written, unsorted, to a run of psrc that
- * the wave reserved (PK_REGION slots at a time, fewer for a wave with few
- * owners left, or the owner's candidate count when larger, so an owner's
- * sources stay contiguous). psrc is split into PK_SLICES equal slices, wave w
- * reserving in slice w % PK_SLICES from that slice's counter, so that no one
- * address takes every reservation (with one owner per wave, as in a small
- * step, a single counter serialises the whole pass). Per owner: the slot count
- * (pcount, by id) and the run's start and length (pkrun, leaf order); band
- * combinations are listed as (probe, other) for the host; segments longer
- * than the place pass sorts go to `big` or `huge`. A reservation beyond its
- * slice writes nothing and sets pk_over (the host grows psrc and repeats the
- * pass; pk_used tells by how much). */
-__global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t *__restrict__ pcount,
+/* the wave's LDS accesses so far complete before its next ones */
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ inline uint64_t wave_lane_u64(unsigned long long v, uint32_t lane) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)lane);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+/* a band combination of owner a as (probe, other): the border point probes in a reverse-list combination */
+__device__ inline void list_band(uint32_t src, uint32_t a, const PairGeo &g, uint2 *amb, uint32_t amb_cap, Counters *cnt) {
+    const bool rev = (src & SRC_REV) != 0;
+    const uint32_t o = rev ? g.rev_pid[src & ~SRC_REV] : g.lp[src];
+    const unsigned long long k = atomicAdd(&cnt->ambiguous, 1ull);
+    if (k < amb_cap) amb[k] = rev ? make_uint2(o, a) : make_uint2(a, o);
+}
+
+/* what the collect pass leaves for owner a, at place w in leaf order: its slots and their run */
+__device__ inline void collect_owner(uint32_t a, uint32_t w, uint32_t run, uint32_t slots, uint32_t *pcount,
+                                     uint2 *pkrun, uint32_t *big, uint32_t *huge, Counters *cnt) {
+    pcount[a] = slots;
+    pkrun[w] = make_uint2(run, slots);
+    if (slots > WCAP) {
+        if (slots <= WSORT_CAP) big[atomicAdd(&cnt->big, 1u)] = a;
+        else huge[atomicAdd(&cnt->huge, 1u)] = a;
+    }
+}
+
+#define CB_SEGS 128u /* source ranges a collecting wave lists at a time */
+
+struct CollectLds {          /* one wave's: the source ranges of the owners at hand, and the owners' positions */
+    uint4 seg[CB_SEGS];      /* first combination, first index (with SRC_REV), owner lane */
+    double2 pos[STC_WAVE];
+    double inv[STC_WAVE];    /* 1 / dpm_lon */
+};
+
+/* The pair pass: every combination of the step (the list above) is decided
+ * once; those that are pairs or lie in the guard band take a slot of their
+ * owner's segment and their sources (the other point's index in the
+ * leaf-ordered arrays or SRC_REV | its reverse-list index, with SRC_AMB on
+ * band combinations) are written, unsorted, to a run of psrc per owner.
+ *
+ * A wave takes `batch` owners that follow one another in leaf order, one per
+ * lane, and lays the combinations of all of them end to end, owner after
+ * owner and source after source (own leaf, cross units, reverse list), so
+ * that every lane of every round but a group's last decides one. The source
+ * ranges are listed in LDS with their first combination; the starts inside a
+ * round's 64 combinations form a 64-bit mask, and the set bits up to a lane
+ * tell its range. Takes are compacted in that order, so each owner's run is
+ * contiguous; the takes ahead of an owner's first combination are counted by
+ * its lane. What bounds it: the issue of some hundred instructions a round,
+ * the positions coming from cache. With an owner per wave instead, the set-up
+ * of an owner and the unfilled lanes of its last round took most of the time
+ * where owners have few combinations (50k objects, 26 each: 137 us, now 22;
+ * 1M, 97 each: 529 us, now 333; 5M, 145 each: 3.76 ms, now 2.42; 10M, 220 each:
+ * 8.5 ms, now 7.6).
+ *
+ * Space: a wave reserves PK_REGION slots of psrc at a time (what its owners
+ * can need when that is less, an owner's combinations when that is more) and
+ * takes on as many owners at once as could fill the rest of it. psrc is split
+ * into PK_SLICES equal slices, wave w reserving in slice w % PK_SLICES from
+ * that slice's counter, so that no one address takes every reservation. Per
+ * owner: the slot count (pcount, by id) and the run's start and length (pkrun,
+ * leaf order); band combinations are listed as (probe, other) for the host;
+ * segments longer than the place pass sorts go to `big` or `huge`. A
+ * reservation beyond its slice writes nothing and sets pk_over (the host grows
+ * psrc and repeats the pass; pk_used tells by how much). */
+__global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t batch, uint32_t *__restrict__ pcount,
                                                       uint2 *__restrict__ pkrun, uint32_t *__restrict__ psrc,
                                                       uint64_t pk_cap, uint2 *__restrict__ amb, uint32_t amb_cap,
                                                       uint32_t *__restrict__ big, uint32_t *__restrict__ huge,
-                                                      Counters *cnt) {
+                                                      uint32_t *__restrict__ many, Counters *cnt) {
+    __shared__ CollectLds wlds[256 / STC_WAVE];
     const int lane = threadIdx.x & (STC_WAVE - 1);
+    CollectLds &ld = wlds[threadIdx.x / STC_WAVE];
     /* wave-uniform values go through readfirstlane: scalar registers, scalar loads, scalar loop control */
-    const uint64_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)((xcd_block_id() * blockDim.x + threadIdx.x) / STC_WAVE));
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / STC_WAVE;
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)((xcd_block_id() * blockDim.x + threadIdx.x) / STC_WAVE));
+    const uint32_t nw = (gridDim.x * blockDim.x) / STC_WAVE;
+    const uint32_t n_batches = (g.n + batch - 1) / batch;
     const uint64_t lt = lanemask_lt(lane);
     unsigned long long cand = 0, total = 0;
     uint64_t rcur = 0, rend = 0; /* the wave's reserved run of psrc */
-    bool over = false;
-    const uint32_t slice_id = (uint32_t)(wid % PK_SLICES);
+    bool over = false, room = true;
+    const uint32_t slice_id = wid % PK_SLICES;
     const uint64_t slice = pk_cap / PK_SLICES, slice_base = slice_id * slice;
-    for (uint64_t w = wid; w < g.n; w += nw) {
-        const uint32_t a = (uint32_t)__builtin_amdgcn_readfirstlane((int)g.lp[w]);
-        bool room = true;
-        uint32_t *out = psrc;
-        auto reserve = [&](uint32_t tot) {
-            if (rend - rcur < tot) {
-                /* PK_REGION slots, or fewer when the wave's remaining owners need less at this
-                 * owner's count each (a wave of a small step has one owner) */
-                const uint64_t left = (g.n - 1 - w) / nw + 1;
-                const uint64_t want = left * tot < PK_REGION ? left * tot : PK_REGION;
-                const uint64_t sz = tot > want ? tot : want;
-                unsigned long long b0 = 0;
-                if (lane == 0) b0 = atomicAdd(&cnt->pk_used[slice_id], (unsigned long long)sz);
-                b0 = __shfl(b0, 0, STC_WAVE);
-                rcur = slice_base + b0;
-                rend = rcur + sz;
-            }
-            room = rend <= slice_base + slice;
-            over |= !room;
-            out = psrc + rcur;
-        };
-        uint32_t fill = 0;
-        auto f = [&](bool v, uint32_t, int dec, uint32_t, float4, uint32_t src) {
-            cand += v;
-            const bool take = v && dec != 0;
-            const uint64_t m = __ballot(take);
-            if (take) {
-                if (room) __builtin_nontemporal_store(dec == 2 ? (src | SRC_AMB) : src, out + fill + (uint32_t)__popcll(m & lt));
-                if (dec == 2) { /* (probe, other): the border point probes in a reverse-list combination */
-                    const bool rev = (src & SRC_REV) != 0;
-                    const uint32_t o = rev ? g.rev_pid[src & ~SRC_REV] : g.lp[src];
-                    const unsigned long long k = atomicAdd(&cnt->ambiguous, 1ull);
-                    if (k < amb_cap) amb[k] = rev ? make_uint2(o, a) : make_uint2(a, o);
-                }
-            }
-            fill += (uint32_t)__popcll(m);
-        };
-        owner_combos<false>((uint32_t)w, a, g, lane, f, reserve);
-        if (lane == 0) {
-            pcount[a] = fill;
-            pkrun[w] = make_uint2((uint32_t)rcur, fill);
-            total += fill;
-            if (fill > WCAP) {
-                if (fill <= WSORT_CAP) big[atomicAdd(&cnt->big, 1u)] = a;
-                else huge[atomicAdd(&cnt->huge, 1u)] = a;
+    for (uint32_t b = wid; b < n_batches; b += nw) {
+        const uint32_t w0 = b * batch, nown = min(batch, g.n - w0);
+        const bool has = (uint32_t)lane < nown;
+        const uint32_t w = w0 + (has ? (uint32_t)lane : 0u);
+        const uint32_t a = g.lp[w];
+        const uint4 pr = has ? g.prange[w] : make_uint4(0, 0, 0, 0);
+        const uint2 un = has ? g.lunits[w] : make_uint2(0, 0);
+        ld.pos[lane] = g.lxy[w];
+        ld.inv[lane] = 1.0 / g.ld[w]; /* the reciprocal of dlon[a] (k_prep) */
+        /* the owner's combinations and non-empty sources, and their prefixes over the batch */
+        uint32_t tot = pr.y + pr.w, ns = (pr.y != 0) + (pr.w != 0);
+        for (uint32_t k = 0; k < un.y; k++) {
+            const uint32_t l = g.urange[un.x + k].y;
+            tot += l;
+            ns += l != 0;
+        }
+        const bool many_src = ns > CB_SEGS; /* more sources than the list holds: left to k_pair_collect_many */
+        if (many_src) {
+            many[atomicAdd(&cnt->many, 1u)] = w;
+            tot = ns = 0;
+        }
+        unsigned long long ptot = tot;
+        uint32_t pns = ns;
+        for (int o = 1; o < STC_WAVE; o <<= 1) {
+            const unsigned long long y = __shfl_up(ptot, o, STC_WAVE);
+            const uint32_t z = __shfl_up(pns, o, STC_WAVE);
+            if (lane >= o) {
+                ptot += y;
+                pns += z;
             }
         }
-        rcur += fill;
+        const uint64_t batch_tot = wave_lane_u64(ptot, STC_WAVE - 1);
+        uint32_t done = 0;
+        while (done < nown) {
+            const uint64_t base = done ? wave_lane_u64(ptot, done - 1) : 0;
+            const uint32_t sbase = done ? (uint32_t)__builtin_amdgcn_readlane((int)pns, (int)done - 1) : 0u;
+            /* the owners from `done` on whose combinations fit in the region and whose sources fit in the list */
+            const uint64_t fits = __ballot((uint32_t)lane >= done && has && ptot - base <= rend - rcur && pns - sbase <= CB_SEGS);
+            const uint32_t gend = done + (uint32_t)__popcll(fits);
+            if (gend == done) { /* not even one owner: a new region, which holds at least one */
+                const uint64_t t1 = (uint32_t)__builtin_amdgcn_readlane((int)tot, (int)done);
+                const uint64_t left = (batch_tot - base) * ((n_batches - 1 - b) / nw + 1);
+                const uint64_t want = left < PK_REGION ? left : PK_REGION;
+                const uint64_t sz = t1 > want ? t1 : want;
+                unsigned long long b0 = 0;
+                if (lane == 0) b0 = atomicAdd(&cnt->pk_used[slice_id], (unsigned long long)sz);
+                rcur = slice_base + wave_lane_u64(b0, 0);
+                rend = rcur + sz;
+                room = rend <= slice_base + slice;
+                over |= !room;
+                continue;
+            }
+            const bool mine = (uint32_t)lane >= done && (uint32_t)lane < gend;
+            const uint32_t gtot = (uint32_t)(wave_lane_u64(ptot, gend - 1) - base);
+            const uint32_t nseg = (uint32_t)__builtin_amdgcn_readlane((int)pns, (int)gend - 1) - sbase;
+            const uint32_t first = (uint32_t)(ptot - tot - base); /* the owner's first combination in the group */
+            if (mine && ns) {
+                uint32_t at = first, sp = pns - ns - sbase;
+                if (pr.y) ld.seg[sp++] = make_uint4(at, pr.x, (uint32_t)lane, 0);
+                at += pr.y;
+                for (uint32_t k = 0; k < un.y; k++) {
+                    const uint2 ur = g.urange[un.x + k];
+                    if (ur.y) ld.seg[sp++] = make_uint4(at, ur.x, (uint32_t)lane, 0);
+                    at += ur.y;
+                }
+                if (pr.w) ld.seg[sp] = make_uint4(at, SRC_REV | pr.z, (uint32_t)lane, 0);
+            }
+            wave_lds_sync();
+            uint32_t fill = 0, sc = 0, ahead = 0; /* ahead: takes before the lane's owner's first combination */
+            uint32_t *out = psrc + rcur;
+            for (uint32_t c0 = 0; c0 < gtot; c0 += STC_WAVE) {
+                const uint32_t c = min(c0 + (uint32_t)lane, gtot - 1);
+                /* the ranges that start inside the round (the first is at combination 0) */
+                const uint32_t st = sc + lane < nseg ? ld.seg[sc + lane].x : ~0u;
+                const uint32_t nb = (uint32_t)__popcll(__ballot(st - c0 < STC_WAVE));
+                uint64_t starts = 0;
+                for (uint32_t i = 0; i < nb; i++)
+                    starts |= 1ull << ((uint32_t)__builtin_amdgcn_readlane((int)st, (int)i) - c0);
+                const uint32_t j = sc - 1 + (uint32_t)__popcll(starts & (lt | (1ull << lane)));
+                sc += nb;
+                const uint4 e = ld.seg[j];
+                const double2 pa = ld.pos[e.z];
+                const bool rev = (e.y & SRC_REV) != 0;
+                const uint32_t idx = (e.y & ~SRC_REV) + (c - e.x);
+                const double2 q = rev ? *(const double2 *)(g.rev + idx) : g.lxy[idx];
+                /* the probe's: the owner, or the border point of the reverse list */
+                double inv = ld.inv[e.z];
+                if (rev) inv = g.rev[idx].il;
+                /* the decision is the same whichever of the two points is subtracted from the other */
+                int dec = 0;
+                if (c0 + lane < gtot)
+                    dec = pair_decide(pa, rev ? g.rev_dl + idx : g.ld + w0 + e.z, inv, q.x, q.y, g);
+                const bool take = dec != 0;
+                const uint64_t m = __ballot(take);
+                if (take) {
+                    const uint32_t src = idx | (e.y & SRC_REV);
+                    if (room) __builtin_nontemporal_store(dec == 2 ? (src | SRC_AMB) : src, out + fill + (uint32_t)__popcll(m & lt));
+                    if (dec == 2) list_band(src, g.lp[w0 + e.z], g, amb, amb_cap, cnt);
+                }
+                if (first - c0 < STC_WAVE) ahead = fill + (uint32_t)__popcll(m & ((1ull << (first - c0)) - 1ull));
+                fill += (uint32_t)__popcll(m);
+            }
+            if (first >= gtot) ahead = fill;
+            const uint32_t next = __shfl_down(ahead, 1, STC_WAVE);
+            const uint32_t got = ((uint32_t)lane + 1 < gend ? next : fill) - ahead;
+            if (mine && !many_src) {
+                total += got;
+                collect_owner(a, w, (uint32_t)(rcur + ahead), got, pcount, pkrun, big, huge, cnt);
+            }
+            if (lane == 0) cand += gtot;
+            rcur += fill;
+            done = gend;
+            wave_lds_sync(); /* the list is rewritten by the next group */
+        }
     }
     /* totals: summed per workgroup, then one update of a counter of 64 (the host adds them), so
      * that no address takes an update per wave */
     __shared__ unsigned long long bsum[256 / STC_WAVE][2];
     cand = wave_sum_u64(cand);
+    total = wave_sum_u64(total);
     if (lane == 0) {
         bsum[threadIdx.x / STC_WAVE][0] = cand;
         bsum[threadIdx.x / STC_WAVE][1] = total;
@@ -942,6 +957,47 @@ __global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t *__
         const uint32_t part = blockIdx.x % PK_SLICES;
         if (c0) atomicAdd(&cnt->cand_part[part], c0);
         if (t0) atomicAdd(&cnt->pairs_part[part], t0);
+    }
+}
+
+/* the collect pass for the owners it left (`many`: their places in leaf order): a wave each, source by source */
+__global__ __launch_bounds__(256) void k_pair_collect_many(PairGeo g, const uint32_t *__restrict__ many, uint32_t n_many,
+                                                           uint32_t *__restrict__ pcount, uint2 *__restrict__ pkrun,
+                                                           uint32_t *__restrict__ psrc, uint64_t pk_cap,
+                                                           uint2 *__restrict__ amb, uint32_t amb_cap,
+                                                           uint32_t *__restrict__ big, uint32_t *__restrict__ huge,
+                                                           Counters *cnt) {
+    const int lane = threadIdx.x & (STC_WAVE - 1);
+    const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) / STC_WAVE));
+    if (k >= n_many) return;
+    const uint64_t lt = lanemask_lt(lane);
+    const uint32_t w = many[k], a = g.lp[w], slice_id = k % PK_SLICES;
+    const uint4 pr = g.prange[w];
+    const uint2 un = g.lunits[w];
+    unsigned long long tot = 0;
+    for (uint32_t u = (uint32_t)lane; u < un.y; u += STC_WAVE) tot += g.urange[un.x + u].y;
+    tot = wave_lane_u64(wave_sum_u64(tot), 0) + pr.y + pr.w;
+    const uint64_t slice = pk_cap / PK_SLICES;
+    unsigned long long b0 = 0;
+    if (lane == 0) b0 = atomicAdd(&cnt->pk_used[slice_id], tot);
+    const uint64_t run = slice_id * slice + wave_lane_u64(b0, 0);
+    const bool room = run + tot <= (slice_id + 1) * slice;
+    uint32_t fill = 0;
+    auto f = [&](bool v, int dec, uint32_t src) {
+        const bool take = v && dec != 0;
+        const uint64_t m = __ballot(take);
+        if (take) {
+            if (room) psrc[run + fill + (uint32_t)__popcll(m & lt)] = dec == 2 ? (src | SRC_AMB) : src;
+            if (dec == 2) list_band(src, a, g, amb, amb_cap, cnt);
+        }
+        fill += (uint32_t)__popcll(m);
+    };
+    owner_combos_by_source(w, a, g, lane, f);
+    if (lane == 0) {
+        if (!room) atomicOr(&cnt->pk_over, 1u);
+        atomicAdd(&cnt->cand_part[slice_id], tot);
+        atomicAdd(&cnt->pairs_part[slice_id], (unsigned long long)fill);
+        collect_owner(a, w, (uint32_t)run, fill, pcount, pkrun, big, huge, cnt);
     }
 }
 
@@ -1106,13 +1162,6 @@ __device__ inline void write_sorted_segment(const uint32_t *srcs, uint32_t slots
             dr += (uint32_t)__popcll(md);
         }
     }
-}
-
-/* the wave's LDS accesses so far complete before its next ones */
-__device__ inline void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 /* The place pass's form of the above, with the wave's LDS buffer lds (64 * K
@@ -2869,11 +2918,15 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
                      c->ucount.p, c->rev_start.p, c->rev_pid.p,
                      c->rev.p, c->rev_dl.p, n, c->buf, r, c->band, r * r * (1.0 - 1e-12),
                      r * r * (1.0 + 1e-12)};
-    /* a multiple of 8 workgroups, for the XCD-aware owner order; at most 32k from 4M objects on (at 10M
-     * objects a step is 0.5 ms shorter than with 16k, measured three times each on one box), else 16k
-     * (with 32k, 64 batched streams of 48k-500k objects stepped 8 % slower) */
-    const uint32_t pcap = n >= (1u << 22) ? 256u * 128u : 256u * 64u;
-    const uint32_t pgrid = (uint32_t)std::min<uint64_t>((blocks_for((uint64_t)n * STC_WAVE, 256) + 7) & ~7ull, pcap);
+    /* the collect pass: owners a wave takes on at a time, and a multiple of 8 workgroups for the XCD-aware
+     * owner order. Fewer owners a wave give more waves, each of which pays its set-up and its space
+     * reservation: at 10k objects 4 (18 us; 1 or 2: 23-36), at 50k 16 (21 us; 8: 28, 4: 42), at 200k 16 (88 us;
+     * 8: 99, 64: 127), at 1M 16 (333 us; 32: 354, 64: 440), at 5M 64 (16 and 32 the same within 3 %). At most
+     * 4k workgroups (1M objects: 333 us, 16k: 378), from 4M objects on 6k (5M: 2.42 ms, 4k: 2.56, 16k: 2.96; 10M:
+     * 7.64 ms, 4k: 7.67, 16k: 8.09) */
+    const uint32_t batch = n < (1u << 15) ? 4 : n < (1u << 22) ? 16 : 64;
+    const uint32_t pgrid = std::min<uint32_t>((blocks_for(blocks_for(n, batch) * (uint64_t)STC_WAVE, 256) + 7) & ~7u,
+                                              n < (1u << 22) ? 4096u : 6144u);
     /* the last run's host copies overlap the collect pass, which computes more than it writes */
     if (queue_run_copies(c)) return fail(c, STC_E_HIP, std::string("run copies: ") + g_last_fail);
     if (c->pkrun.ensure(n)) return fail(c, STC_E_CAPACITY, "pair key runs");
@@ -2884,12 +2937,21 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
         CK(hipMemsetAsync(&cnt->candidates, 0,
                           offsetof(Counters, pk_over) + sizeof(uint32_t) - offsetof(Counters, candidates), s));
         CK(hipEventRecord(c->ev[10], s));
-        hipLaunchKernelGGL(k_pair_collect, dim3(pgrid), dim3(256), 0, s, pg, c->pcount.p, c->pkrun.p, c->psrc.p,
+        hipLaunchKernelGGL(k_pair_collect, dim3(pgrid), dim3(256), 0, s, pg, batch, c->pcount.p, c->pkrun.p, c->psrc.p,
                            (uint64_t)std::min<size_t>(c->psrc.cap, 0xFFFFFFFFu), c->amb.p,
-                           (uint32_t)std::min<size_t>(c->amb.cap, 0xFFFFFFFFu), c->spill_big.p, c->spill_huge.p, cnt);
+                           (uint32_t)std::min<size_t>(c->amb.cap, 0xFFFFFFFFu), c->spill_big.p, c->spill_huge.p,
+                           c->spill_giant.p, cnt);
         CK(hipGetLastError());
         CK(hipEventRecord(c->ev[11], s));
         CKRC(sync_counters(c));
+        if (c->hcnt->many) { /* their list is in spill_giant until the giant segments are listed there */
+            hipLaunchKernelGGL(k_pair_collect_many, dim3(blocks_for((uint64_t)c->hcnt->many * STC_WAVE, 256)), dim3(256), 0, s, pg,
+                               (const uint32_t *)c->spill_giant.p, c->hcnt->many, c->pcount.p, c->pkrun.p, c->psrc.p,
+                               (uint64_t)std::min<size_t>(c->psrc.cap, 0xFFFFFFFFu), c->amb.p,
+                               (uint32_t)std::min<size_t>(c->amb.cap, 0xFFFFFFFFu), c->spill_big.p, c->spill_huge.p, cnt);
+            CK(hipGetLastError());
+            CKRC(sync_counters(c));
+        }
         h = *c->hcnt;
         for (uint32_t k = 0; k < PK_SLICES; k++) {
             h.candidates += h.cand_part[k];
