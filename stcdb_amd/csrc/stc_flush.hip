@@ -698,9 +698,18 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     hipLaunchKernelGGL(k_str_prepare, dim3(1), dim3(1), 0, s, fc, n, split);
     FCK(hipGetLastError());
     /* F2: STR over the full 64-bit key (x high, y low), stable from oid order */
-    FRC(stc_radix_sort_u64(w->mid, w->oids, w->mid_alt, w->oids_alt, n, 0, sc.on ? (int)sc.str_bits : 64, w->scan_temp, s));
+    auto sort_mid = [&](int bits) {
+        bool in_alt = false;
+        const int rc = stc_radix_sort_u64(w->mid, w->oids, w->mid, w->oids, w->mid_alt, w->oids_alt, n, 0, bits, w->scan_temp, &in_alt, s);
+        if (in_alt) {
+            std::swap(w->mid, w->mid_alt);
+            std::swap(w->oids, w->oids_alt);
+        }
+        return rc;
+    };
+    FRC(sort_mid(sc.on ? (int)sc.str_bits : 64));
     hipLaunchKernelGGL(k_strip_keys, dim3(blocks_for(n, B)), dim3(B), 0, s, w->mid, n, sc, fc);
-    FRC(stc_radix_sort_u64(w->mid, w->oids, w->mid_alt, w->oids_alt, n, 0, sc.on ? (int)sc.strip_bits : 40, w->scan_temp, s));
+    FRC(sort_mid(sc.on ? (int)sc.strip_bits : 40));
     hipLaunchKernelGGL(k_make_sid, dim3(blocks_for(n, B)), dim3(B), 0, s, w->oids, n, a->sids, fc);
     /* F3 */
     hipLaunchKernelGGL(k_ctf_capacity, dim3(blocks_for(n, B)), dim3(B), 0, s, w->oids, n, a->sids, a->same_pid_count,
@@ -710,7 +719,9 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     /* F4: object order (key, oid), slot ranges, scatter, rank */
     hipLaunchKernelGGL(k_obj_keys, dim3(blocks_for(n, B)), dim3(B), 0, s, n, a->sids, w->part_tail,
                        a->same_pid_count, w->obj_key, w->obj_id, w->obj_cnt);
-    FRC(stc_radix_sort_u32(w->obj_key, w->obj_id, (uint32_t *)w->mid_alt, w->oids_alt, n, 12, w->scan_temp, s));
+    bool obj_alt = false; /* 12 bits are two passes: back in obj_key, obj_id */
+    FRC(stc_radix_sort_u32(w->obj_key, w->obj_id, w->obj_key, w->obj_id, (uint32_t *)w->mid_alt, w->oids_alt, n, 12, w->scan_temp,
+                           &obj_alt, s));
     hipLaunchKernelGGL(k_gather_counts, dim3(blocks_for(n, B)), dim3(B), 0, s, w->obj_id, a->same_pid_count, n,
                        w->obj_cnt);
     FRC(stc_exclusive_scan_u32(w->obj_cnt, w->obj_cnt, n, nullptr, w->scan_temp, s));

@@ -384,11 +384,6 @@ __global__ void k_amb_gather(const double2 *__restrict__ xy, const uint2 *__rest
     out[i] = make_double4(p.x, p.y, q.x, q.y);
 }
 
-__global__ void k_iota(uint32_t *a, uint32_t n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = i;
-}
-
 /* leaf-ordered SoA and each point's rank within its leaf */
 __global__ void k_gather(const double2 *__restrict__ xy, const double *__restrict__ dlon,
                          const uint32_t *__restrict__ lp, const uint32_t *__restrict__ pt_leaf,
@@ -2398,6 +2393,21 @@ static int ilog2_ceil(uint64_t v) {
     return l;
 }
 
+/* stc_radix_sort_u32/u64 into k/v, whichever of the two pairs of buffers the last pass wrote */
+template <class K>
+static int sort_pairs(const K *kin, const uint32_t *vin, DBuf<K> &k, DBuf<uint32_t> &v, DBuf<K> &ka, DBuf<uint32_t> &va,
+                      uint32_t n, int bits, uint32_t *temp, hipStream_t s) {
+    bool in_alt = false;
+    int rc;
+    if constexpr (sizeof(K) == 4) rc = stc_radix_sort_u32(kin, vin, k.p, v.p, ka.p, va.p, n, bits, temp, &in_alt, s);
+    else rc = stc_radix_sort_u64(kin, vin, k.p, v.p, ka.p, va.p, n, 0, bits, temp, &in_alt, s);
+    if (in_alt) {
+        std::swap(k, ka);
+        std::swap(v, va);
+    }
+    return rc;
+}
+
 /* the last step's pairs (its pair slots without the dead ones), sorted by key */
 static int step_pairs(StcCtx *c, std::vector<PairHit> &ph) {
     ph.resize(c->plen);
@@ -2804,7 +2814,8 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     /* the order the partition walks the points in: Morton order, or with a kept schema the previous
      * step's leaf order (objects move a few metres a step, so it is as coherent, without the sort) */
     const bool reuse_order = c->dyn && c->sch.present && c->lp_valid;
-    if (!reuse_order) CKRC(stc_radix_sort_u32(c->codes.p, c->idx.p, c->codes_alt.p, c->idx_alt.p, n, 28, c->temp.p, s));
+    if (!reuse_order)
+        CKRC(sort_pairs((const uint32_t *)c->codes.p, (const uint32_t *)c->idx.p, c->codes, c->idx, c->codes_alt, c->idx_alt, n, 28, c->temp.p, s));
     const uint32_t *walk = reuse_order ? (const uint32_t *)c->lp.p : (const uint32_t *)c->idx.p;
 
     /* 3: tree: rebuilt from the step's points, or the persistent dynamic schema */
@@ -2842,10 +2853,8 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     CK(hipGetLastError());
     /* 5: leaves in id order */
     CKRC(stc_exclusive_scan_u32(c->leaf_count.p, c->leaf_start.p, n_leaves, nullptr, c->temp.p, s));
-    CK(hipMemcpyAsync(c->lkeys.p, c->pt_leaf.p, 4ull * n, hipMemcpyDeviceToDevice, s));
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(n, 256)), dim3(256), 0, s, c->lp.p, n);
-    CKRC(stc_radix_sort_u32(c->lkeys.p, c->lp.p, c->codes_alt.p, c->idx_alt.p, n,
-                            std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
+    CKRC(sort_pairs((const uint32_t *)c->pt_leaf.p, (const uint32_t *)nullptr, c->lkeys, c->lp, c->codes_alt, c->idx_alt, n,
+                    std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
     hipLaunchKernelGGL(k_gather, dim3(blocks_for(n, 256)), dim3(256), 0, s, xy, c->dlon.p, c->lp.p, c->pt_leaf.p,
                        c->leaf_start.p, n, c->lxy.p, c->ld.p, c->pt_rank.p, c->lleaf.p);
     c->lp_valid = true; /* lp: a permutation of the points, in this step's leaf order */
@@ -2887,8 +2896,8 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
         hipLaunchKernelGGL(k_units_split, dim3(blocks_for(n_units, 256)), dim3(256), 0, s, c->units.p,
                            (uint32_t)n_units, c->rev_leaf.p, c->rev_pid.p);
         CK(hipGetLastError());
-        CKRC(stc_radix_sort_u32(c->rev_leaf.p, c->rev_pid.p, c->rev_leaf_alt.p, c->rev_pid_alt.p, (uint32_t)n_units,
-                                std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
+        CKRC(sort_pairs((const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, c->rev_leaf, c->rev_pid, c->rev_leaf_alt,
+                        c->rev_pid_alt, (uint32_t)n_units, std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
         hipLaunchKernelGGL(k_rev_gather, dim3(blocks_for(n_units, 256)), dim3(256), 0, s, (const uint32_t *)c->rev_pid.p,
                            (uint32_t)n_units, xy, (const double *)c->dlon.p, c->rev.p,
                            c->rev_dl.p);
@@ -3390,8 +3399,8 @@ int stc_step_meetings(void *vc, const stc_meeting_unit *units, uint64_t nu64, ui
         hipLaunchKernelGGL(k_units_decode, dim3(blocks_for(nu, 256)), dim3(256), 0, s, c->units_in.p, nu, c->n,
                            c->ukeys.p, c->uidx.p, cnt);
         CK(hipGetLastError());
-        CKRC(stc_radix_sort_u64(c->ukeys.p, c->uidx.p, c->ukeys_alt.p, c->uidx_alt.p, nu, 0,
-                                32 + std::max(1, ilog2_ceil(c->n)), c->utemp.p, s));
+        CKRC(sort_pairs((const uint64_t *)c->ukeys.p, (const uint32_t *)c->uidx.p, c->ukeys, c->uidx, c->ukeys_alt, c->uidx_alt, nu,
+                        32 + std::max(1, ilog2_ceil(c->n)), c->utemp.p, s));
         hipLaunchKernelGGL(k_units_gather, dim3(blocks_for(nu, 256)), dim3(256), 0, s, c->ukeys.p, c->uidx.p,
                            c->units_in.p, nu, c->pbox.p, cnt);
         CK(hipGetLastError());
@@ -3535,7 +3544,8 @@ int stc_build_schema(void *vc, const double *xy, int32_t xy_on_device) {
     hipLaunchKernelGGL(k_prep, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->s, src, c->n, c->map, c->codes.p,
                        c->idx.p, c->dlon.p, (float2 *)nullptr, c->dcnt); /* posf keeps the last step's positions */
     CK(hipGetLastError());
-    CKRC(stc_radix_sort_u32(c->codes.p, c->idx.p, c->codes_alt.p, c->idx_alt.p, c->n, 28, c->temp.p, c->s));
+    CKRC(sort_pairs((const uint32_t *)c->codes.p, (const uint32_t *)c->idx.p, c->codes, c->idx, c->codes_alt, c->idx_alt, c->n, 28,
+                    c->temp.p, c->s));
     int rc = stc_schema_build(&c->sch, src, c->idx.p, c->n, c->map, c->cap, c->cfg.reach_distance, c->temp.p,
                               c->temp.cap, c->s);
     if (rc) return fail(c, rc, rc == STC_E_ARG ? "root does not split: too few objects for grid_capacity"

@@ -1,42 +1,55 @@
 /*
  * stc_radix.hip — stable LSD radix sort and prefix sums for gfx950.
  *
- * One pass per 8-bit digit, three launches per pass:
- *   histogram : each workgroup counts the digits of its tile of 4096 keys in LDS
- *               and writes them digit-major (digit * tiles + tile);
- *   scan      : exclusive prefix sum over that table (three-phase scan);
- *   scatter   : each workgroup ranks its tile stably, 256 keys per round, with
- *               per-wavefront peer masks built from 8 ballots (64-wide), then
- *               per-digit wave offsets in LDS; 4-byte keys are placed in LDS
- *               in digit order and written out in that order (coalesced),
- *               8-byte keys straight to their global positions.
+ * One pass per 8-bit digit:
+ *   histogram : each workgroup counts the digits of its tile of keys in LDS;
+ *   offsets   : a sort of up to 128 tiles lets every scatter workgroup add up
+ *               the tiles' histograms itself; a larger one writes them
+ *               digit-major (digit * tiles + tile) and scans that table;
+ *   scatter   : each workgroup ranks its tile stably and moves it. A wave holds
+ *               its stretch of the tile in registers, all loads issued before
+ *               the first ranking, and ranks it 64 keys a round by peer masks
+ *               from 8 ballots and digit counts of its own in LDS, without a
+ *               barrier; the waves' counts are added up once at the end. 4-byte
+ *               keys are placed in LDS in digit order and written out in that
+ *               order (coalesced), 8-byte keys straight to their global
+ *               positions.
  * Keys of equal digit keep their input order, so chaining passes from the
  * least significant digit gives a stable sort, as thrust::sort_by_key on
  * primitive keys does in the reference (src/cuda/geometry.cu:1860, 1878-1886).
+ *
+ * What bounds it below a million keys is latency, so the tile is 1024 keys up
+ * to 64k keys (a tile is then 4 rounds, and 50k keys are 49 workgroups instead
+ * of 13), 2048 up to 2M and 4096 above. With 4096-key tiles ranked 256 keys a
+ * round, four barriers and a load in each, a pass over 50k keys took five
+ * launches and 27 us and takes two and 9 us so; one over 1M keys took six and
+ * 37 us and takes four and 22 us.
  */
 #include "stc_internal.h"
 
 #define RS_THREADS 256
-#define RS_ITEMS 16
-#define RS_TILE (RS_THREADS * RS_ITEMS)
+#define RS_WAVES (RS_THREADS / STC_WAVE)
 #define RS_BINS 256
+#define RS_DIRECT 128          /* tiles whose histograms a scatter workgroup adds up itself */
+#define RS_SMALL (64u << 10)   /* keys up to which a tile has 4 keys a thread */
+#define RS_MEDIUM (2u << 20)   /* and 8 */
 #define SCAN_THREADS 1024
 #define SCAN_ITEMS 4
 #define SCAN_TILE (SCAN_THREADS * SCAN_ITEMS)
+#define SCAN_SUMS 4096         /* tile sums that a scan workgroup adds up itself */
 
 static inline uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
+static inline uint32_t rs_items(uint32_t n) { return n <= RS_SMALL ? 4 : n <= RS_MEDIUM ? 8 : 16; }
 
 size_t stc_radix_temp_words(uint32_t n) {
-    uint32_t tiles = ceil_div(n ? n : 1, RS_TILE);
-    size_t hist = (size_t)RS_BINS * tiles;
-    size_t sums = ceil_div(hist, SCAN_TILE);
-    size_t sums2 = ceil_div(sums, SCAN_TILE);
-    /* histogram + scan partials (two levels) + total + slack */
-    size_t scan_n = (n > hist ? n : hist);
-    size_t s1 = ceil_div(scan_n, SCAN_TILE);
-    size_t s2 = ceil_div(s1, SCAN_TILE);
-    (void)sums; (void)sums2;
-    return hist + s1 + s2 + 64;
+    if (!n) n = 1;
+    /* histograms of a sort of up to n keys (the tiles of 2M keys outnumber those of a few more), then
+     * the scans' tile sums, two levels */
+    const uint32_t few = n < RS_MEDIUM ? n : RS_MEDIUM;
+    const size_t t0 = ceil_div(n, RS_THREADS * 16), t1 = ceil_div(few, RS_THREADS * 8), t2 = RS_SMALL / (RS_THREADS * 4);
+    const size_t hist = RS_BINS * (t0 > t1 ? (t0 > t2 ? t0 : t2) : (t1 > t2 ? t1 : t2));
+    const size_t s1 = ceil_div(n > hist ? n : hist, SCAN_TILE);
+    return hist + s1 + ceil_div(s1, SCAN_TILE) + 64;
 }
 
 /* ---------------- exclusive scan ---------------- */
@@ -50,68 +63,77 @@ __device__ inline uint32_t wave_incl_scan(uint32_t v, int lane) {
     return v;
 }
 
-/* block-wide exclusive scan of one value per thread; returns the block total in *total */
+/* block-wide exclusive scan of one value per thread; the block's total to every thread in *total */
 __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t *total) {
-    __shared__ uint32_t wsum[SCAN_THREADS / STC_WAVE];
+    __shared__ uint32_t wsum[SCAN_THREADS / STC_WAVE], all;
     int lane = threadIdx.x & (STC_WAVE - 1), w = threadIdx.x / STC_WAVE;
+    const int nw = (int)(blockDim.x / STC_WAVE);
     uint32_t inc = wave_incl_scan(v, lane);
     if (lane == STC_WAVE - 1) wsum[w] = inc;
     __syncthreads();
     if (w == 0) {
-        uint32_t x = lane < (int)(blockDim.x / STC_WAVE) ? wsum[lane] : 0;
+        uint32_t x = lane < nw ? wsum[lane] : 0;
         uint32_t xi = wave_incl_scan(x, lane);
-        if (lane < (int)(blockDim.x / STC_WAVE)) wsum[lane] = xi - x;
-        if (lane == (int)(blockDim.x / STC_WAVE) - 1) *total = xi;
+        if (lane < nw) wsum[lane] = xi - x;
+        if (lane == nw - 1) all = xi;
     }
     __syncthreads();
     uint32_t r = inc - v + wsum[w];
+    *total = all;
     __syncthreads();
     return r;
 }
 
-__global__ void k_scan_tiles(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *tile_sums) {
-    __shared__ uint32_t tot;
-    uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
+__global__ __launch_bounds__(SCAN_THREADS) void k_scan_sums(const uint32_t *__restrict__ in, uint32_t n,
+                                                             uint32_t *__restrict__ sums) {
+    uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
+    uint32_t s = 0, tot;
+#pragma unroll
+    for (int k = 0; k < SCAN_ITEMS; k++) {
+        const uint64_t i = base + (uint64_t)k * SCAN_THREADS;
+        s += i < n ? in[i] : 0;
+    }
+    block_excl_scan(s, &tot);
+    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
+}
+
+/* One tile per workgroup: the tiles before it (their sums added up here, or
+ * scanned already), then the tile. in may equal out. Up to SCAN_SUMS tiles the
+ * scan is these two launches (before: one per level up and down, one for the
+ * total and a copy of the last value; five for 1M values). */
+__global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(const uint32_t *in, uint32_t *out, uint32_t n,
+                                                              const uint32_t *__restrict__ sums, int scanned,
+                                                              uint32_t *total) {
+    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
     uint32_t v[SCAN_ITEMS];
-    uint32_t s = 0;
+    uint32_t s = 0, before = 0, tot;
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
         v[k] = (base + k < n) ? in[base + k] : 0;
         s += v[k];
     }
-    uint32_t ex = block_excl_scan(s, &tot);
+    if (scanned) {
+        before = sums[blockIdx.x];
+    } else if (blockIdx.x) {
+        uint32_t p = 0;
+        for (uint32_t i = threadIdx.x; i < blockIdx.x; i += SCAN_THREADS) p += sums[i];
+        block_excl_scan(p, &before);
+    }
+    uint32_t ex = before + block_excl_scan(s, &tot);
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
         if (base + k < n) out[base + k] = ex;
         ex += v[k];
     }
-    if (threadIdx.x == 0 && tile_sums) tile_sums[blockIdx.x] = tot;
+    if (total && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = before + tot;
 }
 
-__global__ void k_scan_add(uint32_t *out, uint32_t n, const uint32_t *tile_offsets) {
-    uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
-    uint32_t add = tile_offsets[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++)
-        if (base + k < n) out[base + k] += add;
-}
-
-__global__ void k_scan_total(const uint32_t *in, const uint32_t *out, uint32_t n, uint32_t *total) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *total = n ? out[n - 1] + in[n - 1] : 0;
-}
-
-/* in and out may alias for the first level; totals are recovered before
- * overwriting by scanning into `out` and keeping tile sums separately. */
-static int scan_rec(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *temp, hipStream_t s) {
-    uint32_t tiles = ceil_div(n, SCAN_TILE);
-    if (tiles <= 1) {
-        hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(SCAN_THREADS), 0, s, in, out, n, (uint32_t *)nullptr);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    uint32_t *sums = temp;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(SCAN_THREADS), 0, s, in, out, n, sums);
-    if (scan_rec(sums, sums, tiles, temp + tiles, s)) return -1;
-    hipLaunchKernelGGL(k_scan_add, dim3(tiles), dim3(SCAN_THREADS), 0, s, out, n, sums);
+static int scan_rec(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *total, uint32_t *temp, hipStream_t s) {
+    const uint32_t tiles = ceil_div(n, SCAN_TILE);
+    const bool two = tiles > SCAN_SUMS;
+    if (tiles > 1) hipLaunchKernelGGL(k_scan_sums, dim3(tiles), dim3(SCAN_THREADS), 0, s, in, n, temp);
+    if (two && scan_rec(temp, temp, tiles, nullptr, temp + tiles, s)) return -1;
+    hipLaunchKernelGGL(k_scan_apply, dim3(tiles), dim3(SCAN_THREADS), 0, s, in, out, n, (const uint32_t *)temp, two ? 1 : 0, total);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -121,211 +143,187 @@ int stc_exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint32_t n, uint32
         if (total_dev) hipMemsetAsync(total_dev, 0, 4, s);
         return 0;
     }
-    /* keep the last input value so the total survives an in-place scan */
-    uint32_t *last = temp;
-    STC_CHECK(hipMemcpyAsync(last, in + n - 1, 4, hipMemcpyDeviceToDevice, s));
-    if (scan_rec(in, out, n, temp + 16, s)) return stc_hip_fail(hipGetLastError(), "scan", __FILE__, __LINE__);
-    if (total_dev) hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, s, last, out + n - 1, 1u, total_dev);
-    STC_CHECK(hipGetLastError());
+    if (scan_rec(in, out, n, total_dev, temp, s)) return stc_hip_fail(hipGetLastError(), "scan", __FILE__, __LINE__);
     return 0;
 }
 
 /* ---------------- radix passes ---------------- */
 
-template <typename K>
-__global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const K *keys, uint32_t n, int shift, uint32_t *hist,
-                                                         uint32_t tiles) {
+/* digit counts of each tile, tile after tile (by_tile) or digit-major */
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const K *__restrict__ keys, uint32_t n, int shift,
+                                                         uint32_t *__restrict__ hist, uint32_t tiles, int by_tile) {
     __shared__ uint32_t h[RS_BINS];
     h[threadIdx.x] = 0;
-    __syncthreads();
-    uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
-#pragma unroll 4
-    for (int r = 0; r < RS_ITEMS; r++) {
-        uint64_t i = base + (uint64_t)r * RS_THREADS + threadIdx.x;
-        if (i < n) atomicAdd(&h[(uint32_t)(keys[i] >> shift) & (RS_BINS - 1)], 1u);
+    const uint64_t base = (uint64_t)blockIdx.x * (RS_THREADS * ITEMS) + threadIdx.x;
+    K k[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const uint64_t i = base + (uint64_t)r * RS_THREADS;
+        k[r] = i < n ? keys[i] : (K)0;
     }
     __syncthreads();
-    hist[(uint64_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++)
+        if (base + (uint64_t)r * RS_THREADS < n) atomicAdd(&h[(uint32_t)(k[r] >> shift) & (RS_BINS - 1)], 1u);
+    __syncthreads();
+    hist[by_tile ? (uint64_t)blockIdx.x * RS_BINS + threadIdx.x : (uint64_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
 }
 
-/* Each workgroup ranks its tile stably (256 keys per round, per-wavefront peer
- * masks from 8 ballots, per-digit wave offsets in LDS), places the keys in
- * LDS in digit order, and writes them out in that order: keys of one digit go
- * to consecutive global positions, so the writes are coalesced. */
-template <typename K>
-__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K *kin, const uint32_t *vin, K *kout,
-                                                            uint32_t *vout, uint32_t n, int shift,
-                                                            const uint32_t *offs, uint32_t tiles) {
-    __shared__ uint32_t run[RS_BINS];    /* keys of each digit ranked so far in this tile */
-    __shared__ uint32_t base[RS_BINS];   /* global position of the tile's first key of each digit */
-    __shared__ uint32_t lstart[RS_BINS]; /* position in the tile of its first key of each digit */
-    __shared__ uint32_t wcnt[RS_THREADS / STC_WAVE][RS_BINS];
-    __shared__ K sk[RS_TILE];
-    __shared__ uint32_t sv[RS_TILE];
-    __shared__ uint32_t tile_total;
+/* by_tile: offs holds the tiles' histograms; else the scanned digit-major
+ * table. vin null: the values are the keys' places. */
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                            K *__restrict__ kout, uint32_t *__restrict__ vout, uint32_t n,
+                                                            int shift, const uint32_t *__restrict__ offs, uint32_t tiles,
+                                                            int by_tile) {
+    constexpr uint32_t TILE = RS_THREADS * ITEMS;
+    constexpr bool STAGED = sizeof(K) == 4; /* an LDS tile of 8-byte keys would cost the kernel its occupancy */
+    __shared__ uint32_t base[RS_BINS];   /* global position of the tile's first key of each digit, less its place in LDS */
+    __shared__ uint32_t wcnt[RS_WAVES][RS_BINS];
+    __shared__ K sk[STAGED ? TILE : 1];
+    __shared__ uint32_t sv[STAGED ? TILE : 1];
     const int tid = threadIdx.x, lane = tid & (STC_WAVE - 1), w = tid / STC_WAVE;
-    /* the tile's count of digit tid: the gap to the next entry of the scanned digit-major table */
-    const uint64_t slot = (uint64_t)tid * tiles + blockIdx.x;
-    const uint32_t b0 = offs[slot];
-    const uint32_t b1 = slot + 1 < (uint64_t)RS_BINS * tiles ? offs[slot + 1] : n;
-    base[tid] = b0;
-    run[tid] = 0;
-    lstart[tid] = block_excl_scan(b1 - b0, &tile_total);
+    const uint64_t tile0 = (uint64_t)blockIdx.x * TILE;
+    const uint64_t first = tile0 + (uint64_t)w * (STC_WAVE * ITEMS) + lane; /* the wave's stretch, 64 keys a round */
+    K k[ITEMS];
+    uint32_t v[ITEMS];
 #pragma unroll
-    for (int q = 0; q < RS_THREADS / STC_WAVE; q++) wcnt[q][tid] = 0;
-    __syncthreads();
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (STC_WAVE - lane));
-    const uint64_t tile0 = (uint64_t)blockIdx.x * RS_TILE;
-    for (int r = 0; r < RS_ITEMS; r++) {
-        uint64_t i = tile0 + (uint64_t)r * RS_THREADS + tid;
-        bool valid = i < n;
-        K k = 0;
-        uint32_t v = 0, d = 0;
-        if (valid) {
-            k = kin[i];
-            v = vin[i];
-            d = (uint32_t)(k >> shift) & (RS_BINS - 1);
+    for (int r = 0; r < ITEMS; r++) {
+        const uint64_t i = first + (uint64_t)r * STC_WAVE;
+        k[r] = i < n ? kin[i] : (K)0;
+        v[r] = vin ? (i < n ? vin[i] : 0u) : (uint32_t)i;
+    }
+#pragma unroll
+    for (int q = 0; q < RS_WAVES; q++) wcnt[q][tid] = 0;
+    /* where the tile's keys of digit tid start */
+    uint32_t b0, tot;
+    if (by_tile) {
+        uint32_t pre = 0, all = 0;
+#pragma unroll 16
+        for (uint32_t t = 0; t < tiles; t++) {
+            const uint32_t c = offs[t * RS_BINS + tid];
+            all += c;
+            pre += t < blockIdx.x ? c : 0u;
         }
+        b0 = pre + block_excl_scan(all, &tot);
+    } else {
+        b0 = offs[(uint64_t)tid * tiles + blockIdx.x];
+        __syncthreads();
+    }
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (STC_WAVE - lane));
+    uint32_t rank[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const bool valid = first + (uint64_t)r * STC_WAVE < n;
+        const uint32_t d = (uint32_t)(k[r] >> shift) & (RS_BINS - 1);
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; b++) {
-            bool bit = (d >> b) & 1u;
-            uint64_t m = __ballot(bit);
+            const bool bit = (d >> b) & 1u;
+            const uint64_t m = __ballot(bit);
             peers &= bit ? m : ~m;
         }
-        uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        {
-            uint32_t acc = run[tid];
-#pragma unroll
-            for (int q = 0; q < RS_THREADS / STC_WAVE; q++) {
-                uint32_t c = wcnt[q][tid];
-                wcnt[q][tid] = acc;
-                acc += c;
-            }
-            run[tid] = acc;
-        }
-        __syncthreads();
-        if (valid) {
-            const uint32_t lp = lstart[d] + wcnt[w][d] + rank;
-            sk[lp] = k;
-            sv[lp] = v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < RS_THREADS / STC_WAVE; q++) wcnt[q][tid] = 0;
-        __syncthreads();
+        const uint32_t behind = (uint32_t)__popcll(peers & lt);
+        const uint32_t seen = wcnt[w][d];
+        rank[r] = seen + behind;
+        /* the wave's own counts: its lanes' reads come before the write, its LDS accesses in order */
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (valid && behind == 0) wcnt[w][d] = seen + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-    const uint32_t cnt = (uint32_t)min<uint64_t>(RS_TILE, n - tile0);
-    for (uint32_t p = tid; p < cnt; p += RS_THREADS) {
-        const K k = sk[p];
-        const uint32_t d = (uint32_t)(k >> shift) & (RS_BINS - 1);
-        const uint32_t pos = base[d] + (p - lstart[d]);
-        kout[pos] = k;
-        vout[pos] = sv[p];
-    }
-}
-
-/* The same ranking, each key written straight to its global position: for
- * 8-byte keys, whose LDS tile would cost the kernel its occupancy. */
-template <typename K>
-__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter_direct(const K *kin, const uint32_t *vin, K *kout,
-                                                            uint32_t *vout, uint32_t n, int shift,
-                                                            const uint32_t *offs, uint32_t tiles) {
-    __shared__ uint32_t run[RS_BINS];
-    __shared__ uint32_t base[RS_BINS];
-    __shared__ uint32_t wcnt[RS_THREADS / STC_WAVE][RS_BINS];
-    const int tid = threadIdx.x, lane = tid & (STC_WAVE - 1), w = tid / STC_WAVE;
-    run[tid] = 0;
-    base[tid] = offs[(uint64_t)tid * tiles + blockIdx.x];
-#pragma unroll
-    for (int q = 0; q < RS_THREADS / STC_WAVE; q++) wcnt[q][tid] = 0;
     __syncthreads();
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (STC_WAVE - lane));
-    uint64_t tile0 = (uint64_t)blockIdx.x * RS_TILE;
-    for (int r = 0; r < RS_ITEMS; r++) {
-        uint64_t i = tile0 + (uint64_t)r * RS_THREADS + tid;
-        bool valid = i < n;
-        K k = 0;
-        uint32_t v = 0, d = 0;
-        if (valid) {
-            k = kin[i];
-            v = vin[i];
-            d = (uint32_t)(k >> shift) & (RS_BINS - 1);
-        }
-        uint64_t peers = __ballot(valid);
+    uint32_t acc = 0;
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
-            bool bit = (d >> b) & 1u;
-            uint64_t m = __ballot(bit);
-            peers &= bit ? m : ~m;
-        }
-        uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
+    for (int q = 0; q < RS_WAVES; q++) {
+        const uint32_t c = wcnt[q][tid];
+        wcnt[q][tid] = acc;
+        acc += c;
+    }
+    if constexpr (STAGED) {
+        const uint32_t l0 = block_excl_scan(acc, &tot);
+        base[tid] = b0 - l0;
+#pragma unroll
+        for (int q = 0; q < RS_WAVES; q++) wcnt[q][tid] += l0;
         __syncthreads();
-        {
-            uint32_t acc = run[tid];
 #pragma unroll
-            for (int q = 0; q < RS_THREADS / STC_WAVE; q++) {
-                uint32_t c = wcnt[q][tid];
-                wcnt[q][tid] = acc;
-                acc += c;
+        for (int r = 0; r < ITEMS; r++)
+            if (first + (uint64_t)r * STC_WAVE < n) {
+                const uint32_t at = wcnt[w][(uint32_t)(k[r] >> shift) & (RS_BINS - 1)] + rank[r];
+                sk[at] = k[r];
+                sv[at] = v[r];
             }
-            run[tid] = acc;
-        }
         __syncthreads();
-        if (valid) {
-            uint32_t pos = base[d] + wcnt[w][d] + rank;
-            kout[pos] = k;
-            vout[pos] = v;
+        const uint32_t cnt = (uint32_t)min<uint64_t>(TILE, n - tile0);
+        for (uint32_t p = tid; p < cnt; p += RS_THREADS) {
+            const K key = sk[p];
+            const uint32_t pos = base[(uint32_t)(key >> shift) & (RS_BINS - 1)] + p;
+            kout[pos] = key;
+            vout[pos] = sv[p];
         }
+    } else {
+        base[tid] = b0;
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < RS_THREADS / STC_WAVE; q++) wcnt[q][tid] = 0;
-        __syncthreads();
+        for (int r = 0; r < ITEMS; r++)
+            if (first + (uint64_t)r * STC_WAVE < n) {
+                const uint32_t d = (uint32_t)(k[r] >> shift) & (RS_BINS - 1);
+                const uint32_t pos = base[d] + wcnt[w][d] + rank[r];
+                kout[pos] = k[r];
+                vout[pos] = v[r];
+            }
     }
 }
 
-template <typename K>
-static int radix_sort(K *keys, uint32_t *vals, K *keys_alt, uint32_t *vals_alt, uint32_t n, int lo_bit,
-                      int hi_bit, uint32_t *temp, hipStream_t s) {
-    if (n <= 1 || hi_bit <= lo_bit) return 0;
-    uint32_t tiles = ceil_div(n, RS_TILE);
-    uint32_t *hist = temp;
-    uint32_t *scan_temp = temp + (size_t)RS_BINS * tiles;
-    K *src_k = keys, *dst_k = keys_alt;
-    uint32_t *src_v = vals, *dst_v = vals_alt;
-    int passes = 0;
-    for (int shift = lo_bit; shift < hi_bit; shift += 8, passes++) {
-        hipLaunchKernelGGL(k_rs_hist<K>, dim3(tiles), dim3(RS_THREADS), 0, s, (const K *)src_k, n, shift, hist,
-                           tiles);
-        STC_CHECK(hipGetLastError());
-        int rc = stc_exclusive_scan_u32(hist, hist, RS_BINS * tiles, nullptr, scan_temp, s);
+template <typename K, int ITEMS>
+static int radix_pass(const K *kin, const uint32_t *vin, K *kout, uint32_t *vout, uint32_t n, int shift, uint32_t *temp,
+                      hipStream_t s) {
+    const uint32_t tiles = ceil_div(n, RS_THREADS * ITEMS);
+    const int by_tile = tiles <= RS_DIRECT;
+    hipLaunchKernelGGL((k_rs_hist<K, ITEMS>), dim3(tiles), dim3(RS_THREADS), 0, s, kin, n, shift, temp, tiles, by_tile);
+    STC_CHECK(hipGetLastError());
+    if (!by_tile) {
+        const int rc = stc_exclusive_scan_u32(temp, temp, RS_BINS * tiles, nullptr, temp + (size_t)RS_BINS * tiles, s);
         if (rc) return rc;
-        if constexpr (sizeof(K) == 4)
-            hipLaunchKernelGGL(k_rs_scatter<K>, dim3(tiles), dim3(RS_THREADS), 0, s, (const K *)src_k,
-                               (const uint32_t *)src_v, dst_k, dst_v, n, shift, (const uint32_t *)hist, tiles);
-        else
-            hipLaunchKernelGGL(k_rs_scatter_direct<K>, dim3(tiles), dim3(RS_THREADS), 0, s, (const K *)src_k,
-                               (const uint32_t *)src_v, dst_k, dst_v, n, shift, (const uint32_t *)hist, tiles);
-        STC_CHECK(hipGetLastError());
-        K *tk = src_k; src_k = dst_k; dst_k = tk;
-        uint32_t *tv = src_v; src_v = dst_v; dst_v = tv;
     }
-    if (passes & 1) {
-        STC_CHECK(hipMemcpyAsync(keys, keys_alt, sizeof(K) * (size_t)n, hipMemcpyDeviceToDevice, s));
-        STC_CHECK(hipMemcpyAsync(vals, vals_alt, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL((k_rs_scatter<K, ITEMS>), dim3(tiles), dim3(RS_THREADS), 0, s, kin, vin, kout, vout, n, shift,
+                       (const uint32_t *)temp, tiles, by_tile);
+    STC_CHECK(hipGetLastError());
+    return 0;
+}
+
+template <typename K>
+static int radix_sort(const K *kin, const uint32_t *vin, K *keys, uint32_t *vals, K *keys_alt, uint32_t *vals_alt,
+                      uint32_t n, int lo_bit, int hi_bit, uint32_t *temp, bool *in_alt, hipStream_t s) {
+    *in_alt = false;
+    const bool in_place = kin == keys;
+    if (n == 0 || (in_place && (n == 1 || hi_bit <= lo_bit))) return 0;
+    const K *src_k = kin;
+    const uint32_t *src_v = vin;
+    bool to_alt = in_place;
+    for (int shift = lo_bit; shift < hi_bit || shift == lo_bit; shift += 8, to_alt = !to_alt) {
+        K *dk = to_alt ? keys_alt : keys;
+        uint32_t *dv = to_alt ? vals_alt : vals;
+        const uint32_t items = rs_items(n);
+        const int rc = items == 4   ? radix_pass<K, 4>(src_k, src_v, dk, dv, n, shift, temp, s)
+                       : items == 8 ? radix_pass<K, 8>(src_k, src_v, dk, dv, n, shift, temp, s)
+                                    : radix_pass<K, 16>(src_k, src_v, dk, dv, n, shift, temp, s);
+        if (rc) return rc;
+        src_k = dk;
+        src_v = dv;
+        *in_alt = to_alt;
     }
     return 0;
 }
 
-int stc_radix_sort_u32(uint32_t *keys, uint32_t *vals, uint32_t *keys_alt, uint32_t *vals_alt, uint32_t n,
-                       int bits, uint32_t *temp, hipStream_t s) {
-    return radix_sort<uint32_t>(keys, vals, keys_alt, vals_alt, n, 0, bits, temp, s);
+int stc_radix_sort_u32(const uint32_t *kin, const uint32_t *vin, uint32_t *keys, uint32_t *vals, uint32_t *keys_alt,
+                       uint32_t *vals_alt, uint32_t n, int bits, uint32_t *temp, bool *in_alt, hipStream_t s) {
+    return radix_sort<uint32_t>(kin, vin, keys, vals, keys_alt, vals_alt, n, 0, bits, temp, in_alt, s);
 }
 
-int stc_radix_sort_u64(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt, uint32_t *vals_alt, uint32_t n,
-                       int lo_bit, int hi_bit, uint32_t *temp, hipStream_t s) {
-    return radix_sort<uint64_t>(keys, vals, keys_alt, vals_alt, n, lo_bit, hi_bit, temp, s);
+int stc_radix_sort_u64(const uint64_t *kin, const uint32_t *vin, uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
+                       uint32_t *vals_alt, uint32_t n, int lo_bit, int hi_bit, uint32_t *temp, bool *in_alt, hipStream_t s) {
+    return radix_sort<uint64_t>(kin, vin, keys, vals, keys_alt, vals_alt, n, lo_bit, hi_bit, temp, in_alt, s);
 }
