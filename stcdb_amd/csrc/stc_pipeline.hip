@@ -135,6 +135,7 @@ struct Counters {             /* device-side counters, copied back once per sync
     unsigned long long pk_used[64];    /* psrc slots reserved in each slice by the collecting waves */
     unsigned long long cand_part[64], pairs_part[64]; /* the collect pass's totals, by workgroup mod 64 */
     uint32_t big, huge, giant;         /* segments left to the wave sort, the block sort, the global-scratch sort */
+    uint32_t wide;                     /* nonzero: there are segments of more than 64 slots */
     uint32_t many;                     /* owners with more sources than the collect pass lists */
     uint32_t pk_over;                  /* a collecting wave's reservation exceeded its slice of psrc */
 };
@@ -814,7 +815,7 @@ __global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t bat
     const uint64_t lt = lanemask_lt(lane);
     unsigned long long cand = 0, total = 0;
     uint64_t rcur = 0, rend = 0; /* the wave's reserved run of psrc */
-    bool over = false, room = true;
+    bool over = false, room = true, wide = false;
     const uint32_t slice_id = wid % PK_SLICES;
     const uint64_t slice = pk_cap / PK_SLICES, slice_base = slice_id * slice;
     for (uint32_t b = wid; b < n_batches; b += nw) {
@@ -926,6 +927,7 @@ __global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t bat
                 total += got;
                 collect_owner(a, w, (uint32_t)(rcur + ahead), got, pcount, pkrun, big, huge, cnt);
             }
+            wide |= __ballot(mine && got > STC_WAVE) != 0;
             if (lane == 0) cand += gtot;
             rcur += fill;
             done = gend;
@@ -937,10 +939,14 @@ __global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t bat
     __shared__ unsigned long long bsum[256 / STC_WAVE][2];
     cand = wave_sum_u64(cand);
     total = wave_sum_u64(total);
+    __shared__ uint32_t bwide;
+    if (threadIdx.x == 0) bwide = 0;
+    __syncthreads();
     if (lane == 0) {
         bsum[threadIdx.x / STC_WAVE][0] = cand;
         bsum[threadIdx.x / STC_WAVE][1] = total;
         if (over) atomicOr(&cnt->pk_over, 1u);
+        if (wide) bwide = 1;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -952,6 +958,7 @@ __global__ __launch_bounds__(256, 8) void k_pair_collect(PairGeo g, uint32_t bat
         const uint32_t part = blockIdx.x % PK_SLICES;
         if (c0) atomicAdd(&cnt->cand_part[part], c0);
         if (t0) atomicAdd(&cnt->pairs_part[part], t0);
+        if (bwide) atomicOr(&cnt->wide, 1u);
     }
 }
 
@@ -992,6 +999,7 @@ __global__ __launch_bounds__(256) void k_pair_collect_many(PairGeo g, const uint
         if (!room) atomicOr(&cnt->pk_over, 1u);
         atomicAdd(&cnt->cand_part[slice_id], tot);
         atomicAdd(&cnt->pairs_part[slice_id], (unsigned long long)fill);
+        if (fill > STC_WAVE) atomicOr(&cnt->wide, 1u);
         collect_owner(a, w, (uint32_t)run, fill, pcount, pkrun, big, huge, cnt);
     }
 }
@@ -1183,8 +1191,8 @@ __device__ inline void place_segment(const uint32_t *srcs, uint32_t slots, uint3
     const uint64_t lt = lanemask_lt(lane);
     constexpr uint32_t P = K * STC_WAVE;
     constexpr bool PAIRED = sizeof(T) == 4 && K == 8; /* the key holds slot / 2 */
-    constexpr int SB = sizeof(T) == 8 ? 32 : (K == 1 ? 6 : K == 2 ? 7 : 8);
-    static_assert(K == 1 || K == 2 || K == 4 || K == 8, "segment width");
+    constexpr int SB = sizeof(T) == 8 ? 32 : (K == 2 ? 7 : 8);
+    static_assert(K == 2 || K == 4 || K == 8, "segment width");
     const uint32_t pdead = sizeof(T) == 8 ? DEAD_B : (1u << pbits) - 1u;
     T x[K];
     float2 pf[K];
@@ -1349,14 +1357,116 @@ __global__ void k_huge_expand(PairGeo g, const uint32_t *__restrict__ owners, ui
     }
 }
 
-/* The place pass: per owner (one wave, owners in leaf order) with at most
- * WCAP slots, its collected keys sorted in registers and written to pn as the
- * owner's segment sorted by partner, its live pairs first and its dead slots
- * behind them, so that pn is sorted by key. pbits: the bits of the object
- * count; a segment sorts 32-bit keys when pbits and its slot index (its slot
- * pair index, for 257 to 510 slots) fit in 32. Five waves per SIMD: at six
- * the 32-bit sort of the widest segments spills. */
-__global__ __launch_bounds__(256, 5) void k_pair_place(PairGeo g, const uint32_t *__restrict__ poff,
+/* Several owners' segments at once: the segments of up to 64 slots of owners
+ * that follow one another in leaf order, 64 slots in all, laid end to end over
+ * the wave's lanes and sorted together by (place of the owner, partner, slot).
+ * tab: per segment, in owner order, its run of psrc, its first lane and length
+ * (16 bits each), its place in pn and its owner; starts: the first lanes' bits;
+ * slots: the lanes in use. pbits + 6 bits and those of the segments' number fit
+ * in 32. */
+__device__ inline void place_pack(const uint4 *tab, uint64_t starts, uint32_t slots, const PairGeo &g, const uint32_t *psrc,
+                                  const unsigned long long *acc, uint32_t n_acc, PairSlot *__restrict__ pn, int lane,
+                                  uint32_t pbits) {
+    const bool valid = (uint32_t)lane < slots;
+    const uint64_t lt = lanemask_lt(lane), le = lt | (1ull << lane);
+    const uint32_t j = (uint32_t)__popcll(starts & le) - 1u; /* lane 0 starts the first segment */
+    const uint4 e = tab[j];
+    const uint32_t first = e.y & 0xFFFFu, len = e.y >> 16;
+    const uint32_t pdead = (1u << pbits) - 1u;
+    uint32_t key = ~0u;
+    float px = 0.f, py = 0.f;
+    if (valid) {
+        const uint32_t src = __builtin_nontemporal_load(psrc + e.x + ((uint32_t)lane - first));
+        const uint32_t idx = src & ~(SRC_REV | SRC_AMB);
+        const bool rev = (src & SRC_REV) != 0;
+        uint32_t q = rev ? g.rev[idx].pid : g.lp[idx];
+        const double2 pd = rev ? *(const double2 *)(g.rev + idx) : g.lxy[idx];
+        if ((src & SRC_AMB) && !sorted_contains(acc, n_acc, ((unsigned long long)e.w << 32) | q)) q = pdead;
+        key = (((j << pbits) | q) << 6) | (uint32_t)lane;
+        px = (float)pd.x;
+        py = (float)pd.y;
+    }
+    const uint32_t before = __shfl_up(key, 1, STC_WAVE);
+    uint32_t x[1] = {key};
+    if (__ballot(lane > 0 && key < before)) reg_bitonic<1>(x, lane);
+    /* a segment's slots stay on its lanes */
+    const uint32_t prev = __shfl_up(x[0], 1, STC_WAVE);
+    const uint32_t partner = (x[0] >> 6) & pdead;
+    const bool live = valid && partner != pdead && ((uint32_t)lane == first || (prev >> 6) != (x[0] >> 6));
+    const uint64_t ml = __ballot(live);
+    const uint64_t seg = (len == STC_WAVE ? ~0ull : ((1ull << len) - 1ull)) << first;
+    const float sx = __shfl(px, (int)(x[0] & 63u), STC_WAVE), sy = __shfl(py, (int)(x[0] & 63u), STC_WAVE);
+    if (valid) {
+        const uint32_t at = live ? (uint32_t)__popcll(ml & seg & lt)
+                                 : (uint32_t)__popcll(ml & seg) + (uint32_t)__popcll(~ml & seg & lt);
+        const u32x3u v = {live ? partner : DEAD_B, __float_as_uint(sx), __float_as_uint(sy)};
+        __builtin_nontemporal_store(v, (u32x3u *)(pn + e.z + at));
+    }
+}
+
+/* The place pass: per owner with at most WCAP slots, its collected keys sorted
+ * in registers and written to pn as the owner's segment sorted by partner, its
+ * live pairs first and its dead slots behind them, so that pn is sorted by key.
+ * This kernel takes the segments of up to 64 slots: a wave reads `batch` owners
+ * that follow one another in leaf order, one per lane, and packs their
+ * segments into its lanes (place_pack), as many as 64 lanes and a 32-bit key
+ * hold. pbits: the bits of the object count. Bound by the latency of each
+ * pack's chain (sources, then partners and positions, the sort, the store) at
+ * eight waves per SIMD. With an owner a wave, a segment of ten slots cost as
+ * much as one of 64 (both passes, before and now: 50k objects 15.6 and 5.5 us,
+ * 200k 103 and 44, 1M 372 and 195, 5M 2.72 and 2.33 ms). */
+__global__ __launch_bounds__(256, 8) void k_pair_place(PairGeo g, uint32_t batch, const uint32_t *__restrict__ poff,
+                                                    const uint2 *__restrict__ pkrun,
+                                                    const uint32_t *__restrict__ psrc,
+                                                    const unsigned long long *__restrict__ acc, uint32_t n_acc,
+                                                    PairSlot *__restrict__ pn, uint32_t pbits) {
+    __shared__ uint4 wtab[256 / STC_WAVE][STC_WAVE];
+    const int lane = threadIdx.x & (STC_WAVE - 1);
+    uint4 *tab = wtab[threadIdx.x / STC_WAVE];
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)((xcd_block_id() * blockDim.x + threadIdx.x) / STC_WAVE));
+    const uint32_t nw = (gridDim.x * blockDim.x) / STC_WAVE;
+    const uint32_t n_batches = (g.n + batch - 1) / batch;
+    const uint32_t most = 1u << min(26u - pbits, 6u); /* segments of a pack: pbits, 6 bits of slot, and theirs */
+    for (uint32_t b = wid; b < n_batches; b += nw) {
+        const uint32_t w0 = b * batch, nown = min(batch, g.n - w0);
+        const uint32_t w = w0 + min((uint32_t)lane, nown - 1);
+        const uint2 run = pkrun[w];
+        const uint32_t a = g.lp[w];
+        const uint32_t small = (uint32_t)lane < nown && run.y <= STC_WAVE ? run.y : 0u;
+        const uint32_t base = poff[a];
+        uint32_t incl = small;
+        for (int o = 1; o < STC_WAVE; o <<= 1) {
+            const uint32_t y = __shfl_up(incl, o, STC_WAVE);
+            if (lane >= o) incl += y;
+        }
+        uint64_t left = __ballot(small != 0);
+        const uint32_t nth = (uint32_t)__popcll(left & lanemask_lt(lane)); /* segments before the lane's */
+        while (left) {
+            const int o = __ffsll((long long)left) - 1;
+            const uint32_t at0 = (uint32_t)__builtin_amdgcn_readlane((int)(incl - small), o);
+            const uint32_t n0 = (uint32_t)__builtin_amdgcn_readlane((int)nth, o);
+            const bool in = ((left >> lane) & 1u) && incl - at0 <= STC_WAVE && nth - n0 < most;
+            const uint64_t pack = __ballot(in); /* the first and those that follow, up to the first that does not fit */
+            const uint32_t first = incl - small - at0;
+            if (in) tab[nth - n0] = make_uint4(run.x, first | (small << 16), base, a);
+            uint64_t starts = 0;
+            for (uint64_t m = pack; m; m &= m - 1)
+                starts |= 1ull << (uint32_t)__builtin_amdgcn_readlane((int)first, __ffsll((long long)m) - 1);
+            const uint32_t used = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63 - __clzll((long long)pack)) - at0;
+            wave_lds_sync();
+            place_pack(tab, starts, used, g, psrc, acc, n_acc, pn, lane, pbits);
+            wave_lds_sync(); /* the table is rewritten by the next pack */
+            left &= ~pack;
+        }
+    }
+}
+
+/* The place pass of the segments of 65 to WCAP slots, launched when the
+ * collect pass saw any: a wave each, `batch` owners read at once to find them.
+ * A segment sorts 32-bit keys when pbits and its slot index (its slot pair
+ * index, for 257 to 510 slots) fit in 32. Five waves per SIMD: at six the
+ * 32-bit sort of the widest segments spills. */
+__global__ __launch_bounds__(256, 5) void k_pair_place_wide(PairGeo g, uint32_t batch, const uint32_t *__restrict__ poff,
                                                     const uint2 *__restrict__ pkrun,
                                                     const uint32_t *__restrict__ psrc,
                                                     const unsigned long long *__restrict__ acc, uint32_t n_acc,
@@ -1364,26 +1474,30 @@ __global__ __launch_bounds__(256, 5) void k_pair_place(PairGeo g, const uint32_t
     __shared__ unsigned long long wrun[256 / STC_WAVE][WCAP + WCAP / 2]; /* keys or positions, then partners */
     const int lane = threadIdx.x & (STC_WAVE - 1);
     unsigned long long *runbuf = wrun[threadIdx.x / STC_WAVE];
-    const uint64_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)((xcd_block_id() * blockDim.x + threadIdx.x) / STC_WAVE));
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / STC_WAVE;
-    for (uint64_t w = wid; w < g.n; w += nw) {
-        const uint2 run = pkrun[w];
-        const uint32_t slots = (uint32_t)__builtin_amdgcn_readfirstlane((int)run.y);
-        if (slots == 0 || slots > WCAP) continue;
-        const uint32_t a = (uint32_t)__builtin_amdgcn_readfirstlane((int)g.lp[w]);
-        const uint32_t *keys = psrc + (uint32_t)__builtin_amdgcn_readfirstlane((int)run.x);
-        PairSlot *seg = pn + poff[a];
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)((xcd_block_id() * blockDim.x + threadIdx.x) / STC_WAVE));
+    const uint32_t nw = (gridDim.x * blockDim.x) / STC_WAVE;
+    const uint32_t n_batches = (g.n + batch - 1) / batch;
+    for (uint32_t b = wid; b < n_batches; b += nw) {
+        const uint32_t w0 = b * batch, nown = min(batch, g.n - w0);
+        const uint32_t len = (uint32_t)lane < nown ? pkrun[w0 + lane].y : 0u;
+        for (uint64_t wide = __ballot(len > STC_WAVE && len <= WCAP); wide; wide &= wide - 1) {
+            const uint32_t w = w0 + (uint32_t)__ffsll((long long)wide) - 1;
+            const uint2 run = pkrun[w];
+            const uint32_t slots = (uint32_t)__builtin_amdgcn_readfirstlane((int)run.y);
+            const uint32_t a = (uint32_t)__builtin_amdgcn_readfirstlane((int)g.lp[w]);
+            const uint32_t *keys = psrc + (uint32_t)__builtin_amdgcn_readfirstlane((int)run.x);
+            PairSlot *seg = pn + poff[a];
 #define PLACE(KK, BITS)                                                                                          \
     do {                                                                                                         \
-        if (pbits + (BITS) <= 32u) place_segment<KK, uint32_t>(keys, slots, a, (uint32_t)w, g, acc, n_acc, seg, lane, runbuf, pbits); \
-        else place_segment<KK, unsigned long long>(keys, slots, a, (uint32_t)w, g, acc, n_acc, seg, lane, runbuf, pbits); \
+        if (pbits + (BITS) <= 32u) place_segment<KK, uint32_t>(keys, slots, a, w, g, acc, n_acc, seg, lane, runbuf, pbits); \
+        else place_segment<KK, unsigned long long>(keys, slots, a, w, g, acc, n_acc, seg, lane, runbuf, pbits); \
     } while (0)
-        if (slots <= STC_WAVE) PLACE(1, 6);
-        else if (slots <= 2 * STC_WAVE) PLACE(2, 7);
-        else if (slots <= 4 * STC_WAVE) PLACE(4, 8);
-        else if (slots <= 2 * 255) PLACE(8, 8); /* slot pairs below 255 keep the padding above every key */
-        else place_segment<8, unsigned long long>(keys, slots, a, (uint32_t)w, g, acc, n_acc, seg, lane, runbuf, pbits);
+            if (slots <= 2 * STC_WAVE) PLACE(2, 7);
+            else if (slots <= 4 * STC_WAVE) PLACE(4, 8);
+            else if (slots <= 2 * 255) PLACE(8, 8); /* slot pairs below 255 keep the padding above every key */
+            else place_segment<8, unsigned long long>(keys, slots, a, w, g, acc, n_acc, seg, lane, runbuf, pbits);
 #undef PLACE
+        }
     }
 }
 
@@ -3016,13 +3130,25 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     if (c->pnew.ensure(total + 1) || c->meet[nx].ensure(total + 1))
         return fail(c, STC_E_CAPACITY, "pair and meeting arrays");
     CK(hipEventRecord(c->ev[6], s));
-    /* the place pass runs faster with up to four times the collect pass's workgroups (measured at 10M
-     * objects); both counts are multiples of 8 for the XCD order */
-    const uint32_t wgrid = (uint32_t)std::min<uint64_t>((blocks_for((uint64_t)n * STC_WAVE, 256) + 7) & ~7ull, 65536u);
-    hipLaunchKernelGGL(k_pair_place, dim3(wgrid), dim3(256), 0, s, pg, (const uint32_t *)c->moff[nx].p,
-                       (const uint2 *)c->pkrun.p, (const uint32_t *)c->psrc.p, c->acc.p,
-                       (uint32_t)accepted.size(), c->pnew.p, 32u - (uint32_t)__builtin_clz(c->n));
+    /* the place passes' owners a wave reads at once and workgroups at most. Short segments: 8 owners below
+     * 256k objects (200k: 29 us, 16: 39), 16 above (1M: 144 us, 8: 150, 32: 159), 4k workgroups (1M: 144, 16k:
+     * 178). Long ones, of which a wave with many at once lags behind: 4 and 8k (1M: 50 us, 5M: 1.64 ms; 8:
+     * 47 us, 1.76; 2: 60 us, 1.77; 16: 92 us, 2.1; 64k workgroups of 4: 98 us, 2.0), from 8M objects on 2 and
+     * 16k (both passes at 10M: 7.33 ms; 4 and 8k: 7.72) */
+    const uint32_t nb = n < (1u << 18) ? 8 : 16, wb = n < (1u << 23) ? 4 : 2, wmost = n < (1u << 23) ? 8192 : 16384;
+    const uint32_t pbits = 32u - (uint32_t)__builtin_clz(c->n);
+    auto place_grid = [&](uint32_t batch, uint32_t most) {
+        return std::min<uint32_t>((blocks_for(blocks_for(n, batch) * (uint64_t)STC_WAVE, 256) + 7) & ~7u, most);
+    };
+    hipLaunchKernelGGL(k_pair_place, dim3(place_grid(nb, 4096)), dim3(256), 0, s, pg, nb, (const uint32_t *)c->moff[nx].p,
+                       (const uint2 *)c->pkrun.p, (const uint32_t *)c->psrc.p, c->acc.p, (uint32_t)accepted.size(), c->pnew.p, pbits);
     CK(hipGetLastError());
+    if (h.wide) {
+        hipLaunchKernelGGL(k_pair_place_wide, dim3(place_grid(wb, wmost)), dim3(256), 0, s, pg, wb,
+                           (const uint32_t *)c->moff[nx].p, (const uint2 *)c->pkrun.p, (const uint32_t *)c->psrc.p, c->acc.p,
+                           (uint32_t)accepted.size(), c->pnew.p, pbits);
+        CK(hipGetLastError());
+    }
     CK(hipEventRecord(c->ev[7], s));
     if (h.big) { /* segments longer than the place pass sorts: by waves, by blocks, in global scratch */
         hipLaunchKernelGGL(k_seg_sort_wave, dim3(blocks_for((uint64_t)h.big * STC_WAVE, 256)), dim3(256), 0, s, pg,
