@@ -7,8 +7,9 @@
  *     (end == last step) matched in both directions;
  *   - the memtable records: one thread per record;
  *   - the runs kept in HBM: object and pair queries look the object's CTF up
- *     through the run's sids and binary-search its packed keys, which a CTF
- *     stores sorted by pid (as CTF::search_SSTable does, step_merge.cpp:528);
+ *     through the run's sids and search its packed keys (a wave each, 64 probes
+ *     a round), which a CTF stores sorted by pid (as CTF::search_SSTable does,
+ *     step_merge.cpp:528);
  *     range queries scan the CTFs whose decoded boxes can reach the query box
  *     (one block per query and CTF) and the oversize buffer.
  * Object and pair queries are found per meeting through a small open-addressed
@@ -35,7 +36,10 @@ struct QDev {
     uint32_t n_range;
     const uint32_t *g_start;         /* [QGRID * QGRID + 1] range queries by grid cell */
     const uint32_t *g_list;
-    double x0, y0, dx, dy;
+    const uint32_t *filter;          /* [2^f_bits / 32] a bit per hash of a queried id, then [QGRID * QGRID / 32] a
+                                        bit per grid cell that holds a range query */
+    uint32_t f_bits;
+    double x0, y0, ix, iy;           /* the map's corner and cells per degree */
     stc_hit *hits;
     uint64_t cap;                    /* 0: counts only */
     unsigned long long *n_hits;
@@ -57,6 +61,8 @@ struct QueryBufs {
     uint32_t *g_start = nullptr;
     uint32_t *g_list = nullptr;
     uint32_t g_cap = 0;
+    uint32_t *filter = nullptr;
+    uint32_t f_cap = 0;
     QueryRunDev *runs = nullptr;
     uint32_t runs_cap = 0;
     uint4 *cand = nullptr;
@@ -80,7 +86,7 @@ uint64_t stc_query_bufs_growth(const QueryBufs *b, uint32_t nq, uint64_t cap) {
 
 void stc_query_bufs_free(QueryBufs *b) {
     if (!b) return;
-    void *ptrs[] = {b->q, b->oh_key, b->oh_head, b->q_next, b->oq, b->g_start, b->g_list, b->runs, b->cand,
+    void *ptrs[] = {b->q, b->oh_key, b->oh_head, b->q_next, b->oq, b->g_start, b->g_list, b->filter, b->runs, b->cand,
                     b->hits, b->counters};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -109,11 +115,13 @@ static int grow32(T **p, uint32_t *cap, uint64_t need) {
     return rc;
 }
 
-/* the same arithmetic on the host (registration) and the device (lookup) */
-__host__ __device__ inline int grid_cell(double v, double v0, double d) {
-    double f = floor((v - v0) / d);
+/* The grid cell of a coordinate, the same arithmetic on the host (registration)
+ * and the device (lookup). Any monotone map to cells serves: a meeting and a
+ * query that intersect share the cell of the low corner of their intersection. */
+__host__ __device__ inline int grid_cell(double v, double v0, double inv) {
+    const double f = (v - v0) * inv;
     if (!(f >= 0.0)) return 0;
-    if (f > (double)(QGRID - 1)) return QGRID - 1;
+    if (f >= (double)QGRID) return QGRID - 1;
     return (int)f;
 }
 
@@ -121,27 +129,11 @@ __host__ __device__ inline uint32_t oid_slot(uint32_t oid, uint32_t bits) {
     return (uint32_t)(((uint64_t)oid * 0x9E3779B97F4A7C15ull) >> (64 - bits));
 }
 
-/* per-block query counters: cleared on entry, added to the global counts on
- * exit (one atomic per query and block instead of one per hit) */
-__device__ inline void lc_clear(const QDev &Q, unsigned int *lc) {
-    if (Q.lds)
-        for (uint32_t i = threadIdx.x; i < Q.nq; i += blockDim.x) lc[i] = 0;
-    __syncthreads();
-}
-__device__ inline void lc_flush(const QDev &Q, unsigned int *lc) {
-    __syncthreads();
-    if (Q.lds)
-        for (uint32_t i = threadIdx.x; i < Q.nq; i += blockDim.x)
-            if (lc[i]) atomicAdd(&Q.counts[i], (unsigned long long)lc[i]);
-}
-
-__device__ inline void q_emit(const QDev &Q, unsigned int *lc, uint32_t qi, uint32_t pid, uint32_t target,
-                              uint32_t start, uint32_t end, uint32_t source, const double *m) {
-    if (Q.lds) atomicAdd(&lc[qi], 1u);
-    else atomicAdd(&Q.counts[qi], 1ull);
+/* the hit as the batch's next (all lanes that store together reserve at once: a
+ * counter updated by every hit serialises on its address) */
+__device__ inline void q_store(const QDev &Q, uint32_t qi, uint32_t pid, uint32_t target, uint32_t start, uint32_t end,
+                               uint32_t source, const double *m) {
     if (!Q.cap || (Q.q[qi].flags & STC_QF_COUNT)) return;
-    /* one reservation per call for all lanes that emit together: a counter
-     * updated by every hit serialises on its address */
     const uint64_t act = __ballot(1);
     const int lane = threadIdx.x & (STC_WAVE - 1), leader = __ffsll((long long)act) - 1;
     unsigned long long base = 0;
@@ -164,15 +156,50 @@ __device__ inline void q_emit(const QDev &Q, unsigned int *lc, uint32_t qi, uint
     }
 }
 
+/* A scan's LDS: the per-block query counters (cleared on entry, added to the
+ * global counts on exit: one atomic per query and block instead of one per
+ * hit), then the batch's filter: 2^f_bits bits of id hashes and a bit per grid
+ * cell, which turn away nearly every meeting no query asks for without a read
+ * of the tables. The launch sizes it (q_scan_lds). */
+extern __shared__ uint32_t q_lds[];
+
+__device__ inline uint32_t *q_scan_begin(const QDev &Q) {
+    uint32_t *flt = q_lds + (Q.lds ? Q.nq : 0u);
+    if (Q.lds)
+        for (uint32_t i = threadIdx.x; i < Q.nq; i += blockDim.x) q_lds[i] = 0;
+    const uint32_t words = (1u << Q.f_bits) / 32 + QGRID * QGRID / 32;
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) flt[i] = Q.filter[i];
+    __syncthreads();
+    return flt;
+}
+__device__ inline void q_scan_end(const QDev &Q) {
+    __syncthreads();
+    if (Q.lds)
+        for (uint32_t i = threadIdx.x; i < Q.nq; i += blockDim.x)
+            if (q_lds[i]) atomicAdd(&Q.counts[i], (unsigned long long)q_lds[i]);
+}
+
+__device__ inline void q_emit(const QDev &Q, uint32_t qi, uint32_t pid, uint32_t target, uint32_t start, uint32_t end,
+                              uint32_t source, const double *m) {
+    if (Q.lds) atomicAdd(&q_lds[qi], 1u);
+    else atomicAdd(&Q.counts[qi], 1ull);
+    q_store(Q, qi, pid, target, start, end, source, m);
+}
+
 __device__ inline bool q_time(const stc_query &q, uint32_t s, uint32_t e) { return s <= q.t1 && e >= q.t0; }
 __device__ inline bool q_box(const stc_query &q, const double *m) {
     return m[0] <= q.box[2] && m[2] >= q.box[0] && m[1] <= q.box[3] && m[3] >= q.box[1];
 }
 
+/* may an object or pair query name pid? */
+__device__ inline bool q_may_oid(const QDev &Q, const uint32_t *flt, uint32_t pid) {
+    const uint32_t h = oid_slot(pid, Q.f_bits);
+    return (flt[h >> 5] >> (h & 31)) & 1u;
+}
+
 /* object and pair queries of one meeting seen from pid */
-__device__ inline void match_oid(const QDev &Q, unsigned int *lc, uint32_t pid, uint32_t target, uint32_t s,
-                                 uint32_t e, uint32_t src, const double *m) {
-    if (!Q.oh_bits) return;
+__device__ inline void match_oid(const QDev &Q, uint32_t pid, uint32_t target, uint32_t s, uint32_t e, uint32_t src,
+                                 const double *m) {
     const uint32_t mask = (1u << Q.oh_bits) - 1u;
     uint32_t h = oid_slot(pid, Q.oh_bits);
     for (;;) {
@@ -185,36 +212,46 @@ __device__ inline void match_oid(const QDev &Q, unsigned int *lc, uint32_t pid, 
         const stc_query &q = Q.q[qi];
         if (!q_time(q, s, e)) continue;
         if (q.kind == STC_Q_OID || (q.kind == STC_Q_PAIR && q.oid2 == target))
-            q_emit(Q, lc, (uint32_t)qi, pid, target, s, e, src, m);
+            q_emit(Q, (uint32_t)qi, pid, target, s, e, src, m);
     }
 }
 
 /* range queries of one meeting (called once per meeting) */
-__device__ inline void match_range(const QDev &Q, unsigned int *lc, uint32_t pid, uint32_t target, uint32_t s,
+__device__ inline void match_range(const QDev &Q, const uint32_t *flt, uint32_t pid, uint32_t target, uint32_t s,
                                    uint32_t e, uint32_t src, const double *m) {
-    if (!Q.n_range) return;
-    const int cx0 = grid_cell(m[0], Q.x0, Q.dx), cx1 = grid_cell(m[2], Q.x0, Q.dx);
-    const int cy0 = grid_cell(m[1], Q.y0, Q.dy), cy1 = grid_cell(m[3], Q.y0, Q.dy);
+    const uint32_t *cells = flt + (1u << Q.f_bits) / 32;
+    const int cx0 = grid_cell(m[0], Q.x0, Q.ix), cx1 = grid_cell(m[2], Q.x0, Q.ix);
+    const int cy0 = grid_cell(m[1], Q.y0, Q.iy), cy1 = grid_cell(m[3], Q.y0, Q.iy);
     for (int cy = cy0; cy <= cy1; cy++)
         for (int cx = cx0; cx <= cx1; cx++) {
             const uint32_t cell = (uint32_t)(cy * QGRID + cx);
+            if (!((cells[cell >> 5] >> (cell & 31)) & 1u)) continue;
             for (uint32_t j = Q.g_start[cell]; j < Q.g_start[cell + 1]; j++) {
                 const uint32_t qi = Q.g_list[j];
                 const stc_query &q = Q.q[qi];
                 if (!q_time(q, s, e) || !q_box(q, m)) continue;
-                if (grid_cell(fmax(m[0], q.box[0]), Q.x0, Q.dx) != cx || grid_cell(fmax(m[1], q.box[1]), Q.y0, Q.dy) != cy)
+                if (grid_cell(fmax(m[0], q.box[0]), Q.x0, Q.ix) != cx || grid_cell(fmax(m[1], q.box[1]), Q.y0, Q.iy) != cy)
                     continue;
-                q_emit(Q, lc, qi, pid, target, s, e, src, m);
+                q_emit(Q, qi, pid, target, s, e, src, m);
             }
         }
 }
 
 /* CTF::ctf_get_key_oid, parse_key and new_parse_mbr (step_merge.cpp:325-379)
- * on the little-endian packed key at p */
+ * on the little-endian packed key at p. A key is read as two 8-byte words
+ * wherever it starts (global memory takes unaligned reads; byte by byte a key
+ * is 13 or 14 of them), so up to 15 bytes past its end: the packed keys of a
+ * run are followed in their allocation by its CTF metadata. */
 __device__ inline unsigned __int128 load_packed(const uint8_t *p, uint32_t kb) {
-    unsigned __int128 k = 0;
-    for (uint32_t i = 0; i < kb && i < 16; i++) k |= (unsigned __int128)p[i] << (8 * i);
-    return k;
+    uint64_t w[2];
+    __builtin_memcpy(w, p, 16);
+    if (kb < 8) {
+        w[0] &= (1ull << (8 * kb)) - 1;
+        w[1] = 0;
+    } else if (kb < 16) {
+        w[1] &= (1ull << (8 * (kb - 8))) - 1;
+    }
+    return ((unsigned __int128)w[1] << 64) | w[0];
 }
 
 __device__ inline uint32_t packed_pid(const stc_ctf_meta &c, unsigned __int128 k) {
@@ -265,54 +302,98 @@ __device__ inline void decode_tail(const uint64_t *o_keys, const float4 *o_boxes
     m[3] = b.w;
 }
 
+/* One read of the live meetings, 28 bytes each. Without range queries a lane
+ * reads the ids of four meetings at once and the rest of one only where the id
+ * filter lets it pass; with range queries it reads two whole meetings at once,
+ * so that no read waits for another. Object queries are bound by memory (256M
+ * meetings, 1,000 objects: 3.81 ms when every meeting was read whole and hashed
+ * into the batch's tables in global memory, 2.08 ms = 3.4 TB/s so), range
+ * queries by the cells' arithmetic in 64 bits (42M meetings, 128 mixed queries:
+ * 563 us with divisions by the cell size and a read of the grid for every
+ * meeting, 377 so). */
+template <bool RANGES>
 __global__ __launch_bounds__(256) void k_q_live(const Bucket *__restrict__ t, uint64_t nb, uint32_t last_t, QDev Q) {
-    __shared__ unsigned int lc[QLDS];
-    lc_clear(Q, lc);
+    constexpr int U = RANGES ? 2 : 4;
+    const uint32_t *flt = q_scan_begin(Q);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += stride) {
-        Bucket b = t[i];
-        if (!bucket_live(b)) continue;
-        const uint32_t a = (uint32_t)(b.key >> 32), c = (uint32_t)b.key;
-        double m[4] = {o2f(b.mbr[0]), o2f(b.mbr[1]), o2f(b.mbr[2]), o2f(b.mbr[3])};
-        /* a live meeting ends at the step that built the array */
-        match_oid(Q, lc, a, c, b.start, last_t, 0, m);
-        match_oid(Q, lc, c, a, b.start, last_t, 0, m);
-        match_range(Q, lc, a, c, b.start, last_t, 0, m);
+    const bool oids = Q.oh_bits != 0;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < nb; i0 += stride * U) {
+        Bucket b[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint64_t i = min(i0 + u * stride, nb - 1);
+            if constexpr (RANGES) b[u] = t[i];
+            else b[u].key = t[i].key;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint64_t i = i0 + u * stride;
+            const uint32_t a = (uint32_t)(b[u].key >> 32), c = (uint32_t)b[u].key;
+            if (i >= nb || c == DEAD_B) continue;
+            const bool ma = oids && q_may_oid(Q, flt, a), mc = oids && q_may_oid(Q, flt, c);
+            if (!RANGES) {
+                if (!(ma || mc)) continue;
+                b[u] = t[i];
+            }
+            double m[4] = {o2f(b[u].mbr[0]), o2f(b[u].mbr[1]), o2f(b[u].mbr[2]), o2f(b[u].mbr[3])};
+            /* a live meeting ends at the step that built the array */
+            if (ma) match_oid(Q, a, c, b[u].start, last_t, 0, m);
+            if (mc) match_oid(Q, c, a, b[u].start, last_t, 0, m);
+            if (RANGES) match_range(Q, flt, a, c, b[u].start, last_t, 0, m);
+        }
     }
-    lc_flush(Q, lc);
+    q_scan_end(Q);
 }
 
 __global__ __launch_bounds__(256) void k_q_mem(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes,
                                                uint64_t n, uint32_t base, QDev Q) {
-    __shared__ unsigned int lc[QLDS];
-    lc_clear(Q, lc);
+    const uint32_t *flt = q_scan_begin(Q);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         uint32_t pid, target, start, end;
         double m[4];
         decode_tail(keys, boxes, (uint32_t)i, base, &pid, &target, &start, &end, m);
-        match_oid(Q, lc, pid, target, start, end, 1, m);
-        if (pid < target) match_range(Q, lc, pid, target, start, end, 1, m);
+        if (Q.oh_bits && q_may_oid(Q, flt, pid)) match_oid(Q, pid, target, start, end, 1, m);
+        if (Q.n_range && pid < target) match_range(Q, flt, pid, target, start, end, 1, m);
     }
-    lc_flush(Q, lc);
+    q_scan_end(Q);
 }
 
-/* object and pair queries against one run: the object's CTF by its sid, then a
- * binary search of the CTF's pid-sorted packed keys; oversize objects (sid 1)
- * scan the oversize buffer */
-__device__ inline void run_oid(const QDev &Q, unsigned int *lc, const QueryRunDev &R, uint32_t qi, uint32_t n_objects) {
+/* one query's hits counted by the lanes, added to its count at once */
+__device__ inline void q_count_wave(const QDev &Q, uint32_t qi, uint32_t mine) {
+    for (int o = STC_WAVE / 2; o > 0; o >>= 1) mine += __shfl_down(mine, o, STC_WAVE);
+    if ((threadIdx.x & (STC_WAVE - 1)) == 0 && mine) atomicAdd(&Q.counts[qi], (unsigned long long)mine);
+}
+
+/* Object and pair queries against the runs, a wave per (query, run): the
+ * object's CTF by its sid, the first of its packed keys by 64 probes a round
+ * (two or three dependent reads; a thread's binary search took fifteen, of
+ * fourteen bytes each: 18 us for one query, 5 now; 64 queries, 3 runs: 89 and 8), then its records 64
+ * at a time; oversize objects (sid 1) scan the oversize buffer. */
+__global__ __launch_bounds__(256) void k_q_run_oid(const QueryRunDev *__restrict__ runs, uint32_t nruns,
+                                                   const uint32_t *__restrict__ oq, uint32_t noq, uint32_t n_objects,
+                                                   QDev Q) {
+    const int lane = threadIdx.x & (STC_WAVE - 1);
+    const uint64_t g = (uint64_t)__builtin_amdgcn_readfirstlane((int)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / STC_WAVE));
+    if (g >= (uint64_t)noq * nruns) return;
+    const QueryRunDev R = runs[g / noq];
+    const uint32_t qi = oq[g % noq];
     const stc_query q = Q.q[qi];
     if (q.oid >= n_objects) return;
     const uint16_t sid = R.sids[q.oid];
-    uint32_t pid, target, start, end;
+    uint32_t pid, target, start, end, found = 0;
     double m[4];
     if (sid == 0) return;
     if (sid == 1) {
-        for (uint32_t i = 0; i < R.n_tail; i++) {
+        for (uint32_t i = (uint32_t)lane; i < R.n_tail; i += STC_WAVE) {
             decode_tail(R.o_keys, R.o_boxes, i, R.end_time_min, &pid, &target, &start, &end, m);
             if (pid != q.oid || !q_time(q, start, end)) continue;
-            if (q.kind == STC_Q_OID || target == q.oid2) q_emit(Q, lc, qi, pid, target, start, end, R.source, m);
+            if (q.kind == STC_Q_OID || target == q.oid2) {
+                found++;
+                q_store(Q, qi, pid, target, start, end, R.source, m);
+            }
         }
+        q_count_wave(Q, qi, found);
         return;
     }
     const uint32_t c = sid - 2u;
@@ -320,48 +401,59 @@ __device__ inline void run_oid(const QDev &Q, unsigned int *lc, const QueryRunDe
     const stc_ctf_meta ctf = R.ctfs[c];
     const uint32_t kb = ctf.key_bit / 8;
     const uint8_t *base = R.key_bytes + R.byte_base[c];
-    uint32_t lo = 0, hi = ctf.kv_capacity;
-    while (lo < hi) {
-        uint32_t mid = lo + (hi - lo) / 2;
-        if (packed_pid(ctf, load_packed(base + (uint64_t)mid * kb, kb)) < q.oid) lo = mid + 1;
-        else hi = mid;
+    uint32_t lo = 0, hi = ctf.kv_capacity; /* the first key not below the object's is in [lo, hi] */
+    while (hi - lo > STC_WAVE) {
+        const uint32_t step = (hi - lo) / STC_WAVE, at = lo + (uint32_t)lane * step + step - 1;
+        const uint64_t below = __ballot(packed_pid(ctf, load_packed(base + (uint64_t)at * kb, kb)) < q.oid);
+        const uint32_t k = below == ~0ull ? STC_WAVE : (uint32_t)__ffsll((long long)~below) - 1u;
+        if (k < STC_WAVE) hi = lo + (k + 1) * step - 1;
+        lo += k * step;
     }
-    for (uint32_t i = lo; i < ctf.kv_capacity; i++) {
-        unsigned __int128 k = load_packed(base + (uint64_t)i * kb, kb);
-        if (packed_pid(ctf, k) != q.oid) break;
-        decode_packed(ctf, k, &pid, &target, &start, &end, m);
-        if (!q_time(q, start, end)) continue;
-        if (q.kind == STC_Q_OID || target == q.oid2) q_emit(Q, lc, qi, pid, target, start, end, R.source, m);
+    {
+        const uint32_t at = lo + (uint32_t)lane;
+        const bool below = at < hi && packed_pid(ctf, load_packed(base + (uint64_t)at * kb, kb)) < q.oid;
+        lo += (uint32_t)__popcll(__ballot(below));
     }
-}
-
-__global__ __launch_bounds__(256) void k_q_run_oid(const QueryRunDev *__restrict__ runs, uint32_t nruns,
-                                                   const uint32_t *__restrict__ oq, uint32_t noq, uint32_t n_objects,
-                                                   QDev Q) {
-    __shared__ unsigned int lc[QLDS];
-    lc_clear(Q, lc);
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < (uint64_t)noq * nruns) run_oid(Q, lc, runs[g / noq], oq[g % noq], n_objects);
-    lc_flush(Q, lc);
+    for (uint32_t i0 = lo; i0 < ctf.kv_capacity; i0 += STC_WAVE) {
+        const uint32_t i = i0 + (uint32_t)lane;
+        unsigned __int128 k = 0;
+        bool own = false;
+        if (i < ctf.kv_capacity) {
+            k = load_packed(base + (uint64_t)i * kb, kb);
+            own = packed_pid(ctf, k) == q.oid;
+        }
+        const uint64_t run = __ballot(own);
+        /* the object's records end at the first key that is not its own */
+        const uint32_t len = run == ~0ull ? STC_WAVE : (uint32_t)__ffsll((long long)~run) - 1u;
+        if ((uint32_t)lane < len) {
+            decode_packed(ctf, k, &pid, &target, &start, &end, m);
+            if (q_time(q, start, end) && (q.kind == STC_Q_OID || target == q.oid2)) {
+                found++;
+                q_store(Q, qi, pid, target, start, end, R.source, m);
+            }
+        }
+        if (len < STC_WAVE) break;
+    }
+    q_count_wave(Q, qi, found);
 }
 
 /* range queries: one block per (query, run, CTF) candidate; CTF 0xFFFFFFFF is
  * the run's oversize buffer */
 __global__ __launch_bounds__(256) void k_q_run_range(const QueryRunDev *__restrict__ runs,
                                                      const uint4 *__restrict__ cand, QDev Q) {
-    __shared__ unsigned int lc[QLDS];
-    lc_clear(Q, lc);
     const uint4 cd = cand[blockIdx.x];
     const uint32_t qi = cd.x;
     const stc_query q = Q.q[qi];
     const QueryRunDev R = runs[cd.y];
-    uint32_t pid, target, start, end;
+    uint32_t pid, target, start, end, found = 0;
     double m[4];
     if (cd.z == 0xFFFFFFFFu) {
         for (uint32_t i = threadIdx.x; i < R.n_tail; i += blockDim.x) {
             decode_tail(R.o_keys, R.o_boxes, i, R.end_time_min, &pid, &target, &start, &end, m);
-            if (pid < target && q_time(q, start, end) && q_box(q, m))
-                q_emit(Q, lc, qi, pid, target, start, end, R.source, m);
+            if (pid < target && q_time(q, start, end) && q_box(q, m)) {
+                found++;
+                q_store(Q, qi, pid, target, start, end, R.source, m);
+            }
         }
     } else {
         const stc_ctf_meta ctf = R.ctfs[cd.z];
@@ -369,11 +461,13 @@ __global__ __launch_bounds__(256) void k_q_run_range(const QueryRunDev *__restri
         const uint8_t *base = R.key_bytes + R.byte_base[cd.z];
         for (uint32_t i = threadIdx.x; i < ctf.kv_capacity; i += blockDim.x) {
             decode_packed(ctf, load_packed(base + (uint64_t)i * kb, kb), &pid, &target, &start, &end, m);
-            if (pid < target && q_time(q, start, end) && q_box(q, m))
-                q_emit(Q, lc, qi, pid, target, start, end, R.source, m);
+            if (pid < target && q_time(q, start, end) && q_box(q, m)) {
+                found++;
+                q_store(Q, qi, pid, target, start, end, R.source, m);
+            }
         }
     }
-    lc_flush(Q, lc);
+    q_count_wave(Q, qi, found);
 }
 
 /* one block per CTF: exact union box, time span and forward-record count */
@@ -671,7 +765,16 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
 
     /* grid of the range queries */
     const double x0 = st.map[0], y0 = st.map[1];
-    const double dx = (st.map[2] - st.map[0]) / QGRID, dy = (st.map[3] - st.map[1]) / QGRID;
+    const double ix = QGRID / (st.map[2] - st.map[0]), iy = QGRID / (st.map[3] - st.map[1]);
+    /* the scans' filter: about 16 bits per queried id, at most 2^16 */
+    uint32_t f_bits = 5;
+    if (!oq.empty()) f_bits = std::min(std::max(bits + 3, 10u), 16u);
+    std::vector<uint32_t> filter((1u << f_bits) / 32 + QGRID * QGRID / 32, 0u);
+    for (uint32_t i : oq) {
+        const uint32_t h = oid_slot(q[i].oid, f_bits);
+        filter[h >> 5] |= 1u << (h & 31);
+    }
+    uint32_t *cell_bits = filter.data() + (1u << f_bits) / 32;
     std::vector<uint32_t> rq;
     for (uint32_t i = 0; i < nq; i++)
         if (q[i].kind == STC_Q_RANGE) rq.push_back(i);
@@ -680,13 +783,14 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         std::vector<std::vector<uint32_t>> cells(QGRID * QGRID);
         for (uint32_t qi : rq) {
             const double *b = q[qi].box;
-            int cx0 = grid_cell(b[0], x0, dx), cx1 = grid_cell(b[2], x0, dx);
-            int cy0 = grid_cell(b[1], y0, dy), cy1 = grid_cell(b[3], y0, dy);
+            int cx0 = grid_cell(b[0], x0, ix), cx1 = grid_cell(b[2], x0, ix);
+            int cy0 = grid_cell(b[1], y0, iy), cy1 = grid_cell(b[3], y0, iy);
             for (int cy = cy0; cy <= cy1; cy++)
                 for (int cx = cx0; cx <= cx1; cx++) cells[cy * QGRID + cx].push_back(qi);
         }
         for (int c = 0; c < QGRID * QGRID; c++) {
             start[c + 1] = start[c] + (uint32_t)cells[c].size();
+            if (!cells[c].empty()) cell_bits[c >> 5] |= 1u << (c & 31);
             list.insert(list.end(), cells[c].begin(), cells[c].end());
         }
         uint32_t gc = B->g_cap;
@@ -698,7 +802,12 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         if (!list.empty()) QCK(hipMemcpy(B->g_list, list.data(), list.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
 
+    if (grow32(&B->filter, &B->f_cap, filter.size()))
+        return stc_hip_fail(hipErrorOutOfMemory, "query filter", __FILE__, __LINE__);
+    QCK(hipMemcpy(B->filter, filter.data(), filter.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     QDev Q;
+    Q.filter = B->filter;
+    Q.f_bits = f_bits;
     Q.q = B->q;
     Q.oh_key = B->oh_key;
     Q.oh_head = B->oh_head;
@@ -709,25 +818,27 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     Q.g_list = B->g_list;
     Q.x0 = x0;
     Q.y0 = y0;
-    Q.dx = dx;
-    Q.dy = dy;
+    Q.ix = ix;
+    Q.iy = iy;
     Q.hits = B->hits;
     Q.cap = hits ? cap : 0;
     Q.n_hits = B->counters;
     Q.counts = B->counters + 1;
     Q.nq = nq;
     Q.lds = nq <= QLDS;
+    const size_t q_scan_lds = ((Q.lds ? nq : 0) + filter.size()) * sizeof(uint32_t);
     /* counts a planner adds without a kernel (CTFs wholly inside a range query) */
     std::vector<unsigned long long> planned(nq, 0);
 
     /* live meetings and memtable */
     if (st.stepped && st.table && st.nb) {
         uint32_t g = (uint32_t)std::min<uint64_t>(blocks(st.nb, 256), 8192);
-        hipLaunchKernelGGL(k_q_live, dim3(g), dim3(256), 0, s, st.table, st.nb, st.last_t, Q);
+        if (Q.n_range) hipLaunchKernelGGL(k_q_live<true>, dim3(g), dim3(256), q_scan_lds, s, st.table, st.nb, st.last_t, Q);
+        else hipLaunchKernelGGL(k_q_live<false>, dim3(g), dim3(256), q_scan_lds, s, st.table, st.nb, st.last_t, Q);
         QCK(hipGetLastError());
     }
     if (st.n_rec) {
-        hipLaunchKernelGGL(k_q_mem, dim3(std::min<uint32_t>(blocks(st.n_rec, 256), 8192)), dim3(256), 0, s,
+        hipLaunchKernelGGL(k_q_mem, dim3(std::min<uint32_t>(blocks(st.n_rec, 256), 8192)), dim3(256), q_scan_lds, s,
                            st.rec_keys, st.rec_boxes, st.n_rec, st.end_time_min, Q);
         QCK(hipGetLastError());
     }
@@ -738,7 +849,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
             return stc_hip_fail(hipErrorOutOfMemory, "query runs", __FILE__, __LINE__);
         QCK(hipMemcpy(B->runs, st.runs.data(), nruns * sizeof(QueryRunDev), hipMemcpyHostToDevice));
         if (!oq.empty()) {
-            hipLaunchKernelGGL(k_q_run_oid, dim3(blocks((uint64_t)oq.size() * nruns, 256)), dim3(256), 0, s, B->runs,
+            hipLaunchKernelGGL(k_q_run_oid, dim3(blocks((uint64_t)oq.size() * nruns * STC_WAVE, 256)), dim3(256), 0, s, B->runs,
                                nruns, B->oq, (uint32_t)oq.size(), st.num_objects, Q);
             QCK(hipGetLastError());
         }
