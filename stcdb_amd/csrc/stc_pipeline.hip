@@ -3796,7 +3796,7 @@ static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *
     int rc = 0;
     if (run) {
         if (!c->qb) c->qb = stc_query_bufs_new();
-        rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, c->qs);
+        rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, STC_QUERY_RESERVE, c->qs);
     } else {
         *n_hits = 0;
     }

@@ -71,7 +71,16 @@ struct QueryBufs {
     uint64_t hits_cap = 0;
     unsigned long long *counters = nullptr; /* [0] total hits, [1 ..] per query */
     uint64_t counters_cap = 0;
+    uint8_t *sort = nullptr;         /* keys and places of the hits, and the sort's scratch */
+    uint64_t sort_cap = 0;
+    stc_hit *out[2] = {nullptr, nullptr}; /* pinned: sorted hits on their way to the caller, a chunk each */
+    hipEvent_t out_ev[2] = {nullptr, nullptr};
+    uint32_t *wide = nullptr;        /* pinned: a hit's field did not fit its key bits */
 };
+
+#define QFETCH 65536u /* hits of a chunk */
+#define QSORT_HOST 1024u /* up to this many hits are copied as they are and sorted by the host: the device sort's
+                          * launches cost what that does (about 80 us at 1,000 hits) */
 
 QueryBufs *stc_query_bufs_new() { return new QueryBufs(); }
 
@@ -87,9 +96,14 @@ uint64_t stc_query_bufs_growth(const QueryBufs *b, uint32_t nq, uint64_t cap) {
 void stc_query_bufs_free(QueryBufs *b) {
     if (!b) return;
     void *ptrs[] = {b->q, b->oh_key, b->oh_head, b->q_next, b->oq, b->g_start, b->g_list, b->filter, b->runs, b->cand,
-                    b->hits, b->counters};
+                    b->hits, b->counters, b->sort};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    for (int i = 0; i < 2; i++) {
+        if (b->out[i]) (void)hipHostFree(b->out[i]);
+        if (b->out_ev[i]) (void)hipEventDestroy(b->out_ev[i]);
+    }
+    if (b->wide) (void)hipHostFree(b->wide);
     delete b;
 }
 
@@ -709,6 +723,105 @@ int stc_query_ctf_stats(const QueryRunDev &run, const stc_ctf_meta *host_ctfs, s
     return STC_OK;
 }
 
+/* ---------------- the hits in order ---------------- */
+
+/* how a hit's (query, source, pid, target, start, end) is packed into sort keys */
+struct HitKeyBits {
+    uint32_t q, src, id, t; /* bits of a field */
+    uint32_t two;           /* two keys: (query, source, pid) and (target, start, end); else one of all six */
+};
+
+/* the hits' sort keys, taken in the order idx when there is one; part 0: the low key or the only one, 1: the high key */
+__global__ void k_hit_keys(const stc_hit *__restrict__ hits, const uint32_t *__restrict__ idx, uint32_t n, HitKeyBits b,
+                           int part, uint64_t *__restrict__ keys, uint32_t *__restrict__ wide) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const stc_hit &h = hits[idx ? idx[i] : i];
+    const uint64_t q = h.query, src = h.source, pid = h.pid, tgt = h.target, st = h.start, en = h.end;
+    if ((q >> b.q) | (src >> b.src) | (pid >> b.id) | (tgt >> b.id) | (st >> b.t) | (en >> b.t)) *wide = 1;
+    const uint64_t high = (((q << b.src) | src) << b.id) | pid, low = (((tgt << b.t) | st) << b.t) | en;
+    keys[i] = part ? high : b.two ? low : (high << (b.id + 2 * b.t)) | low;
+}
+
+/* hits[idx[first ..]] to out (host memory), 8 bytes a thread */
+__global__ void k_hit_gather(const uint64_t *__restrict__ hits, const uint32_t *__restrict__ idx, uint32_t first,
+                             uint32_t words, uint64_t *__restrict__ out) {
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w < words) out[w] = hits[(uint64_t)idx[first + w / 7] * 7 + w % 7];
+}
+static_assert(sizeof(stc_hit) == 56, "a hit is seven words");
+
+/* The n stored hits to the caller's `hits`, sorted by (query, source, pid,
+ * target, start, end): a radix sort of the packed fields on the device, then
+ * chunks gathered in order into pinned memory and copied out while the next is
+ * gathered. *done stays false when the fields do not pack, a value does not fit
+ * its bits, or the scratch would leave less than `reserve` bytes of device
+ * memory: the caller then sorts on the host. (330,000 hits: one host thread
+ * sorted them in 17 ms; the sort takes 0.25 ms, the fetch is bound by the link and
+ * the copy into the caller's memory.) */
+static int fetch_sorted(QueryBufs *B, const QueryState &st, uint32_t nq, uint64_t n64, stc_hit *hits, uint64_t reserve,
+                        bool *done, hipStream_t s) {
+    *done = false;
+    auto bits_for = [](uint64_t v) { uint32_t b = 1; while (b < 63 && (v >> b)) b++; return b; };
+    HitKeyBits kb{bits_for(nq - 1), 1, bits_for(st.num_objects - 1), bits_for(st.last_t), 0};
+    for (const QueryRunDev &r : st.runs) kb.src = std::max(kb.src, bits_for(r.source));
+    const uint32_t hb = kb.q + kb.src + kb.id, lb = kb.id + 2 * kb.t;
+    kb.two = hb + lb > 64;
+    if (n64 >= (1ull << 31) || hb > 64 || lb > 64) return STC_OK;
+    const uint32_t n = (uint32_t)n64;
+    const uint64_t bytes = n64 * 24 + stc_radix_temp_words(n) * 4;
+    if (B->sort_cap < bytes) {
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes + bytes / 2 + reserve > free_b + B->sort_cap) return STC_OK;
+        if (grow(&B->sort, &B->sort_cap, bytes)) {
+            (void)hipGetLastError(); /* the host sorts */
+            return STC_OK;
+        }
+    }
+    if (!B->wide) QCK(hipHostMalloc((void **)&B->wide, sizeof(uint32_t), hipHostMallocDefault));
+    for (int i = 0; i < 2; i++) {
+        if (!B->out[i]) QCK(hipHostMalloc((void **)&B->out[i], QFETCH * sizeof(stc_hit), hipHostMallocDefault));
+        if (!B->out_ev[i]) QCK(hipEventCreateWithFlags(&B->out_ev[i], hipEventDisableTiming));
+    }
+    uint64_t *ka = (uint64_t *)B->sort, *kb2 = ka + n;
+    uint32_t *va = (uint32_t *)(kb2 + n), *vb = va + n, *temp = vb + n;
+    *B->wide = 0;
+    bool alt = false;
+    hipLaunchKernelGGL(k_hit_keys, dim3(blocks(n, 256)), dim3(256), 0, s, B->hits, (const uint32_t *)nullptr, n, kb, 0, ka, B->wide);
+    int rc = stc_radix_sort_u64(ka, nullptr, kb2, va, ka, vb, n, 0, (int)(kb.two ? lb : hb + lb), temp, &alt, s);
+    if (rc) return rc;
+    uint32_t *idx = alt ? vb : va;
+    if (kb.two) {
+        uint32_t *other = alt ? va : vb;
+        hipLaunchKernelGGL(k_hit_keys, dim3(blocks(n, 256)), dim3(256), 0, s, B->hits, (const uint32_t *)idx, n, kb, 1, ka, B->wide);
+        bool alt2 = false;
+        rc = stc_radix_sort_u64(ka, idx, ka, idx, kb2, other, n, 0, (int)hb, temp, &alt2, s);
+        if (rc) return rc;
+        if (alt2) idx = other;
+    }
+    QCK(hipGetLastError());
+    const uint32_t chunks = (n + QFETCH - 1) / QFETCH;
+    auto gather = [&](uint32_t c) {
+        const uint32_t first = c * QFETCH, words = std::min(QFETCH, n - first) * 7;
+        hipLaunchKernelGGL(k_hit_gather, dim3(blocks(words, 256)), dim3(256), 0, s, (const uint64_t *)B->hits, (const uint32_t *)idx,
+                           first, words, (uint64_t *)B->out[c & 1]);
+        return hipEventRecord(B->out_ev[c & 1], s);
+    };
+    QCK(gather(0));
+    for (uint32_t c = 0; c < chunks; c++) {
+        if (c + 1 < chunks) QCK(gather(c + 1));
+        QCK(hipEventSynchronize(B->out_ev[c & 1]));
+        if (*(volatile uint32_t *)B->wide) { /* let the gather in flight end before its buffer is used again */
+            QCK(hipStreamSynchronize(s));
+            return STC_OK;
+        }
+        const uint64_t first = (uint64_t)c * QFETCH;
+        memcpy(hits + first, B->out[c & 1], std::min<uint64_t>(QFETCH, n - first) * sizeof(stc_hit));
+    }
+    *done = true;
+    return STC_OK;
+}
+
 /* the decoded boxes of a CTF lie in [low, low + |extent| + longer edge] per
  * axis (new_parse_mbr): a conservative test, widened by 1e-6 degrees for the
  * float/double rounding of the bounds */
@@ -722,7 +835,7 @@ static bool ctf_may_intersect(const stc_ctf_meta &c, const double *box) {
 }
 
 int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap,
-                  uint64_t *n_hits, uint64_t *counts, hipStream_t s) {
+                  uint64_t *n_hits, uint64_t *counts, uint64_t reserve, hipStream_t s) {
     if (nq == 0) {
         *n_hits = 0;
         return STC_OK;
@@ -905,7 +1018,12 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     }
     *n_hits = total;
     uint64_t stored = Q.cap ? std::min<uint64_t>(cnt[0], cap) : 0;
-    if (stored && hits) {
+    bool sorted = false;
+    if (stored > QSORT_HOST && hits) {
+        const int rc = fetch_sorted(B, st, nq, stored, hits, reserve, &sorted, s);
+        if (rc) return rc;
+    }
+    if (stored && hits && !sorted) {
         QCK(hipMemcpy(hits, B->hits, stored * sizeof(stc_hit), hipMemcpyDeviceToHost));
         std::sort(hits, hits + stored, [](const stc_hit &a, const stc_hit &b) {
             if (a.query != b.query) return a.query < b.query;
