@@ -2095,6 +2095,88 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
 
 #define SEG_CAP 4096u  /* LDS sort keys of the four-wave segment sort */
 
+#define LTILE 1024u    /* buckets of an export tile (one workgroup) */
+#define LCHUNK 16u     /* export tiles of a chunk */
+
+/* live buckets of each export tile */
+__global__ __launch_bounds__(256) void k_live_tiles(const Bucket *__restrict__ t, uint64_t n, uint32_t *__restrict__ tiles) {
+    __shared__ uint32_t wsum[256 / STC_WAVE];
+    const int lane = threadIdx.x & (STC_WAVE - 1), wv = threadIdx.x / STC_WAVE;
+    uint32_t c = 0;
+    for (uint32_t r = 0; r < LTILE / 256; r++) {
+        const uint64_t i = (uint64_t)blockIdx.x * LTILE + r * 256 + threadIdx.x;
+        c += (uint32_t)__popcll(__ballot(i < n && (uint32_t)t[i].key != DEAD_B));
+    }
+    if (lane == 0) wsum[wv] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t s = 0;
+        for (uint32_t k = 0; k < 256 / STC_WAVE; k++) s += wsum[k];
+        tiles[blockIdx.x] = s;
+    }
+}
+
+/* The live meetings of the tiles from tile0 on (one per workgroup), in order,
+ * to a chunk of pinned host memory that starts with output base0: as their
+ * fields (keys, starts, MBRs, each an array of the chunk), as the last step's
+ * meeting units (the MBR of the two positions at the step), or as pair keys
+ * alone. tbase: the first output of each tile; null when no bucket is dead.
+ * Bound by the link to the host (28 or 32 bytes a meeting). */
+enum LiveForm { LIVE_FIELDS, LIVE_UNITS, LIVE_KEYS };
+template <LiveForm FORM>
+__global__ __launch_bounds__(256) void k_live_out(const Bucket *__restrict__ t, uint64_t n, uint32_t tile0,
+                                                  const uint32_t *__restrict__ tbase, uint64_t base0,
+                                                  const float2 *__restrict__ posf, uint32_t now, uint8_t *__restrict__ out) {
+    __shared__ uint32_t wsum[256 / STC_WAVE];
+    const int lane = threadIdx.x & (STC_WAVE - 1), wv = threadIdx.x / STC_WAVE;
+    const uint32_t tile = tile0 + blockIdx.x;
+    uint32_t at = (uint32_t)((tbase ? (uint64_t)tbase[tile] : (uint64_t)tile * LTILE) - base0);
+    for (uint32_t r = 0; r < LTILE / 256; r++) {
+        const uint64_t i = (uint64_t)tile * LTILE + r * 256 + threadIdx.x;
+        Bucket b;
+        b.key = DEAD_B;
+        if (i < n) b = t[i];
+        const bool live = bucket_live(b);
+        const uint64_t m = __ballot(live);
+        if (lane == 0) wsum[wv] = (uint32_t)__popcll(m);
+        __syncthreads();
+        uint32_t k = at + (uint32_t)__popcll(m & lanemask_lt(lane));
+        for (int q = 0; q < 256 / STC_WAVE; q++) {
+            if (q < wv) k += wsum[q];
+            at += wsum[q];
+        }
+        __syncthreads();
+        if (!live) continue;
+        if constexpr (FORM == LIVE_FIELDS) {
+            constexpr size_t C = LCHUNK * LTILE;
+            ((uint64_t *)out)[k] = b.key;
+            ((float4 *)(out + 8 * C))[k] = make_float4(o2f(b.mbr[0]), o2f(b.mbr[1]), o2f(b.mbr[2]), o2f(b.mbr[3]));
+            ((uint32_t *)(out + 24 * C))[k] = b.start;
+        } else if constexpr (FORM == LIVE_KEYS) {
+            ((uint64_t *)out)[k] = b.key;
+        } else {
+            const uint64_t x = b.key >> 32, y = b.key & 0xFFFFFFFFull;
+            const float2 p = posf[x], q = posf[y];
+            const float4 mb = pair_mbr(p.x, p.y, q.x, q.y);
+            const uint64_t z = (x + y) * (x + y + 1) / 2 + y;
+            uint4 *d = (uint4 *)(out + 32ull * k);
+            d[0] = make_uint4((uint32_t)z, (uint32_t)(z >> 32), now, now);
+            d[1] = make_uint4(__float_as_uint(mb.x), __float_as_uint(mb.y), __float_as_uint(mb.z), __float_as_uint(mb.w));
+        }
+    }
+}
+
+/* the replayed pairs from first on, as meeting units, to a chunk of pinned host memory */
+__global__ void k_boxed_out(const PairHit *__restrict__ pn, uint64_t first, uint32_t n, uint32_t now, uint4 *__restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const PairHit h = pn[first + i];
+    const uint64_t x = h.key >> 32, y = h.key & 0xFFFFFFFFull, z = (x + y) * (x + y + 1) / 2 + y;
+    out[2 * i] = make_uint4((uint32_t)z, (uint32_t)(z >> 32), now, now);
+    out[2 * i + 1] = make_uint4(__float_as_uint(h.mbr[0]), __float_as_uint(h.mbr[1]), __float_as_uint(h.mbr[2]),
+                                __float_as_uint(h.mbr[3]));
+}
+
 __global__ void k_fill_obox(uint4 *a, uint32_t n) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = make_uint4(100000000u, 100000000u, 0u, 0u); /* cuda_init_o_boxs */
@@ -2370,6 +2452,9 @@ struct StcCtx {
     float flush_done_ms = 0;
     bool drop_pending = false;           /* stc_drop_runs came while a flush thread ran */
     bool lp_valid = false;               /* lp holds a position step's leaf order (a permutation of the points) */
+    uint8_t *xout = nullptr;             /* pinned: two chunks of an export on its way to the caller */
+    hipEvent_t xev[2] = {nullptr, nullptr};
+    DBuf<uint32_t> xtiles;               /* first output of each export tile, and the scan's scratch */
     PinnedPool pinned;
     std::vector<PinnedBlock> deferred;   /* blocks of dropped runs whose host copy is not queued yet */
     QueryBufs *qb = nullptr;
@@ -2522,32 +2607,65 @@ static int sort_pairs(const K *kin, const uint32_t *vin, DBuf<K> &k, DBuf<uint32
     return rc;
 }
 
-/* the last step's pairs (its pair slots without the dead ones), sorted by key */
-static int step_pairs(StcCtx *c, std::vector<PairHit> &ph) {
-    ph.resize(c->plen);
-    if (c->pairs_boxed) {
-        if (c->plen) CK(hipMemcpy(ph.data(), c->pbox.p, c->plen * sizeof(PairHit), hipMemcpyDeviceToHost));
-    } else if (c->plen) { /* slots, owner by owner: the MBR is the box of the owner's and the partner's float positions */
-        std::vector<PairSlot> sl(c->plen);
-        std::vector<float2> pos(c->n);
-        std::vector<uint32_t> off(c->n + 1ull);
-        CK(hipMemcpy(sl.data(), c->pnew.p, c->plen * sizeof(PairSlot), hipMemcpyDeviceToHost));
-        CK(hipMemcpy(pos.data(), c->posf.p, (size_t)c->n * sizeof(float2), hipMemcpyDeviceToHost));
-        CK(hipMemcpy(off.data(), c->moff[c->cur].p, (c->n + 1ull) * 4, hipMemcpyDeviceToHost));
-        for (uint32_t a = 0; a < c->n; a++)
-            for (uint64_t i = off[a]; i < off[a + 1] && i < c->plen; i++) {
-                const float2 o = pos[a];
-                ph[i].key = ((uint64_t)a << 32) | sl[i].partner;
-                ph[i].mbr[0] = std::fmin(o.x, sl[i].px);
-                ph[i].mbr[1] = std::fmin(o.y, sl[i].py);
-                ph[i].mbr[2] = std::fmax(o.x, sl[i].px);
-                ph[i].mbr[3] = std::fmax(o.y, sl[i].py);
-            }
+/* Chunks of an export: launch(k, buffer) fills chunk k of the pinned buffer on the context's stream,
+ * take(k, buffer) copies it to the caller while the next one is filled. */
+template <class Launch, class Take>
+static int export_chunks(StcCtx *c, uint64_t chunks, Launch launch, Take take) {
+    constexpr size_t size = (size_t)LCHUNK * LTILE * 32;
+    if (!c->xout) CK(hipHostMalloc((void **)&c->xout, 2 * size, hipHostMallocDefault));
+    for (int i = 0; i < 2; i++)
+        if (!c->xev[i]) CK(hipEventCreateWithFlags(&c->xev[i], hipEventDisableTiming));
+    auto start = [&](uint64_t k) {
+        launch(k, c->xout + (k & 1) * size);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : hipEventRecord(c->xev[k & 1], c->s);
+    };
+    if (chunks) CK(start(0));
+    for (uint64_t k = 0; k < chunks; k++) {
+        if (k + 1 < chunks) CK(start(k + 1));
+        CK(hipEventSynchronize(c->xev[k & 1]));
+        take(k, c->xout + (k & 1) * size);
     }
-    ph.erase(std::remove_if(ph.begin(), ph.end(), [](const PairHit &e) { return (uint32_t)e.key == DEAD_B; }),
-             ph.end());
-    std::sort(ph.begin(), ph.end(), [](const PairHit &a, const PairHit &b) { return a.key < b.key; });
     return 0;
+}
+
+/* The live meetings of the last step in key order, at most `cap` of them: take(first, count, chunk) for
+ * each chunk of k_live_out's output. The merge counted them (last_live); the pairs of the step are the
+ * same ones. */
+template <LiveForm FORM, class Take>
+static int export_live(StcCtx *c, uint64_t cap, Take take) {
+    const uint64_t want = std::min<uint64_t>(cap, c->last_live);
+    if (!want) return 0;
+    const uint64_t tiles = (c->mlen + LTILE - 1) / LTILE;
+    const uint32_t *tbase = nullptr;
+    std::vector<uint32_t> base; /* first output of each chunk */
+    if (c->last_live != c->mlen) { /* dead buckets: the tiles' outputs by a scan */
+        if (c->xtiles.ensure(tiles + stc_radix_temp_words((uint32_t)tiles))) return fail(c, STC_E_CAPACITY, "export tiles");
+        hipLaunchKernelGGL(k_live_tiles, dim3((uint32_t)tiles), dim3(256), 0, c->s, (const Bucket *)c->meet[c->cur].p, c->mlen, c->xtiles.p);
+        CK(hipGetLastError());
+        CKRC(stc_exclusive_scan_u32(c->xtiles.p, c->xtiles.p, (uint32_t)tiles, nullptr, c->xtiles.p + tiles, c->s));
+        base.resize(tiles);
+        CK(hipMemcpyAsync(base.data(), c->xtiles.p, tiles * 4, hipMemcpyDeviceToHost, c->s));
+        CK(hipStreamSynchronize(c->s));
+        tbase = c->xtiles.p;
+    }
+    auto out_of = [&](uint64_t tile) {
+        return tile >= tiles ? c->last_live : tbase ? (uint64_t)base[tile] : tile * LTILE;
+    };
+    uint64_t chunks = 0; /* up to the one that holds the last wanted meeting */
+    while (out_of(chunks * LCHUNK) < want) chunks++;
+    return export_chunks(
+        c, chunks,
+        [&](uint64_t k, uint8_t *buf) {
+            const uint64_t t0 = k * LCHUNK;
+            hipLaunchKernelGGL(k_live_out<FORM>, dim3((uint32_t)std::min<uint64_t>(LCHUNK, tiles - t0)), dim3(256), 0, c->s,
+                               (const Bucket *)c->meet[c->cur].p, c->mlen, (uint32_t)t0, tbase, out_of(t0),
+                               (const float2 *)c->posf.p, c->last_t, buf);
+        },
+        [&](uint64_t k, const uint8_t *buf) {
+            const uint64_t first = out_of(k * LCHUNK);
+            take(first, std::min(out_of((k + 1) * LCHUNK), want) - first, buf);
+        });
 }
 
 /* A run's pinned block back to the pool. With finish_copy, a host copy owed to
@@ -2846,6 +2964,10 @@ int stc_destroy(void *vc) {
     c->pinned.clear();
     stc_query_bufs_free(c->qb);
     c->qb = nullptr;
+    if (c->xout) (void)hipHostFree(c->xout);
+    for (int i = 0; i < 2; i++)
+        if (c->xev[i]) (void)hipEventDestroy(c->xev[i]);
+    c->xtiles.release();
     for (int i = 0; i < 14; i++) if (c->ev[i]) hipEventDestroy(c->ev[i]);
     stc_schema_free(&c->sch);
     if (c->s) hipStreamDestroy(c->s);
@@ -3562,19 +3684,21 @@ int stc_get_step_meetings(void *vc, stc_meeting_unit *units, uint64_t cap, uint6
     if (!c || !n) return STC_E_ARG;
     if (!c->stepped) return fail(c, STC_E_STATE, "no step processed");
     if (!(c->cfg.keep_pairs & 1)) return fail(c, STC_E_STATE, "pairs are kept only with keep_pairs bit 0 set");
-    std::vector<PairHit> ph;
-    CKRC(step_pairs(c, ph));
-    ph.erase(std::unique(ph.begin(), ph.end(), [](const PairHit &a, const PairHit &b) { return a.key == b.key; }),
-             ph.end());
-    *n = ph.size();
-    if (units)
-        for (uint64_t i = 0; i < std::min<uint64_t>(cap, ph.size()); i++) {
-            const uint64_t a = ph[i].key >> 32, b = ph[i].key & 0xFFFFFFFFull;
-            units[i].key = (a + b) * (a + b + 1) / 2 + b;
-            units[i].start = units[i].end = c->last_t;
-            memcpy(units[i].mbr, ph[i].mbr, sizeof(units[i].mbr));
-        }
-    return STC_OK;
+    *n = c->last_live;
+    if (!units) return STC_OK;
+    if (!c->pairs_boxed)
+        return export_live<LIVE_UNITS>(c, cap, [&](uint64_t first, uint64_t count, const uint8_t *buf) {
+            memcpy(units + first, buf, count * sizeof(stc_meeting_unit));
+        });
+    const uint64_t want = std::min<uint64_t>(cap, c->plen), per = (uint64_t)LCHUNK * LTILE;
+    auto count = [&](uint64_t k) { return std::min(per, want - k * per); };
+    return export_chunks(
+        c, (want + per - 1) / per,
+        [&](uint64_t k, uint8_t *buf) {
+            hipLaunchKernelGGL(k_boxed_out, dim3(blocks_for(count(k), 256)), dim3(256), 0, c->s, (const PairHit *)c->pbox.p, k * per,
+                               (uint32_t)count(k), c->last_t, (uint4 *)buf);
+        },
+        [&](uint64_t k, const uint8_t *buf) { memcpy(units + k * per, buf, count(k) * sizeof(stc_meeting_unit)); });
 }
 
 int stc_get_pairs(void *vc, uint64_t *keys, uint64_t cap, uint64_t *n) {
@@ -3582,33 +3706,26 @@ int stc_get_pairs(void *vc, uint64_t *keys, uint64_t cap, uint64_t *n) {
     if (!c || !n) return STC_E_ARG;
     if (!c->stepped) return fail(c, STC_E_STATE, "no step processed");
     if (!(c->cfg.keep_pairs & 1)) return fail(c, STC_E_STATE, "pairs are kept only with keep_pairs bit 0 set");
-    std::vector<PairHit> ph;
-    CKRC(step_pairs(c, ph));
-    std::vector<uint64_t> k(ph.size());
-    for (size_t i = 0; i < ph.size(); i++) k[i] = ph[i].key;
-    k.erase(std::unique(k.begin(), k.end()), k.end());
-    *n = k.size();
-    if (keys) memcpy(keys, k.data(), std::min<uint64_t>(cap, k.size()) * 8);
-    return STC_OK;
+    *n = c->last_live;
+    if (!keys) return STC_OK;
+    return export_live<LIVE_KEYS>(c, cap, [&](uint64_t first, uint64_t count, const uint8_t *buf) {
+        memcpy(keys + first, buf, count * 8);
+    });
 }
 
 int stc_get_active(void *vc, uint64_t *keys, uint32_t *start, uint32_t *end, float *mbr, uint64_t cap, uint64_t *n) {
     StcCtx *c = (StcCtx *)vc;
     if (!c || !n) return STC_E_ARG;
     if (!c->stepped) return fail(c, STC_E_STATE, "no step processed");
-    std::vector<Bucket> tb(c->mlen);
-    if (c->mlen) CK(hipMemcpy(tb.data(), c->meet[c->cur].p, c->mlen * sizeof(Bucket), hipMemcpyDeviceToHost));
-    std::vector<Bucket> live; /* the array is sorted by key; tombstones trail each segment */
-    for (const Bucket &b : tb)
-        if (bucket_live(b)) live.push_back(b);
-    *n = live.size();
-    for (uint64_t i = 0; i < std::min<uint64_t>(cap, live.size()); i++) {
-        if (keys) keys[i] = live[i].key;
-        if (start) start[i] = live[i].start;
-        if (end) end[i] = c->last_t; /* every live meeting was seen by the last step */
-        if (mbr) for (int q = 0; q < 4; q++) mbr[4 * i + q] = o2f(live[i].mbr[q]);
-    }
-    return STC_OK;
+    *n = c->last_live;
+    if (!keys && !start && !end && !mbr) return STC_OK;
+    return export_live<LIVE_FIELDS>(c, cap, [&](uint64_t first, uint64_t count, const uint8_t *buf) {
+        constexpr size_t C = (size_t)LCHUNK * LTILE;
+        if (keys) memcpy(keys + first, buf, count * 8);
+        if (mbr) memcpy(mbr + 4 * first, buf + 8 * C, count * 16);
+        if (start) memcpy(start + first, buf + 24 * C, count * 4);
+        if (end) std::fill(end + first, end + first + count, c->last_t); /* every live meeting was seen by the last step */
+    });
 }
 
 int stc_get_records(void *vc, uint64_t *keys, float *boxes, uint64_t cap, uint64_t *n) {
