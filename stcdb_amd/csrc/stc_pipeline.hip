@@ -2918,6 +2918,7 @@ int stc_create(const stc_config *cfg, const stc_box *mbr, void **out) {
     hipLaunchKernelGGL(k_fill_obox, dim3(blocks_for(n, 256)), dim3(256), 0, c->s, c->o_boxs, n);
     if (ensure_records(c, std::max<uint64_t>(1 << 16, (uint64_t)cfg->kv_restriction + 2))) return bad("records");
     if (stc_flush_init(&c->flushw, n, C)) return bad("flush buffers");
+    c->qb = stc_query_bufs_new();
     if (hipStreamSynchronize(c->s) != hipSuccess) return bad("init sync");
     *out = c;
     return STC_OK;
@@ -3912,7 +3913,6 @@ static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *
     }
     int rc = 0;
     if (run) {
-        if (!c->qb) c->qb = stc_query_bufs_new();
         rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, STC_QUERY_RESERVE, c->qs);
     } else {
         *n_hits = 0;

@@ -48,29 +48,49 @@ struct QDev {
     uint32_t lds;                    /* nq <= QLDS: per-block counters in LDS */
 };
 
+/* host tables on their way to the device: built in pinned memory, sent with one copy */
+struct QueryUpload {
+    uint8_t *host = nullptr, *dev = nullptr;
+    uint64_t cap = 0, used = 0;
+    /* room for `bytes`, and nothing in it */
+    int begin(uint64_t bytes) {
+        used = 0;
+        if (bytes <= cap) return 0;
+        release();
+        const uint64_t nc = bytes + bytes / 2 + 4096;
+        if (hipHostMalloc((void **)&host, nc, hipHostMallocDefault) != hipSuccess || hipMalloc((void **)&dev, nc) != hipSuccess) {
+            release();
+            return -1;
+        }
+        cap = nc;
+        return 0;
+    }
+    static uint64_t room(uint64_t bytes) { return (bytes + 15) & ~15ull; }
+    /* a table of n (from src, or zeros), and where it will be on the device */
+    template <typename T>
+    T *put(const T *src, uint64_t n) {
+        uint8_t *at = host + used;
+        T *d = (T *)(dev + used);
+        if (src) memcpy(at, src, n * sizeof(T));
+        else memset(at, 0, n * sizeof(T));
+        used += room(n * sizeof(T));
+        return d;
+    }
+    hipError_t send(hipStream_t s) { return hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, s); }
+    void release() {
+        if (host) (void)hipHostFree(host);
+        if (dev) (void)hipFree(dev);
+        host = dev = nullptr;
+        cap = 0;
+    }
+};
+
 struct QueryBufs {
-    stc_query *q = nullptr;
-    uint32_t q_cap = 0;
-    uint32_t *oh_key = nullptr;
-    int32_t *oh_head = nullptr;
-    uint32_t oh_cap = 0;
-    int32_t *q_next = nullptr;
-    uint32_t qn_cap = 0;
-    uint32_t *oq = nullptr;          /* object and pair queries */
-    uint32_t oq_cap = 0;
-    uint32_t *g_start = nullptr;
-    uint32_t *g_list = nullptr;
-    uint32_t g_cap = 0;
-    uint32_t *filter = nullptr;
-    uint32_t f_cap = 0;
-    QueryRunDev *runs = nullptr;
-    uint32_t runs_cap = 0;
-    uint4 *cand = nullptr;
-    uint64_t cand_cap = 0;
+    QueryUpload batch, runs;         /* the batch's tables and zeroed counters; the runs and their candidates */
+    uint64_t *res = nullptr;         /* pinned: the counters, then the first hits */
+    uint64_t res_cap = 0;
     stc_hit *hits = nullptr;
     uint64_t hits_cap = 0;
-    unsigned long long *counters = nullptr; /* [0] total hits, [1 ..] per query */
-    uint64_t counters_cap = 0;
     uint8_t *sort = nullptr;         /* keys and places of the hits, and the sort's scratch */
     uint64_t sort_cap = 0;
     stc_hit *out[2] = {nullptr, nullptr}; /* pinned: sorted hits on their way to the caller, a chunk each */
@@ -82,23 +102,22 @@ struct QueryBufs {
 #define QSORT_HOST 1024u /* up to this many hits are copied as they are and sorted by the host: the device sort's
                           * launches cost what that does (about 80 us at 1,000 hits) */
 
-QueryBufs *stc_query_bufs_new() { return new QueryBufs(); }
 
 uint64_t stc_query_bufs_growth(const QueryBufs *b, uint32_t nq, uint64_t cap) {
     uint64_t need = 0;
-    const uint64_t q_cap = b ? b->q_cap : 0, c_cap = b ? b->counters_cap : 0, h_cap = b ? b->hits_cap : 0;
-    if (nq > q_cap) need += (uint64_t)nq * sizeof(stc_query) * 3 / 2;
-    if (nq + 1ull > c_cap) need += (nq + 1ull) * 8 * 3 / 2;
+    const uint64_t h_cap = b ? b->hits_cap : 0, list = nq * (sizeof(stc_query) + 8ull) + 8;
+    if (list > (b ? b->batch.cap : 0)) need += list * 3 / 2;
     if (cap > h_cap) need += cap * sizeof(stc_hit) * 3 / 2;
     return need;
 }
 
 void stc_query_bufs_free(QueryBufs *b) {
     if (!b) return;
-    void *ptrs[] = {b->q, b->oh_key, b->oh_head, b->q_next, b->oq, b->g_start, b->g_list, b->filter, b->runs, b->cand,
-                    b->hits, b->counters, b->sort};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    b->batch.release();
+    b->runs.release();
+    if (b->res) (void)hipHostFree(b->res);
+    if (b->hits) (void)hipFree(b->hits);
+    if (b->sort) (void)hipFree(b->sort);
     for (int i = 0; i < 2; i++) {
         if (b->out[i]) (void)hipHostFree(b->out[i]);
         if (b->out_ev[i]) (void)hipEventDestroy(b->out_ev[i]);
@@ -121,12 +140,15 @@ static int grow(T **p, uint64_t *cap, uint64_t need) {
     *cap = nc;
     return 0;
 }
-template <typename T>
-static int grow32(T **p, uint32_t *cap, uint64_t need) {
-    uint64_t c = *cap;
-    int rc = grow(p, &c, need);
-    *cap = (uint32_t)std::min<uint64_t>(c, 0xFFFFFFFFu);
-    return rc;
+/* with room for an ordinary batch, so that a context's first one allocates nothing */
+QueryBufs *stc_query_bufs_new() {
+    QueryBufs *b = new QueryBufs();
+    (void)b->batch.begin(64u << 10);
+    (void)b->runs.begin(32u << 10);
+    if (hipHostMalloc((void **)&b->res, (QSORT_HOST * 7 + 4096) * 8, hipHostMallocDefault) == hipSuccess) b->res_cap = QSORT_HOST * 7 + 4096;
+    (void)grow(&b->hits, &b->hits_cap, 12u << 10);
+    (void)hipGetLastError(); /* what could not be had now is asked for by the batch that needs it */
+    return b;
 }
 
 /* The grid cell of a coordinate, the same arithmetic on the host (registration)
@@ -723,6 +745,14 @@ int stc_query_ctf_stats(const QueryRunDev &run, const stc_ctf_meta *host_ctfs, s
     return STC_OK;
 }
 
+/* the counters and the first hits (at most `most`) to host memory: one launch, and the only wait of a small batch */
+__global__ void k_q_finish(const unsigned long long *__restrict__ counters, uint32_t nq, const uint64_t *__restrict__ hits,
+                           uint64_t most, uint64_t *__restrict__ out) {
+    const uint64_t c = min<uint64_t>(counters[0], most), words = nq + 1ull + c * 7;
+    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += (uint64_t)gridDim.x * blockDim.x)
+        out[w] = w <= nq ? counters[w] : hits[w - nq - 1];
+}
+
 /* ---------------- the hits in order ---------------- */
 
 /* how a hit's (query, source, pid, target, start, end) is packed into sort keys */
@@ -840,24 +870,20 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         *n_hits = 0;
         return STC_OK;
     }
-    /* queries */
-    if (grow32(&B->q, &B->q_cap, nq) || grow(&B->counters, &B->counters_cap, (uint64_t)nq + 1) ||
-        grow(&B->hits, &B->hits_cap, std::max<uint64_t>(cap, 1)))
-        return stc_hip_fail(hipErrorOutOfMemory, "query buffers", __FILE__, __LINE__);
-    QCK(hipMemcpyAsync(B->q, q, nq * sizeof(stc_query), hipMemcpyHostToDevice, s));
-    QCK(hipMemsetAsync(B->counters, 0, ((uint64_t)nq + 1) * sizeof(unsigned long long), s));
-
     /* hash of the queried ids (object and pair queries) */
     std::vector<uint32_t> oq;
     for (uint32_t i = 0; i < nq; i++)
         if (q[i].kind == STC_Q_OID || q[i].kind == STC_Q_PAIR) oq.push_back(i);
     uint32_t bits = 0;
+    std::vector<uint32_t> key;
+    std::vector<int32_t> head, next;
     if (!oq.empty()) {
         bits = 6;
         while ((1ull << bits) < 2ull * oq.size()) bits++;
         const uint32_t size = 1u << bits, mask = size - 1;
-        std::vector<uint32_t> key(size, 0xFFFFFFFFu);
-        std::vector<int32_t> head(size, -1), next(nq, -1);
+        key.assign(size, 0xFFFFFFFFu);
+        head.assign(size, -1);
+        next.assign(nq, -1);
         for (size_t j = oq.size(); j-- > 0;) { /* insert in reverse: lists keep query order */
             uint32_t qi = oq[j], id = q[qi].oid, h = oid_slot(id, bits);
             while (key[h] != 0xFFFFFFFFu && key[h] != id) h = (h + 1) & mask;
@@ -865,15 +891,6 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
             next[qi] = head[h];
             head[h] = (int32_t)qi;
         }
-        uint32_t hc = B->oh_cap, nc = B->oh_cap;
-        if (grow32(&B->oh_key, &hc, size) || grow32(&B->oh_head, &nc, size) ||
-            grow32(&B->q_next, &B->qn_cap, nq) || grow32(&B->oq, &B->oq_cap, oq.size()))
-            return stc_hip_fail(hipErrorOutOfMemory, "query id hash", __FILE__, __LINE__);
-        B->oh_cap = std::min(hc, nc);
-        QCK(hipMemcpy(B->oh_key, key.data(), size * sizeof(uint32_t), hipMemcpyHostToDevice));
-        QCK(hipMemcpy(B->oh_head, head.data(), size * sizeof(int32_t), hipMemcpyHostToDevice));
-        QCK(hipMemcpy(B->q_next, next.data(), nq * sizeof(int32_t), hipMemcpyHostToDevice));
-        QCK(hipMemcpy(B->oq, oq.data(), oq.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
 
     /* grid of the range queries */
@@ -891,55 +908,67 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     std::vector<uint32_t> rq;
     for (uint32_t i = 0; i < nq; i++)
         if (q[i].kind == STC_Q_RANGE) rq.push_back(i);
-    if (!rq.empty()) {
-        std::vector<uint32_t> start(QGRID * QGRID + 1, 0), list;
-        std::vector<std::vector<uint32_t>> cells(QGRID * QGRID);
-        for (uint32_t qi : rq) {
+    std::vector<uint32_t> start, list;
+    if (!rq.empty()) { /* counted per cell, then listed in query order */
+        start.assign(QGRID * QGRID + 1, 0);
+        auto cells = [&](uint32_t qi, auto &&f) {
             const double *b = q[qi].box;
-            int cx0 = grid_cell(b[0], x0, ix), cx1 = grid_cell(b[2], x0, ix);
-            int cy0 = grid_cell(b[1], y0, iy), cy1 = grid_cell(b[3], y0, iy);
+            const int cx0 = grid_cell(b[0], x0, ix), cx1 = grid_cell(b[2], x0, ix);
+            const int cy0 = grid_cell(b[1], y0, iy), cy1 = grid_cell(b[3], y0, iy);
             for (int cy = cy0; cy <= cy1; cy++)
-                for (int cx = cx0; cx <= cx1; cx++) cells[cy * QGRID + cx].push_back(qi);
-        }
+                for (int cx = cx0; cx <= cx1; cx++) f(cy * QGRID + cx);
+        };
+        for (uint32_t qi : rq) cells(qi, [&](int c) { start[c + 1]++; });
         for (int c = 0; c < QGRID * QGRID; c++) {
-            start[c + 1] = start[c] + (uint32_t)cells[c].size();
-            if (!cells[c].empty()) cell_bits[c >> 5] |= 1u << (c & 31);
-            list.insert(list.end(), cells[c].begin(), cells[c].end());
+            if (start[c + 1]) cell_bits[c >> 5] |= 1u << (c & 31);
+            start[c + 1] += start[c];
         }
-        uint32_t gc = B->g_cap;
-        if (grow32(&B->g_list, &gc, std::max<size_t>(list.size(), 1)))
-            return stc_hip_fail(hipErrorOutOfMemory, "query grid", __FILE__, __LINE__);
-        B->g_cap = gc;
-        if (!B->g_start) QCK(hipMalloc((void **)&B->g_start, (QGRID * QGRID + 1) * sizeof(uint32_t)));
-        QCK(hipMemcpy(B->g_start, start.data(), start.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-        if (!list.empty()) QCK(hipMemcpy(B->g_list, list.data(), list.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        list.resize(start.back());
+        std::vector<uint32_t> at(start.begin(), start.end() - 1);
+        for (uint32_t qi : rq) cells(qi, [&](int c) { list[at[c]++] = qi; });
     }
 
-    if (grow32(&B->filter, &B->f_cap, filter.size()))
-        return stc_hip_fail(hipErrorOutOfMemory, "query filter", __FILE__, __LINE__);
-    QCK(hipMemcpy(B->filter, filter.data(), filter.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    /* one copy for all of it (each table was a copy of its own, waited for: 10 us and more a piece) */
+    uint64_t bytes = 0;
+    for (uint64_t b : std::initializer_list<uint64_t>{(nq + 1ull) * 8, nq * sizeof(stc_query), key.size() * 4, head.size() * 4,
+                                                      next.size() * 4, oq.size() * 4, start.size() * 4, list.size() * 4, filter.size() * 4})
+        bytes += QueryUpload::room(b);
+    const uint64_t most = hits ? std::min<uint64_t>(cap, QSORT_HOST) : 0, res_words = nq + 1ull + most * 7;
+    if (B->batch.begin(bytes) || grow(&B->hits, &B->hits_cap, std::max<uint64_t>(cap, 1)))
+        return stc_hip_fail(hipErrorOutOfMemory, "query buffers", __FILE__, __LINE__);
+    if (B->res_cap < res_words) {
+        if (B->res) (void)hipHostFree(B->res);
+        B->res = nullptr;
+        B->res_cap = 0;
+        QCK(hipHostMalloc((void **)&B->res, (res_words + res_words / 2) * 8, hipHostMallocDefault));
+        B->res_cap = res_words + res_words / 2;
+    }
+    QueryUpload &U = B->batch;
     QDev Q;
-    Q.filter = B->filter;
+    unsigned long long *counters = U.put((const unsigned long long *)nullptr, nq + 1ull); /* total hits, then per query */
+    Q.q = U.put(q, nq);
+    Q.oh_key = U.put(key.data(), key.size());
+    Q.oh_head = U.put(head.data(), head.size());
+    Q.q_next = U.put(next.data(), next.size());
+    const uint32_t *oq_dev = U.put(oq.data(), oq.size());
+    Q.g_start = U.put(start.data(), start.size());
+    Q.g_list = U.put(list.data(), list.size());
+    Q.filter = U.put(filter.data(), filter.size());
     Q.f_bits = f_bits;
-    Q.q = B->q;
-    Q.oh_key = B->oh_key;
-    Q.oh_head = B->oh_head;
-    Q.q_next = B->q_next;
     Q.oh_bits = bits;
     Q.n_range = (uint32_t)rq.size();
-    Q.g_start = B->g_start;
-    Q.g_list = B->g_list;
     Q.x0 = x0;
     Q.y0 = y0;
     Q.ix = ix;
     Q.iy = iy;
     Q.hits = B->hits;
     Q.cap = hits ? cap : 0;
-    Q.n_hits = B->counters;
-    Q.counts = B->counters + 1;
+    Q.n_hits = counters;
+    Q.counts = counters + 1;
     Q.nq = nq;
     Q.lds = nq <= QLDS;
     const size_t q_scan_lds = ((Q.lds ? nq : 0) + filter.size()) * sizeof(uint32_t);
+    QCK(U.send(s));
     /* counts a planner adds without a kernel (CTFs wholly inside a range query) */
     std::vector<unsigned long long> planned(nq, 0);
 
@@ -958,16 +987,8 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     /* runs */
     const uint32_t nruns = (uint32_t)st.runs.size();
     if (nruns) {
-        if (grow32(&B->runs, &B->runs_cap, nruns))
-            return stc_hip_fail(hipErrorOutOfMemory, "query runs", __FILE__, __LINE__);
-        QCK(hipMemcpy(B->runs, st.runs.data(), nruns * sizeof(QueryRunDev), hipMemcpyHostToDevice));
-        if (!oq.empty()) {
-            hipLaunchKernelGGL(k_q_run_oid, dim3(blocks((uint64_t)oq.size() * nruns * STC_WAVE, 256)), dim3(256), 0, s, B->runs,
-                               nruns, B->oq, (uint32_t)oq.size(), st.num_objects, Q);
-            QCK(hipGetLastError());
-        }
-        if (!rq.empty()) {
-            std::vector<uint4> cand;
+        std::vector<uint4> cand;
+        if (!rq.empty()) { /* while the scans run */
             for (uint32_t qi : rq) {
                 const stc_query &qq = q[qi];
                 for (uint32_t r = 0; r < nruns; r++) {
@@ -996,20 +1017,29 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
                     if (st.runs[r].n_tail) cand.push_back(make_uint4(qi, r, 0xFFFFFFFFu, 0));
                 }
             }
-            if (!cand.empty()) {
-                if (grow(&B->cand, &B->cand_cap, cand.size()))
-                    return stc_hip_fail(hipErrorOutOfMemory, "query candidates", __FILE__, __LINE__);
-                QCK(hipMemcpy(B->cand, cand.data(), cand.size() * sizeof(uint4), hipMemcpyHostToDevice));
-                hipLaunchKernelGGL(k_q_run_range, dim3((uint32_t)cand.size()), dim3(256), 0, s, B->runs, B->cand, Q);
-                QCK(hipGetLastError());
-            }
+        }
+        if (!oq.empty() || !cand.empty()) {
+            if (B->runs.begin(QueryUpload::room(nruns * sizeof(QueryRunDev)) + QueryUpload::room(cand.size() * sizeof(uint4))))
+                return stc_hip_fail(hipErrorOutOfMemory, "query runs", __FILE__, __LINE__);
+            const QueryRunDev *runs = B->runs.put(st.runs.data(), nruns);
+            const uint4 *cand_dev = B->runs.put(cand.data(), cand.size());
+            QCK(B->runs.send(s));
+            if (!oq.empty())
+                hipLaunchKernelGGL(k_q_run_oid, dim3(blocks((uint64_t)oq.size() * nruns * STC_WAVE, 256)), dim3(256), 0, s, runs,
+                                   nruns, oq_dev, (uint32_t)oq.size(), st.num_objects, Q);
+            QCK(hipGetLastError());
+            if (!cand.empty())
+                hipLaunchKernelGGL(k_q_run_range, dim3((uint32_t)cand.size()), dim3(256), 0, s, runs, cand_dev, Q);
+            QCK(hipGetLastError());
         }
     }
 
     /* results */
-    std::vector<unsigned long long> cnt((uint64_t)nq + 1);
-    QCK(hipMemcpyAsync(cnt.data(), B->counters, cnt.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_q_finish, dim3(std::min<uint32_t>(blocks(res_words, 256), 256)), dim3(256), 0, s, counters, nq,
+                       (const uint64_t *)B->hits, most, B->res);
+    QCK(hipGetLastError());
     QCK(hipStreamSynchronize(s));
+    const uint64_t *cnt = B->res;
     uint64_t total = 0; /* the hits of the queries that store theirs */
     for (uint32_t i = 0; i < nq; i++) {
         const uint64_t ci = cnt[i + 1] + planned[i];
@@ -1024,7 +1054,8 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         if (rc) return rc;
     }
     if (stored && hits && !sorted) {
-        QCK(hipMemcpy(hits, B->hits, stored * sizeof(stc_hit), hipMemcpyDeviceToHost));
+        if (stored <= most) memcpy(hits, cnt + nq + 1, stored * sizeof(stc_hit));
+        else QCK(hipMemcpy(hits, B->hits, stored * sizeof(stc_hit), hipMemcpyDeviceToHost));
         std::sort(hits, hits + stored, [](const stc_hit &a, const stc_hit &b) {
             if (a.query != b.query) return a.query < b.query;
             if (a.source != b.source) return a.source < b.source;

@@ -38,6 +38,7 @@ HIT_DTYPE = np.dtype([("query", "<u4"), ("pid", "<u4"), ("target", "<u4"), ("sta
                       ("source", "<u4"), ("mbr", "<f8", (4,))])
 Q_OID, Q_RANGE, Q_PAIR = 1, 2, 3
 QF_COUNT = 1  # STC_QF_COUNT: count the query's hits, store none
+FETCH_ROWS = 1 << 14  # hits a query without a capacity has room for at first
 # stc_meeting_unit: the reference's 32-byte meeting_unit (src/tracing/workbench.h:62-83)
 MEETING_UNIT_DTYPE = np.dtype([("key", "<u8"), ("start", "<u4"), ("end", "<u4"), ("mbr", "<f4", (4,))])
 assert MEETING_UNIT_DTYPE.itemsize == 32
@@ -252,13 +253,26 @@ class Pipeline:
         `into`: a HIT_DTYPE array of at least cap entries to store them in."""
         q = np.ascontiguousarray(q, dtype=QUERY_DTYPE)
         counts = np.zeros(len(q), dtype=np.uint64)
-        n = C.c_uint64()
         if cap is None:
-            _check(self.lib.stc_query_batch(self.ctx, _ptr(q), len(q), None, 0, C.byref(n), _ptr(counts)), self.ctx)
-            cap = n.value
+            hits = self._fetch(FETCH_ROWS, into, lambda h, n: self.lib.stc_query_batch(
+                self.ctx, _ptr(q), len(q), _ptr(h), len(h), C.byref(n), _ptr(counts)))
+            return hits, counts
+        n = C.c_uint64()
         hits = into if into is not None and len(into) >= cap else np.zeros(cap, dtype=HIT_DTYPE)
         _check(self.lib.stc_query_batch(self.ctx, _ptr(q), len(q), _ptr(hits), cap, C.byref(n), _ptr(counts)), self.ctx)
         return hits[:min(n.value, cap)], counts
+
+    def _fetch(self, rows, into, call):
+        """all hits of call(buffer, n): one call where they fit in `into`, or
+        in a first guess of `rows`, else a second with room for all"""
+        n = C.c_uint64()
+        hits = into if into is not None and len(into) else np.empty(rows, dtype=HIT_DTYPE)
+        _check(call(hits, n), self.ctx)
+        if n.value <= len(hits):
+            return hits[:n.value] if hits is into else hits[:n.value].copy()
+        hits = np.empty(n.value, dtype=HIT_DTYPE)
+        _check(call(hits, n), self.ctx)
+        return hits[:min(n.value, len(hits))]
 
     def query_at(self, q, into):
         """a query batch over the last published state (safe while another
@@ -276,12 +290,8 @@ class Pipeline:
         """established live contacts of the given objects (stc_live_search);
         hits as HIT_DTYPE with `query` the index into pids"""
         pids = np.ascontiguousarray(pids, dtype=np.uint32)
-        n = C.c_uint64()
-        _check(self.lib.stc_live_search(self.ctx, _ptr(pids), len(pids), None, 0, C.byref(n)), self.ctx)
-        hits = np.zeros(n.value, dtype=HIT_DTYPE)
-        _check(self.lib.stc_live_search(self.ctx, _ptr(pids), len(pids), _ptr(hits), len(hits), C.byref(n)),
-               self.ctx)
-        return hits
+        return self._fetch(1024 + 8 * len(pids), None, lambda h, n: self.lib.stc_live_search(
+            self.ctx, _ptr(pids), len(pids), _ptr(h), len(h), C.byref(n)))
 
     def dump_run(self, i, directory, prefix, ctb):
         """write run i in the reference's file layout (stc_dump_run)"""
