@@ -385,13 +385,15 @@ __global__ void k_amb_gather(const double2 *__restrict__ xy, const uint2 *__rest
     out[i] = make_double4(p.x, p.y, q.x, q.y);
 }
 
-/* leaf-ordered SoA and each point's rank within its leaf */
+/* leaf-ordered SoA and each point's rank within its leaf; and, a thread per leaf, the points beyond its buffer */
 __global__ void k_gather(const double2 *__restrict__ xy, const double *__restrict__ dlon,
                          const uint32_t *__restrict__ lp, const uint32_t *__restrict__ pt_leaf,
                          const uint32_t *__restrict__ leaf_start, uint32_t n, double2 *__restrict__ lxy,
                          double *__restrict__ ld, uint32_t *__restrict__ pt_rank,
-                         uint32_t *__restrict__ lleaf) {
+                         uint32_t *__restrict__ lleaf, const uint32_t *__restrict__ leaf_count, uint32_t nl, uint32_t buf,
+                         Counters *cnt) {
     uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < nl && leaf_count[j] > buf) atomicAdd(&cnt->overflow, leaf_count[j] - buf);
     if (j >= n) return;
     uint32_t p = lp[j];
     double2 q = xy[p];
@@ -402,51 +404,22 @@ __global__ void k_gather(const double2 *__restrict__ xy, const double *__restric
     lleaf[j] = L;
 }
 
-/* each point's cross units in leaf order (first unit, count) */
-__global__ void k_units_lorder(const uint32_t *__restrict__ lp, const uint32_t *__restrict__ uoffset,
-                               const uint32_t *__restrict__ ucount, uint32_t n, uint2 *__restrict__ lunits) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t p = lp[j];
-    lunits[j] = make_uint2(uoffset[p], ucount[p]);
-}
-
-__global__ void k_overflow(const uint32_t *leaf_count, uint32_t nl, uint32_t buf, Counters *cnt) {
-    uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t over = 0;
-    if (l < nl && leaf_count[l] > buf) over = leaf_count[l] - buf;
-    if (over) atomicAdd(&cnt->overflow, over);
-}
-
 /* ------------------------------------------------------------------ */
-/* border lookup (two passes)                                          */
+/* border lookup                                                       */
 /* ------------------------------------------------------------------ */
 
-/* One thread per point, points in leaf order: a wave's points share a leaf
- * and mostly the same subtrees, so their descents stay together. Outputs are
- * per point id (count[p], units from offset[p]). */
-template <bool EMIT>
-__global__ void k_lookup(const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy,
-                         const double *__restrict__ ld, uint32_t n,
-                         const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r, double band,
-                         uint32_t *__restrict__ count, const uint32_t *__restrict__ offset,
-                         uint2 *__restrict__ units, Counters *cnt) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t p = lp[j];
-    uint32_t lv = pt_lv[p];
-    if (lv == 0xFFFFFFFFu) {
-        if (!EMIT) count[p] = 0;
-        return;
-    }
-    const double2 q = lxy[j];
-    const double dl = ld[j];
+#define LK_KEPT 4u /* leaves of a point that the lookup keeps for the emission */
+
+/* the leaves within reach of a border point on its top or right: f(leaf) in
+ * descent order below lv; returns how many box distances lie in the guard
+ * band, sets *full when the stack was */
+template <class F>
+__device__ inline uint32_t lookup_leaves(double2 q, double dl, uint32_t lv, const Node *__restrict__ nodes, double r,
+                                         double band, bool *full, F f) {
     uint32_t stk[STACK_DEPTH];
     int sp = 0;
     stk[sp++] = lv;
-    uint32_t found = 0, amb = 0;
-    bool full = false;
-    uint32_t out = EMIT ? offset[p] : 0;
+    uint32_t amb = 0;
     while (sp > 0) {
         uint32_t cur = stk[--sp];
         const Node &nd = nodes[cur];
@@ -457,22 +430,86 @@ __global__ void k_lookup(const uint32_t *__restrict__ lp, const double2 *__restr
             if (fabs(d - r) <= band) amb++;
             if (d <= r) {
                 if (ch.type == T_LEAF) {
-                    if (q.y < ch.lo1 || (q.y < ch.hi1 && q.x < ch.lo0)) {
-                        if (EMIT) units[out + found] = make_uint2(p, ch.leaf);
-                        found++;
-                    }
+                    if (q.y < ch.lo1 || (q.y < ch.hi1 && q.x < ch.lo0)) f(ch.leaf);
                 } else if (sp < STACK_DEPTH) {
                     stk[sp++] = c;
                 } else {
-                    full = true;
+                    *full = true;
                 }
             }
         }
     }
-    if (!EMIT) {
-        count[p] = found;
+    return amb;
+}
+
+/* One thread per point, points in leaf order: a wave's points share a leaf
+ * and mostly the same subtrees, so their descents stay together. count[p] per
+ * point id; the first LK_KEPT leaves of the point at place j in kept[j]. */
+__global__ void k_lookup(const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy,
+                         const double *__restrict__ ld, uint32_t n,
+                         const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r, double band,
+                         uint32_t *__restrict__ count, uint4 *__restrict__ kept, Counters *cnt) {
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const uint32_t p = lp[j];
+    uint32_t lv = pt_lv[p];
+    uint32_t found = 0;
+    if (lv != 0xFFFFFFFFu) {
+        bool full = false;
+        uint4 k = make_uint4(0, 0, 0, 0);
+        const uint32_t amb = lookup_leaves(lxy[j], ld[j], lv, nodes, r, band, &full, [&](uint32_t leaf) {
+            if (found == 0) k.x = leaf;
+            else if (found == 1) k.y = leaf;
+            else if (found == 2) k.z = leaf;
+            else if (found == 3) k.w = leaf;
+            found++;
+        });
+        if (found) kept[j] = k;
         if (amb) atomicAdd(&cnt->ambiguous_nodes, (unsigned long long)amb);
         if (full) atomicAdd(&cnt->lookup_overflow, 1u);
+    }
+    count[p] = found;
+}
+
+/* The cross units (point, leaf) in point order, and all that is kept of each:
+ * the leaf and the point for the reverse lists, the leaf's kept members above
+ * the point (an index range into the leaf-ordered arrays); and each point's
+ * first unit and count in leaf order. The leaves come from the lookup; a point
+ * with more than it keeps descends again. (A second descent for every point,
+ * then a pass each for the reverse lists, the ranges and the leaf order: 23 +
+ * 10 us at 50k objects, 97 + 44 at 1M; 6.5 and 54 us so.) */
+__global__ void k_units_emit(const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy, const double *__restrict__ ld,
+                             uint32_t n, const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r,
+                             double band, const uint32_t *__restrict__ count, const uint32_t *__restrict__ offset,
+                             const uint4 *__restrict__ kept, const uint32_t *__restrict__ leaf_start,
+                             const uint32_t *__restrict__ leaf_count, uint32_t buf, uint2 *__restrict__ units,
+                             uint32_t *__restrict__ rev_leaf, uint32_t *__restrict__ rev_pid, uint2 *__restrict__ urange,
+                             uint2 *__restrict__ lunits) {
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const uint32_t p = lp[j], c = count[p];
+    uint32_t u = offset[p];
+    lunits[j] = make_uint2(u, c);
+    if (!c) return;
+    auto emit = [&](uint32_t leaf) {
+        uint32_t s2 = leaf_count[leaf];
+        if (s2 > buf) s2 = buf;
+        const uint32_t st2 = leaf_start[leaf], m0 = lower_bound_u32(lp + st2, s2, p + 1);
+        units[u] = make_uint2(p, leaf);
+        rev_leaf[u] = leaf;
+        rev_pid[u] = p;
+        urange[u] = make_uint2(st2 + m0, s2 - m0);
+        u++;
+    };
+    if (c <= LK_KEPT) {
+        const uint4 k = kept[j];
+        emit(k.x);
+        if (c > 1) emit(k.y);
+        if (c > 2) emit(k.z);
+        if (c > 3) emit(k.w);
+    } else {
+        bool full = false;
+        lookup_leaves(lxy[j], ld[j], pt_lv[p], nodes, r, band, &full, emit);
     }
 }
 
@@ -643,54 +680,26 @@ __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const Pair
     }
 }
 
-/* split the cross units into (leaf, pid) key/value arrays for the reverse lists */
-__global__ void k_units_split(const uint2 *__restrict__ units, uint32_t nu, uint32_t *__restrict__ leaf,
-                              uint32_t *__restrict__ pid) {
+/* The reverse lists' finish: the border points' data in list order, so that
+ * owners read it coalesced, and each leaf's first entry (rev_start[n_leaves] = nr). */
+__global__ void k_rev_finish(const uint32_t *__restrict__ rev_leaf, const uint32_t *__restrict__ rev_pid, uint32_t nr,
+                             uint32_t n_leaves, const double2 *__restrict__ xy, const double *__restrict__ dlon,
+                             RevPt *__restrict__ rev, double *__restrict__ rev_dl, uint32_t *__restrict__ rev_start) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nu) return;
-    const uint2 u = units[i];
-    leaf[i] = u.y;
-    pid[i] = u.x;
-}
-
-/* each leaf's first entry in the leaf-sorted reverse lists (rev_start[n_leaves] = nu) */
-__global__ void k_rev_starts(const uint32_t *__restrict__ sorted_leaf, uint32_t nu, uint32_t n_leaves,
-                             uint32_t *__restrict__ rev_start) {
-    const uint32_t L = blockIdx.x * blockDim.x + threadIdx.x;
-    if (L <= n_leaves) rev_start[L] = lower_bound_u32(sorted_leaf, nu, L);
-}
-
-/* the border points' data in reverse-list order, so that owners read it coalesced */
-__global__ void k_rev_gather(const uint32_t *__restrict__ rev_pid, uint32_t nr, const double2 *__restrict__ xy,
-                             const double *__restrict__ dlon, RevPt *__restrict__ rev, double *__restrict__ rev_dl) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nr) return;
-    const uint32_t p = rev_pid[i];
-    const double2 q = xy[p];
-    const double d = dlon[p];
-    RevPt r;
-    r.x = q.x;
-    r.y = q.y;
-    r.il = 1.0 / d; /* the reciprocal of dlon[p], as the owners' loops compute theirs */
-    r.pid = p;
-    r.pad = 0;
-    rev[i] = r;
-    rev_dl[i] = d;
-}
-
-/* per cross unit (p, leaf): the leaf's kept members above p, as an index range
- * into the leaf-ordered arrays */
-__global__ void k_unit_ranges(const uint2 *__restrict__ units, uint32_t nu, const uint32_t *__restrict__ leaf_start,
-                              const uint32_t *__restrict__ leaf_count, const uint32_t *__restrict__ lp, uint32_t buf,
-                              uint2 *__restrict__ urange) {
-    const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= nu) return;
-    const uint2 un = units[u];
-    uint32_t s2 = leaf_count[un.y];
-    if (s2 > buf) s2 = buf;
-    const uint32_t st2 = leaf_start[un.y];
-    const uint32_t m0 = lower_bound_u32(lp + st2, s2, un.x + 1);
-    urange[u] = make_uint2(st2 + m0, s2 - m0);
+    if (i < nr) {
+        const uint32_t p = rev_pid[i];
+        const double2 q = xy[p];
+        const double d = dlon[p];
+        RevPt r;
+        r.x = q.x;
+        r.y = q.y;
+        r.il = 1.0 / d; /* the reciprocal of dlon[p], as the owners' loops compute theirs */
+        r.pid = p;
+        r.pad = 0;
+        rev[i] = r;
+        rev_dl[i] = d;
+    }
+    if (i <= n_leaves) rev_start[i] = lower_bound_u32(rev_leaf, nr, i);
 }
 
 /* per point in leaf order: its later kept members in its leaf, and (when it is
@@ -3092,19 +3101,19 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     CKRC(stc_exclusive_scan_u32(c->leaf_count.p, c->leaf_start.p, n_leaves, nullptr, c->temp.p, s));
     CKRC(sort_pairs((const uint32_t *)c->pt_leaf.p, (const uint32_t *)nullptr, c->lkeys, c->lp, c->codes_alt, c->idx_alt, n,
                     std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
-    hipLaunchKernelGGL(k_gather, dim3(blocks_for(n, 256)), dim3(256), 0, s, xy, c->dlon.p, c->lp.p, c->pt_leaf.p,
-                       c->leaf_start.p, n, c->lxy.p, c->ld.p, c->pt_rank.p, c->lleaf.p);
-    c->lp_valid = true; /* lp: a permutation of the points, in this step's leaf order */
-    hipLaunchKernelGGL(k_overflow, dim3(blocks_for(n_leaves, 256)), dim3(256), 0, s, c->leaf_count.p, n_leaves,
+    hipLaunchKernelGGL(k_gather, dim3(blocks_for(std::max(n, n_leaves), 256)), dim3(256), 0, s, xy, c->dlon.p, c->lp.p, c->pt_leaf.p,
+                       c->leaf_start.p, n, c->lxy.p, c->ld.p, c->pt_rank.p, c->lleaf.p, (const uint32_t *)c->leaf_count.p, n_leaves,
                        c->buf, cnt);
+    c->lp_valid = true; /* lp: a permutation of the points, in this step's leaf order */
     CK(hipGetLastError());
     CK(hipEventRecord(c->ev[1], s));
 
     /* 6: border lookup (count, scan, emit) */
     double r = c->cfg.reach_distance;
-    hipLaunchKernelGGL(k_lookup<false>, dim3(blocks_for(n, 128)), dim3(128), 0, s, (const uint32_t *)c->lp.p,
+    uint4 *kept = c->prange.p; /* the lookup's leaves, until k_point_ranges fills it */
+    hipLaunchKernelGGL(k_lookup, dim3(blocks_for(n, 128)), dim3(128), 0, s, (const uint32_t *)c->lp.p,
                        (const double2 *)c->lxy.p, (const double *)c->ld.p, n, (const Node *)tree_nodes(c),
-                       c->pt_lv.p, r, c->band, c->ucount.p, (const uint32_t *)nullptr, (uint2 *)nullptr, cnt);
+                       (const uint32_t *)c->pt_lv.p, r, c->band, c->ucount.p, kept, cnt);
     CK(hipGetLastError());
     uint32_t *units_total = (uint32_t *)((char *)cnt + offsetof(Counters, units));
     CKRC(stc_exclusive_scan_u32(c->ucount.p, c->uoffset.p, n, units_total, c->temp.p, s));
@@ -3114,45 +3123,35 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     if (h.lookup_overflow) return fail(c, STC_E_CAPACITY, "border lookup: node stack depth exceeded");
     uint64_t n_units = (uint32_t)h.units;
     if (n_units >= (1u << 30)) return fail(c, STC_E_CAPACITY, "2^30 or more cross units in one step");
-    if (c->units.ensure(n_units + 1)) return fail(c, STC_E_CAPACITY, "unit buffer allocation failed");
-    hipLaunchKernelGGL(k_lookup<true>, dim3(blocks_for(n, 128)), dim3(128), 0, s, (const uint32_t *)c->lp.p,
+    if (c->units.ensure(n_units + 1) || c->urange.ensure(n_units + 1) || c->rev_leaf.ensure(n_units + 1) ||
+        c->rev_pid.ensure(n_units + 1))
+        return fail(c, STC_E_CAPACITY, "unit buffer allocation failed");
+    hipLaunchKernelGGL(k_units_emit, dim3(blocks_for(n, 128)), dim3(128), 0, s, (const uint32_t *)c->lp.p,
                        (const double2 *)c->lxy.p, (const double *)c->ld.p, n, (const Node *)tree_nodes(c),
-                       c->pt_lv.p, r, c->band, c->ucount.p, (const uint32_t *)c->uoffset.p, c->units.p, cnt);
+                       (const uint32_t *)c->pt_lv.p, r, c->band, (const uint32_t *)c->ucount.p, (const uint32_t *)c->uoffset.p,
+                       (const uint4 *)kept, (const uint32_t *)c->leaf_start.p, (const uint32_t *)c->leaf_count.p, c->buf,
+                       c->units.p, c->rev_leaf.p, c->rev_pid.p, c->urange.p, c->lunits.p);
     CK(hipGetLastError());
     CK(hipEventRecord(c->ev[2], s));
 
     /* 7: reverse cross units: per leaf, the border points with a cross unit to it, by pid */
-    if (c->rev_leaf.ensure(n_units + 1) || c->rev_pid.ensure(n_units + 1) || c->rev_leaf_alt.ensure(n_units + 1) ||
+    if (c->rev_leaf_alt.ensure(n_units + 1) ||
         c->rev.ensure(n_units + 1) || c->rev_dl.ensure(n_units + 1) ||
         c->rev_pid_alt.ensure(n_units + 1) ||
         c->rev_start.ensure(n_leaves + 1ull) ||
         c->temp.ensure(stc_radix_temp_words((uint32_t)std::max<uint64_t>(std::max<uint64_t>(n_units, n),
                                                                           std::max<size_t>(c->nodes.cap, c->sch.cap))) + 64))
         return fail(c, STC_E_CAPACITY, "reverse unit buffers");
-    if (n_units) {
-        hipLaunchKernelGGL(k_units_split, dim3(blocks_for(n_units, 256)), dim3(256), 0, s, c->units.p,
-                           (uint32_t)n_units, c->rev_leaf.p, c->rev_pid.p);
-        CK(hipGetLastError());
+    if (n_units)
         CKRC(sort_pairs((const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, c->rev_leaf, c->rev_pid, c->rev_leaf_alt,
                         c->rev_pid_alt, (uint32_t)n_units, std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
-        hipLaunchKernelGGL(k_rev_gather, dim3(blocks_for(n_units, 256)), dim3(256), 0, s, (const uint32_t *)c->rev_pid.p,
-                           (uint32_t)n_units, xy, (const double *)c->dlon.p, c->rev.p,
-                           c->rev_dl.p);
-        CK(hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_rev_starts, dim3(blocks_for(n_leaves + 1ull, 256)), dim3(256), 0, s,
-                       (const uint32_t *)c->rev_leaf.p, (uint32_t)n_units, n_leaves, c->rev_start.p);
+    hipLaunchKernelGGL(k_rev_finish, dim3(blocks_for(std::max<uint64_t>(n_units, n_leaves + 1ull), 256)), dim3(256), 0, s,
+                       (const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, (uint32_t)n_units, n_leaves, xy,
+                       (const double *)c->dlon.p, c->rev.p, c->rev_dl.p, c->rev_start.p);
     CK(hipGetLastError());
 
     /* 8: the pairs owner by owner: count (a band combination reserves a slot),
      * the band decided on the host, segment offsets, write */
-    hipLaunchKernelGGL(k_units_lorder, dim3(blocks_for(n, 256)), dim3(256), 0, s, (const uint32_t *)c->lp.p,
-                       (const uint32_t *)c->uoffset.p, (const uint32_t *)c->ucount.p, n, c->lunits.p);
-    if (c->urange.ensure(n_units + 1)) return fail(c, STC_E_CAPACITY, "unit ranges");
-    if (n_units)
-        hipLaunchKernelGGL(k_unit_ranges, dim3(blocks_for(n_units, 256)), dim3(256), 0, s, (const uint2 *)c->units.p,
-                           (uint32_t)n_units, (const uint32_t *)c->leaf_start.p, (const uint32_t *)c->leaf_count.p,
-                           (const uint32_t *)c->lp.p, c->buf, c->urange.p);
     hipLaunchKernelGGL(k_point_ranges, dim3(blocks_for(n, 256)), dim3(256), 0, s, (const uint32_t *)c->lp.p,
                        (const uint32_t *)c->lleaf.p, n, (const uint32_t *)c->leaf_start.p,
                        (const uint32_t *)c->leaf_count.p, (const uint32_t *)c->rev_start.p,
