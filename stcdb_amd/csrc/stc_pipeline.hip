@@ -81,7 +81,7 @@ int stc_hip_fail(hipError_t e, const char *expr, const char *file, int line) {
 /* device structures                                                   */
 /* ------------------------------------------------------------------ */
 
-struct FrontierItem { uint32_t node, code; };
+struct FrontierItem { uint32_t node, code, lo, hi; }; /* a branch block and its range of the sorted cell codes */
 
 struct PairHit {              /* 24 B: key and the float MBR of the two positions (replayed meeting units) */
     unsigned long long key;
@@ -213,57 +213,48 @@ __device__ inline uint32_t lower_bound_u32(const uint32_t *a, uint32_t n, uint32
     return lo;
 }
 
-__global__ void k_tree_root(Node *nodes, MapBox m, FrontierItem *frontier, Counters *cnt, uint32_t n, uint32_t cap) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    Node nd;
-    block_box(nd, m, 0, 0, 1);
-    nd.type = T_BRANCH;
-    nd.leaf = 0;
-    nd.code = 0;
-    nd.level = NLEVELS - 1;
-    for (int c = 0; c < 4; c++) nd.child[c] = 0;
-    nodes[0] = nd;
-    cnt->nodes = 1;
-    cnt->leaves = 0;
-    for (int l = 0; l <= NLEVELS; l++) cnt->frontier[l] = 0;
-    if (n > cap) {
-        frontier[0].node = 0;
-        frontier[0].code = 0;
-        cnt->frontier[NLEVELS - 1] = 1;
-    }
-}
-
-/* expand the branch blocks of level L (L >= 1): each of the four sub-blocks
- * becomes a branch when it holds more than cap points, else a halving leaf */
-__global__ void k_tree_level(Node *nodes, MapBox m, const uint32_t *sorted_codes, uint32_t n, uint32_t cap, int L,
-                             const FrontierItem *fin, FrontierItem *fout, Counters *cnt, uint32_t node_cap,
-                             uint32_t front_cap) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= cnt->frontier[L]) return;
-    FrontierItem f = fin[i];
+/* Expand a branch block of level L (L >= 1): each of its four sub-blocks
+ * becomes a branch when it holds more than cap points, else a halving leaf.
+ * The sub-blocks' counts come from three searches inside the block's own range
+ * of the sorted codes. take_nodes(), take_leaves(k) and take_front(k) give the
+ * first of as many new entries; false: the node or frontier arrays are full. */
+template <class N, class F, class T>
+__device__ inline bool expand_block(FrontierItem f, Node *nodes, MapBox m, const uint32_t *sorted_codes, uint32_t cap, int L,
+                                    FrontierItem *fout, uint32_t *leaf_node, uint32_t node_cap, uint32_t front_cap,
+                                    N take_nodes, F take_leaves, T take_front) {
     Node parent = nodes[f.node];
     int Lc = L - 1;
     uint32_t xdim = ONE_DIM >> Lc;
-    uint32_t child_ids[4];
-    uint32_t nb = 0;
+    uint32_t nb = 0, at[5] = {f.lo, 0, 0, 0, f.hi};
     bool is_branch[4];
+    { /* the three searches side by side: one read's latency a halving, not three */
+        uint32_t end[4];
+        for (int c = 1; c < 4; c++) {
+            at[c] = f.lo;
+            end[c] = f.hi;
+        }
+        for (uint32_t span = f.hi - f.lo; span; span >>= 1) { /* halvings enough for f.hi - f.lo + 1 places */
+            uint32_t v[4];
+            for (int c = 1; c < 4; c++) v[c] = sorted_codes[min((at[c] + end[c]) >> 1, f.hi - 1)];
+            for (int c = 1; c < 4; c++) {
+                if (at[c] >= end[c]) continue;
+                const uint32_t mid = (at[c] + end[c]) >> 1;
+                if (v[c] < ((f.code << 2) | (uint32_t)c) << (2 * Lc)) at[c] = mid + 1;
+                else end[c] = mid;
+            }
+        }
+    }
     for (int c = 0; c < 4; c++) {
-        uint32_t sub = (f.code << 2) | (uint32_t)c;
-        uint32_t lo = sub << (2 * Lc);
-        uint32_t a = lower_bound_u32(sorted_codes, n, lo);
-        uint32_t b = lower_bound_u32(sorted_codes, n, lo + (1u << (2 * Lc)));
-        is_branch[c] = (b - a) > cap;
+        is_branch[c] = at[c + 1] - at[c] > cap;
         nb += is_branch[c];
     }
-    uint32_t base = atomicAdd(&cnt->nodes, 4u);
-    if (base + 4 > node_cap) { atomicAdd(&cnt->table_fail, 1u); return; }
-    uint32_t nleaf = 4 - nb;
-    uint32_t lbase = nleaf ? atomicAdd(&cnt->leaves, nleaf) : 0;
-    uint32_t fbase = nb ? atomicAdd(&cnt->frontier[Lc], nb) : 0;
-    if (fbase + nb > front_cap) { atomicAdd(&cnt->table_fail, 1u); return; }
+    uint32_t base = take_nodes();
+    if (base + 4 > node_cap) return false;
+    uint32_t lbase = nb < 4 ? take_leaves(4 - nb) : 0;
+    uint32_t fbase = nb ? take_front(nb) : 0;
+    if (fbase + nb > front_cap) return false;
     for (int c = 0; c < 4; c++) {
         uint32_t id = base + c;
-        child_ids[c] = id;
         Node nd;
         uint32_t sub = (f.code << 2) | (uint32_t)c;
         for (int k = 0; k < 4; k++) nd.child[k] = 0;
@@ -271,32 +262,29 @@ __global__ void k_tree_level(Node *nodes, MapBox m, const uint32_t *sorted_codes
             block_box(nd, m, compact1by1(sub), compact1by1(sub >> 1), xdim);
             nd.type = T_BRANCH;
             nd.leaf = 0;
-            nd.code = sub;
-            nd.level = Lc;
-            fout[fbase].node = id;
-            fout[fbase].code = sub;
-            fbase++;
+            fout[fbase++] = FrontierItem{id, sub, at[c], at[c + 1]};
         } else {
             halving_leaf(nd, parent, c);
             nd.type = T_LEAF;
-            nd.leaf = lbase++;
-            nd.code = sub;
-            nd.level = Lc;
+            nd.leaf = lbase;
+            leaf_node[lbase++] = id;
         }
+        nd.code = sub;
+        nd.level = Lc;
         nodes[id] = nd;
+        nodes[f.node].child[c] = id;
     }
-    for (int c = 0; c < 4; c++) nodes[f.node].child[c] = child_ids[c];
+    return true;
 }
 
-/* finest level: each overfull cell becomes a branch of four halving leaves */
-__global__ void k_tree_finest(Node *nodes, const FrontierItem *fin, Counters *cnt, uint32_t node_cap) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= cnt->frontier[0]) return;
-    FrontierItem f = fin[i];
+/* finest level: an overfull cell becomes a branch of four halving leaves */
+template <class N, class F>
+__device__ inline bool expand_cell(FrontierItem f, Node *nodes, uint32_t *leaf_node, uint32_t node_cap, N take_nodes,
+                                   F take_leaves) {
     Node parent = nodes[f.node];
-    uint32_t base = atomicAdd(&cnt->nodes, 4u);
-    if (base + 4 > node_cap) { atomicAdd(&cnt->table_fail, 1u); return; }
-    uint32_t lbase = atomicAdd(&cnt->leaves, 4u);
+    uint32_t base = take_nodes();
+    if (base + 4 > node_cap) return false;
+    uint32_t lbase = take_leaves(4u);
     for (int c = 0; c < 4; c++) {
         Node nd;
         halving_leaf(nd, parent, c);
@@ -307,13 +295,77 @@ __global__ void k_tree_finest(Node *nodes, const FrontierItem *fin, Counters *cn
         nd.level = 0;
         nodes[base + c] = nd;
         nodes[f.node].child[c] = base + c;
+        leaf_node[lbase + c] = base + c;
+    }
+    return true;
+}
+
+/* The tree's root and its levels down to `last` (0: the finest cells too),
+ * where no level can hold more than TREE_TOP branches: one workgroup, level by
+ * level, the counters in LDS. What bounds it is the latency of each level's
+ * searches; as a launch per level, each searching all codes eight times per
+ * block, the whole tree took 91 us at 10k objects and 374 us at 1M; 24 us and 172 us so. */
+#define TREE_TOP 1024u
+__global__ __launch_bounds__(1024) void k_tree_top(Node *nodes, MapBox m, const uint32_t *sorted_codes, uint32_t n, uint32_t cap,
+                                                   int last, FrontierItem *fin, FrontierItem *fout, uint32_t *leaf_node,
+                                                   Counters *cnt, uint32_t node_cap, uint32_t front_cap) {
+    __shared__ uint32_t n_nodes, n_leaves, n_in, n_out, bad;
+    if (threadIdx.x == 0) {
+        Node nd;
+        block_box(nd, m, 0, 0, 1);
+        nd.type = T_BRANCH;
+        nd.leaf = 0;
+        nd.code = 0;
+        nd.level = NLEVELS - 1;
+        for (int c = 0; c < 4; c++) nd.child[c] = 0;
+        nodes[0] = nd;
+        n_nodes = 1;
+        n_leaves = 0;
+        bad = 0;
+        n_in = n > cap ? 1 : 0;
+        if (n > cap) fin[0] = FrontierItem{0, 0, 0, n};
+    }
+    auto take_nodes = [&] { return atomicAdd(&n_nodes, 4u); };
+    auto take_leaves = [&](uint32_t k) { return atomicAdd(&n_leaves, k); };
+    auto take_front = [&](uint32_t k) { return atomicAdd(&n_out, k); };
+    int L = NLEVELS - 1;
+    for (; L >= last; L--) {
+        if (threadIdx.x == 0) n_out = 0;
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < n_in; i += blockDim.x)
+            if (!(L ? expand_block(fin[i], nodes, m, sorted_codes, cap, L, fout, leaf_node, node_cap, front_cap, take_nodes,
+                                   take_leaves, take_front)
+                    : expand_cell(fin[i], nodes, leaf_node, node_cap, take_nodes, take_leaves)))
+                bad = 1;
+        __syncthreads();
+        if (bad) break; /* the same for every thread: set before the barrier */
+        if (threadIdx.x == 0) n_in = n_out;
+        FrontierItem *t = fin;
+        fin = fout;
+        fout = t;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        cnt->nodes = n_nodes;
+        cnt->leaves = n_leaves;
+        if (bad) cnt->table_fail = 1;
+        for (int l = 0; l <= NLEVELS; l++) cnt->frontier[l] = 0;
+        if (L >= 0 && !bad) cnt->frontier[L] = n_in;
     }
 }
 
-__global__ void k_leaf_nodes(const Node *nodes, uint32_t n_nodes, uint32_t *leaf_node) {
+/* the branch blocks of one level below those */
+__global__ void k_tree_level(Node *nodes, MapBox m, const uint32_t *sorted_codes, uint32_t cap, int L,
+                             const FrontierItem *fin, FrontierItem *fout, uint32_t *leaf_node, Counters *cnt,
+                             uint32_t node_cap, uint32_t front_cap) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_nodes) return;
-    if (nodes[i].type == T_LEAF) leaf_node[nodes[i].leaf] = i;
+    if (i >= cnt->frontier[L]) return;
+    auto take_nodes = [&] { return atomicAdd(&cnt->nodes, 4u); };
+    auto take_leaves = [&](uint32_t k) { return atomicAdd(&cnt->leaves, k); };
+    const bool ok = L ? expand_block(fin[i], nodes, m, sorted_codes, cap, L, fout, leaf_node, node_cap, front_cap, take_nodes,
+                                     take_leaves, [&](uint32_t k) { return atomicAdd(&cnt->frontier[L - 1], k); })
+                      : expand_cell(fin[i], nodes, leaf_node, node_cap, take_nodes, take_leaves);
+    if (!ok) atomicAdd(&cnt->table_fail, 1u);
 }
 
 /* Workgroups go to the 8 XCDs in turn (workgroup b to XCD b % 8), each XCD
@@ -3019,18 +3071,19 @@ static int rebuild_tree(StcCtx *c, uint32_t *n_nodes, uint32_t *n_leaves) {
     hipStream_t s = c->s;
     Counters *cnt = c->dcnt;
     uint32_t node_cap = (uint32_t)c->nodes.cap;
-    hipLaunchKernelGGL(k_tree_root, dim3(1), dim3(64), 0, s, c->nodes.p, c->map, c->frontier_a.p, cnt, n, c->cap);
     FrontierItem *fin = c->frontier_a.p, *fout = c->frontier_b.p;
-    for (int L = NLEVELS - 1; L >= 1; L--) {
-        uint64_t bound = std::min<uint64_t>(1ull << (2 * (NLEVELS - 1 - L)), c->frontier_a.cap);
-        hipLaunchKernelGGL(k_tree_level, dim3(blocks_for(bound, 128)), dim3(128), 0, s, c->nodes.p, c->map,
-                           c->codes.p, n, c->cap, L, fin, fout, cnt, node_cap, (uint32_t)c->frontier_a.cap);
+    /* branches of a level hold more than cap points each */
+    auto most = [&](int L) { return std::min<uint64_t>(1ull << (2 * (NLEVELS - 1 - L)), n / (c->cap + 1ull) + 1); };
+    int L = NLEVELS - 1;
+    while (L > 0 && most(L - 1) <= TREE_TOP) L--;
+    hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(1024), 0, s, c->nodes.p, c->map, (const uint32_t *)c->codes.p, n, c->cap, L, fin,
+                       fout, c->leaf_node.p, cnt, node_cap, (uint32_t)c->frontier_a.cap);
+    if ((NLEVELS - L) & 1) std::swap(fin, fout);
+    for (L--; L >= 0; L--) {
+        hipLaunchKernelGGL(k_tree_level, dim3(blocks_for(most(L), 64)), dim3(64), 0, s, c->nodes.p, c->map,
+                           (const uint32_t *)c->codes.p, c->cap, L, (const FrontierItem *)fin, fout, c->leaf_node.p, cnt, node_cap,
+                           (uint32_t)c->frontier_a.cap);
         std::swap(fin, fout);
-    }
-    {
-        uint64_t bound = c->frontier_a.cap;
-        hipLaunchKernelGGL(k_tree_finest, dim3(blocks_for(bound, 128)), dim3(128), 0, s, c->nodes.p, fin, cnt,
-                           node_cap);
     }
     CK(hipGetLastError());
     CKRC(sync_counters(c));
@@ -3091,9 +3144,6 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
 
     /* 4: partition */
     CK(hipMemsetAsync(c->leaf_count.p, 0, 4ull * n_leaves, s));
-    if (!c->dyn)
-        hipLaunchKernelGGL(k_leaf_nodes, dim3(blocks_for(n_nodes, 256)), dim3(256), 0, s, c->nodes.p, n_nodes,
-                           c->leaf_node.p);
     hipLaunchKernelGGL(k_partition, dim3(blocks_for(n, 256)), dim3(256), 0, s, xy, walk, n,
                        (const Node *)tree_nodes(c), c->x_buffer, c->y_buffer, c->pt_leaf.p, c->pt_lv.p, c->leaf_count.p, cnt);
     CK(hipGetLastError());
