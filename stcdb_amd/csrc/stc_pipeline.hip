@@ -1646,38 +1646,44 @@ __device__ inline void write_meeting_records(const Bucket &b, uint32_t end, unsi
     }
 }
 
-/* per-object memtable state of the records [from, to) (geometry.cu:705-733):
+/* per-object memtable state of the step's records, from `from` on (geometry.cu:705-733):
  * record counts, quantised MBRs, and oversize meetings (one per record pair)
  * marking both objects. The objects with records are counted by the flush.
  * A box bound is updated only when the record moves it past the value read
  * first: within a memtable the bounds only shrink (low) or grow (high), so a
  * value read before another thread's update still proves an update redundant. */
 __global__ void k_records_account(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes, uint64_t from,
-                                  uint64_t to, uint32_t max_meet, MemtableDev mt, Counters *cnt) {
-    const uint64_t i = from + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                  uint32_t max_meet, MemtableDev mt, Counters *cnt) {
+    const uint64_t to = cnt->kv_count;
+    if (to > mt.cap) return; /* the merge is run again with more room */
     const int lane = threadIdx.x & (STC_WAVE - 1);
-    bool oversize = false;
-    if (i < to) {
-        const uint64_t lo = keys[2 * i], hi = keys[2 * i + 1];
-        const uint32_t a = (uint32_t)(hi >> 26) & 0x3FFFFFFu, c = (uint32_t)hi & 0x3FFFFFFu;
-        const uint32_t duration = (uint32_t)(lo >> 32);
-        if (((i - from) & 1) == 0 && duration > max_meet) {
-            oversize = true;
-            mt.sids[a] = 1;
-            mt.sids[c] = 1;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    uint32_t n_over = 0;
+    for (uint64_t i0 = from + (uint64_t)blockIdx.x * blockDim.x; i0 < to; i0 += stride) {
+        const uint64_t i = i0 + threadIdx.x;
+        bool oversize = false;
+        if (i < to) {
+            const uint64_t lo = keys[2 * i], hi = keys[2 * i + 1];
+            const uint32_t a = (uint32_t)(hi >> 26) & 0x3FFFFFFu, c = (uint32_t)hi & 0x3FFFFFFu;
+            const uint32_t duration = (uint32_t)(lo >> 32);
+            if (((i - from) & 1) == 0 && duration > max_meet) {
+                oversize = true;
+                mt.sids[a] = 1;
+                mt.sids[c] = 1;
+            }
+            const float4 b = boxes[i];
+            atomicAdd(&mt.same_pid_count[a], 1u);
+            const uint4 cur = mt.o_boxs[a];
+            const uint32_t q0 = f2q(b.x), q1 = f2q(b.y), q2 = f2q(b.z), q3 = f2q(b.w);
+            if (q0 < cur.x) atomicMin(&mt.o_boxs[a].x, q0);
+            if (q2 > cur.z) atomicMax(&mt.o_boxs[a].z, q2);
+            if (q1 < cur.y) atomicMin(&mt.o_boxs[a].y, q1);
+            if (q3 > cur.w) atomicMax(&mt.o_boxs[a].w, q3);
         }
-        const float4 b = boxes[i];
-        atomicAdd(&mt.same_pid_count[a], 1u);
-        const uint4 cur = mt.o_boxs[a];
-        const uint32_t q0 = f2q(b.x), q1 = f2q(b.y), q2 = f2q(b.z), q3 = f2q(b.w);
-        if (q0 < cur.x) atomicMin(&mt.o_boxs[a].x, q0);
-        if (q2 > cur.z) atomicMax(&mt.o_boxs[a].z, q2);
-        if (q1 < cur.y) atomicMin(&mt.o_boxs[a].y, q1);
-        if (q3 > cur.w) atomicMax(&mt.o_boxs[a].w, q3);
+        n_over += (uint32_t)__popcll(__ballot(oversize));
     }
     /* one counter update per wave: a counter updated by every thread serialises on its address */
-    const uint64_t om = __ballot(oversize);
-    if (lane == 0 && om) atomicAdd(&cnt->oversize_oid_count, (uint32_t)__popcll(om));
+    if (lane == 0 && n_over) atomicAdd(&cnt->oversize_oid_count, n_over);
 }
 
 /* ascending bitonic sort of s[0, P) (P a power of two) by a block */
@@ -3183,8 +3189,6 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
                        c->units.p, c->rev_leaf.p, c->rev_pid.p, c->urange.p, c->lunits.p);
     CK(hipGetLastError());
     CK(hipEventRecord(c->ev[2], s));
-
-    /* 7: reverse cross units: per leaf, the border points with a cross unit to it, by pid */
     if (c->rev_leaf_alt.ensure(n_units + 1) ||
         c->rev.ensure(n_units + 1) || c->rev_dl.ensure(n_units + 1) ||
         c->rev_pid_alt.ensure(n_units + 1) ||
@@ -3192,6 +3196,13 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
         c->temp.ensure(stc_radix_temp_words((uint32_t)std::max<uint64_t>(std::max<uint64_t>(n_units, n),
                                                                           std::max<size_t>(c->nodes.cap, c->sch.cap))) + 64))
         return fail(c, STC_E_CAPACITY, "reverse unit buffers");
+    if (c->dyn) { /* the update's splits and merges follow from the partition: their numbers come with the collect pass's */
+        const int rc = stc_schema_plan(&c->sch, c->leaf_count.p, c->cap, c->cfg.reach_distance, c->cfg.schema_update_delay,
+                                       c->temp.p, c->temp.cap, s);
+        if (rc) return fail(c, rc, std::string("schema update: ") + g_last_fail);
+    }
+
+    /* 7: reverse cross units: per leaf, the border points with a cross unit to it, by pid */
     if (n_units)
         CKRC(sort_pairs((const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, c->rev_leaf, c->rev_pid, c->rev_leaf_alt,
                         c->rev_pid_alt, (uint32_t)n_units, std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
@@ -3228,9 +3239,9 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     if (!c->psrc.p && c->psrc.ensure(std::max<size_t>((size_t)n * 16, 1u << 20)))
         return fail(c, STC_E_CAPACITY, "pair sources");
     for (int attempt = 0;; attempt++) {
-        /* one clear for candidates .. pk_over (a fill launch can wait behind the run copies) */
-        CK(hipMemsetAsync(&cnt->candidates, 0,
-                          offsetof(Counters, pk_over) + sizeof(uint32_t) - offsetof(Counters, candidates), s));
+        if (attempt) /* candidates .. pk_over; the step's first counters are clear */
+            CK(hipMemsetAsync(&cnt->candidates, 0,
+                              offsetof(Counters, pk_over) + sizeof(uint32_t) - offsetof(Counters, candidates), s));
         CK(hipEventRecord(c->ev[10], s));
         hipLaunchKernelGGL(k_pair_collect, dim3(pgrid), dim3(256), 0, s, pg, batch, c->pcount.p, c->pkrun.p, c->psrc.p,
                            (uint64_t)std::min<size_t>(c->psrc.cap, 0xFFFFFFFFu), c->amb.p,
@@ -3360,7 +3371,9 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
                            h.giant, (const uint32_t *)c->moff[nx].p, (const PairSlot *)c->ptmp.p, c->pnew.p,
                            (uint32_t *)nullptr, (uint32_t *)nullptr, c->gsrt.p, gcap, cnt);
         CK(hipGetLastError());
+        CKRC(sync_counters(c));
     }
+    if (c->hcnt->table_fail) return fail(c, STC_E_HIP, "a pair segment was longer than its sort's scratch");
     c->plen = total;
     c->pairs_boxed = false;
     CK(hipEventRecord(c->ev[3], s));
@@ -3388,10 +3401,8 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     if (ensure_records(c, kv_before + 2 * std::max<uint64_t>(c->last_expired + c->last_expired / 4, 1 << 16) + 2))
         return fail(c, STC_E_CAPACITY, "record buffer allocation failed");
     const MergeArgs ma{t, c->cfg.min_meet_time, c->cfg.max_meet_time, c->end_time_min, c->map, c->last_t};
-    CKRC(sync_counters(c));
-    Counters h = *c->hcnt;
-    if (h.table_fail) return fail(c, STC_E_HIP, "a pair segment was longer than its sort's scratch");
-    const Counters before = h;
+    const Counters before = *c->hcnt; /* as read last: nothing since has changed them */
+    Counters h;
     /* tiles of the step's pairs and their ranges in the previous meetings */
     const uint32_t n_tiles = (uint32_t)std::max<uint64_t>((c->plen + MTILE - 1) / MTILE, 1);
     if (c->tbounds.ensure(n_tiles + 1ull) || c->towner.ensure(n_tiles)) return fail(c, STC_E_CAPACITY, "merge tile bounds");
@@ -3416,12 +3427,16 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         std::min<uint32_t>((n_tiles + 3) / 4, std::min<uint32_t>(std::max<uint32_t>(n_tiles / 40, 2048), 65536)), 1);
     /* the merge writes meet[nx] and, after a flush emptied the memtable, records from index 0 */
     wait_readers(c, nx, kv_before == 0);
+    const bool schema_step = c->dyn && g.nodes;
+    int schema_rc = STC_OK;
     for (int attempt = 0;; attempt++) {
         /* the merge rewrites the same buckets, so a re-run with more record room is exact */
-        *c->hinit = before;
-        memset(c->hinit->meet_part, 0, sizeof(c->hinit->meet_part));
-        c->hinit->kv_count = kv_before;
-        CK(hipMemcpyAsync(cnt, c->hinit, sizeof(Counters), hipMemcpyHostToDevice, s));
+        if (attempt) {
+            *c->hinit = before;
+            memset(c->hinit->meet_part, 0, sizeof(c->hinit->meet_part));
+            c->hinit->kv_count = kv_before;
+            CK(hipMemcpyAsync(cnt, c->hinit, sizeof(Counters), hipMemcpyHostToDevice, s));
+        }
         const MemtableDev mt{c->rec_keys, c->rec_boxes, c->rec_cap, c->same_pid_count, c->o_boxs, c->sids};
         CK(hipEventRecord(c->ev[8], s));
         if (c->pairs_boxed)
@@ -3436,22 +3451,24 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
                                (const uint32_t *)c->towner.p, c->n, cnt);
         CK(hipGetLastError());
         CK(hipEventRecord(c->ev[9], s));
-        CKRC(sync_counters(c));
+        /* per-object memtable state of the new records, about as many as the last step's; a thread each at most */
+        const uint32_t agrid = std::max<uint32_t>(std::min<uint64_t>(blocks_for(2 * c->last_expired, 256), 1u << 16), 64);
+        hipLaunchKernelGGL(k_records_account, dim3(agrid), dim3(256), 0, s, (const uint64_t *)c->rec_keys,
+                           (const float4 *)c->rec_boxes, kv_before, c->cfg.max_meet_time, mt, cnt);
+        CK(hipGetLastError());
+        CK(hipEventRecord(c->ev[4], s));
+        if (schema_step && !attempt) { /* the dynamic schema's update for the next step (geometry.cu:2159-2182) */
+            CK(hipEventRecord(c->ev[12], s));
+            schema_rc = stc_schema_apply(&c->sch, s);
+            CK(hipEventRecord(c->ev[13], s));
+        }
+        CK(hipEventRecord(c->ev[5], s));
+        CKRC(sync_counters(c)); /* the step's last wait, unless it flushes */
         h = *c->hcnt;
         if (h.table_fail) return fail(c, STC_E_HIP, "merge: the step's pairs are not sorted by key");
         if (h.kv_count <= c->rec_cap) break;
         if (attempt >= 2 || ensure_records(c, h.kv_count + h.kv_count / 4 + 2))
             return fail(c, STC_E_CAPACITY, "record buffer allocation failed");
-    }
-    /* per-object memtable state of the new records */
-    if (h.kv_count > kv_before) {
-        const MemtableDev mt{c->rec_keys, c->rec_boxes, c->rec_cap, c->same_pid_count, c->o_boxs, c->sids};
-        hipLaunchKernelGGL(k_records_account, dim3(blocks_for(h.kv_count - kv_before, 256)), dim3(256), 0, s,
-                           (const uint64_t *)c->rec_keys, (const float4 *)c->rec_boxes, kv_before, (uint64_t)h.kv_count,
-                           c->cfg.max_meet_time, mt, cnt);
-        CK(hipGetLastError());
-        CKRC(sync_counters(c));
-        h = *c->hcnt;
     }
     c->kv_count = h.kv_count;
     c->oversize_oid_count = h.oversize_oid_count;
@@ -3467,11 +3484,12 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     c->cur = nx;
     c->mlen = c->plen;
     g.pairs = met.live;
-    CK(hipEventRecord(c->ev[4], s));
+    if (schema_rc) return fail(c, schema_rc, std::string("schema update: ") + g_last_fail);
 
     /* 10: flush */
     uint32_t flushed = 0;
     if (c->kv_count > c->cfg.kv_restriction) {
+        CK(hipEventRecord(c->ev[4], s));
         FlushArgs fa{};
         fa.n = n;
         fa.ctf_count = c->cfg.ctf_count;
@@ -3541,17 +3559,10 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         c->epoch++;
         flushed = 1;
     }
-    /* 11: the dynamic schema's update for the next step (geometry.cu:2159-2182) */
-    const bool schema_step = c->dyn && g.nodes;
-    if (schema_step) {
-        CK(hipEventRecord(c->ev[12], s));
-        int rc = stc_schema_update(&c->sch, c->leaf_count.p, c->cap, c->cfg.reach_distance,
-                                   c->cfg.schema_update_delay, c->temp.p, c->temp.cap, s);
-        if (rc) return fail(c, rc, std::string("schema update: ") + g_last_fail);
-        CK(hipEventRecord(c->ev[13], s));
+    if (flushed) {
+        CK(hipEventRecord(c->ev[5], s));
+        CK(hipEventSynchronize(c->ev[5]));
     }
-    CK(hipEventRecord(c->ev[5], s));
-    CK(hipEventSynchronize(c->ev[5]));
 
     c->stepped = true;
     c->last_t = t;

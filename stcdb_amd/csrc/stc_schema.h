@@ -35,6 +35,7 @@ struct MapBox { double lo0, lo1, hi0, hi1; };
 struct SchemaState {
     Node *nodes = nullptr;
     uint32_t *nstate = nullptr;        /* overflow_count | underflow_count << 16 */
+    uint32_t *nstate_next = nullptr;   /* a planned update's */
     uint32_t *fstack = nullptr;        /* free slots */
     uint32_t *fs = nullptr, *fm = nullptr, *rs = nullptr, *rm = nullptr; /* per-slot flags and ranks */
     uint32_t *pnode = nullptr;         /* initial build: each point's node (bit 31: settled) */
@@ -61,8 +62,11 @@ int stc_schema_get(SchemaState *S, stc_qtnode *nodes, uint64_t cap, uint64_t *n,
 /* leaf ids 0..n_leaves-1 in slot order; leaf_node[leaf] = slot */
 int stc_schema_number_leaves(SchemaState *S, uint32_t *leaf_node, uint32_t *temp, size_t temp_words,
                              hipStream_t s);
-/* the update after a step from its leaf counts (all points of each leaf) */
-int stc_schema_update(SchemaState *S, const uint32_t *leaf_count, uint32_t cap, double r, uint32_t delay,
-                      uint32_t *temp, size_t temp_words, hipStream_t s);
+/* The update after a step from its leaf counts (all points of each leaf), in two parts: the plan marks and
+ * ranks the splits and merges and queues their numbers for the host, and can go as soon as the points are
+ * partitioned; once the stream has been waited for, the update is applied after the step's last use of the tree. */
+int stc_schema_plan(SchemaState *S, const uint32_t *leaf_count, uint32_t cap, double r, uint32_t delay,
+                    uint32_t *temp, size_t temp_words, hipStream_t s);
+int stc_schema_apply(SchemaState *S, hipStream_t s);
 
 #endif

@@ -173,8 +173,8 @@ __global__ void k_leaf_assign(Node *__restrict__ nodes, uint32_t hwm, const uint
 /* ------------------------------------------------------------------ */
 
 /* cuda_update_schema_collect (geometry.cu:1193-1234) */
-__global__ void k_schema_collect(const Node *__restrict__ nodes, uint32_t hwm, uint32_t *__restrict__ nstate,
-                                 const uint32_t *__restrict__ leaf_count, uint32_t cap, double r2, uint32_t delay,
+__global__ void k_schema_collect(const Node *__restrict__ nodes, uint32_t hwm, const uint32_t *__restrict__ nstate,
+                                 uint32_t *__restrict__ nstate_next, const uint32_t *__restrict__ leaf_count, uint32_t cap, double r2, uint32_t delay,
                                  uint32_t *__restrict__ fs, uint32_t *__restrict__ fm) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= hwm) return;
@@ -204,7 +204,7 @@ __global__ void k_schema_collect(const Node *__restrict__ nodes, uint32_t hwm, u
             unf = 0;
         }
     }
-    nstate[i] = ovf | (unf << 16);
+    nstate_next[i] = ovf | (unf << 16);
     fs[i] = s;
     fm[i] = m;
 }
@@ -277,6 +277,7 @@ static int reserve_slots(SchemaState *S, uint32_t need, hipStream_t s) {
     uint32_t nc = std::max<uint32_t>(need + need / 2, 1024);
     /* flags and ranks too: an update grows the slots between its scans and its splits */
     if (grow_copy(S->nodes, S->cap, nc, true, s) || grow_copy(S->nstate, S->cap, nc, true, s) ||
+        grow_copy(S->nstate_next, S->cap, nc, false, s) ||
         grow_copy(S->fstack, S->cap, nc, true, s) || grow_copy(S->fs, S->cap, nc, true, s) ||
         grow_copy(S->fm, S->cap, nc, true, s) || grow_copy(S->rs, S->cap, nc, true, s) ||
         grow_copy(S->rm, S->cap, nc, true, s) || grow_copy(S->cnt, S->cap, nc, true, s))
@@ -296,7 +297,7 @@ int stc_schema_init(SchemaState *S, uint32_t n_points, uint32_t slots) {
 }
 
 void stc_schema_free(SchemaState *S) {
-    void *d[] = {S->nodes, S->nstate, S->fstack, S->fs, S->fm, S->rs, S->rm, S->pnode, S->cnt, S->dcount, S->amb};
+    void *d[] = {S->nodes, S->nstate, S->nstate_next, S->fstack, S->fs, S->fm, S->rs, S->rm, S->pnode, S->cnt, S->dcount, S->amb};
     for (void *p : d)
         if (p) (void)hipFree(p);
     if (S->hcount) (void)hipHostFree(S->hcount);
@@ -463,19 +464,25 @@ int stc_schema_number_leaves(SchemaState *S, uint32_t *leaf_node, uint32_t *temp
     return 0;
 }
 
-int stc_schema_update(SchemaState *S, const uint32_t *leaf_count, uint32_t cap, double r, uint32_t delay,
-                      uint32_t *temp, size_t temp_words, hipStream_t s) {
+int stc_schema_plan(SchemaState *S, const uint32_t *leaf_count, uint32_t cap, double r, uint32_t delay,
+                    uint32_t *temp, size_t temp_words, hipStream_t s) {
     const uint32_t hwm = S->hwm;
     if (temp_words < stc_radix_temp_words(hwm)) return STC_E_CAPACITY;
-    STC_CHECK(hipMemsetAsync(S->dcount, 0, DC_WORDS * 4, s));
     hipLaunchKernelGGL(k_schema_collect, dim3(nblk(hwm, 256)), dim3(256), 0, s, (const Node *)S->nodes, hwm,
-                       S->nstate, leaf_count, cap, 2 * r, delay ? delay : 1u, S->fs, S->fm);
+                       (const uint32_t *)S->nstate, S->nstate_next, leaf_count, cap, 2 * r, delay ? delay : 1u, S->fs, S->fm);
     STC_CHECK(hipGetLastError());
     int rc = stc_exclusive_scan_u32(S->fs, S->rs, hwm, S->dcount + DC_SPLITS, temp, s);
     if (!rc) rc = stc_exclusive_scan_u32(S->fm, S->rm, hwm, S->dcount + DC_MERGES, temp, s);
     if (rc) return rc;
-    { int rc_ = read_counts(S, s); if (rc_) return rc_; }
+    STC_CHECK(hipMemcpyAsync(S->hcount, S->dcount, DC_WORDS * 4, hipMemcpyDeviceToHost, s));
+    return 0;
+}
+
+int stc_schema_apply(SchemaState *S, hipStream_t s) {
+    const uint32_t hwm = S->hwm;
     const uint32_t ns = S->hcount[DC_SPLITS], nm = S->hcount[DC_MERGES];
+    int rc;
+    std::swap(S->nstate, S->nstate_next);
     if (ns) {
         const uint32_t need = 4 * ns;
         const uint32_t new_hwm = hwm + (need > S->n_free ? need - S->n_free : 0);
