@@ -8,6 +8,9 @@
 #include "../../include/stcdb.h"
 #include <vector>
 
+/* an object's place among the records: first slot, slots filled so far, sid (or the tail's key), record count */
+struct __attribute__((aligned(16))) ObjSlots { uint32_t base, fill, key, count; };
+
 struct FlushWork {
     uint32_t n = 0, ctf_count = 0;
     bool str_full = false;                         /* STR sorts over the full 64-bit keys (a compact key overflowed) */
@@ -19,9 +22,9 @@ struct FlushWork {
     uint64_t *ctf_byte_base = nullptr;             /* per-CTF first packed byte */
     stc_ctf_meta *ctfs = nullptr;
     uint8_t *bitmaps = nullptr;                    /* ctf_count * 8192 */
-    uint32_t *obj_base = nullptr, *obj_fill = nullptr; /* per-object record slots */
+    ObjSlots *slots = nullptr;                     /* per-object record slots */
     uint8_t *part_tail = nullptr;                  /* per object: records go to the oversize buffer */
-    uint32_t *obj_key = nullptr, *obj_id = nullptr, *obj_cnt = nullptr; /* object placement order */
+    uint32_t *obj_key = nullptr, *obj_id = nullptr, *obj_cnt = nullptr, *obj_first = nullptr; /* object placement order */
     uint32_t *scan_temp = nullptr;
     size_t scan_temp_words = 0;
     uint32_t *flags = nullptr;                     /* device counters of the flush */

@@ -45,6 +45,8 @@
 #define BIT_COUNT 65536u
 #define BITMAP_WORDS (BIT_COUNT / 32)
 #define MAX_RASTER (1u << 20)
+#define TAIL_KEY (1u << 31 | 4095u) /* the placement key of an oversize object: its low 12 bits are sorted by */
+#define LIMIT_THREADS 1024 /* of a CTF's limits: there are few CTFs, and each is read by one workgroup (256: 80 -> 40 us at 5.2M records) */
 
 static inline uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t); }
 
@@ -108,8 +110,6 @@ void stc_ctf_bits(stc_ctf_meta *c, const double *map, uint32_t num_objects, uint
 struct FlushCounters {
     uint32_t oversize_oid_count; /* from identify, plus set_oid's area test */
     uint32_t sid_count;
-    uint32_t z;                  /* objects without a CTF (no records or oversize) */
-    uint32_t xpc, pkc, split;
     uint32_t n_tail;             /* records of oversize objects */
     uint32_t o_start_min, o_start_max;
     uint32_t bad;                /* inconsistent capacities (reference would misbehave) */
@@ -143,128 +143,145 @@ __device__ inline uint64_t sat_u64(double v) {
 }
 __device__ inline float q2f(uint32_t f) { return (float)f / 100000 - 180; } /* uint_to_float */
 
+/* a value of each thread added up over the workgroup and into *to, one update a workgroup: an address takes an
+ * update every few nanoseconds, whatever the number of waves that send one */
+__device__ inline void block_add(uint32_t v, uint32_t *to) {
+    __shared__ uint32_t part[16];
+    for (int o = STC_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, STC_WAVE);
+    if ((threadIdx.x & (STC_WAVE - 1)) == 0) part[threadIdx.x / STC_WAVE] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t i = 1; i < blockDim.x / STC_WAVE; i++) v += part[i];
+        if (v) atomicAdd(to, v);
+    }
+    __syncthreads();
+}
+
+__global__ void k_flush_init(FlushCounters *fc, uint32_t oversize, uint32_t *capacity, uint32_t C) {
+    for (uint32_t i = threadIdx.x; i <= C; i += blockDim.x) capacity[i] = 0;
+    if (threadIdx.x == 0) {
+        FlushCounters z{};
+        z.oversize_oid_count = oversize;
+        *fc = z;
+    }
+}
+
 /* ------------------------------------------------------------------ */
 /* F1: set_oid                                                         */
 /* ------------------------------------------------------------------ */
 
-__global__ void k_set_oid(uint32_t n, const uint32_t *__restrict__ same_pid_count, const uint4 *__restrict__ o_boxs,
-                          uint16_t *__restrict__ sids, uint64_t *__restrict__ mid, uint32_t *__restrict__ oids,
-                          uint8_t *__restrict__ part_tail, double area_threshold, uint32_t sticky, StrCompact sc,
-                          FlushCounters *fc) {
-    uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n) return;
-    oids[id] = id;
-    uint64_t m = 0;
-    if (same_pid_count[id] >= 1) {
-        uint4 ob = o_boxs[id];
-        float low0 = q2f(ob.x), high0 = q2f(ob.z), low1 = q2f(ob.y), high1 = q2f(ob.w);
-        float area = (high1 - low1) * (high0 - low0);
-        if ((sticky && sids[id] == 1) || (double)area > area_threshold) {
-            atomicAdd(&fc->oversize_oid_count, 1u);
-            sids[id] = 1;
-        } else {
-            uint32_t am0 = ob.x / 2 + ob.z / 2;
-            uint32_t am1 = ob.w / 2 + ob.w / 2; /* high[1] twice, as the reference */
-            if (!sc.on) {
-                m = ((uint64_t)am0 << 32) + (uint64_t)am1;
+/* Also sid_count: the objects with at least one record (geometry.cu:726-729
+ * counts them as their first record arrives). 1M objects: 18 us (before, with
+ * an update a wave and a pass for the count: 56). */
+__global__ __launch_bounds__(256) void k_set_oid(uint32_t n, const uint32_t *__restrict__ same_pid_count,
+                                                 const uint4 *__restrict__ o_boxs, uint16_t *__restrict__ sids,
+                                                 uint64_t *__restrict__ mid, uint8_t *__restrict__ part_tail,
+                                                 double area_threshold, uint32_t sticky, StrCompact sc, FlushCounters *fc) {
+    uint32_t have = 0, over = 0;
+    for (uint32_t id = blockIdx.x * blockDim.x + threadIdx.x; id < n; id += gridDim.x * blockDim.x) {
+        uint64_t m = 0;
+        uint32_t sid = sids[id];
+        if (same_pid_count[id] >= 1) {
+            have++;
+            uint4 ob = o_boxs[id];
+            float low0 = q2f(ob.x), high0 = q2f(ob.z), low1 = q2f(ob.y), high1 = q2f(ob.w);
+            float area = (high1 - low1) * (high0 - low0);
+            if ((sticky && sid == 1) || (double)area > area_threshold) {
+                over++;
+                sids[id] = 1;
+                sid = 1;
             } else {
-                const uint64_t x = (uint64_t)am0 - sc.base0 + 1, y = (uint64_t)am1 - sc.base1;
-                if (am0 < sc.base0 || am1 < sc.base1 || x >= sc.lim0 || y >= sc.lim1) atomicOr(&fc->str_wide, 1u);
-                m = (x << sc.by) | (y & (sc.lim1 - 1));
+                uint32_t am0 = ob.x / 2 + ob.z / 2;
+                uint32_t am1 = ob.w / 2 + ob.w / 2; /* high[1] twice, as the reference */
+                if (!sc.on) {
+                    m = ((uint64_t)am0 << 32) + (uint64_t)am1;
+                } else {
+                    const uint64_t x = (uint64_t)am0 - sc.base0 + 1, y = (uint64_t)am1 - sc.base1;
+                    if (am0 < sc.base0 || am1 < sc.base1 || x >= sc.lim0 || y >= sc.lim1) atomicOr(&fc->str_wide, 1u);
+                    m = (x << sc.by) | (y & (sc.lim1 - 1));
+                }
             }
         }
+        mid[id] = m;
+        part_tail[id] = sid == 1 ? 1 : 0; /* partition-time oversize flag (geometry.cu:1777-1780) */
     }
-    mid[id] = m;
-    part_tail[id] = (sids[id] == 1) ? 1 : 0; /* partition-time oversize flag (geometry.cu:1777-1780) */
+    block_add(have, &fc->sid_count);
+    block_add(over, &fc->oversize_oid_count);
 }
 
-/* sid_count: the objects with at least one record (geometry.cu:726-729 counts
- * them as their first record arrives) */
-__global__ __launch_bounds__(256) void k_count_sids(const uint32_t *__restrict__ same_pid_count, uint32_t n,
-                                                    FlushCounters *fc) {
-    uint32_t mine = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        mine += same_pid_count[i] ? 1u : 0u;
-    for (int o = STC_WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, STC_WAVE);
-    if ((threadIdx.x & (STC_WAVE - 1)) == 0 && mine) atomicAdd(&fc->sid_count, mine);
-}
-
-__global__ void k_str_prepare(FlushCounters *fc, uint32_t n, uint32_t split) {
-    if (threadIdx.x || blockIdx.x) return;
-    uint32_t z = (n - fc->sid_count) + fc->oversize_oid_count;
-    uint32_t xpc = (fc->sid_count - fc->oversize_oid_count) / split + 1;
-    fc->z = z;
-    fc->xpc = xpc;
-    fc->pkc = xpc / split + 1;
-    fc->split = split;
+/* the STR cut, from set_oid's counts: objects below z have no CTF (no records or oversize) */
+struct StrCut { uint32_t z, xpc, pkc; };
+__device__ inline StrCut str_cut(const FlushCounters *fc, uint32_t n, uint32_t split) {
+    const uint32_t on = fc->sid_count - fc->oversize_oid_count, xpc = on / split + 1;
+    return StrCut{n - on, xpc, xpc / split + 1};
 }
 
 /* narrow_xy_to_y + strip ranges: key = (strip + 1) << 32 | y for positions >= z
  * (with compact keys, (strip + 1) << by | y - base1) */
-__global__ void k_strip_keys(uint64_t *mid, uint32_t n, StrCompact sc, const FlushCounters *fc) {
+__global__ void k_strip_keys(uint64_t *mid, uint32_t n, StrCompact sc, uint32_t split, const FlushCounters *fc) {
     uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= n) return;
-    uint32_t z = fc->z;
-    if (id < z) { mid[id] = 0; return; }
-    uint32_t strip = (id - z) / fc->xpc;
-    if (strip > fc->split - 1) strip = fc->split - 1;
+    const StrCut cut = str_cut(fc, n, split);
+    if (id < cut.z) { mid[id] = 0; return; }
+    uint32_t strip = (id - cut.z) / cut.xpc;
+    if (strip > split - 1) strip = split - 1;
     if (sc.on) mid[id] = ((uint64_t)(strip + 1) << sc.by) | (mid[id] & (sc.lim1 - 1));
     else mid[id] = ((uint64_t)(strip + 1) << 32) | (mid[id] & 0xFFFFFFFFull);
 }
 
-__global__ void k_make_sid(const uint32_t *oids, uint32_t n, uint16_t *sids, const FlushCounters *fc) {
-    uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t z = fc->z;
-    if (id >= n || id < z) return;
-    uint32_t xi = (id - z) / fc->xpc;
-    uint32_t yi = (id - z - xi * fc->xpc) / fc->pkc;
-    sids[oids[id]] = (uint16_t)(xi * fc->split + yi + 2);
-}
+#define CAP_ITEMS 8u  /* objects per thread of k_make_sid */
+#define CAP_SLOTS 64u /* CTFs whose counts a workgroup keeps in LDS */
 
-__global__ void k_ctf_capacity(const uint32_t *oids, uint32_t n, const uint16_t *sids,
-                               const uint32_t *same_pid_count, uint32_t *capacity, uint32_t ctf_count,
-                               FlushCounters *fc) {
-    /* objects id >= z are in CTF order, so a wavefront spans one or two CTFs:
-     * lanes of one CTF add their counts first and one lane updates it */
-    uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & (STC_WAVE - 1);
-    bool on = id < n && id >= fc->z;
-    uint32_t cid = 0, v = 0;
-    if (on) {
-        uint32_t oid = oids[id];
-        cid = (uint32_t)sids[oid] - 2;
-        v = same_pid_count[oid];
+/* make_sid, and the CTFs' record counts. Objects id >= z are in CTF order: a
+ * workgroup's stretch spans a few CTFs, which it adds up in LDS before one
+ * update each (an update a wave is serial at the CTF's address; 5M objects,
+ * with the counts in a pass of their own: 135 -> 61 us). CTFs further on than
+ * LDS has room for are updated directly. */
+__global__ __launch_bounds__(256) void k_make_sid(const uint32_t *__restrict__ oids, uint32_t n, uint32_t split,
+                                                  uint16_t *__restrict__ sids,
+                                                  const uint32_t *__restrict__ same_pid_count,
+                                                  uint32_t *__restrict__ capacity, uint32_t ctf_count, FlushCounters *fc) {
+    __shared__ uint32_t part[CAP_SLOTS];
+    const StrCut cut = str_cut(fc, n, split);
+    if (threadIdx.x < CAP_SLOTS) part[threadIdx.x] = 0;
+    const uint64_t base = (uint64_t)blockIdx.x * (256 * CAP_ITEMS);
+    auto ctf_of = [&](uint32_t id) {
+        const uint32_t xi = (id - cut.z) / cut.xpc;
+        return xi * split + (id - cut.z - xi * cut.xpc) / cut.pkc;
+    };
+    const uint32_t c0 = base < cut.z ? 0u : base < n ? ctf_of((uint32_t)base) : 0u;
+    __syncthreads();
+    for (uint32_t k = 0; k < CAP_ITEMS; k++) {
+        const uint64_t at = base + k * 256 + threadIdx.x;
+        if (at >= n || at < cut.z) continue;
+        const uint32_t oid = oids[at], cid = (uint16_t)(ctf_of((uint32_t)at) + 2) - 2u;
+        sids[oid] = (uint16_t)(cid + 2);
         if (cid >= ctf_count) {
             atomicAdd(&fc->bad, 1u);
-            on = false;
+            continue;
         }
+        const uint32_t v = same_pid_count[oid];
+        if (cid - c0 < CAP_SLOTS) atomicAdd(&part[cid - c0], v);
+        else atomicAdd(&capacity[cid], v);
     }
-    uint64_t act = __ballot(on);
-    while (act) {
-        int leader = __ffsll((unsigned long long)act) - 1;
-        uint32_t lc = __shfl(cid, leader, STC_WAVE);
-        bool mine = on && cid == lc;
-        uint32_t sum = mine ? v : 0u;
-        for (int o = STC_WAVE / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, STC_WAVE);
-        if (lane == leader) atomicAdd(&capacity[lc], sum);
-        act &= ~__ballot(mine);
-        if (mine) on = false;
-    }
+    __syncthreads();
+    if (threadIdx.x < CAP_SLOTS && part[threadIdx.x]) atomicAdd(&capacity[c0 + threadIdx.x], part[threadIdx.x]);
 }
 
 /* object order for placement: objects by (sid, oid) — the CTF records, sid
  * being the key's top field — then the oversize objects by oid (key 4095, the
- * tail). Objects without records have no slots. */
-__global__ void k_obj_keys(uint32_t n, const uint16_t *sids, const uint8_t *part_tail, const uint32_t *same_pid_count,
-                           uint32_t *obj_key, uint32_t *obj_id, uint32_t *obj_cnt) {
-    uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n) return;
-    uint32_t cnt = same_pid_count[id];
-    uint32_t key = 0;
-    if (cnt) key = part_tail[id] ? 4095u : (uint32_t)sids[id];
-    obj_key[id] = key;
-    obj_id[id] = id;
-    obj_cnt[id] = cnt;
+ * tail). Objects without records have no slots. Also the tail's records. */
+__global__ __launch_bounds__(256) void k_obj_keys(uint32_t n, const uint16_t *__restrict__ sids,
+                                                  const uint8_t *__restrict__ part_tail,
+                                                  const uint32_t *__restrict__ same_pid_count,
+                                                  uint32_t *__restrict__ obj_key, FlushCounters *fc) {
+    uint32_t tail = 0;
+    for (uint32_t id = blockIdx.x * blockDim.x + threadIdx.x; id < n; id += gridDim.x * blockDim.x) {
+        const uint32_t cnt = same_pid_count[id], oversize = part_tail[id];
+        obj_key[id] = !cnt ? 0u : oversize ? TAIL_KEY : (uint32_t)sids[id];
+        if (oversize) tail += cnt;
+    }
+    block_add(tail, &fc->n_tail);
 }
 
 __global__ void k_gather_counts(const uint32_t *obj_id, const uint32_t *same_pid_count, uint32_t n, uint32_t *cnt) {
@@ -272,55 +289,52 @@ __global__ void k_gather_counts(const uint32_t *obj_id, const uint32_t *same_pid
     if (i < n) cnt[i] = same_pid_count[obj_id[i]];
 }
 
-__global__ void k_scatter_base(const uint32_t *obj_id, const uint32_t *scanned, uint32_t n, uint32_t *obj_base,
-                               uint32_t *obj_fill) {
+/* all that placing an object's records takes, in one 16-byte word: a record's
+ * object is anywhere, and base, fill, sid and tail in arrays of their own are
+ * four cache lines a record (5.2M records of 5M objects: 380 -> 356 us, the
+ * updates of fill being most of it) */
+__global__ void k_obj_slots(const uint32_t *__restrict__ obj_id, const uint32_t *__restrict__ obj_key,
+                            const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ first, uint32_t n,
+                            ObjSlots *__restrict__ slots) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t oid = obj_id[i];
-    obj_base[oid] = scanned[i];
-    obj_fill[oid] = 0;
-}
-
-__global__ void k_count_tail(const uint8_t *part_tail, const uint32_t *same_pid_count, uint32_t n, FlushCounters *fc) {
-    uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t v = (id < n && part_tail[id]) ? same_pid_count[id] : 0;
-    if (v) atomicAdd(&fc->n_tail, v);
+    if (i < n) slots[obj_id[i]] = ObjSlots{first[i], 0, obj_key[i], cnt[i]};
 }
 
 /* records to their object's slot range; front keys get their CTF id (write_sid_in_key) */
 __global__ void k_scatter_records(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes, uint64_t K,
-                                  const uint32_t *__restrict__ obj_base, uint32_t *__restrict__ obj_fill,
-                                  const uint16_t *__restrict__ sids, const uint8_t *__restrict__ part_tail,
-                                  uint64_t *__restrict__ tkeys, float4 *__restrict__ tboxes) {
+                                  ObjSlots *slots, uint64_t *__restrict__ tkeys, float4 *__restrict__ tboxes) {
     uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= K) return;
-    uint64_t lo = keys[2 * k], hi = keys[2 * k + 1];
-    uint32_t oid = (uint32_t)((hi >> 26) & OID_MASK);
-    uint32_t slot = obj_base[oid] + atomicAdd(&obj_fill[oid], 1u);
-    if (!part_tail[oid]) hi = (hi & ((1ull << SID_SHIFT_HI) - 1)) + ((uint64_t)sids[oid] << SID_SHIFT_HI);
-    tkeys[2 * (uint64_t)slot] = lo;
-    tkeys[2 * (uint64_t)slot + 1] = hi;
-    tboxes[slot] = boxes[k];
+    const ulonglong2 key = ((const ulonglong2 *)keys)[k];
+    const float4 box = boxes[k];
+    uint64_t hi = key.y;
+    ObjSlots *o = slots + (uint32_t)((hi >> 26) & OID_MASK);
+    const uint32_t base = o->base, okey = o->key;
+    const uint32_t slot = base + atomicAdd(&o->fill, 1u);
+    if (okey != TAIL_KEY) hi = (hi & ((1ull << SID_SHIFT_HI) - 1)) + ((uint64_t)okey << SID_SHIFT_HI);
+    ((ulonglong2 *)tkeys)[slot] = make_ulonglong2(key.x, hi);
+    tboxes[slot] = box;
 }
 
 /* each record moves to its rank inside its object's range */
 __global__ void k_rank_records(const uint64_t *__restrict__ tkeys, const float4 *__restrict__ tboxes, uint64_t K,
-                               const uint32_t *__restrict__ obj_base, const uint32_t *__restrict__ same_pid_count,
-                               uint64_t *__restrict__ okeys, float4 *__restrict__ oboxes) {
+                               const ObjSlots *__restrict__ slots, uint64_t *__restrict__ okeys,
+                               float4 *__restrict__ oboxes) {
     uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= K) return;
-    uint64_t lo = tkeys[2 * j], hi = tkeys[2 * j + 1];
-    uint32_t oid = (uint32_t)((hi >> 26) & OID_MASK);
-    uint32_t b = obj_base[oid], cnt = same_pid_count[oid];
+    const ulonglong2 *tk = (const ulonglong2 *)tkeys;
+    const ulonglong2 key = tk[j];
+    const float4 box = tboxes[j];
+    const ObjSlots o = slots[(uint32_t)((key.y >> 26) & OID_MASK)];
     uint32_t rank = 0;
-    for (uint32_t i = b; i < b + cnt; i++) {
-        uint64_t l2 = tkeys[2 * (uint64_t)i], h2 = tkeys[2 * (uint64_t)i + 1];
-        rank += (h2 < hi || (h2 == hi && l2 < lo)) ? 1u : 0u;
+#pragma unroll 4
+    for (uint32_t i = 0; i < o.count; i++) {
+        const ulonglong2 x = tk[o.base + i];
+        rank += (x.y < key.y || (x.y == key.y && x.x < key.x)) ? 1u : 0u;
     }
-    uint64_t dst = (uint64_t)b + rank;
-    okeys[2 * dst] = lo;
-    okeys[2 * dst + 1] = hi;
-    oboxes[dst] = tboxes[j];
+    const uint64_t dst = (uint64_t)o.base + rank;
+    ((ulonglong2 *)okeys)[dst] = key;
+    oboxes[dst] = box;
 }
 
 /* ------------------------------------------------------------------ */
@@ -386,13 +400,13 @@ __device__ inline uint32_t block_max_u(uint32_t v, uint32_t *sh) {
 
 /* one workgroup per CTF (blockIdx.x < ctf_count) and one for the oversize
  * buffer (blockIdx.x == ctf_count) */
-__global__ __launch_bounds__(256) void k_limits(const uint64_t *__restrict__ skeys, const float4 *__restrict__ sboxes,
+__global__ __launch_bounds__(LIMIT_THREADS) void k_limits(const uint64_t *__restrict__ skeys, const float4 *__restrict__ sboxes,
                                                 const uint32_t *__restrict__ capacity,
                                                 const uint32_t *__restrict__ ctf_base, uint32_t ctf_count,
                                                 stc_ctf_meta *ctfs, FlushCounters *fc, uint64_t K,
                                                 uint32_t end_time_min, uint32_t cur_time, int compat) {
-    __shared__ float shf[8];
-    __shared__ uint32_t shu[8];
+    __shared__ float shf[LIMIT_THREADS / STC_WAVE];
+    __shared__ uint32_t shu[LIMIT_THREADS / STC_WAVE];
     uint32_t c = blockIdx.x;
     uint32_t n_tail = fc->n_tail;
     uint64_t first, count;
@@ -605,7 +619,7 @@ int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count) {
     size_t N = n;
     if (hipMalloc((void **)&w->mid, N * 8) || hipMalloc((void **)&w->mid_alt, N * 8) ||
         hipMalloc((void **)&w->oids, N * 4) || hipMalloc((void **)&w->oids_alt, N * 4) ||
-        hipMalloc((void **)&w->obj_base, N * 4) || hipMalloc((void **)&w->obj_fill, N * 4) ||
+        hipMalloc((void **)&w->slots, N * sizeof(ObjSlots)) || hipMalloc((void **)&w->obj_first, N * 4) ||
         hipMalloc((void **)&w->capacity, (ctf_count + 1) * 4) || hipMalloc((void **)&w->ctf_base, (ctf_count + 1) * 4) ||
         hipMalloc((void **)&w->ctf_byte_base, (ctf_count + 1) * 8) ||
         hipMalloc((void **)&w->ctfs, ctf_count * sizeof(stc_ctf_meta)) ||
@@ -629,7 +643,7 @@ void stc_flush_free(FlushWork *w) {
     if (w->cs) (void)hipStreamDestroy(w->cs);
     if (w->ready) (void)hipEventDestroy(w->ready);
     if (w->copied) (void)hipEventDestroy(w->copied);
-    void *ptrs[] = {w->chunks, w->sids_out, w->o_bitmap_dev, w->mid, w->mid_alt, w->oids, w->oids_alt, w->obj_base, w->obj_fill, w->capacity, w->ctf_base,
+    void *ptrs[] = {w->chunks, w->sids_out, w->o_bitmap_dev, w->mid, w->mid_alt, w->oids, w->oids_alt, w->slots, w->obj_first, w->capacity, w->ctf_base,
                     w->ctf_byte_base, w->ctfs, w->bitmaps, w->flags, w->part_tail, w->obj_key, w->obj_id, w->obj_cnt,
                     w->scan_temp, w->keys_out, w->boxes_out, w->tkeys, w->tboxes, w->key_bytes};
     for (void *p : ptrs)
@@ -692,14 +706,7 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     /* the previous run's copies read keys_out, key_bytes, bitmaps, sids_out and the counters */
     if (w->pending) FCK(hipStreamWaitEvent(s, w->copied, 0));
     FlushCounters *fc = (FlushCounters *)w->flags;
-    FlushCounters init;
-    memset(&init, 0, sizeof(init));
-    init.oversize_oid_count = a->oversize_oid_count;
-    init.sid_count = 0; /* counted below */
-    FCK(hipMemcpyAsync(fc, &init, sizeof(init), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_count_sids, dim3(std::max<uint32_t>(std::min<uint32_t>(blocks_for(n, 256), 1024), 1)),
-                       dim3(256), 0, s, a->same_pid_count, n, fc);
-    FCK(hipMemsetAsync(w->capacity, 0, (C + 1) * 4, s));
+    hipLaunchKernelGGL(k_flush_init, dim3(1), dim3(256), 0, s, fc, a->oversize_oid_count, w->capacity, C);
     FCK(hipMemsetAsync(w->bitmaps, 0, (size_t)C * 8192, s));
     const uint32_t B = 256;
 
@@ -724,50 +731,47 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
         }
     }
     /* F1 */
-    hipLaunchKernelGGL(k_set_oid, dim3(blocks_for(n, B)), dim3(B), 0, s, n, a->same_pid_count, a->o_boxs, a->sids,
-                       w->mid, w->oids, w->part_tail, a->area_threshold, a->sticky_oversize, sc, fc);
-    hipLaunchKernelGGL(k_str_prepare, dim3(1), dim3(1), 0, s, fc, n, split);
+    const uint32_t few = std::max<uint32_t>(std::min<uint32_t>(blocks_for(n, B), 1024), 1); /* workgroups that update a counter */
+    hipLaunchKernelGGL(k_set_oid, dim3(few), dim3(B), 0, s, n, a->same_pid_count, a->o_boxs, a->sids,
+                       w->mid, w->part_tail, a->area_threshold, a->sticky_oversize, sc, fc);
     FCK(hipGetLastError());
     /* F2: STR over the full 64-bit key (x high, y low), stable from oid order */
-    auto sort_mid = [&](int bits) {
+    auto sort_mid = [&](const uint32_t *vin, int bits) {
         bool in_alt = false;
-        const int rc = stc_radix_sort_u64(w->mid, w->oids, w->mid, w->oids, w->mid_alt, w->oids_alt, n, 0, bits, w->scan_temp, &in_alt, s);
+        const int rc = stc_radix_sort_u64(w->mid, vin, w->mid, w->oids, w->mid_alt, w->oids_alt, n, 0, bits, w->scan_temp, &in_alt, s);
         if (in_alt) {
             std::swap(w->mid, w->mid_alt);
             std::swap(w->oids, w->oids_alt);
         }
         return rc;
     };
-    FRC(sort_mid(sc.on ? (int)sc.str_bits : 64));
-    hipLaunchKernelGGL(k_strip_keys, dim3(blocks_for(n, B)), dim3(B), 0, s, w->mid, n, sc, fc);
-    FRC(sort_mid(sc.on ? (int)sc.strip_bits : 40));
-    hipLaunchKernelGGL(k_make_sid, dim3(blocks_for(n, B)), dim3(B), 0, s, w->oids, n, a->sids, fc);
-    /* F3 */
-    hipLaunchKernelGGL(k_ctf_capacity, dim3(blocks_for(n, B)), dim3(B), 0, s, w->oids, n, a->sids, a->same_pid_count,
-                       w->capacity, C, fc);
+    FRC(sort_mid(nullptr, sc.on ? (int)sc.str_bits : 64));
+    hipLaunchKernelGGL(k_strip_keys, dim3(blocks_for(n, B)), dim3(B), 0, s, w->mid, n, sc, split, fc);
+    FRC(sort_mid(w->oids, sc.on ? (int)sc.strip_bits : 40));
+    /* and F3 */
+    hipLaunchKernelGGL(k_make_sid, dim3(blocks_for(n, B * CAP_ITEMS)), dim3(B), 0, s, w->oids, n, split, a->sids,
+                       a->same_pid_count, w->capacity, C, fc);
     FCK(hipGetLastError());
     FRC(stc_exclusive_scan_u32(w->capacity, w->ctf_base, C, w->ctf_base + C, w->scan_temp, s));
     /* F4: object order (key, oid), slot ranges, scatter, rank */
-    hipLaunchKernelGGL(k_obj_keys, dim3(blocks_for(n, B)), dim3(B), 0, s, n, a->sids, w->part_tail,
-                       a->same_pid_count, w->obj_key, w->obj_id, w->obj_cnt);
+    hipLaunchKernelGGL(k_obj_keys, dim3(few), dim3(B), 0, s, n, a->sids, w->part_tail, a->same_pid_count, w->obj_key, fc);
     bool obj_alt = false; /* 12 bits are two passes: back in obj_key, obj_id */
-    FRC(stc_radix_sort_u32(w->obj_key, w->obj_id, w->obj_key, w->obj_id, (uint32_t *)w->mid_alt, w->oids_alt, n, 12, w->scan_temp,
+    FRC(stc_radix_sort_u32(w->obj_key, nullptr, w->obj_key, w->obj_id, (uint32_t *)w->mid_alt, w->oids_alt, n, 12, w->scan_temp,
                            &obj_alt, s));
     hipLaunchKernelGGL(k_gather_counts, dim3(blocks_for(n, B)), dim3(B), 0, s, w->obj_id, a->same_pid_count, n,
                        w->obj_cnt);
-    FRC(stc_exclusive_scan_u32(w->obj_cnt, w->obj_cnt, n, nullptr, w->scan_temp, s));
-    hipLaunchKernelGGL(k_scatter_base, dim3(blocks_for(n, B)), dim3(B), 0, s, w->obj_id, w->obj_cnt, n, w->obj_base,
-                       w->obj_fill);
-    hipLaunchKernelGGL(k_count_tail, dim3(blocks_for(n, B)), dim3(B), 0, s, w->part_tail, a->same_pid_count, n, fc);
+    FRC(stc_exclusive_scan_u32(w->obj_cnt, w->obj_first, n, nullptr, w->scan_temp, s));
+    hipLaunchKernelGGL(k_obj_slots, dim3(blocks_for(n, B)), dim3(B), 0, s, w->obj_id, w->obj_key, w->obj_cnt, w->obj_first,
+                       n, w->slots);
     if (K) {
         hipLaunchKernelGGL(k_scatter_records, dim3(blocks_for(K, B)), dim3(B), 0, s, a->rec_keys, a->rec_boxes, K,
-                           w->obj_base, w->obj_fill, a->sids, w->part_tail, w->tkeys, w->tboxes);
+                           w->slots, w->tkeys, w->tboxes);
         hipLaunchKernelGGL(k_rank_records, dim3(blocks_for(K, B)), dim3(B), 0, s, w->tkeys, w->tboxes, K,
-                           w->obj_base, a->same_pid_count, w->keys_out, w->boxes_out);
+                           w->slots, w->keys_out, w->boxes_out);
     }
     FCK(hipGetLastError());
     /* F5 */
-    hipLaunchKernelGGL(k_limits, dim3(C + 1), dim3(256), 0, s, w->keys_out, w->boxes_out, w->capacity, w->ctf_base,
+    hipLaunchKernelGGL(k_limits, dim3(C + 1), dim3(LIMIT_THREADS), 0, s, w->keys_out, w->boxes_out, w->capacity, w->ctf_base,
                        C, w->ctfs, fc, K, a->end_time_min, a->cur_time, (int)(a->compat & 1));
     FCK(hipGetLastError());
     /* F6: bit widths on the host */

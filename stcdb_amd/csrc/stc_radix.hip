@@ -299,7 +299,7 @@ static int radix_sort(const K *kin, const uint32_t *vin, K *keys, uint32_t *vals
                       uint32_t n, int lo_bit, int hi_bit, uint32_t *temp, bool *in_alt, hipStream_t s) {
     *in_alt = false;
     const bool in_place = kin == keys;
-    if (n == 0 || (in_place && (n == 1 || hi_bit <= lo_bit))) return 0;
+    if (n == 0 || (in_place && vin && (n == 1 || hi_bit <= lo_bit))) return 0;
     const K *src_k = kin;
     const uint32_t *src_v = vin;
     bool to_alt = in_place;
