@@ -47,7 +47,8 @@ struct FlushWork {
     size_t chunks_cap = 0;
     uint8_t *o_bitmap_dev = nullptr;               /* oversize bitmap as of the flush */
     hipStream_t cs = nullptr;
-    hipEvent_t ready = nullptr, copied = nullptr;
+    hipEvent_t ready = nullptr, copied = nullptr, planned = nullptr;
+    void *head = nullptr;                          /* pinned: the counters, totals and CTFs that the host waits for */
     bool pending = false;                          /* copies queued on cs, maybe still running */
     struct Job {                                   /* copies of the last flush not yet queued */
         uint8_t *dst;

@@ -25,13 +25,18 @@
  *                    (get_o_limit, :926-984). compat bit 0 reduces only the
  *                    records whose in-CTF index mod 64 is below 32, as the
  *                    reference's reduction does.
- *   F6 bits          CTF::get_ctf_bits on the host (step_merge.cpp:140-186)
+ *   F6 bits          CTF::get_ctf_bits (step_merge.cpp:140-186), the CTFs' byte offsets and
+ *                    the chunks of F7
  *   F7 bitmaps+keys  per CTF workgroup: rasterize record boxes into the CTF
  *                    bitmap staged in LDS (cuda_write_bitmap, :986-1021) and
  *                    pack each key to key_bit/8 little-endian bytes
  *                    (write_key_and_mbr, :1073-1107, serialize_mbr :161-171).
- *                    The oversize bitmap (:904-924) is drawn first into CTF 0's
- *                    slot, copied out and cleared, as the reference does.
+ *                    The oversize bitmap (:904-924) is drawn beside them: the
+ *                    reference draws it into CTF 0's slot, copies it out and
+ *                    clears that slot, so that bits past the slot stay in the
+ *                    following CTFs' bitmaps.
+ * Nothing up to F7 needs the host, which waits once, for the widths and the
+ * totals, while F7 runs.
  */
 #include "stc_flush.h"
 #include "stc_table.h"
@@ -45,31 +50,31 @@
 #define BIT_COUNT 65536u
 #define BITMAP_WORDS (BIT_COUNT / 32)
 #define MAX_RASTER (1u << 20)
+#define BK_CHUNK 512u /* records per block of k_bitmap_keys */
 #define TAIL_KEY (1u << 31 | 4095u) /* the placement key of an oversize object: its low 12 bits are sorted by */
 #define LIMIT_THREADS 1024 /* of a CTF's limits: there are few CTFs, and each is read by one workgroup (256: 80 -> 40 us at 5.2M records) */
 
 static inline uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t); }
 
 /* ------------------------------------------------------------------ */
-/* host arithmetic of get_ctf_bits                                     */
+/* arithmetic of get_ctf_bits: IEEE operations, the same on both sides */
 /* ------------------------------------------------------------------ */
 
-static inline uint32_t x86_d2u32(double v) {
+__host__ __device__ static inline uint32_t x86_d2u32(double v) {
     /* host double -> uint32 as x86-64 compilers emit it (cvttsd2si into a
      * 64-bit register, low 32 bits kept) */
     if (!(v > -9223372036854775808.0 && v < 9223372036854775808.0)) return 0;
     return (uint32_t)(uint64_t)(int64_t)v;
 }
-static inline int32_t x86_d2i32(double v) {
+__host__ __device__ static inline int32_t x86_d2i32(double v) {
     if (!(v > -2147483649.0 && v < 2147483648.0)) return (int32_t)0x80000000u;
     return (int32_t)v;
 }
-static inline uint32_t min_bits(uint32_t v) { /* min_bits_to_store (util.h:527-533) */
-    if (v == 0) return 1;
-    return (uint32_t)std::log2((double)v) + 1;
+__host__ __device__ static inline uint32_t min_bits(uint32_t v) { /* min_bits_to_store (util.h:527-533): log2(v) + 1 */
+    return v == 0 ? 1 : 32 - (uint32_t)__builtin_clz(v);
 }
 
-void stc_ctf_bits(stc_ctf_meta *c, const double *map, uint32_t num_objects, uint32_t max_meet_time) {
+__host__ __device__ static void ctf_bits(stc_ctf_meta *c, const double *map, uint32_t num_objects, uint32_t max_meet_time) {
     c->flags &= ~1u;
     c->id_bit = (uint16_t)min_bits(num_objects);
     c->duration_bit = (uint16_t)min_bits(max_meet_time - 1);
@@ -101,6 +106,10 @@ void stc_ctf_bits(stc_ctf_meta *c, const double *map, uint32_t num_objects, uint
     }
     c->bitmap_size = ((uint32_t)c->x_grid * c->y_grid + 7) / 8;
     if (!(c->bitmap_size < 8192)) c->flags |= 1;
+}
+
+void stc_ctf_bits(stc_ctf_meta *c, const double *map, uint32_t num_objects, uint32_t max_meet_time) {
+    ctf_bits(c, map, num_objects, max_meet_time);
 }
 
 /* ------------------------------------------------------------------ */
@@ -157,8 +166,9 @@ __device__ inline void block_add(uint32_t v, uint32_t *to) {
     __syncthreads();
 }
 
-__global__ void k_flush_init(FlushCounters *fc, uint32_t oversize, uint32_t *capacity, uint32_t C) {
+__global__ void k_flush_init(FlushCounters *fc, uint32_t oversize, uint32_t *capacity, uint32_t C, uint32_t *o_bitmap) {
     for (uint32_t i = threadIdx.x; i <= C; i += blockDim.x) capacity[i] = 0;
+    for (uint32_t i = threadIdx.x; i < BITMAP_WORDS; i += blockDim.x) o_bitmap[i] = 0;
     if (threadIdx.x == 0) {
         FlushCounters z{};
         z.oversize_oid_count = oversize;
@@ -398,13 +408,16 @@ __device__ inline uint32_t block_max_u(uint32_t v, uint32_t *sh) {
     return r;
 }
 
+struct MapExtent { double v[4]; };
+
 /* one workgroup per CTF (blockIdx.x < ctf_count) and one for the oversize
  * buffer (blockIdx.x == ctf_count) */
 __global__ __launch_bounds__(LIMIT_THREADS) void k_limits(const uint64_t *__restrict__ skeys, const float4 *__restrict__ sboxes,
                                                 const uint32_t *__restrict__ capacity,
                                                 const uint32_t *__restrict__ ctf_base, uint32_t ctf_count,
                                                 stc_ctf_meta *ctfs, FlushCounters *fc, uint64_t K,
-                                                uint32_t end_time_min, uint32_t cur_time, int compat) {
+                                                uint32_t end_time_min, uint32_t cur_time, int compat, MapExtent map,
+                                                uint32_t n, uint32_t max_meet_time) {
     __shared__ float shf[LIMIT_THREADS / STC_WAVE];
     __shared__ uint32_t shu[LIMIT_THREADS / STC_WAVE];
     uint32_t c = blockIdx.x;
@@ -449,6 +462,7 @@ __global__ __launch_bounds__(LIMIT_THREADS) void k_limits(const uint64_t *__rest
             m.start_time_max = smax;
             m.end_time_min = end_time_min;
             m.end_time_max = cur_time;
+            ctf_bits(&m, map.v, n, max_meet_time);
             ctfs[c] = m;
         } else {
             fc->o_start_min = smin;
@@ -457,26 +471,92 @@ __global__ __launch_bounds__(LIMIT_THREADS) void k_limits(const uint64_t *__rest
     }
 }
 
-/* oversize bitmap into CTF 0's slot (geometry.cu:904-924) */
-__global__ void k_o_bitmap(const float4 *__restrict__ sboxes, uint64_t tail_first, const FlushCounters *fc,
-                           uint32_t *__restrict__ words, uint64_t total_bits, double m0, double m1, double m2,
-                           double m3) {
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= fc->n_tail) return;
-    float4 b = sboxes[tail_first + k];
-    uint32_t low0 = sat_u32(((double)b.x - m0) / (m2 - m0) * 256);
-    uint32_t low1 = sat_u32(((double)b.y - m1) / (m3 - m1) * 256);
-    uint32_t high0 = sat_u32(((double)b.z - m0) / (m2 - m0) * 256);
-    uint32_t high1 = sat_u32(((double)b.w - m1) / (m3 - m1) * 256);
-    for (uint64_t i = low0; i <= high0 && i < total_bits; i++)
-        for (uint64_t j = low1; j <= high1 && i + j * 256 < total_bits; j++) {
-            uint32_t bit = (uint32_t)(i + j * 256);
-            atomicOr(&words[bit >> 5], 1u << (bit & 31));
+/* What the host needs of a flush, in pinned memory; the CTFs follow. */
+struct FlushHead {
+    FlushCounters fc;
+    uint32_t records;            /* in CTFs */
+    uint64_t key_bytes;
+};
+
+/* The CTFs' first packed bytes and the chunks of k_bitmap_keys (of at most
+ * BK_CHUNK records, CTF by CTF), and all of it that the host needs. One
+ * workgroup: two scans over the CTFs, 1024 at a time, and each chunk finding
+ * its CTF among them. */
+__global__ __launch_bounds__(1024) void k_layout(const FlushCounters *__restrict__ fc, const stc_ctf_meta *__restrict__ ctfs,
+                                                 const uint32_t *__restrict__ capacity, const uint32_t *__restrict__ ctf_base,
+                                                 uint32_t C, uint64_t *__restrict__ byte_base, uint4 *__restrict__ chunks,
+                                                 uint32_t chunks_cap, uint32_t *__restrict__ n_chunks, FlushHead *head) {
+    __shared__ uint64_t wbytes[16];
+    __shared__ uint32_t wchunks[16], first[1024];
+    const uint32_t tid = threadIdx.x, lane = tid & (STC_WAVE - 1), wv = tid / STC_WAVE;
+    uint64_t bytes0 = 0;
+    uint32_t chunk0 = 0;
+    for (uint32_t c0 = 0; c0 < C; c0 += 1024) {
+        const uint32_t c = c0 + tid, cap = c < C ? capacity[c] : 0;
+        const uint64_t mine = c < C ? (uint64_t)cap * ctfs[c].key_bit / 8 : 0;
+        const uint32_t nch = cap / BK_CHUNK + (cap % BK_CHUNK != 0);
+        uint64_t b = mine;
+        uint32_t k = nch;
+        for (int o = 1; o < STC_WAVE; o <<= 1) {
+            const uint64_t ub = __shfl_up(b, o, STC_WAVE);
+            const uint32_t uk = __shfl_up(k, o, STC_WAVE);
+            if (lane >= (uint32_t)o) { b += ub; k += uk; }
         }
+        if (lane == STC_WAVE - 1) { wbytes[wv] = b; wchunks[wv] = k; }
+        __syncthreads();
+        uint64_t tb = 0;
+        uint32_t tk = 0;
+        for (uint32_t w = 0; w < 16; w++) {
+            if (w < wv) { b += wbytes[w]; k += wchunks[w]; }
+            tb += wbytes[w];
+            tk += wchunks[w];
+        }
+        if (c < C) byte_base[c] = bytes0 + b - mine;
+        first[tid] = k - nch;
+        __syncthreads();
+        for (uint32_t i = tid; i < tk && chunk0 + i < chunks_cap; i += 1024) {
+            uint32_t lo = 0; /* the last CTF that starts at or before chunk i: those without records start with their successor */
+            for (uint32_t step = 512; step; step >>= 1)
+                if (first[lo + step] <= i) lo += step;
+            const uint32_t at = (i - first[lo]) * BK_CHUNK;
+            chunks[chunk0 + i] = make_uint4(c0 + lo, at, min(BK_CHUNK, capacity[c0 + lo] - at), 0);
+        }
+        bytes0 += tb;
+        chunk0 += tk;
+        __syncthreads();
+    }
+    if (tid == 0) {
+        byte_base[C] = bytes0;
+        *n_chunks = min(chunk0, chunks_cap);
+        head->fc = *fc;
+        head->records = ctf_base[C];
+        head->key_bytes = bytes0;
+    }
+    const uint32_t *src = (const uint32_t *)ctfs;
+    uint32_t *dst = (uint32_t *)(head + 1);
+    for (uint64_t i = tid; i < (uint64_t)C * (sizeof(stc_ctf_meta) / 4); i += 1024) dst[i] = src[i];
+}
+
+/* oversize bitmap (geometry.cu:904-924); bits past its end, into the CTFs' bitmaps after CTF 0's */
+__global__ void k_o_bitmap(const float4 *__restrict__ sboxes, uint64_t K, const FlushCounters *fc,
+                           uint32_t *__restrict__ o_bitmap, uint32_t *__restrict__ words, uint64_t total_bits, MapExtent map) {
+    const uint32_t n_tail = fc->n_tail;
+    const double m0 = map.v[0], m1 = map.v[1], m2 = map.v[2], m3 = map.v[3];
+    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n_tail; k += (uint64_t)gridDim.x * blockDim.x) {
+        float4 b = sboxes[K - n_tail + k];
+        uint32_t low0 = sat_u32(((double)b.x - m0) / (m2 - m0) * 256);
+        uint32_t low1 = sat_u32(((double)b.y - m1) / (m3 - m1) * 256);
+        uint32_t high0 = sat_u32(((double)b.z - m0) / (m2 - m0) * 256);
+        uint32_t high1 = sat_u32(((double)b.w - m1) / (m3 - m1) * 256);
+        for (uint64_t i = low0; i <= high0 && i < total_bits; i++)
+            for (uint64_t j = low1; j <= high1 && i + j * 256 < total_bits; j++) {
+                uint32_t bit = (uint32_t)(i + j * 256);
+                atomicOr(bit < BIT_COUNT ? &o_bitmap[bit >> 5] : &words[bit >> 5], 1u << (bit & 31));
+            }
+    }
 }
 
 /* F7: bitmap and key packing, one workgroup per CTF */
-#define BK_CHUNK 512u /* records per block of k_bitmap_keys */
 
 /* the bits [from, to) of an LDS bitmap (reading a word first, to leave it alone where it has them, took longer) */
 __device__ inline void set_bits_lds(uint32_t *bm, uint32_t from, uint32_t to) {
@@ -506,11 +586,14 @@ __global__ __launch_bounds__(256) void k_bitmap_keys(const uint64_t *__restrict_
                                                      const uint32_t *__restrict__ ctf_base,
                                                      const uint64_t *__restrict__ ctf_byte_base,
                                                      const stc_ctf_meta *__restrict__ ctfs, uint32_t ctf_count,
-                                                     uint64_t nf, uint32_t *__restrict__ words,
-                                                     uint8_t *__restrict__ key_bytes, FlushCounters *fcw) {
+                                                     const uint32_t *__restrict__ n_chunks, uint64_t K, uint64_t room_bytes,
+                                                     uint32_t *__restrict__ words, uint8_t *__restrict__ key_bytes,
+                                                     FlushCounters *fcw) {
     __shared__ uint32_t bm[BITMAP_WORDS];
     __shared__ uint32_t kst[BK_CHUNK * 4 + 1]; /* packed keys, byte after byte */
+    if (blockIdx.x >= *n_chunks || ctf_byte_base[ctf_count] > room_bytes) return; /* the host fails the flush for the latter */
     const uint4 ch = chunks[blockIdx.x];
+    const uint64_t nf = K - fcw->n_tail;
     const uint32_t c = ch.x, k0 = ch.y, kn = ch.z;
     for (uint32_t i = threadIdx.x; i < BITMAP_WORDS; i += blockDim.x) bm[i] = 0;
     __syncthreads();
@@ -593,9 +676,13 @@ __global__ __launch_bounds__(256) void k_bitmap_keys(const uint64_t *__restrict_
         if (bm[i]) atomicOr(&gw[i], bm[i]);
 }
 
-__global__ void k_fill_obox2(uint4 *a, uint32_t n) {
+/* the memtable's per-object state, empty (geometry.cu:2111-2131) */
+__global__ void k_reset_objects(uint32_t n, uint32_t *same_pid_count, uint16_t *sids, uint4 *o_boxs) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = make_uint4(100000000u, 100000000u, 0u, 0u);
+    if (i >= n) return;
+    same_pid_count[i] = 0;
+    sids[i] = 0;
+    o_boxs[i] = make_uint4(100000000u, 100000000u, 0u, 0u);
 }
 
 /* ------------------------------------------------------------------ */
@@ -630,7 +717,9 @@ int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count) {
         return STC_E_HIP;
     if (hipStreamCreateWithFlags(&w->cs, hipStreamNonBlocking) ||
         hipEventCreateWithFlags(&w->ready, hipEventDisableTiming) ||
-        hipEventCreateWithFlags(&w->copied, hipEventDisableTiming))
+        hipEventCreateWithFlags(&w->copied, hipEventDisableTiming) ||
+        hipEventCreateWithFlags(&w->planned, hipEventDisableTiming) ||
+        hipHostMalloc((void **)&w->head, sizeof(FlushHead) + ctf_count * sizeof(stc_ctf_meta), hipHostMallocDefault))
         return STC_E_HIP;
     w->scan_temp_words = stc_radix_temp_words(n) + 64;
     if (hipMalloc((void **)&w->scan_temp, w->scan_temp_words * 4)) return STC_E_HIP;
@@ -643,6 +732,8 @@ void stc_flush_free(FlushWork *w) {
     if (w->cs) (void)hipStreamDestroy(w->cs);
     if (w->ready) (void)hipEventDestroy(w->ready);
     if (w->copied) (void)hipEventDestroy(w->copied);
+    if (w->planned) (void)hipEventDestroy(w->planned);
+    if (w->head) (void)hipHostFree(w->head);
     void *ptrs[] = {w->chunks, w->sids_out, w->o_bitmap_dev, w->mid, w->mid_alt, w->oids, w->oids_alt, w->slots, w->obj_first, w->capacity, w->ctf_base,
                     w->ctf_byte_base, w->ctfs, w->bitmaps, w->flags, w->part_tail, w->obj_key, w->obj_id, w->obj_cnt,
                     w->scan_temp, w->keys_out, w->boxes_out, w->tkeys, w->tboxes, w->key_bytes};
@@ -706,8 +797,10 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     /* the previous run's copies read keys_out, key_bytes, bitmaps, sids_out and the counters */
     if (w->pending) FCK(hipStreamWaitEvent(s, w->copied, 0));
     FlushCounters *fc = (FlushCounters *)w->flags;
-    hipLaunchKernelGGL(k_flush_init, dim3(1), dim3(256), 0, s, fc, a->oversize_oid_count, w->capacity, C);
+    hipLaunchKernelGGL(k_flush_init, dim3(1), dim3(256), 0, s, fc, a->oversize_oid_count, w->capacity, C,
+                       (uint32_t *)w->o_bitmap_dev);
     FCK(hipMemsetAsync(w->bitmaps, 0, (size_t)C * 8192, s));
+    const MapExtent map{{a->map[0], a->map[1], a->map[2], a->map[3]}};
     const uint32_t B = 256;
 
     /* compact STR keys from the map box: every record box lies inside it, so every object's quantised
@@ -772,61 +865,44 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     FCK(hipGetLastError());
     /* F5 */
     hipLaunchKernelGGL(k_limits, dim3(C + 1), dim3(LIMIT_THREADS), 0, s, w->keys_out, w->boxes_out, w->capacity, w->ctf_base,
-                       C, w->ctfs, fc, K, a->end_time_min, a->cur_time, (int)(a->compat & 1));
+                       C, w->ctfs, fc, K, a->end_time_min, a->cur_time, (int)(a->compat & 1), map, n, a->max_meet_time);
+    /* F6 */
+    const uint64_t most = K / BK_CHUNK + C; /* chunks */
+    if (most > w->chunks_cap) {
+        if (w->chunks) FCK(hipFree(w->chunks));
+        w->chunks = nullptr;
+        w->chunks_cap = 0;
+        FCK(hipMalloc((void **)&w->chunks, (most + most / 2) * sizeof(uint4)));
+        w->chunks_cap = most + most / 2;
+    }
+    uint32_t *n_chunks = (uint32_t *)(fc + 1);
+    hipLaunchKernelGGL(k_layout, dim3(1), dim3(1024), 0, s, fc, w->ctfs, w->capacity, w->ctf_base, C, w->ctf_byte_base,
+                       w->chunks, (uint32_t)most, n_chunks, (FlushHead *)w->head);
     FCK(hipGetLastError());
-    /* F6: bit widths on the host */
-    FlushCounters hfc;
-    std::vector<stc_ctf_meta> ctfs(C);
-    std::vector<uint32_t> cap(C + 1), base(C + 1);
-    FCK(hipMemcpyAsync(&hfc, fc, sizeof(hfc), hipMemcpyDeviceToHost, s));
-    FCK(hipMemcpyAsync(ctfs.data(), w->ctfs, C * sizeof(stc_ctf_meta), hipMemcpyDeviceToHost, s));
-    FCK(hipMemcpyAsync(cap.data(), w->capacity, C * 4, hipMemcpyDeviceToHost, s));
-    FCK(hipMemcpyAsync(base.data(), w->ctf_base, (C + 1) * 4, hipMemcpyDeviceToHost, s));
-    FCK(hipStreamSynchronize(s));
+    FCK(hipEventRecord(w->planned, s));
+    /* F7 */
+    uint32_t *words = (uint32_t *)w->bitmaps;
+    hipLaunchKernelGGL(k_o_bitmap, dim3(64), dim3(B), 0, s, w->boxes_out, K, fc, (uint32_t *)w->o_bitmap_dev, words,
+                       (uint64_t)C * BIT_COUNT, map);
+    hipLaunchKernelGGL(k_bitmap_keys, dim3((uint32_t)most), dim3(256), 0, s, w->keys_out, w->boxes_out, w->chunks,
+                       w->ctf_base, w->ctf_byte_base, w->ctfs, C, n_chunks, K, w->rec_cap * 16, words, w->key_bytes, fc);
+    FCK(hipGetLastError());
+    FCK(hipEventSynchronize(w->planned));
+    const FlushHead head = *(const FlushHead *)w->head;
+    const FlushCounters &hfc = head.fc;
     if (hfc.str_wide && sc.on) { /* cannot happen for records inside the map; redone over the full keys */
         w->str_full = true;
         return stc_flush_run(w, a, out, s);
     }
-    std::vector<uint64_t> byte_base(C + 1, 0);
-    for (uint32_t c = 0; c < C; c++) {
-        stc_ctf_bits(&ctfs[c], a->map, n, a->max_meet_time);
-        byte_base[c + 1] = byte_base[c] + (uint64_t)cap[c] * ctfs[c].key_bit / 8;
-    }
+    const stc_ctf_meta *hctfs = (const stc_ctf_meta *)((const FlushHead *)w->head + 1);
+    std::vector<stc_ctf_meta> ctfs(hctfs, hctfs + C);
     const uint64_t n_tail = hfc.n_tail, nf = K - n_tail;
     uint32_t flags = 0;
     if (hfc.bad) flags |= 2;
     if (!(n_tail < a->kv_restriction / 100)) flags |= 4;
-    if (base[C] != nf) flags |= 2;
+    if (head.records != nf) flags |= 2;
     for (auto &m : ctfs) m.flags |= flags;
-    if (byte_base[C] > w->rec_cap * 16) return stc_hip_fail(hipErrorOutOfMemory, "key bytes", __FILE__, __LINE__);
-    FCK(hipMemcpyAsync(w->ctfs, ctfs.data(), C * sizeof(stc_ctf_meta), hipMemcpyHostToDevice, s));
-    FCK(hipMemcpyAsync(w->ctf_byte_base, byte_base.data(), (C + 1) * 8, hipMemcpyHostToDevice, s));
-    /* F7: oversize bitmap first (CTF 0's slot, then copied out and cleared) */
-    uint32_t *words = (uint32_t *)w->bitmaps;
-    uint64_t total_bits = (uint64_t)C * BIT_COUNT;
-    if (n_tail)
-        hipLaunchKernelGGL(k_o_bitmap, dim3(blocks_for(n_tail, B)), dim3(B), 0, s, w->boxes_out, nf, fc, words,
-                           total_bits, a->map[0], a->map[1], a->map[2], a->map[3]);
-    FCK(hipMemcpyAsync(w->o_bitmap_dev, w->bitmaps, 8192, hipMemcpyDeviceToDevice, s));
-    FCK(hipMemsetAsync(w->bitmaps, 0, 8192, s));
-    /* chunks of at most BK_CHUNK records, CTF by CTF */
-    std::vector<uint4> chunks;
-    for (uint32_t c = 0; c < C; c++)
-        for (uint32_t k = 0; k < cap[c]; k += BK_CHUNK) chunks.push_back(make_uint4(c, k, std::min(BK_CHUNK, cap[c] - k), 0));
-    if (!chunks.empty()) {
-        if (chunks.size() > w->chunks_cap) {
-            if (w->chunks) FCK(hipFree(w->chunks));
-            w->chunks = nullptr;
-            w->chunks_cap = 0;
-            size_t nc = chunks.size() + chunks.size() / 2 + 64;
-            FCK(hipMalloc((void **)&w->chunks, nc * sizeof(uint4)));
-            w->chunks_cap = nc;
-        }
-        FCK(hipMemcpyAsync(w->chunks, chunks.data(), chunks.size() * sizeof(uint4), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_bitmap_keys, dim3((uint32_t)chunks.size()), dim3(256), 0, s, w->keys_out, w->boxes_out,
-                           w->chunks, w->ctf_base, w->ctf_byte_base, w->ctfs, C, nf, words, w->key_bytes, fc);
-        FCK(hipGetLastError());
-    }
+    if (head.key_bytes > w->rec_cap * 16) return stc_hip_fail(hipErrorOutOfMemory, "key bytes", __FILE__, __LINE__);
     FCK(hipMemcpyAsync(w->sids_out, a->sids, (size_t)n * 2, hipMemcpyDeviceToDevice, s));
 
     /* outputs: one pinned block, filled on the copy stream */
@@ -835,7 +911,7 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     RunLayout &L = out->lay;
     size_t off = 0;
     auto place = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
-    L.key_bytes = place(byte_base[C]);
+    L.key_bytes = place(head.key_bytes);
     L.bitmaps = place((size_t)C * 8192);
     L.o_bitmap = place(8192);
     L.sids = place((size_t)n * 2);
@@ -847,10 +923,8 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     L.total = off;
     out->blk = out->acquire(out->acquire_ctx, L.total);
     if (!out->blk.p) return stc_hip_fail(hipErrorOutOfMemory, "pinned run buffer", __FILE__, __LINE__);
-    if (a->reset_memtable) { /* geometry.cu:2111-2131 */
-        FCK(hipMemsetAsync(a->same_pid_count, 0, 4ull * n, s));
-        FCK(hipMemsetAsync(a->sids, 0, 2ull * n, s));
-        hipLaunchKernelGGL(k_fill_obox2, dim3(blocks_for(n, 256)), dim3(256), 0, s, a->o_boxs, n);
+    if (a->reset_memtable) {
+        hipLaunchKernelGGL(k_reset_objects, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a->same_pid_count, a->sids, a->o_boxs);
         FCK(hipGetLastError());
     }
     /* the copies to the pinned block wait for stc_flush_release */
@@ -859,7 +933,7 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     j.key_bytes_at = L.key_bytes; j.bitmaps_at = L.bitmaps; j.o_bitmap_at = L.o_bitmap; j.sids_at = L.sids;
     j.o_keys_at = L.o_keys; j.o_boxes_at = L.o_boxes; j.sorted_keys_at = L.sorted_keys;
     j.sorted_boxes_at = L.sorted_boxes; j.counters_at = L.counters;
-    j.key_bytes = byte_base[C];
+    j.key_bytes = head.key_bytes;
     j.nf = nf;
     j.n_tail = n_tail;
     j.ctf_count = C;
@@ -881,7 +955,7 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     info.cur_time = a->cur_time;
     info.sid_count = hfc.sid_count;
     info.oversize_oid_count = hfc.oversize_oid_count;
-    info.key_bytes = byte_base[C];
+    info.key_bytes = head.key_bytes;
     return 0;
 }
 
