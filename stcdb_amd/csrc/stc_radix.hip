@@ -5,7 +5,9 @@
  *   histogram : each workgroup counts the digits of its tile of keys in LDS;
  *   offsets   : a sort of up to 128 tiles lets every scatter workgroup add up
  *               the tiles' histograms itself; a larger one writes them
- *               digit-major (digit * tiles + tile) and scans that table;
+ *               digit-major (digit * tiles + tile) and scans each digit's row
+ *               with a workgroup of its own, the 256 totals being added up by
+ *               the scatter;
  *   scatter   : each workgroup ranks its tile stably and moves it. A wave holds
  *               its stretch of the tile in registers, all loads issued before
  *               the first ranking, and ranks it 64 keys a round by peer masks
@@ -23,7 +25,7 @@
  * of 13), 2048 up to 2M and 4096 above. With 4096-key tiles ranked 256 keys a
  * round, four barriers and a load in each, a pass over 50k keys took five
  * launches and 27 us and takes two and 9 us so; one over 1M keys took six and
- * 37 us and takes four and 22 us.
+ * 37 us and takes three and 19 us (four and 22 with a scan of the whole table).
  */
 #include "stc_internal.h"
 
@@ -49,7 +51,7 @@ size_t stc_radix_temp_words(uint32_t n) {
     const size_t t0 = ceil_div(n, RS_THREADS * 16), t1 = ceil_div(few, RS_THREADS * 8), t2 = RS_SMALL / (RS_THREADS * 4);
     const size_t hist = RS_BINS * (t0 > t1 ? (t0 > t2 ? t0 : t2) : (t1 > t2 ? t1 : t2));
     const size_t s1 = ceil_div(n > hist ? n : hist, SCAN_TILE);
-    return hist + s1 + ceil_div(s1, SCAN_TILE) + 64;
+    return hist + RS_BINS + s1 + ceil_div(s1, SCAN_TILE) + 64;
 }
 
 /* ---------------- exclusive scan ---------------- */
@@ -170,8 +172,32 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const K *__restrict__ ke
     hist[by_tile ? (uint64_t)blockIdx.x * RS_BINS + threadIdx.x : (uint64_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
 }
 
-/* by_tile: offs holds the tiles' histograms; else the scanned digit-major
- * table. vin null: the values are the keys' places. */
+/* Each digit's row of the digit-major table (a workgroup each) to the keys of
+ * the digit in the tiles before, and the rows' totals. */
+__global__ __launch_bounds__(RS_THREADS) void k_rs_rows(uint32_t *__restrict__ hist, uint32_t tiles, uint32_t *__restrict__ totals) {
+    uint32_t *row = hist + (uint64_t)blockIdx.x * tiles;
+    uint32_t before = 0;
+    for (uint32_t t0 = 0; t0 < tiles; t0 += RS_THREADS * SCAN_ITEMS) {
+        const uint32_t base = t0 + threadIdx.x * SCAN_ITEMS;
+        uint32_t v[SCAN_ITEMS], s = 0, tot;
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; k++) {
+            v[k] = base + k < tiles ? row[base + k] : 0;
+            s += v[k];
+        }
+        uint32_t ex = before + block_excl_scan(s, &tot);
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; k++) {
+            if (base + k < tiles) row[base + k] = ex;
+            ex += v[k];
+        }
+        before += tot;
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = before;
+}
+
+/* by_tile: offs holds the tiles' histograms; else the digit-major table of
+ * k_rs_rows and behind it the totals. vin null: the values are the keys' places. */
 template <typename K, int ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                             K *__restrict__ kout, uint32_t *__restrict__ vout, uint32_t n,
@@ -208,8 +234,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K *__restrict__
         }
         b0 = pre + block_excl_scan(all, &tot);
     } else {
-        b0 = offs[(uint64_t)tid * tiles + blockIdx.x];
-        __syncthreads();
+        const uint32_t pre = offs[(uint64_t)tid * tiles + blockIdx.x];
+        b0 = pre + block_excl_scan(offs[(uint64_t)RS_BINS * tiles + tid], &tot);
     }
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (STC_WAVE - lane));
     uint32_t rank[ITEMS];
@@ -285,8 +311,8 @@ static int radix_pass(const K *kin, const uint32_t *vin, K *kout, uint32_t *vout
     hipLaunchKernelGGL((k_rs_hist<K, ITEMS>), dim3(tiles), dim3(RS_THREADS), 0, s, kin, n, shift, temp, tiles, by_tile);
     STC_CHECK(hipGetLastError());
     if (!by_tile) {
-        const int rc = stc_exclusive_scan_u32(temp, temp, RS_BINS * tiles, nullptr, temp + (size_t)RS_BINS * tiles, s);
-        if (rc) return rc;
+        hipLaunchKernelGGL(k_rs_rows, dim3(RS_BINS), dim3(RS_THREADS), 0, s, temp, tiles, temp + (size_t)RS_BINS * tiles);
+        STC_CHECK(hipGetLastError());
     }
     hipLaunchKernelGGL((k_rs_scatter<K, ITEMS>), dim3(tiles), dim3(RS_THREADS), 0, s, kin, vin, kout, vout, n, shift,
                        (const uint32_t *)temp, tiles, by_tile);
