@@ -59,8 +59,7 @@
 #include <vector>
 #include <type_traits>
 
-/* 4-byte aligned vectors for the streaming stores of the 12-byte slots and 28-byte buckets */
-typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+/* a 4-byte aligned vector for the streaming stores of the 12-byte slots */
 typedef uint32_t u32x3u __attribute__((ext_vector_type(3), aligned(4)));
 
 #define ONE_DIM 16384u
@@ -569,7 +568,7 @@ __global__ void k_units_emit(const uint32_t *__restrict__ lp, const double2 *__r
 /* meetings: pairs grouped by owner, merged with the live meetings      */
 /* ------------------------------------------------------------------ */
 /*
- * The live meetings after a step are an array of 28 B buckets sorted by key
+ * The live meetings after a step are arrays (28 B a meeting) sorted by key
  * (oid1 << 32 | oid2): one segment per owner oid1 (the pair's smaller id), in
  * owner order, each segment's live buckets followed by tombstones for the
  * step's duplicate or rejected pairs. A step finds its pairs owner by owner,
@@ -1828,7 +1827,7 @@ __global__ void k_tile_owner(const uint32_t *__restrict__ poff, uint32_t n, uint
  * two segments mostly hold the same partners) and widens by doubling steps
  * until it brackets the key, so a few dependent reads usually suffice. */
 template <class S>
-__global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const Bucket *__restrict__ mold,
+__global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const unsigned long long *__restrict__ mold,
                               const uint32_t *__restrict__ ooff, const uint32_t *__restrict__ poff, uint64_t n_o,
                               uint32_t n_tiles, const uint32_t *__restrict__ towner, uint32_t *__restrict__ tb) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1847,11 +1846,11 @@ __global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const Buck
     if (hi > lo && np_a) {
         /* bracket [lo, hi) around the scaled guess g: keys below lo are < key, keys from hi on are >= key */
         const uint32_t g = lo + (uint32_t)(((uint64_t)(first - p0) * (hi - lo)) / np_a);
-        if (g < hi && mold[g].key < key) {
+        if (g < hi && mold[g] < key) {
             uint32_t step = 1, l = g + 1;
             while (l < hi) {
                 const uint32_t probe = min(l + step - 1, hi - 1);
-                if (mold[probe].key < key) {
+                if (mold[probe] < key) {
                     l = probe + 1;
                     step <<= 1;
                 } else {
@@ -1864,7 +1863,7 @@ __global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const Buck
             uint32_t step = 1, r = g; /* mold[r] >= key or r == hi */
             while (r > lo) {
                 const uint32_t probe = r - min(step, r - lo);
-                if (mold[probe].key < key) {
+                if (mold[probe] < key) {
                     lo = probe + 1;
                     break;
                 }
@@ -1876,7 +1875,7 @@ __global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const Buck
     }
     while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (mold[mid].key < key) lo = mid + 1;
+        if (mold[mid] < key) lo = mid + 1;
         else hi = mid;
     }
     tb[t] = lo;
@@ -1892,11 +1891,25 @@ __device__ inline uint32_t lower_bound_u64(const unsigned long long *s, uint32_t
     return lo;
 }
 
-__device__ inline uint32_t lower_bound_bucket(const Bucket *s, uint32_t n, unsigned long long v) {
+/* a tile's previous meetings where they are staged, or in device memory from `first` on */
+struct StagedMeets {
+    const Bucket *p;
+    __device__ inline unsigned long long key(uint32_t i) const { return p[i].key; }
+    __device__ inline Bucket at(uint32_t i) const { return p[i]; }
+};
+struct MeetsFrom {
+    Meets m;
+    uint64_t first;
+    __device__ inline unsigned long long key(uint32_t i) const { return m.key(first + i); }
+    __device__ inline Bucket at(uint32_t i) const { return m.at(first + i); }
+};
+
+template <class M>
+__device__ inline uint32_t lower_bound_bucket(const M &s, uint32_t n, unsigned long long v) {
     uint32_t lo = 0, hi = n;
     while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (s[mid].key < v) lo = mid + 1;
+        if (s.key(mid) < v) lo = mid + 1;
         else hi = mid;
     }
     return lo;
@@ -1917,8 +1930,11 @@ __device__ inline uint32_t lower_bound_bucket(const Bucket *s, uint32_t n, unsig
 
 template <class S>
 __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, uint64_t n_p,
-                                                    const Bucket *__restrict__ mold, const uint32_t *__restrict__ tb,
-                                                    uint32_t n_tiles, Bucket *__restrict__ mnew, MergeArgs ma,
+                                                    const unsigned long long *__restrict__ okey,
+                                                    const uint32_t *__restrict__ ostart, const uint4 *__restrict__ ombr,
+                                                    const uint32_t *__restrict__ tb, uint32_t n_tiles,
+                                                    unsigned long long *__restrict__ nkey, uint32_t *__restrict__ nstart,
+                                                    uint4 *__restrict__ nmbr, MergeArgs ma,
                                                     MemtableDev mt, const float2 *__restrict__ posf,
                                                     const uint32_t *__restrict__ poff, const uint32_t *__restrict__ towner,
                                                     uint32_t n_obj, Counters *cnt) {
@@ -1969,7 +1985,11 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
         for (int k = 0; k < SPF; k++) ps[k] = pn[min<uint64_t>(i0 + lane + k * STC_WAVE, plast)];
         const uint32_t olast = o1 > o0 ? o1 - 1 : (n_o ? min(o0, n_o - 1) : 0u);
 #pragma unroll
-        for (int k = 0; k < OPF; k++) po[k] = mold[min(o0 + lane + k * STC_WAVE, olast)];
+        for (int k = 0; k < OPF; k++) {
+            const uint32_t i = min(o0 + lane + k * STC_WAVE, olast);
+            const uint4 m = ombr[i];
+            po[k] = Bucket{okey[i], ostart[i], {m.x, m.y, m.z, m.w}};
+        }
         /* the starts of the 64 owners after a0 (a0 owns the tile's first slot), read with the rest */
         uint32_t bst = 0;
         if constexpr (SLOTS) {
@@ -2040,7 +2060,7 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
         }
         /* the join, instantiated for previous meetings in LDS and, for a range longer than
          * OCAP, in global memory (so the LDS searches wait on nothing but LDS) */
-        auto join = [&](const Bucket *obk) {
+        auto join = [&](auto obk) {
             /* every lane joins its slots, in range or not (lanes past np store nothing), so that no
              * load of the tile is moved behind a branch */
 #pragma unroll
@@ -2054,7 +2074,7 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
                 const uint32_t j = lower_bound_bucket(obk, no, key);
                 const uint4 q = slot_mbr(e, posf, own[k]);
                 const uint32_t q0 = q.x, q1 = q.y, q2 = q.z, q3 = q.w;
-                const Bucket ob = obk[j < no ? j : (no ? no - 1 : 0u)];
+                const Bucket ob = obk.at(j < no ? j : (no ? no - 1 : 0u));
                 const bool cont = j < no && ob.key == key;
                 Bucket nb;
                 nb.key = key;
@@ -2069,12 +2089,12 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
                         if (cont) n_cont++;
                         else n_fresh++;
                     }
-                    /* streamed out past the caches: the array is read again only by the next step */
-                    uint32_t *d = (uint32_t *)(mnew + i0 + i);
-                    const u32x4u lo = {(uint32_t)nb.key, (uint32_t)(nb.key >> 32), nb.start, nb.mbr[0]};
-                    const u32x3u hi = {nb.mbr[1], nb.mbr[2], nb.mbr[3]};
-                    __builtin_nontemporal_store(lo, (u32x4u *)d);
-                    __builtin_nontemporal_store(hi, (u32x3u *)(d + 4));
+                    /* streamed out past the caches: the arrays are read again only by the next step */
+                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                    const u32x4 mb = {nb.mbr[0], nb.mbr[1], nb.mbr[2], nb.mbr[3]};
+                    __builtin_nontemporal_store(nb.key, nkey + i0 + i);
+                    __builtin_nontemporal_store(nb.start, nstart + i0 + i);
+                    __builtin_nontemporal_store(mb, (u32x4 *)(nmbr + i0 + i));
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -2083,12 +2103,12 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
                 bool emit = false;
                 Bucket ob;
                 if (j < no) {
-                    const unsigned long long key = obk[j].key;
+                    const unsigned long long key = obk.key(j);
                     if ((uint32_t)key != DEAD_B) {
                         const uint32_t k = lower_bound_u64(pk, np, key);
                         if (!(k < np && pk[k] == key)) {
                             n_exp++;
-                            ob = obk[j];
+                            ob = obk.at(j);
                             emit = meeting_emits(ob, ma);
                         }
                     }
@@ -2116,8 +2136,8 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
                 }
             }
         };
-        if (oin) join(ob_l);
-        else join(mold + o0);
+        if (oin) join(StagedMeets{ob_l});
+        else join(MeetsFrom{Meets{okey, ostart, ombr}, o0});
         __builtin_amdgcn_wave_barrier(); /* the wave's LDS is reused by its next tile */
     }
     /* the waves' last staged meetings with one reservation, and one update of each counter, per
@@ -2166,13 +2186,13 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
 #define LCHUNK 16u     /* export tiles of a chunk */
 
 /* live buckets of each export tile */
-__global__ __launch_bounds__(256) void k_live_tiles(const Bucket *__restrict__ t, uint64_t n, uint32_t *__restrict__ tiles) {
+__global__ __launch_bounds__(256) void k_live_tiles(const unsigned long long *__restrict__ keys, uint64_t n, uint32_t *__restrict__ tiles) {
     __shared__ uint32_t wsum[256 / STC_WAVE];
     const int lane = threadIdx.x & (STC_WAVE - 1), wv = threadIdx.x / STC_WAVE;
     uint32_t c = 0;
     for (uint32_t r = 0; r < LTILE / 256; r++) {
         const uint64_t i = (uint64_t)blockIdx.x * LTILE + r * 256 + threadIdx.x;
-        c += (uint32_t)__popcll(__ballot(i < n && (uint32_t)t[i].key != DEAD_B));
+        c += (uint32_t)__popcll(__ballot(i < n && (uint32_t)keys[i] != DEAD_B));
     }
     if (lane == 0) wsum[wv] = c;
     __syncthreads();
@@ -2191,7 +2211,7 @@ __global__ __launch_bounds__(256) void k_live_tiles(const Bucket *__restrict__ t
  * Bound by the link to the host (28 or 32 bytes a meeting). */
 enum LiveForm { LIVE_FIELDS, LIVE_UNITS, LIVE_KEYS };
 template <LiveForm FORM>
-__global__ __launch_bounds__(256) void k_live_out(const Bucket *__restrict__ t, uint64_t n, uint32_t tile0,
+__global__ __launch_bounds__(256) void k_live_out(Meets t, uint64_t n, uint32_t tile0,
                                                   const uint32_t *__restrict__ tbase, uint64_t base0,
                                                   const float2 *__restrict__ posf, uint32_t now, uint8_t *__restrict__ out) {
     __shared__ uint32_t wsum[256 / STC_WAVE];
@@ -2202,7 +2222,10 @@ __global__ __launch_bounds__(256) void k_live_out(const Bucket *__restrict__ t, 
         const uint64_t i = (uint64_t)tile * LTILE + r * 256 + threadIdx.x;
         Bucket b;
         b.key = DEAD_B;
-        if (i < n) b = t[i];
+        if (i < n) {
+            if constexpr (FORM == LIVE_FIELDS) b = t.at(i);
+            else b.key = t.key(i);
+        }
         const bool live = bucket_live(b);
         const uint64_t m = __ballot(live);
         if (lane == 0) wsum[wv] = (uint32_t)__popcll(m);
@@ -2333,11 +2356,11 @@ __device__ inline void na_match(uint8_t *sc, uint32_t n, uint32_t pid, uint32_t 
 }
 
 /* live meetings of the last step established by t_est (start <= t_est) */
-__global__ void k_na_live(const Bucket *__restrict__ t, uint64_t nb, uint32_t last_t, uint32_t t_est, uint8_t *sc,
+__global__ void k_na_live(Meets t, uint64_t nb, uint32_t last_t, uint32_t t_est, uint8_t *sc,
                           uint32_t n) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += stride) {
-        const Bucket b = t[i];
+        const Bucket b = t.at(i);
         if (!bucket_live(b) || b.start > t_est) continue;
         const uint32_t a = (uint32_t)(b.key >> 32), c = (uint32_t)b.key;
         na_match(sc, n, a, c, b, last_t);
@@ -2358,6 +2381,16 @@ struct DBuf {
         return 0;
     }
     void release() { if (p) hipFree(p); p = nullptr; cap = 0; }
+};
+
+/* a step's meetings */
+struct MeetBuf {
+    DBuf<unsigned long long> keys;
+    DBuf<uint32_t> starts;
+    DBuf<uint4> mbrs;
+    int ensure(size_t n) { return keys.ensure(n) || starts.ensure(n) || mbrs.ensure(n) ? -1 : 0; }
+    void release() { keys.release(); starts.release(); mbrs.release(); }
+    Meets view() const { return Meets{keys.p, starts.p, mbrs.p}; }
 };
 
 /* A flushed run: metadata on the host, payload in a pinned block that the
@@ -2473,7 +2506,7 @@ struct StcCtx {
     bool pairs_boxed = false;            /* the last step's pairs are in pbox (replayed units), not pnew */
     DBuf<uint32_t> psrc;                 /* collected pair sources, a run per owner */
     DBuf<uint2> pkrun;                   /* per owner in leaf order: its run of psrc (start, length) */
-    DBuf<Bucket> meet[2];
+    MeetBuf meet[2];
     DBuf<uint32_t> moff[2];
     DBuf<uint32_t> tbounds;              /* merge tiles' ranges in the previous meetings */
     DBuf<uint32_t> towner;               /* merge tiles' first owners (the slots carry no owner) */
@@ -2552,7 +2585,7 @@ struct StcCtx {
 /* publish the state after a step (or a change of the runs) to queries */
 static void publish(StcCtx *c) {
     QueryState st;
-    st.table = c->meet[c->cur].p;
+    st.meets = c->meet[c->cur].view();
     st.nb = c->mlen;
     st.last_t = c->last_t;
     st.stepped = c->stepped ? 1 : 0;
@@ -2708,7 +2741,8 @@ static int export_live(StcCtx *c, uint64_t cap, Take take) {
     std::vector<uint32_t> base; /* first output of each chunk */
     if (c->last_live != c->mlen) { /* dead buckets: the tiles' outputs by a scan */
         if (c->xtiles.ensure(tiles + stc_radix_temp_words((uint32_t)tiles))) return fail(c, STC_E_CAPACITY, "export tiles");
-        hipLaunchKernelGGL(k_live_tiles, dim3((uint32_t)tiles), dim3(256), 0, c->s, (const Bucket *)c->meet[c->cur].p, c->mlen, c->xtiles.p);
+        hipLaunchKernelGGL(k_live_tiles, dim3((uint32_t)tiles), dim3(256), 0, c->s,
+                           (const unsigned long long *)c->meet[c->cur].keys.p, c->mlen, c->xtiles.p);
         CK(hipGetLastError());
         CKRC(stc_exclusive_scan_u32(c->xtiles.p, c->xtiles.p, (uint32_t)tiles, nullptr, c->xtiles.p + tiles, c->s));
         base.resize(tiles);
@@ -2726,7 +2760,7 @@ static int export_live(StcCtx *c, uint64_t cap, Take take) {
         [&](uint64_t k, uint8_t *buf) {
             const uint64_t t0 = k * LCHUNK;
             hipLaunchKernelGGL(k_live_out<FORM>, dim3((uint32_t)std::min<uint64_t>(LCHUNK, tiles - t0)), dim3(256), 0, c->s,
-                               (const Bucket *)c->meet[c->cur].p, c->mlen, (uint32_t)t0, tbase, out_of(t0),
+                               c->meet[c->cur].view(), c->mlen, (uint32_t)t0, tbase, out_of(t0),
                                (const float2 *)c->posf.p, c->last_t, buf);
         },
         [&](uint64_t k, const uint8_t *buf) {
@@ -3408,14 +3442,14 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     if (c->tbounds.ensure(n_tiles + 1ull) || c->towner.ensure(n_tiles)) return fail(c, STC_E_CAPACITY, "merge tile bounds");
     if (c->pairs_boxed) {
         hipLaunchKernelGGL(k_tile_bounds<PairHit>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairHit *)c->pbox.p, c->plen, (const Bucket *)c->meet[cu].p,
+                           (const PairHit *)c->pbox.p, c->plen, (const unsigned long long *)c->meet[cu].keys.p,
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)nullptr, c->tbounds.p);
     } else {
         hipLaunchKernelGGL(k_tile_owner, dim3(blocks_for(c->n, 256)), dim3(256), 0, s, (const uint32_t *)c->moff[nx].p,
                            c->n, c->towner.p);
         hipLaunchKernelGGL(k_tile_bounds<PairSlot>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairSlot *)c->pnew.p, c->plen, (const Bucket *)c->meet[cu].p,
+                           (const PairSlot *)c->pnew.p, c->plen, (const unsigned long long *)c->meet[cu].keys.p,
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)c->towner.p, c->tbounds.p);
     }
@@ -3438,16 +3472,17 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
             CK(hipMemcpyAsync(cnt, c->hinit, sizeof(Counters), hipMemcpyHostToDevice, s));
         }
         const MemtableDev mt{c->rec_keys, c->rec_boxes, c->rec_cap, c->same_pid_count, c->o_boxs, c->sids};
+        const Meets mo = c->meet[cu].view();
         CK(hipEventRecord(c->ev[8], s));
         if (c->pairs_boxed)
             hipLaunchKernelGGL(k_meet_merge<PairHit>, dim3(mgrid), dim3(256), 0, s, (const PairHit *)c->pbox.p,
-                               c->plen, (const Bucket *)c->meet[cu].p, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].p, ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
+                               c->plen, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
+                               c->meet[nx].keys.p, c->meet[nx].starts.p, c->meet[nx].mbrs.p, ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
                                (const uint32_t *)nullptr, c->n, cnt);
         else
             hipLaunchKernelGGL(k_meet_merge<PairSlot>, dim3(mgrid), dim3(256), 0, s, (const PairSlot *)c->pnew.p,
-                               c->plen, (const Bucket *)c->meet[cu].p, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].p, ma, mt, (const float2 *)c->posf.p, (const uint32_t *)c->moff[nx].p,
+                               c->plen, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
+                               c->meet[nx].keys.p, c->meet[nx].starts.p, c->meet[nx].mbrs.p, ma, mt, (const float2 *)c->posf.p, (const uint32_t *)c->moff[nx].p,
                                (const uint32_t *)c->towner.p, c->n, cnt);
         CK(hipGetLastError());
         CK(hipEventRecord(c->ev[9], s));
@@ -4028,7 +4063,7 @@ int stc_live_search_noalloc(void *vc, const uint32_t *pids, uint32_t n, stc_hit 
     CK(hipGetLastError());
     if (c->mlen) {
         const uint32_t g = (uint32_t)std::min<uint64_t>(blocks_for(c->mlen, 256), 8192);
-        hipLaunchKernelGGL(k_na_live, dim3(g), dim3(256), 0, s, (const Bucket *)c->meet[c->cur].p, c->mlen, t, t - m,
+        hipLaunchKernelGGL(k_na_live, dim3(g), dim3(256), 0, s, c->meet[c->cur].view(), c->mlen, t, t - m,
                            sc, n);
         CK(hipGetLastError());
     }

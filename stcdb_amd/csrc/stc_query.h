@@ -35,7 +35,7 @@ struct CtfStats {
 };
 
 struct QueryState {
-    const Bucket *table;
+    Meets meets;
     uint64_t nb;
     uint32_t last_t;
     uint32_t stepped;

@@ -24,6 +24,8 @@
 #include <cstring>
 
 #define QGRID 64
+#define QFINE 256 /* cells a side of the scans' range filter */
+#define QSTAGE 48 /* hits a wave gathers before it reserves room for them */
 #define QLDS 4096 /* batches up to this many queries count in LDS, block by block */
 #define MASK26 ((1u << 26) - 1u)
 
@@ -46,6 +48,7 @@ struct QDev {
     unsigned long long *counts;
     uint32_t nq;
     uint32_t lds;                    /* nq <= QLDS: per-block counters in LDS */
+    float fx[2], fy[2], fix, fiy;    /* range filter: the map's low corner in two parts, cells per degree */
 };
 
 /* host tables on their way to the device: built in pinned memory, sent with one copy */
@@ -196,14 +199,15 @@ __device__ inline void q_store(const QDev &Q, uint32_t qi, uint32_t pid, uint32_
  * global counts on exit: one atomic per query and block instead of one per
  * hit), then the batch's filter: 2^f_bits bits of id hashes and a bit per grid
  * cell, which turn away nearly every meeting no query asks for without a read
- * of the tables. The launch sizes it (q_scan_lds). */
+ * of the tables, and with range queries a bit per cell of a finer grid, of the
+ * cells at and around their boxes. The launch sizes it (q_scan_lds). */
 extern __shared__ uint32_t q_lds[];
 
 __device__ inline uint32_t *q_scan_begin(const QDev &Q) {
     uint32_t *flt = q_lds + (Q.lds ? Q.nq : 0u);
     if (Q.lds)
         for (uint32_t i = threadIdx.x; i < Q.nq; i += blockDim.x) q_lds[i] = 0;
-    const uint32_t words = (1u << Q.f_bits) / 32 + QGRID * QGRID / 32;
+    const uint32_t words = (1u << Q.f_bits) / 32 + QGRID * QGRID / 32 + (Q.n_range ? QFINE * QFINE / 32 : 0);
     for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) flt[i] = Q.filter[i];
     __syncthreads();
     return flt;
@@ -215,12 +219,73 @@ __device__ inline void q_scan_end(const QDev &Q) {
             if (q_lds[i]) atomicAdd(&Q.counts[i], (unsigned long long)q_lds[i]);
 }
 
-__device__ inline void q_emit(const QDev &Q, uint32_t qi, uint32_t pid, uint32_t target, uint32_t start, uint32_t end,
-                              uint32_t source, const double *m) {
+/* A wave's hits on their way out, in LDS. A reservation per group of lanes that
+ * hit together was an update of one address every few hits, 4 ns each in a
+ * row, which bounded the scans of crowded boxes. */
+struct QStage {
+    stc_hit *h;
+    uint32_t *n;
+};
+
+__device__ inline void q_emit(const QDev &Q, const QStage &st, uint32_t qi, uint32_t pid, uint32_t target, uint32_t start,
+                              uint32_t end, uint32_t source, const double *m) {
     if (Q.lds) atomicAdd(&q_lds[qi], 1u);
     else atomicAdd(&Q.counts[qi], 1ull);
-    q_store(Q, qi, pid, target, start, end, source, m);
+    if (!Q.cap || (Q.q[qi].flags & STC_QF_COUNT)) return;
+    const uint32_t at = atomicAdd(st.n, 1u);
+    if (at < QSTAGE) st.h[at] = stc_hit{qi, pid, target, start, end, source, {m[0], m[1], m[2], m[3]}};
+    else q_store(Q, qi, pid, target, start, end, source, m);
 }
+
+/* n staged hits to the batch's hits from `base` on, by a wave */
+__device__ inline void q_stage_out(const QDev &Q, const QStage &st, uint32_t n, unsigned long long base) {
+    constexpr uint32_t W = sizeof(stc_hit) / 8;
+    const uint64_t keep = base < Q.cap ? min<uint64_t>(n, Q.cap - base) : 0;
+    uint64_t *dst = (uint64_t *)(Q.hits + base);
+    const uint64_t *src = (const uint64_t *)st.h;
+    for (uint32_t i = threadIdx.x & (STC_WAVE - 1); i < keep * W; i += STC_WAVE) dst[i] = src[i];
+}
+
+/* all lanes of the wave: its hits out where half its room is taken */
+__device__ inline void q_stage_drain(const QDev &Q, const QStage &st) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)*(volatile uint32_t *)st.n);
+    if (n < QSTAGE / 2) return;
+    const uint32_t k = min(n, (uint32_t)QSTAGE);
+    unsigned long long base = 0;
+    if ((threadIdx.x & (STC_WAVE - 1)) == 0) base = atomicAdd(Q.n_hits, (unsigned long long)k);
+    base = __shfl(base, 0, STC_WAVE);
+    q_stage_out(Q, st, k, base);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    *(volatile uint32_t *)st.n = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+/* the workgroup's last hits, one reservation; n: its waves' counts */
+__device__ inline void q_stage_end(const QDev &Q, const QStage &st, const uint32_t *n) {
+    __shared__ unsigned long long base;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t all = 0;
+        for (uint32_t w = 0; w < blockDim.x / STC_WAVE; w++) all += min(n[w], (uint32_t)QSTAGE);
+        base = all ? atomicAdd(Q.n_hits, (unsigned long long)all) : 0ull;
+    }
+    __syncthreads();
+    unsigned long long b = base;
+    const uint32_t wv = threadIdx.x / STC_WAVE;
+    for (uint32_t w = 0; w < wv; w++) b += min(n[w], (uint32_t)QSTAGE);
+    q_stage_out(Q, st, min(n[wv], (uint32_t)QSTAGE), b);
+}
+
+#define Q_STAGE(st)                                                   \
+    __shared__ stc_hit st##_h[256 / STC_WAVE][QSTAGE];                \
+    __shared__ uint32_t st##_n[256 / STC_WAVE];                       \
+    const QStage st{st##_h[threadIdx.x / STC_WAVE], st##_n + threadIdx.x / STC_WAVE}; \
+    if ((threadIdx.x & (STC_WAVE - 1)) == 0) *st.n = 0;               \
+    __syncthreads()
 
 __device__ inline bool q_time(const stc_query &q, uint32_t s, uint32_t e) { return s <= q.t1 && e >= q.t0; }
 __device__ inline bool q_box(const stc_query &q, const double *m) {
@@ -233,31 +298,52 @@ __device__ inline bool q_may_oid(const QDev &Q, const uint32_t *flt, uint32_t pi
     return (flt[h >> 5] >> (h & 31)) & 1u;
 }
 
-/* object and pair queries of one meeting seen from pid */
-__device__ inline void match_oid(const QDev &Q, uint32_t pid, uint32_t target, uint32_t s, uint32_t e, uint32_t src,
-                                 const double *m) {
+/* may a range query reach a box? In 32 bits: the low corner's cell of the fine
+ * grid comes within a thousandth of a cell, and the filter's bits are those of
+ * the cells that a query's box covers and of their neighbours, so a box of up
+ * to half a cell is never missed; a larger one (or NaN) passes. */
+__device__ inline int fine_cell(float v, const float *v0, float inv) {
+    const float f = ((v - v0[0]) - v0[1]) * inv;
+    if (!(f >= 0.0f)) return 0;
+    return f >= (float)QFINE ? QFINE - 1 : (int)f;
+}
+__device__ inline bool q_may_box(const QDev &Q, const uint32_t *flt, float lo0, float lo1, float hi0, float hi1) {
+    if (!((hi0 - lo0) * Q.fix <= 0.5f && (hi1 - lo1) * Q.fiy <= 0.5f)) return true;
+    const uint32_t *fine = flt + (1u << Q.f_bits) / 32 + QGRID * QGRID / 32;
+    const uint32_t cell = (uint32_t)(fine_cell(lo1, Q.fy, Q.fiy) * QFINE + fine_cell(lo0, Q.fx, Q.fix));
+    return (fine[cell >> 5] >> (cell & 31)) & 1u;
+}
+
+/* the object and pair queries that name pid: the first of their list, -1 when there are none */
+__device__ inline int32_t oid_queries(const QDev &Q, uint32_t pid) {
     const uint32_t mask = (1u << Q.oh_bits) - 1u;
     uint32_t h = oid_slot(pid, Q.oh_bits);
     for (;;) {
         uint32_t k = Q.oh_key[h];
-        if (k == pid) break;
-        if (k == 0xFFFFFFFFu) return;
+        if (k == pid) return Q.oh_head[h];
+        if (k == 0xFFFFFFFFu) return -1;
         h = (h + 1) & mask;
     }
-    for (int32_t qi = Q.oh_head[h]; qi >= 0; qi = Q.q_next[qi]) {
+}
+
+/* the queries of that list for one meeting seen from pid */
+__device__ inline void match_oid(const QDev &Q, const QStage &st, int32_t qi, uint32_t pid, uint32_t target, uint32_t s,
+                                 uint32_t e, uint32_t src, const double *m) {
+    for (; qi >= 0; qi = Q.q_next[qi]) {
         const stc_query &q = Q.q[qi];
         if (!q_time(q, s, e)) continue;
         if (q.kind == STC_Q_OID || (q.kind == STC_Q_PAIR && q.oid2 == target))
-            q_emit(Q, (uint32_t)qi, pid, target, s, e, src, m);
+            q_emit(Q, st, (uint32_t)qi, pid, target, s, e, src, m);
     }
 }
 
 /* range queries of one meeting (called once per meeting) */
-__device__ inline void match_range(const QDev &Q, const uint32_t *flt, uint32_t pid, uint32_t target, uint32_t s,
+__device__ inline void match_range(const QDev &Q, const QStage &st, const uint32_t *flt, uint32_t pid, uint32_t target, uint32_t s,
                                    uint32_t e, uint32_t src, const double *m) {
     const uint32_t *cells = flt + (1u << Q.f_bits) / 32;
     const int cx0 = grid_cell(m[0], Q.x0, Q.ix), cx1 = grid_cell(m[2], Q.x0, Q.ix);
     const int cy0 = grid_cell(m[1], Q.y0, Q.iy), cy1 = grid_cell(m[3], Q.y0, Q.iy);
+    const bool one = cx0 == cx1 && cy0 == cy1;
     for (int cy = cy0; cy <= cy1; cy++)
         for (int cx = cx0; cx <= cx1; cx++) {
             const uint32_t cell = (uint32_t)(cy * QGRID + cx);
@@ -266,9 +352,9 @@ __device__ inline void match_range(const QDev &Q, const uint32_t *flt, uint32_t 
                 const uint32_t qi = Q.g_list[j];
                 const stc_query &q = Q.q[qi];
                 if (!q_time(q, s, e) || !q_box(q, m)) continue;
-                if (grid_cell(fmax(m[0], q.box[0]), Q.x0, Q.ix) != cx || grid_cell(fmax(m[1], q.box[1]), Q.y0, Q.iy) != cy)
-                    continue;
-                q_emit(Q, qi, pid, target, s, e, src, m);
+                if (!one && (grid_cell(fmax(m[0], q.box[0]), Q.x0, Q.ix) != cx || grid_cell(fmax(m[1], q.box[1]), Q.y0, Q.iy) != cy))
+                    continue; /* counted in the cell of the intersection's low corner */
+                q_emit(Q, st, qi, pid, target, s, e, src, m);
             }
         }
 }
@@ -338,60 +424,104 @@ __device__ inline void decode_tail(const uint64_t *o_keys, const float4 *o_boxes
     m[3] = b.w;
 }
 
-/* One read of the live meetings, 28 bytes each. Without range queries a lane
- * reads the ids of four meetings at once and the rest of one only where the id
- * filter lets it pass; with range queries it reads two whole meetings at once,
- * so that no read waits for another. Object queries are bound by memory (256M
- * meetings, 1,000 objects: 3.81 ms when every meeting was read whole and hashed
- * into the batch's tables in global memory, 2.08 ms = 3.4 TB/s so), range
- * queries by the cells' arithmetic in 64 bits (42M meetings, 128 mixed queries:
- * 563 us with divisions by the cell size and a read of the grid for every
- * meeting, 377 so). */
-template <bool RANGES>
-__global__ __launch_bounds__(256) void k_q_live(const Bucket *__restrict__ t, uint64_t nb, uint32_t last_t, QDev Q) {
-    constexpr int U = RANGES ? 2 : 4;
+/* One read of the live meetings, several at once so that no read waits for
+ * another: the ids for object queries, the boxes for range queries. A meeting
+ * that the filters let pass waits in the wave's LDS until 64 of them are looked
+ * up together: nearly every wave has one or two in every round, and the
+ * lookup's chain of reads for those few was what bounded the scan. With 28-byte
+ * meetings read whole or looked up one by one: 1,000 objects among 128M
+ * meetings 2.10 -> 0.83 ms (8 bytes each at 1.2 TB/s; the id filter and the
+ * table now bound it), one among 10M 52 -> 25 us, 48 crowded boxes with 446,000
+ * hits 465 -> 257 us (with the hits' reservations, at q_emit); 128 mixed
+ * queries, bound by the lookups, 408 -> 429. */
+template <bool OIDS, bool RANGES>
+__global__ __launch_bounds__(256) void k_q_live(Meets t, uint64_t nb, uint32_t last_t, QDev Q) {
+    constexpr int U = RANGES ? 4 : 8;
+    __shared__ uint64_t wait[256 / STC_WAVE][2 * STC_WAVE];
     const uint32_t *flt = q_scan_begin(Q);
+    Q_STAGE(st);
+    uint64_t *wq = wait[threadIdx.x / STC_WAVE];
+    uint32_t waiting = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const bool oids = Q.oh_bits != 0;
-    for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < nb; i0 += stride * U) {
-        Bucket b[U];
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(STC_WAVE - 1u));
+    const uint32_t lane = threadIdx.x & (STC_WAVE - 1);
+    const uint64_t lt = (1ull << lane) - 1ull;
+    auto look_up = [&](uint32_t n) { /* the last n of the waiting */
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        waiting -= n;
+        if (lane < n) {
+            const uint64_t i = wq[waiting + lane];
+            const Bucket b = t.at(i);
+            const uint32_t a = (uint32_t)(b.key >> 32), c = (uint32_t)b.key;
+            if (c != DEAD_B) {
+                const double m[4] = {o2f(b.mbr[0]), o2f(b.mbr[1]), o2f(b.mbr[2]), o2f(b.mbr[3])};
+                /* a live meeting ends at the step that built the arrays */
+                if constexpr (OIDS) {
+                    match_oid(Q, st, oid_queries(Q, a), a, c, b.start, last_t, 0, m);
+                    match_oid(Q, st, oid_queries(Q, c), c, a, b.start, last_t, 0, m);
+                }
+                if constexpr (RANGES) match_range(Q, st, flt, a, c, b.start, last_t, 0, m);
+            }
+        }
+        q_stage_drain(Q, st);
+    };
+    for (uint64_t i0 = first; i0 < nb; i0 += stride * U) {
+        unsigned long long key[U];
+        uint4 mbr[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const uint64_t i = min(i0 + u * stride, nb - 1);
-            if constexpr (RANGES) b[u] = t[i];
-            else b[u].key = t[i].key;
+            const uint64_t i = min(i0 + lane + u * stride, nb - 1);
+            if constexpr (OIDS) key[u] = t.keys[i];
+            if constexpr (RANGES) mbr[u] = t.mbrs[i];
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const uint64_t i = i0 + u * stride;
-            const uint32_t a = (uint32_t)(b[u].key >> 32), c = (uint32_t)b[u].key;
-            if (i >= nb || c == DEAD_B) continue;
-            const bool ma = oids && q_may_oid(Q, flt, a), mc = oids && q_may_oid(Q, flt, c);
-            if (!RANGES) {
-                if (!(ma || mc)) continue;
-                b[u] = t[i];
+            const uint64_t i = i0 + lane + u * stride;
+            bool pass = false;
+            if constexpr (RANGES) pass = q_may_box(Q, flt, o2f(mbr[u].x), o2f(mbr[u].y), o2f(mbr[u].z), o2f(mbr[u].w));
+            if constexpr (OIDS) {
+                pass = pass || q_may_oid(Q, flt, (uint32_t)(key[u] >> 32)) || q_may_oid(Q, flt, (uint32_t)key[u]);
+                pass = pass && (uint32_t)key[u] != DEAD_B;
             }
-            double m[4] = {o2f(b[u].mbr[0]), o2f(b[u].mbr[1]), o2f(b[u].mbr[2]), o2f(b[u].mbr[3])};
-            /* a live meeting ends at the step that built the array */
-            if (ma) match_oid(Q, a, c, b[u].start, last_t, 0, m);
-            if (mc) match_oid(Q, c, a, b[u].start, last_t, 0, m);
-            if (RANGES) match_range(Q, flt, a, c, b[u].start, last_t, 0, m);
+            pass = pass && i < nb;
+            const uint64_t passing = __ballot(pass);
+            if (pass) wq[waiting + (uint32_t)__popcll(passing & lt)] = i;
+            waiting += (uint32_t)__popcll(passing);
+            if (waiting >= STC_WAVE) look_up(STC_WAVE);
         }
     }
+    look_up(waiting);
+    q_stage_end(Q, st, st_n);
     q_scan_end(Q);
 }
 
 __global__ __launch_bounds__(256) void k_q_mem(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes,
                                                uint64_t n, uint32_t base, QDev Q) {
     const uint32_t *flt = q_scan_begin(Q);
+    Q_STAGE(st);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        uint32_t pid, target, start, end;
-        double m[4];
-        decode_tail(keys, boxes, (uint32_t)i, base, &pid, &target, &start, &end, m);
-        if (Q.oh_bits && q_may_oid(Q, flt, pid)) match_oid(Q, pid, target, start, end, 1, m);
-        if (Q.n_range && pid < target) match_range(Q, flt, pid, target, start, end, 1, m);
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(STC_WAVE - 1u)), lane = threadIdx.x & (STC_WAVE - 1);
+    for (uint64_t i0 = first; i0 < n; i0 += stride) {
+        const uint64_t i = i0 + lane;
+        if (i < n) {
+            const uint64_t hi = keys[2 * i + 1];
+            const uint32_t pid = (uint32_t)(hi >> 26) & MASK26, target = (uint32_t)hi & MASK26;
+            float4 b = make_float4(0, 0, 0, 0);
+            if (Q.n_range) b = boxes[i];
+            const int32_t qo = Q.oh_bits && q_may_oid(Q, flt, pid) ? oid_queries(Q, pid) : -1;
+            const bool mr = Q.n_range && pid < target && q_may_box(Q, flt, b.x, b.y, b.z, b.w);
+            if (qo >= 0 || mr) {
+                uint32_t p, c, start, end;
+                double m[4];
+                decode_tail(keys, boxes, (uint32_t)i, base, &p, &c, &start, &end, m);
+                match_oid(Q, st, qo, pid, target, start, end, 1, m);
+                if (mr) match_range(Q, st, flt, pid, target, start, end, 1, m);
+            }
+        }
+        q_stage_drain(Q, st);
     }
+    q_stage_end(Q, st, st_n);
     q_scan_end(Q);
 }
 
@@ -483,26 +613,37 @@ __global__ __launch_bounds__(256) void k_q_run_range(const QueryRunDev *__restri
     const QueryRunDev R = runs[cd.y];
     uint32_t pid, target, start, end, found = 0;
     double m[4];
+    Q_STAGE(st);
+    const bool store = Q.cap && !(q.flags & STC_QF_COUNT);
+    auto hit = [&]() {
+        found++;
+        if (!store) return;
+        const uint32_t at = atomicAdd(st.n, 1u);
+        if (at < QSTAGE) st.h[at] = stc_hit{qi, pid, target, start, end, R.source, {m[0], m[1], m[2], m[3]}};
+        else q_store(Q, qi, pid, target, start, end, R.source, m);
+    };
+    const uint32_t first = threadIdx.x & ~(STC_WAVE - 1u), lane = threadIdx.x & (STC_WAVE - 1);
     if (cd.z == 0xFFFFFFFFu) {
-        for (uint32_t i = threadIdx.x; i < R.n_tail; i += blockDim.x) {
-            decode_tail(R.o_keys, R.o_boxes, i, R.end_time_min, &pid, &target, &start, &end, m);
-            if (pid < target && q_time(q, start, end) && q_box(q, m)) {
-                found++;
-                q_store(Q, qi, pid, target, start, end, R.source, m);
+        for (uint32_t i0 = first; i0 < R.n_tail; i0 += blockDim.x) {
+            if (i0 + lane < R.n_tail) {
+                decode_tail(R.o_keys, R.o_boxes, i0 + lane, R.end_time_min, &pid, &target, &start, &end, m);
+                if (pid < target && q_time(q, start, end) && q_box(q, m)) hit();
             }
+            if (store) q_stage_drain(Q, st);
         }
     } else {
         const stc_ctf_meta ctf = R.ctfs[cd.z];
         const uint32_t kb = ctf.key_bit / 8;
         const uint8_t *base = R.key_bytes + R.byte_base[cd.z];
-        for (uint32_t i = threadIdx.x; i < ctf.kv_capacity; i += blockDim.x) {
-            decode_packed(ctf, load_packed(base + (uint64_t)i * kb, kb), &pid, &target, &start, &end, m);
-            if (pid < target && q_time(q, start, end) && q_box(q, m)) {
-                found++;
-                q_store(Q, qi, pid, target, start, end, R.source, m);
+        for (uint32_t i0 = first; i0 < ctf.kv_capacity; i0 += blockDim.x) {
+            if (i0 + lane < ctf.kv_capacity) {
+                decode_packed(ctf, load_packed(base + (uint64_t)(i0 + lane) * kb, kb), &pid, &target, &start, &end, m);
+                if (pid < target && q_time(q, start, end) && q_box(q, m)) hit();
             }
+            if (store) q_stage_drain(Q, st);
         }
     }
+    if (store) q_stage_end(Q, st, st_n);
     q_count_wave(Q, qi, found);
 }
 
@@ -896,18 +1037,18 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     /* grid of the range queries */
     const double x0 = st.map[0], y0 = st.map[1];
     const double ix = QGRID / (st.map[2] - st.map[0]), iy = QGRID / (st.map[3] - st.map[1]);
-    /* the scans' filter: about 16 bits per queried id, at most 2^16 */
+    /* the scans' filter: 64 bits or more per queried id, 2^16 (8 KB of LDS) at most */
     uint32_t f_bits = 5;
-    if (!oq.empty()) f_bits = std::min(std::max(bits + 3, 10u), 16u);
-    std::vector<uint32_t> filter((1u << f_bits) / 32 + QGRID * QGRID / 32, 0u);
+    if (!oq.empty()) f_bits = std::min(bits + 5, 16u);
+    std::vector<uint32_t> rq;
+    for (uint32_t i = 0; i < nq; i++)
+        if (q[i].kind == STC_Q_RANGE) rq.push_back(i);
+    std::vector<uint32_t> filter((1u << f_bits) / 32 + QGRID * QGRID / 32 + (rq.empty() ? 0 : QFINE * QFINE / 32), 0u);
     for (uint32_t i : oq) {
         const uint32_t h = oid_slot(q[i].oid, f_bits);
         filter[h >> 5] |= 1u << (h & 31);
     }
     uint32_t *cell_bits = filter.data() + (1u << f_bits) / 32;
-    std::vector<uint32_t> rq;
-    for (uint32_t i = 0; i < nq; i++)
-        if (q[i].kind == STC_Q_RANGE) rq.push_back(i);
     std::vector<uint32_t> start, list;
     if (!rq.empty()) { /* counted per cell, then listed in query order */
         start.assign(QGRID * QGRID + 1, 0);
@@ -926,6 +1067,22 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         list.resize(start.back());
         std::vector<uint32_t> at(start.begin(), start.end() - 1);
         for (uint32_t qi : rq) cells(qi, [&](int c) { list[at[c]++] = qi; });
+        /* the fine grid's cells at and around the boxes; all of them where the map is too small for 32 bits */
+        uint32_t *fine = cell_bits + QGRID * QGRID / 32;
+        const double fine_per = (double)QFINE / QGRID;
+        auto fine_of = [&](double v, double v0, double inv, int off) {
+            const double f = (v - v0) * inv * fine_per;
+            return std::min(std::max((!(f >= 0.0) ? 0 : f >= (double)QFINE ? QFINE - 1 : (int)f) + off, 0), QFINE - 1);
+        };
+        if (!(ix < 1e30 && iy < 1e30)) std::fill(fine, fine + QFINE * QFINE / 32, ~0u);
+        else
+            for (uint32_t qi : rq) {
+                const double *b = q[qi].box;
+                const int x0c = fine_of(b[0], x0, ix, -1), x1c = fine_of(b[2], x0, ix, 1);
+                for (int y = fine_of(b[1], y0, iy, -1); y <= fine_of(b[3], y0, iy, 1); y++)
+                    for (int w = x0c >> 5; w <= x1c >> 5; w++)
+                        fine[y * (QFINE / 32) + w] |= (w == x0c >> 5 ? ~0u << (x0c & 31) : ~0u) & (w == x1c >> 5 ? ~0u >> (31 - (x1c & 31)) : ~0u);
+            }
     }
 
     /* one copy for all of it (each table was a copy of its own, waited for: 10 us and more a piece) */
@@ -961,6 +1118,12 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     Q.y0 = y0;
     Q.ix = ix;
     Q.iy = iy;
+    Q.fx[0] = (float)x0;
+    Q.fx[1] = (float)(x0 - (double)Q.fx[0]);
+    Q.fy[0] = (float)y0;
+    Q.fy[1] = (float)(y0 - (double)Q.fy[0]);
+    Q.fix = (float)(ix * (QFINE / QGRID));
+    Q.fiy = (float)(iy * (QFINE / QGRID));
     Q.hits = B->hits;
     Q.cap = hits ? cap : 0;
     Q.n_hits = counters;
@@ -973,14 +1136,15 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     std::vector<unsigned long long> planned(nq, 0);
 
     /* live meetings and memtable */
-    if (st.stepped && st.table && st.nb) {
-        uint32_t g = (uint32_t)std::min<uint64_t>(blocks(st.nb, 256), 8192);
-        if (Q.n_range) hipLaunchKernelGGL(k_q_live<true>, dim3(g), dim3(256), q_scan_lds, s, st.table, st.nb, st.last_t, Q);
-        else hipLaunchKernelGGL(k_q_live<false>, dim3(g), dim3(256), q_scan_lds, s, st.table, st.nb, st.last_t, Q);
+    if (st.stepped && st.meets.keys && st.nb) {
+        const dim3 g((uint32_t)std::min<uint64_t>(blocks(st.nb, 256), 4096));
+        if (Q.n_range && bits) hipLaunchKernelGGL((k_q_live<true, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
+        else if (Q.n_range) hipLaunchKernelGGL((k_q_live<false, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
+        else if (bits) hipLaunchKernelGGL((k_q_live<true, false>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
         QCK(hipGetLastError());
     }
     if (st.n_rec) {
-        hipLaunchKernelGGL(k_q_mem, dim3(std::min<uint32_t>(blocks(st.n_rec, 256), 8192)), dim3(256), q_scan_lds, s,
+        hipLaunchKernelGGL(k_q_mem, dim3(std::min<uint32_t>(blocks(st.n_rec, 256), 4096)), dim3(256), q_scan_lds, s,
                            st.rec_keys, st.rec_boxes, st.n_rec, st.end_time_min, Q);
         QCK(hipGetLastError());
     }

@@ -7,7 +7,10 @@
  * order-preserving u32 images of the f32 bounds so that min/max updates are
  * integer ops. Keys are oid1 << 32 | oid2 with oid1 < oid2 < 2^26.
  *
- * The live meetings after a step are one array of buckets sorted by key, one
+ * The live meetings after a step are the buckets' keys, starts and MBRs, an
+ * array each (a search by object then reads 8 bytes a meeting, not the lines
+ * of all 28: a lookup among 10M meetings 52 -> 25 us; the merge, which reads
+ * and writes all, takes as long either way), sorted by key, one
  * segment per owner oid1 (a pair's smaller id). Bucket i of a step's array is
  * built from the step's pair slot i, so a slot that held a duplicate pair or
  * a rejected band pair leaves a dead bucket: key oid1 << 32 | DEAD_B (it sorts
@@ -25,13 +28,25 @@
 
 #define DEAD_B 0xFFFFFFFFu /* partner word of a dead slot or bucket */
 
-/* packed to 28 bytes (4-byte aligned): the merge streams two arrays of them per step */
+/* one meeting at hand */
 struct __attribute__((packed, aligned(4))) Bucket {
     unsigned long long key;
     uint32_t start;
     uint32_t mbr[4];          /* ordered ints of low0, low1, high0, high1 */
 };
 static_assert(sizeof(Bucket) == 28, "a bucket is 28 bytes");
+
+/* a step's meetings in device memory, all to be read only */
+struct Meets {
+    const unsigned long long *keys;
+    const uint32_t *starts;
+    const uint4 *mbrs;
+    __device__ inline unsigned long long key(uint64_t i) const { return keys[i]; }
+    __device__ inline Bucket at(uint64_t i) const {
+        const uint4 m = mbrs[i];
+        return Bucket{keys[i], starts[i], {m.x, m.y, m.z, m.w}};
+    }
+};
 
 /* a bucket that holds a live meeting (not a dead slot) */
 __host__ __device__ inline bool bucket_live(const Bucket &b) { return (uint32_t)b.key != DEAD_B; }
