@@ -459,47 +459,88 @@ __global__ void k_gather(const double2 *__restrict__ xy, const double *__restric
 /* border lookup                                                       */
 /* ------------------------------------------------------------------ */
 
-#define LK_KEPT 4u /* leaves of a point that the lookup keeps for the emission */
+#define LK_KEPT 4u    /* leaves of a point that the lookup keeps for the emission */
+#define LK_THREADS 128
+#define LK_STACK 8u   /* nodes to visit that a thread keeps in LDS; further ones (a wide reach in a deep tree) go to memory */
 
 /* the leaves within reach of a border point on its top or right: f(leaf) in
  * descent order below lv; returns how many box distances lie in the guard
- * band, sets *full when the stack was */
+ * band, sets *full when the stack was.
+ * Most descents are a path with a branch here and there: the next node stays
+ * in a register, the others wait in LDS, and a child's own children are read
+ * with its box, so that a level is one wait for memory. A box is decided by its
+ * squared distance with reciprocals where that is clear of the guard band by
+ * far more than its rounding, by the division and root of the formula
+ * otherwise. */
 template <class F>
 __device__ inline uint32_t lookup_leaves(double2 q, double dl, uint32_t lv, const Node *__restrict__ nodes, double r,
                                          double band, bool *full, F f) {
-    uint32_t stk[STACK_DEPTH];
+    __shared__ uint32_t wait[LK_STACK][LK_THREADS];
+    uint32_t rest[STACK_DEPTH - LK_STACK];
+    const double il = 1.0 / dl, out = r + 2 * band, in = r - 2 * band;
+    const double s_out = out * out * (1.0 + 1e-9), s_in = in > 0 ? in * in * (1.0 - 1e-9) : -1.0;
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
     int sp = 0;
-    stk[sp++] = lv;
     uint32_t amb = 0;
-    while (sp > 0) {
-        uint32_t cur = stk[--sp];
-        const Node &nd = nodes[cur];
+    uint4 kids = *(const uint4 *)nodes[lv].child;
+    for (;;) {
+        uint4 next_kids = make_uint4(0, 0, 0, 0);
+        uint32_t next = NONE;
+        const uint32_t kid[4] = {kids.x, kids.y, kids.z, kids.w};
+#pragma unroll
         for (int i = 0; i < 4; i++) {
-            uint32_t c = nd.child[i];
+            const uint32_t c = kid[i];
             const Node &ch = nodes[c];
-            double d = stc_box_dist(ch.lo0, ch.lo1, ch.hi0, ch.hi1, q.x, q.y, dl);
-            if (fabs(d - r) <= band) amb++;
-            if (d <= r) {
-                if (ch.type == T_LEAF) {
-                    if (q.y < ch.lo1 || (q.y < ch.hi1 && q.x < ch.lo0)) f(ch.leaf);
-                } else if (sp < STACK_DEPTH) {
-                    stk[sp++] = c;
+            const double lo0 = ch.lo0, lo1 = ch.lo1, hi0 = ch.hi0, hi1 = ch.hi1;
+            const uint4 grand = *(const uint4 *)ch.child;
+            const uint32_t type = ch.type, leaf = ch.leaf;
+            const double dx = fmax(fabs(q.x - (lo0 + hi0) / 2) - (hi0 - lo0) / 2, 0.0);
+            const double dy = fmax(fabs(q.y - (lo1 + hi1) / 2) - (hi1 - lo1) / 2, 0.0);
+            const double ax = dx * il, ay = dy * STC_INV_DPM_LAT, s2 = ax * ax + ay * ay;
+            bool reach = s2 < s_in;
+            if (!reach && !(s2 > s_out)) {
+                const double d = stc_box_dist(lo0, lo1, hi0, hi1, q.x, q.y, dl);
+                if (fabs(d - r) <= band) amb++;
+                reach = d <= r;
+            }
+            if (reach) {
+                if (type == T_LEAF) {
+                    if (q.y < lo1 || (q.y < hi1 && q.x < lo0)) f(leaf);
+                } else if (sp + (next != NONE ? 1 : 0) < STACK_DEPTH) {
+                    if (next != NONE) {
+                        if ((uint32_t)sp < LK_STACK) wait[sp][threadIdx.x] = next;
+                        else rest[sp - LK_STACK] = next;
+                        sp++;
+                    }
+                    next = c;
+                    next_kids = grand;
                 } else {
                     *full = true;
                 }
             }
         }
+        if (next == NONE) {
+            if (sp == 0) break;
+            sp--;
+            next = (uint32_t)sp < LK_STACK ? wait[sp][threadIdx.x] : rest[sp - LK_STACK];
+            next_kids = *(const uint4 *)nodes[next].child;
+        }
+        kids = next_kids;
     }
     return amb;
 }
 
 /* One thread per point, points in leaf order: a wave's points share a leaf
  * and mostly the same subtrees, so their descents stay together. count[p] per
- * point id; the first LK_KEPT leaves of the point at place j in kept[j]. */
-__global__ void k_lookup(const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy,
-                         const double *__restrict__ ld, uint32_t n,
-                         const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r, double band,
-                         uint32_t *__restrict__ count, uint4 *__restrict__ kept, Counters *cnt) {
+ * point id; the first LK_KEPT leaves of the point at place j in kept[j]. Bound
+ * by the descent's chain of reads at a few 10,000 points and by its 64-bit
+ * arithmetic at millions: with the stack in memory, two reads a level and every
+ * distance divided and rooted, 50k objects 25.6 us, 5M 460; 14.2 and 373 so. */
+__global__ __launch_bounds__(LK_THREADS) void k_lookup(const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy,
+                                                       const double *__restrict__ ld, uint32_t n,
+                                                       const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv,
+                                                       double r, double band, uint32_t *__restrict__ count,
+                                                       uint4 *__restrict__ kept, Counters *cnt) {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const uint32_t p = lp[j];
@@ -522,45 +563,80 @@ __global__ void k_lookup(const uint32_t *__restrict__ lp, const double2 *__restr
     count[p] = found;
 }
 
-/* The cross units (point, leaf) in point order, and all that is kept of each:
- * the leaf and the point for the reverse lists, the leaf's kept members above
+/* The cross units in point order, and all that is kept of each: the leaf and
+ * the point, from which the reverse lists are sorted, and the leaf's kept members above
  * the point (an index range into the leaf-ordered arrays); and each point's
  * first unit and count in leaf order. The leaves come from the lookup; a point
  * with more than it keeps descends again. (A second descent for every point,
  * then a pass each for the reverse lists, the ranges and the leaf order: 23 +
- * 10 us at 50k objects, 97 + 44 at 1M; 6.5 and 54 us so.) */
-__global__ void k_units_emit(const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy, const double *__restrict__ ld,
-                             uint32_t n, const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r,
-                             double band, const uint32_t *__restrict__ count, const uint32_t *__restrict__ offset,
-                             const uint4 *__restrict__ kept, const uint32_t *__restrict__ leaf_start,
-                             const uint32_t *__restrict__ leaf_count, uint32_t buf, uint2 *__restrict__ units,
-                             uint32_t *__restrict__ rev_leaf, uint32_t *__restrict__ rev_pid, uint2 *__restrict__ urange,
-                             uint2 *__restrict__ lunits) {
+ * 10 us at 50k objects, 97 + 44 at 1M; 6.5 and 54 us so.) Bound by writes in
+ * point order, a line for each array: leaf and point were written twice, 517 us
+ * at 5M objects; 347 without that and with a point's searches side by side. */
+__global__ __launch_bounds__(LK_THREADS) void k_units_emit(
+    const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy, const double *__restrict__ ld, uint32_t n,
+    const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r, double band,
+    const uint32_t *__restrict__ count, const uint32_t *__restrict__ offset, const uint4 *__restrict__ kept,
+    const uint32_t *__restrict__ leaf_start, const uint32_t *__restrict__ leaf_count, uint32_t buf,
+    uint32_t *__restrict__ unit_leaf, uint32_t *__restrict__ unit_pid, uint2 *__restrict__ urange, uint2 *__restrict__ lunits) {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const uint32_t p = lp[j], c = count[p];
     uint32_t u = offset[p];
     lunits[j] = make_uint2(u, c);
     if (!c) return;
-    auto emit = [&](uint32_t leaf) {
-        uint32_t s2 = leaf_count[leaf];
-        if (s2 > buf) s2 = buf;
-        const uint32_t st2 = leaf_start[leaf], m0 = lower_bound_u32(lp + st2, s2, p + 1);
-        units[u] = make_uint2(p, leaf);
-        rev_leaf[u] = leaf;
-        rev_pid[u] = p;
-        urange[u] = make_uint2(st2 + m0, s2 - m0);
-        u++;
-    };
     if (c <= LK_KEPT) {
         const uint4 k = kept[j];
-        emit(k.x);
-        if (c > 1) emit(k.y);
-        if (c > 2) emit(k.z);
-        if (c > 3) emit(k.w);
+        const uint32_t leaf[LK_KEPT] = {k.x, k.y, k.z, k.w};
+        uint32_t first[LK_KEPT], have[LK_KEPT], lo[LK_KEPT], hi[LK_KEPT];
+        const bool some[LK_KEPT] = {true, __any(c > 1) != 0, __any(c > 2) != 0, __any(c > 3) != 0}; /* of the wave */
+#pragma unroll
+        for (uint32_t i = 0; i < LK_KEPT; i++) {
+            first[i] = have[i] = 0;
+            if (some[i]) {
+                const uint32_t l = leaf[i < c ? i : 0];
+                first[i] = leaf_start[l];
+                have[i] = min(leaf_count[l], buf);
+            }
+            lo[i] = 0;
+            hi[i] = i < c ? have[i] : 0;
+        }
+        /* the point's place among the members of each leaf, the searches side by side */
+        for (;;) {
+            uint32_t v[LK_KEPT];
+            bool more = false;
+#pragma unroll
+            for (uint32_t i = 0; i < LK_KEPT; i++) {
+                v[i] = 0;
+                if (some[i]) v[i] = lp[min(first[i] + (lo[i] + hi[i]) / 2, n - 1)];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < LK_KEPT; i++) {
+                const uint32_t mid = (lo[i] + hi[i]) / 2;
+                if (lo[i] < hi[i]) {
+                    if (v[i] <= p) lo[i] = mid + 1;
+                    else hi[i] = mid;
+                }
+                more |= lo[i] < hi[i];
+            }
+            if (!__any(more)) break;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < LK_KEPT; i++)
+            if (i < c) {
+                unit_leaf[u + i] = leaf[i];
+                unit_pid[u + i] = p;
+                urange[u + i] = make_uint2(first[i] + lo[i], have[i] - lo[i]);
+            }
     } else {
         bool full = false;
-        lookup_leaves(lxy[j], ld[j], pt_lv[p], nodes, r, band, &full, emit);
+        lookup_leaves(lxy[j], ld[j], pt_lv[p], nodes, r, band, &full, [&](uint32_t leaf) {
+            const uint32_t s2 = min(leaf_count[leaf], buf);
+            const uint32_t st2 = leaf_start[leaf], m0 = lower_bound_u32(lp + st2, s2, p + 1);
+            unit_leaf[u] = leaf;
+            unit_pid[u] = p;
+            urange[u] = make_uint2(st2 + m0, s2 - m0);
+            u++;
+        });
     }
 }
 
@@ -606,7 +682,7 @@ struct PairGeo {
     const uint2 *urange;                 /* per cross unit: its leaf's kept members above the unit's point (first, count) */
     const uint4 *prange;                 /* per point in leaf order: its later leaf members and the border
                                             points above it with a unit to its leaf (first, count, first, count) */
-    const uint2 *units;                  /* cross units (pid, leaf), point after point */
+    const uint32_t *units;               /* the cross units' leaves, point after point */
     const uint32_t *uoffset, *ucount;    /* a point's cross units: units[uoffset[p] ..] */
     const uint32_t *rev_start, *rev_pid; /* per leaf, by pid: the border points with a cross unit to it */
     const RevPt *rev;                    /* their positions, 1/dpm_lon and ids, in rev_pid order */
@@ -700,7 +776,7 @@ __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const Pair
     const uint2 un = g.lunits[w];
     const uint32_t u0 = un.x, nu = un.y;
     for (uint32_t k = 0; k < nu; k++) {
-        const uint32_t L2 = g.units[u0 + k].y;
+        const uint32_t L2 = g.units[u0 + k];
         uint32_t s2 = g.leaf_count[L2];
         if (s2 > g.buf) s2 = g.buf;
         const uint32_t st2 = g.leaf_start[L2];
@@ -2491,7 +2567,7 @@ struct StcCtx {
     DBuf<uint2> urange;                  /* per cross unit: member range above its point */
     DBuf<uint4> prange;                  /* per point in leaf order: own-leaf and reverse-list ranges */
     DBuf<uint32_t> ucount, uoffset;
-    DBuf<uint2> units;
+    DBuf<uint32_t> units;                /* cross units' leaves */
     DBuf<uint2> amb;                     /* band combinations (probe, other) for the host */
     DBuf<double4> amb_xy;                /* their positions (probe x, y, other x, y) */
     /* per leaf, by pid: the border points with a cross unit to it */
@@ -3201,7 +3277,7 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     /* 6: border lookup (count, scan, emit) */
     double r = c->cfg.reach_distance;
     uint4 *kept = c->prange.p; /* the lookup's leaves, until k_point_ranges fills it */
-    hipLaunchKernelGGL(k_lookup, dim3(blocks_for(n, 128)), dim3(128), 0, s, (const uint32_t *)c->lp.p,
+    hipLaunchKernelGGL(k_lookup, dim3(blocks_for(n, LK_THREADS)), dim3(LK_THREADS), 0, s, (const uint32_t *)c->lp.p,
                        (const double2 *)c->lxy.p, (const double *)c->ld.p, n, (const Node *)tree_nodes(c),
                        (const uint32_t *)c->pt_lv.p, r, c->band, c->ucount.p, kept, cnt);
     CK(hipGetLastError());
@@ -3214,18 +3290,17 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     uint64_t n_units = (uint32_t)h.units;
     if (n_units >= (1u << 30)) return fail(c, STC_E_CAPACITY, "2^30 or more cross units in one step");
     if (c->units.ensure(n_units + 1) || c->urange.ensure(n_units + 1) || c->rev_leaf.ensure(n_units + 1) ||
-        c->rev_pid.ensure(n_units + 1))
+        c->rev_pid.ensure(n_units + 1) || c->rev_pid_alt.ensure(n_units + 1))
         return fail(c, STC_E_CAPACITY, "unit buffer allocation failed");
-    hipLaunchKernelGGL(k_units_emit, dim3(blocks_for(n, 128)), dim3(128), 0, s, (const uint32_t *)c->lp.p,
+    hipLaunchKernelGGL(k_units_emit, dim3(blocks_for(n, LK_THREADS)), dim3(LK_THREADS), 0, s, (const uint32_t *)c->lp.p,
                        (const double2 *)c->lxy.p, (const double *)c->ld.p, n, (const Node *)tree_nodes(c),
                        (const uint32_t *)c->pt_lv.p, r, c->band, (const uint32_t *)c->ucount.p, (const uint32_t *)c->uoffset.p,
                        (const uint4 *)kept, (const uint32_t *)c->leaf_start.p, (const uint32_t *)c->leaf_count.p, c->buf,
-                       c->units.p, c->rev_leaf.p, c->rev_pid.p, c->urange.p, c->lunits.p);
+                       c->units.p, c->rev_pid_alt.p, c->urange.p, c->lunits.p); /* the sort below reads the points there first */
     CK(hipGetLastError());
     CK(hipEventRecord(c->ev[2], s));
     if (c->rev_leaf_alt.ensure(n_units + 1) ||
         c->rev.ensure(n_units + 1) || c->rev_dl.ensure(n_units + 1) ||
-        c->rev_pid_alt.ensure(n_units + 1) ||
         c->rev_start.ensure(n_leaves + 1ull) ||
         c->temp.ensure(stc_radix_temp_words((uint32_t)std::max<uint64_t>(std::max<uint64_t>(n_units, n),
                                                                           std::max<size_t>(c->nodes.cap, c->sch.cap))) + 64))
@@ -3238,7 +3313,7 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
 
     /* 7: reverse cross units: per leaf, the border points with a cross unit to it, by pid */
     if (n_units)
-        CKRC(sort_pairs((const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, c->rev_leaf, c->rev_pid, c->rev_leaf_alt,
+        CKRC(sort_pairs((const uint32_t *)c->units.p, (const uint32_t *)c->rev_pid_alt.p, c->rev_leaf, c->rev_pid, c->rev_leaf_alt,
                         c->rev_pid_alt, (uint32_t)n_units, std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
     hipLaunchKernelGGL(k_rev_finish, dim3(blocks_for(std::max<uint64_t>(n_units, n_leaves + 1ull), 256)), dim3(256), 0, s,
                        (const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, (uint32_t)n_units, n_leaves, xy,
