@@ -140,6 +140,33 @@ struct Counters {             /* device-side counters, copied back once per sync
 };
 
 
+/* a step's counters, clear, and the kept schema's leaf counts */
+__global__ __launch_bounds__(256) void k_step_begin(Counters *cnt, unsigned long long kv_count, uint32_t oversize,
+                                                    uint32_t *leaf_count, uint32_t n_leaves) {
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (uint32_t i = i0; i < n_leaves; i += stride) leaf_count[i] = 0;
+    if (blockIdx.x) return;
+    for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 4; i += blockDim.x) ((uint32_t *)cnt)[i] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        cnt->kv_count = kv_count;
+        cnt->oversize_oid_count = oversize;
+    }
+}
+
+/* the counters, and those of the schema, where the host reads them, then the number of this wait: a host that looks for it sees it some
+ * microseconds before a copy and the stream's end would let it go on */
+__global__ __launch_bounds__(256) void k_counters_out(const Counters *__restrict__ cnt, Counters *host,
+                                                      const uint32_t *schema, uint32_t *schema_host, uint32_t *flag, uint32_t seq) {
+    for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 8; i += blockDim.x)
+        ((unsigned long long *)host)[i] = ((const unsigned long long *)cnt)[i];
+    if (schema && threadIdx.x < DC_WORDS) schema_host[threadIdx.x] = schema[threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+static_assert(sizeof(Counters) % 8 == 0, "copied in 8-byte words");
+
 __device__ inline uint32_t part1by1(uint32_t x) {
     x &= 0x0000ffff;
     x = (x | (x << 8)) & 0x00FF00FF;
@@ -2601,6 +2628,8 @@ struct StcCtx {
     uint16_t *sids = nullptr;
     Counters *dcnt = nullptr;
     Counters *hcnt = nullptr;  /* pinned */
+    uint32_t *hseq = nullptr;  /* pinned: the last wait whose counters are in hcnt */
+    uint32_t seq = 0;
     Counters *hinit = nullptr; /* pinned: initial counter values of a step */
     uint32_t oversize_oid_count = 0;
     uint32_t end_time_min = 0;
@@ -2734,8 +2763,22 @@ static inline uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n
         if (jrc_) return jrc_;         \
     } while (0)
 
+/* The step's counters on the host. The kernel's number is looked for during the time that a step of some 10,000
+ * objects takes; a longer step, or one that failed, is waited for as usual. With
+ * copies and the stream's end (and a copy of the first counters) a step of 10k objects 376 us, of 50k 328, 16 streams
+ * together 2.69 ms; 305, 283 and 2.49 so. */
 static int sync_counters(StcCtx *c) {
-    CK(hipMemcpyAsync(c->hcnt, c->dcnt, sizeof(Counters), hipMemcpyDeviceToHost, c->s));
+    const uint32_t seq = ++c->seq;
+    hipLaunchKernelGGL(k_counters_out, dim3(1), dim3(256), 0, c->s, (const Counters *)c->dcnt, c->hcnt,
+                       (const uint32_t *)c->sch.dcount, c->sch.hcount, c->hseq, seq);
+    CK(hipGetLastError());
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(300);
+    do {
+        for (int k = 0; k < 32; k++) {
+            if (__atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) == seq) return 0;
+            __builtin_ia32_pause();
+        }
+    } while (std::chrono::steady_clock::now() < until);
     CK(hipStreamSynchronize(c->s));
     return 0;
 }
@@ -3080,8 +3123,10 @@ int stc_create(const stc_config *cfg, const stc_box *mbr, void **out) {
         return bad("device allocation failed");
     if (hipMalloc((void **)&c->dcnt, sizeof(Counters)) != hipSuccess) return bad("counters");
     if (hipHostMalloc((void **)&c->hcnt, sizeof(Counters), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&c->hseq, 64, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&c->hinit, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
         return bad("pinned");
+    *c->hseq = 0;
     /* no meetings yet: every segment of the current array is empty */
     uint64_t nb = cfg->num_meeting_buckets ? cfg->num_meeting_buckets : 2ull * n;
     if (c->pnew.ensure(nb) || c->meet[0].ensure(nb) || c->meet[1].ensure(nb))
@@ -3130,6 +3175,7 @@ int stc_destroy(void *vc) {
     if (c->sids) hipFree(c->sids);
     if (c->dcnt) hipFree(c->dcnt);
     if (c->hcnt) hipHostFree(c->hcnt);
+    if (c->hseq) hipHostFree(c->hseq);
     if (c->hinit) hipHostFree(c->hinit);
     stc_flush_free(&c->flushw);
     for (auto &r : c->runs) {
@@ -3216,10 +3262,11 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     const uint32_t n = c->n;
     hipStream_t s = c->s;
     Counters *cnt = c->dcnt;
-    memset(c->hinit, 0, sizeof(Counters));
-    c->hinit->kv_count = c->kv_count;
-    c->hinit->oversize_oid_count = c->oversize_oid_count;
-    CK(hipMemcpyAsync(cnt, c->hinit, sizeof(Counters), hipMemcpyHostToDevice, s));
+    /* the kept schema's leaves are those of the last step's update, and their counts have room unless it grew */
+    const uint32_t cleared = c->dyn && c->sch.present && c->leaf_count.cap > c->sch.n_leaves ? c->sch.n_leaves : 0;
+    hipLaunchKernelGGL(k_step_begin, dim3(std::min<uint32_t>(blocks_for(cleared, 256) + 1, 256)), dim3(256), 0, s, cnt,
+                       (unsigned long long)c->kv_count, c->oversize_oid_count, c->leaf_count.p, cleared);
+    CK(hipGetLastError());
     CK(hipEventRecord(c->ev[0], s));
 
     /* 1-2: cells, Morton codes, dpm_lon; sort codes */
@@ -3259,7 +3306,7 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     c->last_leaves = n_leaves;
 
     /* 4: partition */
-    CK(hipMemsetAsync(c->leaf_count.p, 0, 4ull * n_leaves, s));
+    if (cleared != n_leaves) CK(hipMemsetAsync(c->leaf_count.p, 0, 4ull * n_leaves, s));
     hipLaunchKernelGGL(k_partition, dim3(blocks_for(n, 256)), dim3(256), 0, s, xy, walk, n,
                        (const Node *)tree_nodes(c), c->x_buffer, c->y_buffer, c->pt_leaf.p, c->pt_lv.p, c->leaf_count.p, cnt);
     CK(hipGetLastError());
@@ -3697,6 +3744,7 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         out->table_occupied = met.live + met.expired;
         out->flushed = flushed;
         out->rebuilt = 0;
+        CK(hipEventSynchronize(c->ev[5])); /* reached already: the counters were written after it */
         hipEventElapsedTime(&out->ms_partition, c->ev[0], c->ev[1]);
         hipEventElapsedTime(&out->ms_filter, c->ev[1], c->ev[2]);
         hipEventElapsedTime(&out->ms_refine, c->ev[2], c->ev[3]);

@@ -429,8 +429,8 @@ __device__ inline void decode_tail(const uint64_t *o_keys, const float4 *o_boxes
  * that the filters let pass waits in the wave's LDS until 64 of them are looked
  * up together: nearly every wave has one or two in every round, and the
  * lookup's chain of reads for those few was what bounded the scan. With 28-byte
- * meetings read whole or looked up one by one: 1,000 objects among 128M
- * meetings 2.10 -> 0.83 ms (8 bytes each at 1.2 TB/s; the id filter and the
+ * meetings read whole or looked up one by one: 1,000 objects among 256M
+ * meetings 2.10 -> 0.83 ms (8 bytes each at 2.5 TB/s; the id filter and the
  * table now bound it), one among 10M 52 -> 25 us, 48 crowded boxes with 446,000
  * hits 465 -> 257 us (with the hits' reservations, at q_emit); 128 mixed
  * queries, bound by the lookups, 408 -> 429. */

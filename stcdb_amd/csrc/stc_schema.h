@@ -28,6 +28,8 @@ struct Node {                 /* QTSchema (src/index/QTree.h:49-62) without its 
     uint32_t code, level;     /* Morton code of a rebuilt block; depth of a dynamic node */
 };
 
+enum { DC_SPLITS = 0, DC_MERGES = 1, DC_AMB = 2, DC_LEAVES = 3, DC_WORDS = 8 }; /* words of SchemaState::dcount */
+
 struct MapBox { double lo0, lo1, hi0, hi1; };
 
 /* The persistent tree: nodes in slots [0, hwm), free slots listed in fstack,

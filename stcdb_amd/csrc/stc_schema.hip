@@ -38,7 +38,6 @@
 #define SB_MAX_DEPTH 60
 #define SB_AMB_CAP 4096u
 
-enum { DC_SPLITS = 0, DC_MERGES = 1, DC_AMB = 2, DC_LEAVES = 3, DC_WORDS = 8 };
 
 /* degree_per_meter_longitude of the host (util.h:59-66), here with the
  * correctly rounded sine of stc_geo.h */
@@ -473,9 +472,7 @@ int stc_schema_plan(SchemaState *S, const uint32_t *leaf_count, uint32_t cap, do
     STC_CHECK(hipGetLastError());
     int rc = stc_exclusive_scan_u32(S->fs, S->rs, hwm, S->dcount + DC_SPLITS, temp, s);
     if (!rc) rc = stc_exclusive_scan_u32(S->fm, S->rm, hwm, S->dcount + DC_MERGES, temp, s);
-    if (rc) return rc;
-    STC_CHECK(hipMemcpyAsync(S->hcount, S->dcount, DC_WORDS * 4, hipMemcpyDeviceToHost, s));
-    return 0;
+    return rc; /* the numbers go to the host with the step's counters */
 }
 
 int stc_schema_apply(SchemaState *S, hipStream_t s) {
