@@ -8,8 +8,8 @@
 #include "../../include/stcdb.h"
 #include <vector>
 
-/* an object's place among the records: first slot, slots filled so far, sid (or the tail's key), record count */
-struct __attribute__((aligned(16))) ObjSlots { uint32_t base, fill, key, count; };
+/* an object's place among the records: first slot, first record as grouped, sid (or the tail's key), record count */
+struct __attribute__((aligned(16))) ObjSlots { uint32_t base, group, key, count; };
 
 struct FlushWork {
     uint32_t n = 0, ctf_count = 0;
@@ -25,6 +25,7 @@ struct FlushWork {
     ObjSlots *slots = nullptr;                     /* per-object record slots */
     uint8_t *part_tail = nullptr;                  /* per object: records go to the oversize buffer */
     uint32_t *obj_key = nullptr, *obj_id = nullptr, *obj_cnt = nullptr, *obj_first = nullptr; /* object placement order */
+    uint32_t *group = nullptr;                     /* per object: its first record in tkeys, tboxes */
     uint32_t *scan_temp = nullptr;
     size_t scan_temp_words = 0;
     uint32_t *flags = nullptr;                     /* device counters of the flush */
@@ -77,7 +78,7 @@ struct FlushArgs {
     uint64_t *rec_keys;      /* (lo, hi) per record */
     float4 *rec_boxes;
     uint32_t *same_pid_count;
-    uint4 *o_boxs;
+    uint32_t *rec_ord;       /* per record: its place among its object's, any order */
     uint16_t *sids;
 };
 

@@ -3,7 +3,9 @@
  * ctf_count CTFs (process_with_gpu's flush chain, src/cuda/geometry.cu:1752-2137).
  *
  * Order of the work, and what each step reproduces:
- *   F1 set_oid       per object: oversize test on the quantized object MBR
+ *   F0 groups        records to their object's range (a prefix sum of the record
+ *                    counts; each record's place in it came with its count)
+ *   F1 set_oid       per object: its quantized MBR from its records, oversize test on the quantized object MBR
  *                    and the STR key (geometry.cu:739-767, including the
  *                    high[1]-twice y term of :764)
  *   F2 STR           stable radix sort of (STR key, oid) over all objects, then
@@ -184,16 +186,27 @@ __global__ void k_flush_init(FlushCounters *fc, uint32_t oversize, uint32_t *cap
  * counts them as their first record arrives). 1M objects: 18 us (before, with
  * an update a wave and a pass for the count: 56). */
 __global__ __launch_bounds__(256) void k_set_oid(uint32_t n, const uint32_t *__restrict__ same_pid_count,
-                                                 const uint4 *__restrict__ o_boxs, uint16_t *__restrict__ sids,
+                                                 const uint32_t *__restrict__ group, const float4 *__restrict__ tboxes,
+                                                 uint16_t *__restrict__ sids,
                                                  uint64_t *__restrict__ mid, uint8_t *__restrict__ part_tail,
                                                  double area_threshold, uint32_t sticky, StrCompact sc, FlushCounters *fc) {
     uint32_t have = 0, over = 0;
     for (uint32_t id = blockIdx.x * blockDim.x + threadIdx.x; id < n; id += gridDim.x * blockDim.x) {
         uint64_t m = 0;
         uint32_t sid = sids[id];
-        if (same_pid_count[id] >= 1) {
+        const uint32_t cnt = same_pid_count[id];
+        if (cnt >= 1) {
             have++;
-            uint4 ob = o_boxs[id];
+            uint4 ob = make_uint4(100000000u, 100000000u, 0u, 0u);
+            const float4 *b = tboxes + group[id];
+#pragma unroll 4
+            for (uint32_t r = 0; r < cnt; r++) {
+                const float4 x = b[r];
+                ob.x = min(ob.x, f2q(x.x));
+                ob.y = min(ob.y, f2q(x.y));
+                ob.z = max(ob.z, f2q(x.z));
+                ob.w = max(ob.w, f2q(x.w));
+            }
             float low0 = q2f(ob.x), high0 = q2f(ob.z), low1 = q2f(ob.y), high1 = q2f(ob.w);
             float area = (high1 - low1) * (high0 - low0);
             if ((sticky && sid == 1) || (double)area > area_threshold) {
@@ -299,49 +312,48 @@ __global__ void k_gather_counts(const uint32_t *obj_id, const uint32_t *same_pid
     if (i < n) cnt[i] = same_pid_count[obj_id[i]];
 }
 
-/* all that placing an object's records takes, in one 16-byte word: a record's
- * object is anywhere, and base, fill, sid and tail in arrays of their own are
- * four cache lines a record (5.2M records of 5M objects: 380 -> 356 us, the
- * updates of fill being most of it) */
+/* all that placing an object's records takes, in one 16-byte word (in arrays
+ * of their own they are four cache lines a record) */
 __global__ void k_obj_slots(const uint32_t *__restrict__ obj_id, const uint32_t *__restrict__ obj_key,
-                            const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ first, uint32_t n,
-                            ObjSlots *__restrict__ slots) {
+                            const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ first,
+                            const uint32_t *__restrict__ group, uint32_t n, ObjSlots *__restrict__ slots) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) slots[obj_id[i]] = ObjSlots{first[i], 0, obj_key[i], cnt[i]};
+    if (i < n) slots[obj_id[i]] = ObjSlots{first[i], group[obj_id[i]], obj_key[i], cnt[i]};
 }
 
-/* records to their object's slot range; front keys get their CTF id (write_sid_in_key) */
-__global__ void k_scatter_records(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes, uint64_t K,
-                                  ObjSlots *slots, uint64_t *__restrict__ tkeys, float4 *__restrict__ tboxes) {
+/* records to their object's group: a random 32-byte write each (with the slot
+ * taken by an update of the object's, 356 us for 5.2M records of 5M objects;
+ * 178 so, and the objects' MBRs 164 in k_set_oid instead of four updates a
+ * record in the step) */
+__global__ void k_group_records(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes,
+                                const uint32_t *__restrict__ ord, uint64_t K, const uint32_t *__restrict__ group,
+                                uint64_t *__restrict__ tkeys, float4 *__restrict__ tboxes) {
     uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= K) return;
     const ulonglong2 key = ((const ulonglong2 *)keys)[k];
     const float4 box = boxes[k];
-    uint64_t hi = key.y;
-    ObjSlots *o = slots + (uint32_t)((hi >> 26) & OID_MASK);
-    const uint32_t base = o->base, okey = o->key;
-    const uint32_t slot = base + atomicAdd(&o->fill, 1u);
-    if (okey != TAIL_KEY) hi = (hi & ((1ull << SID_SHIFT_HI) - 1)) + ((uint64_t)okey << SID_SHIFT_HI);
-    ((ulonglong2 *)tkeys)[slot] = make_ulonglong2(key.x, hi);
+    const uint32_t slot = group[(uint32_t)((key.y >> 26) & OID_MASK)] + ord[k];
+    ((ulonglong2 *)tkeys)[slot] = key;
     tboxes[slot] = box;
 }
 
-/* each record moves to its rank inside its object's range */
+/* each record moves to its rank inside its object's slot range; front keys get their CTF id (write_sid_in_key) */
 __global__ void k_rank_records(const uint64_t *__restrict__ tkeys, const float4 *__restrict__ tboxes, uint64_t K,
                                const ObjSlots *__restrict__ slots, uint64_t *__restrict__ okeys,
                                float4 *__restrict__ oboxes) {
     uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= K) return;
     const ulonglong2 *tk = (const ulonglong2 *)tkeys;
-    const ulonglong2 key = tk[j];
+    ulonglong2 key = tk[j];
     const float4 box = tboxes[j];
     const ObjSlots o = slots[(uint32_t)((key.y >> 26) & OID_MASK)];
     uint32_t rank = 0;
 #pragma unroll 4
     for (uint32_t i = 0; i < o.count; i++) {
-        const ulonglong2 x = tk[o.base + i];
+        const ulonglong2 x = tk[o.group + i];
         rank += (x.y < key.y || (x.y == key.y && x.x < key.x)) ? 1u : 0u;
     }
+    if (o.key != TAIL_KEY) key.y = (key.y & ((1ull << SID_SHIFT_HI) - 1)) + ((uint64_t)o.key << SID_SHIFT_HI);
     const uint64_t dst = (uint64_t)o.base + rank;
     ((ulonglong2 *)okeys)[dst] = key;
     oboxes[dst] = box;
@@ -677,12 +689,11 @@ __global__ __launch_bounds__(256) void k_bitmap_keys(const uint64_t *__restrict_
 }
 
 /* the memtable's per-object state, empty (geometry.cu:2111-2131) */
-__global__ void k_reset_objects(uint32_t n, uint32_t *same_pid_count, uint16_t *sids, uint4 *o_boxs) {
+__global__ void k_reset_objects(uint32_t n, uint32_t *same_pid_count, uint16_t *sids) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     same_pid_count[i] = 0;
     sids[i] = 0;
-    o_boxs[i] = make_uint4(100000000u, 100000000u, 0u, 0u);
 }
 
 /* ------------------------------------------------------------------ */
@@ -706,7 +717,7 @@ int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count) {
     size_t N = n;
     if (hipMalloc((void **)&w->mid, N * 8) || hipMalloc((void **)&w->mid_alt, N * 8) ||
         hipMalloc((void **)&w->oids, N * 4) || hipMalloc((void **)&w->oids_alt, N * 4) ||
-        hipMalloc((void **)&w->slots, N * sizeof(ObjSlots)) || hipMalloc((void **)&w->obj_first, N * 4) ||
+        hipMalloc((void **)&w->slots, N * sizeof(ObjSlots)) || hipMalloc((void **)&w->obj_first, N * 4) || hipMalloc((void **)&w->group, N * 4) ||
         hipMalloc((void **)&w->capacity, (ctf_count + 1) * 4) || hipMalloc((void **)&w->ctf_base, (ctf_count + 1) * 4) ||
         hipMalloc((void **)&w->ctf_byte_base, (ctf_count + 1) * 8) ||
         hipMalloc((void **)&w->ctfs, ctf_count * sizeof(stc_ctf_meta)) ||
@@ -734,7 +745,7 @@ void stc_flush_free(FlushWork *w) {
     if (w->copied) (void)hipEventDestroy(w->copied);
     if (w->planned) (void)hipEventDestroy(w->planned);
     if (w->head) (void)hipHostFree(w->head);
-    void *ptrs[] = {w->chunks, w->sids_out, w->o_bitmap_dev, w->mid, w->mid_alt, w->oids, w->oids_alt, w->slots, w->obj_first, w->capacity, w->ctf_base,
+    void *ptrs[] = {w->chunks, w->sids_out, w->o_bitmap_dev, w->mid, w->mid_alt, w->oids, w->oids_alt, w->slots, w->obj_first, w->group, w->capacity, w->ctf_base,
                     w->ctf_byte_base, w->ctfs, w->bitmaps, w->flags, w->part_tail, w->obj_key, w->obj_id, w->obj_cnt,
                     w->scan_temp, w->keys_out, w->boxes_out, w->tkeys, w->tboxes, w->key_bytes};
     for (void *p : ptrs)
@@ -823,9 +834,13 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
             sc.strip_bits = by + bits_for(split);
         }
     }
-    /* F1 */
+    /* F0, F1 */
     const uint32_t few = std::max<uint32_t>(std::min<uint32_t>(blocks_for(n, B), 1024), 1); /* workgroups that update a counter */
-    hipLaunchKernelGGL(k_set_oid, dim3(few), dim3(B), 0, s, n, a->same_pid_count, a->o_boxs, a->sids,
+    FRC(stc_exclusive_scan_u32(a->same_pid_count, w->group, n, nullptr, w->scan_temp, s));
+    if (K)
+        hipLaunchKernelGGL(k_group_records, dim3(blocks_for(K, B)), dim3(B), 0, s, a->rec_keys, a->rec_boxes, a->rec_ord, K,
+                           w->group, w->tkeys, w->tboxes);
+    hipLaunchKernelGGL(k_set_oid, dim3(few), dim3(B), 0, s, n, a->same_pid_count, w->group, w->tboxes, a->sids,
                        w->mid, w->part_tail, a->area_threshold, a->sticky_oversize, sc, fc);
     FCK(hipGetLastError());
     /* F2: STR over the full 64-bit key (x high, y low), stable from oid order */
@@ -855,10 +870,8 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
                        w->obj_cnt);
     FRC(stc_exclusive_scan_u32(w->obj_cnt, w->obj_first, n, nullptr, w->scan_temp, s));
     hipLaunchKernelGGL(k_obj_slots, dim3(blocks_for(n, B)), dim3(B), 0, s, w->obj_id, w->obj_key, w->obj_cnt, w->obj_first,
-                       n, w->slots);
+                       w->group, n, w->slots);
     if (K) {
-        hipLaunchKernelGGL(k_scatter_records, dim3(blocks_for(K, B)), dim3(B), 0, s, a->rec_keys, a->rec_boxes, K,
-                           w->slots, w->tkeys, w->tboxes);
         hipLaunchKernelGGL(k_rank_records, dim3(blocks_for(K, B)), dim3(B), 0, s, w->tkeys, w->tboxes, K,
                            w->slots, w->keys_out, w->boxes_out);
     }
@@ -924,7 +937,7 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     out->blk = out->acquire(out->acquire_ctx, L.total);
     if (!out->blk.p) return stc_hip_fail(hipErrorOutOfMemory, "pinned run buffer", __FILE__, __LINE__);
     if (a->reset_memtable) {
-        hipLaunchKernelGGL(k_reset_objects, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a->same_pid_count, a->sids, a->o_boxs);
+        hipLaunchKernelGGL(k_reset_objects, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a->same_pid_count, a->sids);
         FCK(hipGetLastError());
     }
     /* the copies to the pinned block wait for stc_flush_release */

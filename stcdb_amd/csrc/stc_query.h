@@ -65,7 +65,7 @@ int stc_query_run(QueryBufs *b, const QueryState &st, const stc_query *q, uint32
  * counts, quantised MBRs, and sids[o] = 1 where R had o oversize. A record
  * whose ids are not below num_objects sets *bad and is not counted. */
 int stc_compact_decode(const QueryRunDev &R, uint64_t kv_count, uint32_t num_objects, uint32_t base, uint64_t out0,
-                       uint64_t *keys, float4 *boxes, uint32_t *same_pid_count, uint4 *o_boxs, uint16_t *sids,
+                       uint64_t *keys, float4 *boxes, uint32_t *same_pid_count, uint32_t *ord, uint16_t *sids,
                        uint32_t *bad, hipStream_t s);
 
 /* decode every record of a run kept in HBM once and summarise each CTF */

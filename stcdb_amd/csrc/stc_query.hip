@@ -743,18 +743,16 @@ __device__ inline float4 decode_fbox(const stc_ctf_meta &c, uint64_t vm) {
 }
 
 /* A run's records are grouped by object, so the lanes of a wave mostly share
- * a few objects: their per-object counts and box bounds are combined across
- * each run of equal ids first, and the run's first lane makes the atomic
- * updates (64 updates of one address would be serialised). */
+ * a few objects: the first lane of each run of equal ids adds up the run's
+ * length (64 updates of one address would be serialised), and its lanes take
+ * the records' places among their objects' from there. */
 __global__ __launch_bounds__(256) void k_compact_decode(QueryRunDev R, uint64_t kv_count, uint32_t num_objects,
                                                         uint32_t base, uint64_t out0, uint64_t *__restrict__ keys,
                                                         float4 *__restrict__ boxes, uint32_t *__restrict__ same_pid_count,
-                                                        uint4 *__restrict__ o_boxs, uint32_t *__restrict__ bad) {
+                                                        uint32_t *__restrict__ ord, uint32_t *__restrict__ bad) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & (STC_WAVE - 1);
     uint32_t pid = 0xFFFFFFFFu; /* no object: lanes past the end and bad records */
-    uint32_t cnt = 0;
-    uint4 q = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u);
     if (i < kv_count + R.n_tail) {
         uint32_t p, target, dur, end;
         float4 b;
@@ -795,31 +793,18 @@ __global__ __launch_bounds__(256) void k_compact_decode(QueryRunDev R, uint64_t 
             atomicOr(bad, 1u);
         } else {
             pid = p;
-            cnt = 1;
-            q = make_uint4(f2q(b.x), f2q(b.y), f2q(b.z), f2q(b.w));
-        }
-    }
-    /* lane l ends up holding the combination over lanes [l, end of its run of equal ids) */
-    for (int o = 1; o < STC_WAVE; o <<= 1) {
-        const uint32_t op = __shfl_down(pid, o, STC_WAVE), oc = __shfl_down(cnt, o, STC_WAVE);
-        const uint32_t o0 = __shfl_down(q.x, o, STC_WAVE), o1 = __shfl_down(q.y, o, STC_WAVE);
-        const uint32_t o2 = __shfl_down(q.z, o, STC_WAVE), o3 = __shfl_down(q.w, o, STC_WAVE);
-        if (lane + o < STC_WAVE && op == pid) {
-            cnt += oc;
-            q.x = min(q.x, o0);
-            q.y = min(q.y, o1);
-            q.z = max(q.z, o2);
-            q.w = max(q.w, o3);
         }
     }
     const uint32_t prev = __shfl_up(pid, 1, STC_WAVE);
-    if (pid != 0xFFFFFFFFu && (lane == 0 || prev != pid)) {
-        atomicAdd(&same_pid_count[pid], cnt);
-        atomicMin(&o_boxs[pid].x, q.x);
-        atomicMax(&o_boxs[pid].z, q.z);
-        atomicMin(&o_boxs[pid].y, q.y);
-        atomicMax(&o_boxs[pid].w, q.w);
-    }
+    const bool head = lane == 0 || prev != pid;
+    const uint64_t heads = __ballot(head), upto = heads & (~0ull >> (STC_WAVE - 1 - lane));
+    const int first = STC_WAVE - 1 - __clzll((long long)upto);
+    const uint64_t after = lane == STC_WAVE - 1 ? 0ull : heads >> (lane + 1);
+    uint32_t at = 0;
+    if (head && pid != 0xFFFFFFFFu)
+        at = atomicAdd(&same_pid_count[pid], after ? (uint32_t)__ffsll((long long)after) : (uint32_t)(STC_WAVE - lane));
+    at = (uint32_t)__shfl((int)at, first, STC_WAVE) + (uint32_t)(lane - first);
+    if (pid != 0xFFFFFFFFu) ord[out0 + i] = at;
 }
 
 __global__ void k_compact_sids(const uint16_t *__restrict__ run_sids, uint32_t n, uint16_t *__restrict__ sids) {
@@ -828,11 +813,11 @@ __global__ void k_compact_sids(const uint16_t *__restrict__ run_sids, uint32_t n
 }
 
 int stc_compact_decode(const QueryRunDev &R, uint64_t kv_count, uint32_t num_objects, uint32_t base, uint64_t out0,
-                       uint64_t *keys, float4 *boxes, uint32_t *same_pid_count, uint4 *o_boxs, uint16_t *sids,
+                       uint64_t *keys, float4 *boxes, uint32_t *same_pid_count, uint32_t *ord, uint16_t *sids,
                        uint32_t *bad, hipStream_t s) {
     if (kv_count + R.n_tail)
         hipLaunchKernelGGL(k_compact_decode, dim3(blocks(kv_count + R.n_tail, 256)), dim3(256), 0, s, R, kv_count,
-                           num_objects, base, out0, keys, boxes, same_pid_count, o_boxs, bad);
+                           num_objects, base, out0, keys, boxes, same_pid_count, ord, bad);
     QCK(hipGetLastError());
     hipLaunchKernelGGL(k_compact_sids, dim3(blocks(num_objects, 256)), dim3(256), 0, s, R.sids, num_objects, sids);
     QCK(hipGetLastError());
