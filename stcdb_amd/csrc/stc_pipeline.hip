@@ -3709,10 +3709,8 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         c->epoch++;
         flushed = 1;
     }
-    if (flushed) {
-        CK(hipEventRecord(c->ev[5], s));
-        CK(hipEventSynchronize(c->ev[5]));
-    }
+    if (flushed) CK(hipEventRecord(c->ev[5], s));
+    CK(hipEventSynchronize(c->ev[5])); /* without a flush reached already: the counters were written after it */
 
     c->stepped = true;
     c->last_t = t;
@@ -3737,7 +3735,6 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         out->table_occupied = met.live + met.expired;
         out->flushed = flushed;
         out->rebuilt = 0;
-        CK(hipEventSynchronize(c->ev[5])); /* reached already: the counters were written after it */
         hipEventElapsedTime(&out->ms_partition, c->ev[0], c->ev[1]);
         hipEventElapsedTime(&out->ms_filter, c->ev[1], c->ev[2]);
         hipEventElapsedTime(&out->ms_refine, c->ev[2], c->ev[3]);
