@@ -347,6 +347,16 @@ typedef struct stc_hit {
 
 int stc_query_batch(void *ctx, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap, uint64_t *n_hits,
               uint64_t *counts);
+/* The same for a caller that wants every hit and does not know how many there
+ * are: up to cap go to hits; of more, room(arg, n) is asked for an array of
+ * n, which takes them all, where the context's own hit buffer (as long as the
+ * largest cap so far, and half again) held them. Where it did not, or room
+ * gave null, *n_hits > cap and *all = 0: nothing is stored, and the batch is
+ * asked again with cap = *n_hits. room is called on the calling thread, at
+ * most once, and must not call into the context. */
+typedef stc_hit *(*stc_room)(void *arg, uint64_t n);
+int stc_query_batch_room(void *ctx, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap, stc_room room, void *arg,
+              uint64_t *n_hits, uint64_t *counts, int32_t *all);
 /* Serving. A query batch answers over the state the last completed step
  * published (its meetings, memtable and runs) and runs on the context's own
  * query stream, so batches issued from another host thread overlap the next

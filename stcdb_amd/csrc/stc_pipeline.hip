@@ -4091,7 +4091,7 @@ int stc_sync(void *vc) {
 extern "C++" {
 template <class Make>
 static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap, uint64_t *n_hits,
-                           uint64_t *counts, uint32_t *state_step, Make make) {
+                           uint64_t *counts, uint32_t *state_step, Make make, QueryRoom *more = nullptr) {
     std::lock_guard<std::mutex> ql(c->q_mu);
     /* admission: what the batch's query list, counters and hit buffer add to the query buffers */
     const uint64_t need = stc_query_bufs_growth(c->qb, nq, hits ? cap : 0);
@@ -4121,7 +4121,7 @@ static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *
     }
     int rc = 0;
     if (run) {
-        rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, STC_QUERY_RESERVE, c->qs);
+        rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, STC_QUERY_RESERVE, more, c->qs);
     } else {
         *n_hits = 0;
     }
@@ -4450,6 +4450,18 @@ int stc_query_batch_at(void *vc, const stc_query *q, uint32_t nq, stc_hit *hits,
 int stc_query_batch(void *vc, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap, uint64_t *n_hits,
                     uint64_t *counts) {
     return stc_query_batch_at(vc, q, nq, hits, cap, n_hits, counts, nullptr);
+}
+
+int stc_query_batch_room(void *vc, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap, stc_room room, void *arg,
+                         uint64_t *n_hits, uint64_t *counts, int32_t *all) {
+    StcCtx *c = (StcCtx *)vc;
+    if (!c || (!q && nq) || !n_hits || !all || !room || (!hits && cap)) return STC_E_ARG;
+    for (uint32_t i = 0; i < nq; i++)
+        if (q[i].kind < STC_Q_OID || q[i].kind > STC_Q_PAIR) return fail(c, STC_E_ARG, "unknown query kind");
+    QueryRoom more{room, arg, false};
+    const int rc = query_published(c, q, nq, hits, cap, n_hits, counts, nullptr, nullptr, &more);
+    *all = rc == STC_OK && more.all;
+    return rc;
 }
 
 } /* extern "C" */

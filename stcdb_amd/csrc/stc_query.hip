@@ -991,9 +991,10 @@ static bool ctf_may_intersect(const stc_ctf_meta &c, const double *box) {
 }
 
 int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap,
-                  uint64_t *n_hits, uint64_t *counts, uint64_t reserve, hipStream_t s) {
+                  uint64_t *n_hits, uint64_t *counts, uint64_t reserve, QueryRoom *more, hipStream_t s) {
     if (nq == 0) {
         *n_hits = 0;
+        if (more) more->all = true;
         return STC_OK;
     }
     /* hash of the queried ids (object and pair queries) */
@@ -1110,7 +1111,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     Q.fix = (float)(ix * (QFINE / QGRID));
     Q.fiy = (float)(iy * (QFINE / QGRID));
     Q.hits = B->hits;
-    Q.cap = hits ? cap : 0;
+    Q.cap = more ? B->hits_cap : hits ? cap : 0;
     Q.n_hits = counters;
     Q.counts = counters + 1;
     Q.nq = nq;
@@ -1196,6 +1197,16 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         if (counts) counts[i] = ci;
     }
     *n_hits = total;
+    if (more) {
+        more->all = total <= Q.cap;
+        if (more->all && total > cap) {
+            stc_hit *all = more->room(more->arg, total);
+            more->all = all != nullptr;
+            hits = all;
+            cap = total;
+        }
+        if (!more->all) return STC_OK;
+    }
     uint64_t stored = Q.cap ? std::min<uint64_t>(cnt[0], cap) : 0;
     bool sorted = false;
     if (stored > QSORT_HOST && hits) {

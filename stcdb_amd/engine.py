@@ -254,13 +254,32 @@ class Pipeline:
         q = np.ascontiguousarray(q, dtype=QUERY_DTYPE)
         counts = np.zeros(len(q), dtype=np.uint64)
         if cap is None:
-            hits = self._fetch(FETCH_ROWS, into, lambda h, n: self.lib.stc_query_batch(
-                self.ctx, _ptr(q), len(q), _ptr(h), len(h), C.byref(n), _ptr(counts)))
-            return hits, counts
+            return self._query_all(q, counts, into), counts
         n = C.c_uint64()
         hits = into if into is not None and len(into) >= cap else np.zeros(cap, dtype=HIT_DTYPE)
         _check(self.lib.stc_query_batch(self.ctx, _ptr(q), len(q), _ptr(hits), cap, C.byref(n), _ptr(counts)), self.ctx)
         return hits[:min(n.value, cap)], counts
+
+    def _query_all(self, q, counts, into):
+        """all hits of a batch, in `into` or a first guess where they fit, else in an array of their number: at once
+        where the device held them all, by a second call where its buffer has to grow first"""
+        n, all_ = C.c_uint64(), C.c_int32()
+        hits = into if into is not None and len(into) else np.empty(FETCH_ROWS, dtype=HIT_DTYPE)
+        more = []
+
+        def room(_, count):
+            more.append(np.empty(count, dtype=HIT_DTYPE))
+            return more[0].ctypes.data
+
+        _check(self.lib.stc_query_batch_room(self.ctx, _ptr(q), len(q), _ptr(hits), len(hits), L.ROOM(room), None, C.byref(n),
+                                             _ptr(counts), C.byref(all_)), self.ctx)
+        if all_.value and more:
+            return more[0]
+        if all_.value:
+            return hits[:n.value] if hits is into else hits[:n.value].copy()
+        hits = np.empty(n.value, dtype=HIT_DTYPE)
+        _check(self.lib.stc_query_batch(self.ctx, _ptr(q), len(q), _ptr(hits), len(hits), C.byref(n), _ptr(counts)), self.ctx)
+        return hits[:min(n.value, len(hits))]
 
     def _fetch(self, rows, into, call):
         """all hits of call(buffer, n): one call where they fit in `into`, or

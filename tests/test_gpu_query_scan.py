@@ -45,3 +45,28 @@ def test_scan_edges(cells):
     assert found > 2000
     gpu.close()
     orc.close()
+
+
+@pytest.mark.parametrize("rows", [1, 1 << 14])
+def test_more_hits_than_the_first_guess(rows, monkeypatch):
+    """the hits of places, asked again and again: by a second call while the device's buffer is short, at once after it"""
+    import stcdb_amd.engine as engine
+    monkeypatch.setattr(engine, "FETCH_ROWS", rows)
+    w = workload("c1", num_objects=2500, kv_restriction=400, min_meet_time=2, device_runs=1, reach_distance=12.0)
+    w["gen"].update(n_hotspots=2, hotspot_frac=0.8, hotspot_sigma=120.0)
+    gpu, orc = Pipeline(w["cfg"], w["box"]), O.Oracle(w["cfg"], w["box"])
+    for t, xy in HostTrace(w["gen"]).steps(12):
+        gpu.step(xy, t)
+        orc.step(xy, t)
+    q = make_queries(orc, w, np.random.default_rng(1), 3)[:1].repeat(24)
+    q["kind"], q["t0"], q["t1"] = 2, 0, 20
+    q["box"] = boxes(np.random.default_rng(2), w["box"], len(q))
+    sizes = []
+    for n in (4, 24, 24, 8, 1):
+        sizes.append(compare(gpu, orc, q[:n], f"{n} places, {rows} rows"))
+    assert max(sizes) > 2 * (1 << 14) and min(sizes) > 0
+    into = np.zeros(5, dtype=engine.HIT_DTYPE)
+    hits, _ = gpu.query(q, into=into)
+    assert len(hits) == sizes[1] and np.array_equal(hits.view(np.uint8), orc.query(q)[0].view(np.uint8))
+    gpu.close()
+    orc.close()
