@@ -3,8 +3,8 @@
  *
  * Object-history, square-range and pair queries (semantics at stc_query_batch in
  * include/stcdb.h) are answered from three sources in one pass each:
- *   - the meeting table: a grid-stride scan over the buckets, live buckets
- *     (end == last step) matched in both directions;
+ *   - the live meetings: a grid-stride scan over their ids, boxes or both, live
+ *     ones (end == last step) matched in both directions;
  *   - the memtable records: one thread per record;
  *   - the runs kept in HBM: object and pair queries look the object's CTF up
  *     through the run's sids and search its packed keys (a wave each, 64 probes
@@ -102,8 +102,9 @@ struct QueryBufs {
 };
 
 #define QFETCH 65536u /* hits of a chunk */
-#define QSORT_HOST 1024u /* up to this many hits are copied as they are and sorted by the host: the device sort's
-                          * launches cost what that does (about 80 us at 1,000 hits) */
+#define QSORT_HOST 256u /* up to this many hits come with the counters and are sorted by the host: the device's ranking
+                         * costs a wait more (some 30 us; the host takes about 80 at 1,000 hits) */
+#define QRANK 16384u    /* and up to this many are ranked by comparing all with all */
 
 
 uint64_t stc_query_bufs_growth(const QueryBufs *b, uint32_t nq, uint64_t cap) {
@@ -907,8 +908,45 @@ __global__ void k_hit_gather(const uint64_t *__restrict__ hits, const uint32_t *
 }
 static_assert(sizeof(stc_hit) == 56, "a hit is seven words");
 
+/* rank[i] += the hits of the workgroup's tile that come before hit i: (query,
+ * source, pid, target, start, end) as three words, equal ones in the order they
+ * were found. A radix sort of a few thousand hits is some twenty launches and
+ * nothing but latency; all with all is n^2 / 2^16 workgroups of 256 short
+ * rounds (128 queries with some 3,000 hits: 714 -> 672 us, a step with 1,200
+ * contacts 1,679 -> 1,646). */
+__global__ __launch_bounds__(256) void k_hit_rank(const stc_hit *__restrict__ hits, uint32_t n, uint32_t *__restrict__ rank) {
+    __shared__ uint64_t ka[256], kb[256], kc[256];
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, j0 = blockIdx.y * 256, j = j0 + threadIdx.x;
+    auto load = [&](uint32_t k, uint64_t *a, uint64_t *b, uint64_t *c) {
+        const stc_hit &h = hits[min(k, n - 1)];
+        *a = (uint64_t)h.query << 32 | h.source;
+        *b = (uint64_t)h.pid << 32 | h.target;
+        *c = (uint64_t)h.start << 32 | h.end;
+    };
+    uint64_t a, b, c;
+    load(j, &ka[threadIdx.x], &kb[threadIdx.x], &kc[threadIdx.x]);
+    load(i, &a, &b, &c);
+    __syncthreads();
+    const uint32_t m = min(256u, n - j0);
+    uint32_t before = 0;
+#pragma unroll 4
+    for (uint32_t k = 0; k < m; k++) {
+        const uint64_t x = ka[k], y = kb[k], z = kc[k];
+        const bool last = z < c || (z == c && j0 + k < i);
+        before += (x < a || (x == a && (y < b || (y == b && last)))) ? 1u : 0u;
+    }
+    if (i < n && before) atomicAdd(&rank[i], before);
+}
+
+/* the hits to their ranks in out (host memory), 8 bytes a thread */
+__global__ void k_hit_place(const uint64_t *__restrict__ hits, const uint32_t *__restrict__ rank, uint32_t words,
+                            uint64_t *__restrict__ out) {
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w < words) out[(uint64_t)rank[w / 7] * 7 + w % 7] = hits[w];
+}
+
 /* The n stored hits to the caller's `hits`, sorted by (query, source, pid,
- * target, start, end): a radix sort of the packed fields on the device, then
+ * target, start, end): up to QRANK of them ranked, more by a radix sort of the packed fields on the device, then
  * chunks gathered in order into pinned memory and copied out while the next is
  * gathered. *done stays false when the fields do not pack, a value does not fit
  * its bits, or the scratch would leave less than `reserve` bytes of device
@@ -923,9 +961,10 @@ static int fetch_sorted(QueryBufs *B, const QueryState &st, uint32_t nq, uint64_
     for (const QueryRunDev &r : st.runs) kb.src = std::max(kb.src, bits_for(r.source));
     const uint32_t hb = kb.q + kb.src + kb.id, lb = kb.id + 2 * kb.t;
     kb.two = hb + lb > 64;
-    if (n64 >= (1ull << 31) || hb > 64 || lb > 64) return STC_OK;
+    const bool ranked = n64 <= QRANK;
+    if (!ranked && (n64 >= (1ull << 31) || hb > 64 || lb > 64)) return STC_OK;
     const uint32_t n = (uint32_t)n64;
-    const uint64_t bytes = n64 * 24 + stc_radix_temp_words(n) * 4;
+    const uint64_t bytes = ranked ? n64 * 4 : n64 * 24 + stc_radix_temp_words(n) * 4;
     if (B->sort_cap < bytes) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes + bytes / 2 + reserve > free_b + B->sort_cap) return STC_OK;
@@ -938,6 +977,18 @@ static int fetch_sorted(QueryBufs *B, const QueryState &st, uint32_t nq, uint64_
     for (int i = 0; i < 2; i++) {
         if (!B->out[i]) QCK(hipHostMalloc((void **)&B->out[i], QFETCH * sizeof(stc_hit), hipHostMallocDefault));
         if (!B->out_ev[i]) QCK(hipEventCreateWithFlags(&B->out_ev[i], hipEventDisableTiming));
+    }
+    if (ranked) {
+        uint32_t *rank = (uint32_t *)B->sort;
+        QCK(hipMemsetAsync(rank, 0, n * 4ull, s));
+        hipLaunchKernelGGL(k_hit_rank, dim3(blocks(n, 256), blocks(n, 256)), dim3(256), 0, s, B->hits, n, rank);
+        hipLaunchKernelGGL(k_hit_place, dim3(blocks(n * 7ull, 256)), dim3(256), 0, s, (const uint64_t *)B->hits,
+                           (const uint32_t *)rank, n * 7, (uint64_t *)B->out[0]);
+        QCK(hipGetLastError());
+        QCK(hipStreamSynchronize(s));
+        memcpy(hits, B->out[0], n64 * sizeof(stc_hit));
+        *done = true;
+        return STC_OK;
     }
     uint64_t *ka = (uint64_t *)B->sort, *kb2 = ka + n;
     uint32_t *va = (uint32_t *)(kb2 + n), *vb = va + n, *temp = vb + n;
