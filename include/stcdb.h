@@ -365,8 +365,8 @@ int stc_query_batch_room(void *ctx, const stc_query *q, uint32_t nq, stc_hit *hi
  * start after a flush). Batches are admitted by free device memory: one whose
  * query list and hit buffer would leave less than 1 GiB free returns
  * STC_E_CAPACITY (split it and retry). stc_query_batch_at also reports the
- * timestep of the state it answered. Only stc_query_batch, stc_query_batch_at
- * and stc_live_search may run concurrently with stc_step on one context;
+ * timestep of the state it answered. Only stc_query_batch, stc_query_batch_room,
+ * stc_query_batch_at and stc_live_search may run concurrently with stc_step on one context;
  * stc_drop_runs and stc_compact_runs wait for batches in flight. The
  * reference answers its live search from the command thread between steps
  * (process.cpp:350-371, 443-495). */
