@@ -464,12 +464,13 @@ __global__ void k_amb_gather(const double2 *__restrict__ xy, const uint2 *__rest
 }
 
 /* leaf-ordered SoA and each point's rank within its leaf; and, a thread per leaf, the points beyond its buffer */
+/* Positions and scales in leaf order; the points' leaves in that order are the
+ * sort's keys. Bound by the two reads at the points' ids, a line each (with the
+ * leaf read there too and each point's rank written there, 5M objects 350 us;
+ * 197 so). */
 __global__ void k_gather(const double2 *__restrict__ xy, const double *__restrict__ dlon,
-                         const uint32_t *__restrict__ lp, const uint32_t *__restrict__ pt_leaf,
-                         const uint32_t *__restrict__ leaf_start, uint32_t n, double2 *__restrict__ lxy,
-                         double *__restrict__ ld, uint32_t *__restrict__ pt_rank,
-                         uint32_t *__restrict__ lleaf, const uint32_t *__restrict__ leaf_count, uint32_t nl, uint32_t buf,
-                         Counters *cnt) {
+                         const uint32_t *__restrict__ lp, uint32_t n, double2 *__restrict__ lxy, double *__restrict__ ld,
+                         const uint32_t *__restrict__ leaf_count, uint32_t nl, uint32_t buf, Counters *cnt) {
     uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < nl && leaf_count[j] > buf) atomicAdd(&cnt->overflow, leaf_count[j] - buf);
     if (j >= n) return;
@@ -477,9 +478,6 @@ __global__ void k_gather(const double2 *__restrict__ xy, const double *__restric
     double2 q = xy[p];
     lxy[j] = q;
     ld[j] = dlon[p];
-    const uint32_t L = pt_leaf[p];
-    pt_rank[p] = j - leaf_start[L];
-    lleaf[j] = L;
 }
 
 /* ------------------------------------------------------------------ */
@@ -702,7 +700,7 @@ struct PairGeo {
     const double2 *xy;
     const double *dlon;
     const double2 *lxy;                  /* positions in leaf order (one 16-byte read per candidate) */
-    const uint32_t *pt_leaf, *pt_rank, *leaf_start, *leaf_count, *lp;
+    const uint32_t *pt_leaf, *leaf_start, *leaf_count, *lp;
     const double *ld;                    /* dpm_lon in leaf order */
     const uint32_t *lleaf;               /* leaf of each point, in leaf order */
     const uint2 *lunits;                 /* (first cross unit, count) of each point, in leaf order */
@@ -778,6 +776,12 @@ __device__ inline uint32_t wave_upper_bound(const uint32_t *arr, uint32_t n, uin
         hi = nhi;
     }
     return lo;
+}
+
+/* the place in leaf order of an object, by the whole wave: its leaf's points are in id order */
+__device__ inline uint32_t place_of(const PairGeo &g, uint32_t a, int lane) {
+    const uint32_t L = g.pt_leaf[a], st = g.leaf_start[L];
+    return st + wave_upper_bound(g.lp + st, g.leaf_count[L], a, lane) - 1;
 }
 
 template <class F>
@@ -1487,7 +1491,7 @@ __global__ __launch_bounds__(256, 5) void k_seg_sort_wave(PairGeo g, const uint3
     for (uint32_t oi = wid; oi < n_owners; oi += nw) {
         const uint32_t a = owners[oi];
         const uint32_t base = poff[a], slots = poff[a + 1] - base;
-        const uint32_t w = g.leaf_start[g.pt_leaf[a]] + g.pt_rank[a]; /* a's place in leaf order */
+        const uint32_t w = place_of(g, a, lane);
         write_sorted_segment<WSORT_CAP / STC_WAVE>(psrc + pkrun[w].x, slots, a, w, g, acc, n_acc, pn + base, lane);
     }
 }
@@ -1505,7 +1509,7 @@ __global__ void k_huge_expand(PairGeo g, const uint32_t *__restrict__ owners, ui
     for (uint32_t oi = wid; oi < n_owners; oi += nw) {
         const uint32_t a = owners[oi];
         const uint32_t base = poff[a], slots = poff[a + 1] - base;
-        const uint32_t w = g.leaf_start[g.pt_leaf[a]] + g.pt_rank[a];
+        const uint32_t w = place_of(g, a, lane);
         const uint32_t *srcs = psrc + pkrun[w].x;
         for (uint32_t i = lane; i < slots; i += STC_WAVE) {
             const unsigned long long k = settle_key(srcs[i], a, g, acc, n_acc);
@@ -2577,8 +2581,8 @@ struct StcCtx {
     DBuf<Node> nodes;
     DBuf<FrontierItem> frontier_a, frontier_b;
     DBuf<uint32_t> leaf_count, leaf_start, leaf_node;
-    DBuf<uint32_t> pt_leaf, pt_lv, pt_rank, lp, lkeys;
-    DBuf<uint32_t> lleaf;                /* leaf of each point, in leaf order */
+    DBuf<uint32_t> pt_leaf, pt_lv, lp;
+    DBuf<uint32_t> lkeys;                /* leaf of each point, in leaf order */
     DBuf<uint2> lunits;                  /* first cross unit and count of each point, in leaf order */
     DBuf<uint2> urange;                  /* per cross unit: member range above its point */
     DBuf<uint4> prange;                  /* per point in leaf order: own-leaf and reverse-list ranges */
@@ -3106,8 +3110,8 @@ int stc_create(const stc_config *cfg, const stc_box *mbr, void **out) {
     if (c->xy_in.ensure(n) || c->codes.ensure(n) || c->idx.ensure(n) || c->codes_alt.ensure(n) ||
         c->idx_alt.ensure(n) || c->dlon.ensure(n) || c->posf.ensure(n) || c->lxy.ensure(n) || c->ld.ensure(n) ||
         c->nodes.ensure(node_cap) || c->frontier_a.ensure(front_cap) || c->frontier_b.ensure(front_cap) ||
-        c->pt_leaf.ensure(n) || c->pt_lv.ensure(n) || c->pt_rank.ensure(n) || c->lp.ensure(n) ||
-        c->lleaf.ensure(n) || c->lunits.ensure(n) || c->prange.ensure(n) ||
+        c->pt_leaf.ensure(n) || c->pt_lv.ensure(n) || c->lp.ensure(n) ||
+        c->lunits.ensure(n) || c->prange.ensure(n) ||
         c->lkeys.ensure(n) || c->ucount.ensure(n) || c->uoffset.ensure(n) || c->units.ensure(4ull * n) ||
         c->amb.ensure(1 << 16) || c->pcount.ensure(n) || c->moff[0].ensure(n + 1ull) || c->moff[1].ensure(n + 1ull) ||
         c->spill_big.ensure(n) || c->spill_huge.ensure(n) || c->spill_giant.ensure(n) ||
@@ -3148,8 +3152,8 @@ int stc_destroy(void *vc) {
     c->xy_in.release(); c->codes.release(); c->idx.release(); c->codes_alt.release(); c->idx_alt.release();
     c->temp.release(); c->dlon.release(); c->posf.release(); c->lxy.release(); c->ld.release(); c->nodes.release();
     c->frontier_a.release(); c->frontier_b.release(); c->leaf_count.release(); c->leaf_start.release();
-    c->leaf_node.release(); c->pt_leaf.release(); c->pt_lv.release(); c->pt_rank.release(); c->lp.release();
-    c->lleaf.release(); c->lunits.release(); c->urange.release(); c->prange.release();
+    c->leaf_node.release(); c->pt_leaf.release(); c->pt_lv.release(); c->lp.release();
+    c->lunits.release(); c->urange.release(); c->prange.release();
     c->lkeys.release(); c->ucount.release(); c->uoffset.release(); c->units.release();
     c->amb.release(); c->amb_xy.release();
     c->rev_leaf.release(); c->rev_pid.release(); c->rev_leaf_alt.release(); c->rev_pid_alt.release();
@@ -3307,8 +3311,8 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     CKRC(stc_exclusive_scan_u32(c->leaf_count.p, c->leaf_start.p, n_leaves, nullptr, c->temp.p, s));
     CKRC(sort_pairs((const uint32_t *)c->pt_leaf.p, (const uint32_t *)nullptr, c->lkeys, c->lp, c->codes_alt, c->idx_alt, n,
                     std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
-    hipLaunchKernelGGL(k_gather, dim3(blocks_for(std::max(n, n_leaves), 256)), dim3(256), 0, s, xy, c->dlon.p, c->lp.p, c->pt_leaf.p,
-                       c->leaf_start.p, n, c->lxy.p, c->ld.p, c->pt_rank.p, c->lleaf.p, (const uint32_t *)c->leaf_count.p, n_leaves,
+    hipLaunchKernelGGL(k_gather, dim3(blocks_for(std::max(n, n_leaves), 256)), dim3(256), 0, s, xy, c->dlon.p, c->lp.p, n,
+                       c->lxy.p, c->ld.p, (const uint32_t *)c->leaf_count.p, n_leaves,
                        c->buf, cnt);
     c->lp_valid = true; /* lp: a permutation of the points, in this step's leaf order */
     CK(hipGetLastError());
@@ -3363,12 +3367,12 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
     /* 8: the pairs owner by owner: count (a band combination reserves a slot),
      * the band decided on the host, segment offsets, write */
     hipLaunchKernelGGL(k_point_ranges, dim3(blocks_for(n, 256)), dim3(256), 0, s, (const uint32_t *)c->lp.p,
-                       (const uint32_t *)c->lleaf.p, n, (const uint32_t *)c->leaf_start.p,
+                       (const uint32_t *)c->lkeys.p, n, (const uint32_t *)c->leaf_start.p,
                        (const uint32_t *)c->leaf_count.p, (const uint32_t *)c->rev_start.p,
                        (const uint32_t *)c->rev_pid.p, c->buf, c->prange.p);
     CK(hipGetLastError());
-    const PairGeo pg{xy, c->dlon.p, c->lxy.p, c->pt_leaf.p, c->pt_rank.p, c->leaf_start.p,
-                     c->leaf_count.p, c->lp.p, c->ld.p, c->lleaf.p, c->lunits.p, c->urange.p, c->prange.p,
+    const PairGeo pg{xy, c->dlon.p, c->lxy.p, c->pt_leaf.p, c->leaf_start.p,
+                     c->leaf_count.p, c->lp.p, c->ld.p, c->lkeys.p, c->lunits.p, c->urange.p, c->prange.p,
                      c->units.p, c->uoffset.p,
                      c->ucount.p, c->rev_start.p, c->rev_pid.p,
                      c->rev.p, c->rev_dl.p, n, c->buf, r, c->band, r * r * (1.0 - 1e-12),
