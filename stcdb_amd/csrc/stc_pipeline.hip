@@ -589,7 +589,7 @@ __global__ __launch_bounds__(LK_THREADS) void k_lookup(const uint32_t *__restric
 }
 
 /* The cross units in point order, and all that is kept of each: the leaf and
- * the point, from which the reverse lists are sorted, and the leaf's kept members above
+ * the point's place in leaf order, from which the reverse lists are sorted, and the leaf's kept members above
  * the point (an index range into the leaf-ordered arrays); and each point's
  * first unit and count in leaf order. The leaves come from the lookup; a point
  * with more than it keeps descends again. (A second descent for every point,
@@ -602,7 +602,7 @@ __global__ __launch_bounds__(LK_THREADS) void k_units_emit(
     const Node *__restrict__ nodes, const uint32_t *__restrict__ pt_lv, double r, double band,
     const uint32_t *__restrict__ count, const uint32_t *__restrict__ offset, const uint4 *__restrict__ kept,
     const uint32_t *__restrict__ leaf_start, const uint32_t *__restrict__ leaf_count, uint32_t buf,
-    uint32_t *__restrict__ unit_leaf, uint32_t *__restrict__ unit_pid, uint2 *__restrict__ urange, uint2 *__restrict__ lunits) {
+    uint32_t *__restrict__ unit_leaf, uint32_t *__restrict__ unit_place, uint2 *__restrict__ urange, uint2 *__restrict__ lunits) {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const uint32_t p = lp[j], c = count[p];
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(LK_THREADS) void k_units_emit(
         for (uint32_t i = 0; i < LK_KEPT; i++)
             if (i < c) {
                 unit_leaf[u + i] = leaf[i];
-                unit_pid[u + i] = p;
+                unit_place[u + i] = j;
                 urange[u + i] = make_uint2(first[i] + lo[i], have[i] - lo[i]);
             }
     } else {
@@ -658,7 +658,7 @@ __global__ __launch_bounds__(LK_THREADS) void k_units_emit(
             const uint32_t s2 = min(leaf_count[leaf], buf);
             const uint32_t st2 = leaf_start[leaf], m0 = lower_bound_u32(lp + st2, s2, p + 1);
             unit_leaf[u] = leaf;
-            unit_pid[u] = p;
+            unit_place[u] = j;
             urange[u] = make_uint2(st2 + m0, s2 - m0);
             u++;
         });
@@ -839,23 +839,29 @@ __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const Pair
 }
 
 /* The reverse lists' finish: the border points' data in list order, so that
- * owners read it coalesced, and each leaf's first entry (rev_start[n_leaves] = nr). */
-__global__ void k_rev_finish(const uint32_t *__restrict__ rev_leaf, const uint32_t *__restrict__ rev_pid, uint32_t nr,
-                             uint32_t n_leaves, const double2 *__restrict__ xy, const double *__restrict__ dlon,
-                             RevPt *__restrict__ rev, double *__restrict__ rev_dl, uint32_t *__restrict__ rev_start) {
+ * owners read it coalesced, and each leaf's first entry (rev_start[n_leaves] =
+ * nr). rev_pid comes with the points' places in leaf order and leaves with
+ * their ids: a leaf's border points lie in its neighbours, a few stretches of
+ * the leaf-ordered arrays, where by id each was a line of its own (5M objects,
+ * 5.4M units: 220 -> 86 us). */
+__global__ void k_rev_finish(const uint32_t *__restrict__ rev_leaf, uint32_t *__restrict__ rev_pid, uint32_t nr,
+                             uint32_t n_leaves, const uint32_t *__restrict__ lp, const double2 *__restrict__ lxy,
+                             const double *__restrict__ ld, RevPt *__restrict__ rev, double *__restrict__ rev_dl,
+                             uint32_t *__restrict__ rev_start) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nr) {
-        const uint32_t p = rev_pid[i];
-        const double2 q = xy[p];
-        const double d = dlon[p];
+        const uint32_t j = rev_pid[i];
+        const double2 q = lxy[j];
+        const double d = ld[j];
         RevPt r;
         r.x = q.x;
         r.y = q.y;
-        r.il = 1.0 / d; /* the reciprocal of dlon[p], as the owners' loops compute theirs */
-        r.pid = p;
+        r.il = 1.0 / d; /* the reciprocal of the point's dlon, as the owners' loops compute theirs */
+        r.pid = lp[j];
         r.pad = 0;
         rev[i] = r;
         rev_dl[i] = d;
+        rev_pid[i] = r.pid;
     }
     if (i <= n_leaves) rev_start[i] = lower_bound_u32(rev_leaf, nr, i);
 }
@@ -3360,8 +3366,8 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
         CKRC(sort_pairs((const uint32_t *)c->units.p, (const uint32_t *)c->rev_pid_alt.p, c->rev_leaf, c->rev_pid, c->rev_leaf_alt,
                         c->rev_pid_alt, (uint32_t)n_units, std::max(1, ilog2_ceil(n_leaves)), c->temp.p, s));
     hipLaunchKernelGGL(k_rev_finish, dim3(blocks_for(std::max<uint64_t>(n_units, n_leaves + 1ull), 256)), dim3(256), 0, s,
-                       (const uint32_t *)c->rev_leaf.p, (const uint32_t *)c->rev_pid.p, (uint32_t)n_units, n_leaves, xy,
-                       (const double *)c->dlon.p, c->rev.p, c->rev_dl.p, c->rev_start.p);
+                       (const uint32_t *)c->rev_leaf.p, c->rev_pid.p, (uint32_t)n_units, n_leaves, (const uint32_t *)c->lp.p,
+                       (const double2 *)c->lxy.p, (const double *)c->ld.p, c->rev.p, c->rev_dl.p, c->rev_start.p);
     CK(hipGetLastError());
 
     /* 8: the pairs owner by owner: count (a band combination reserves a slot),
