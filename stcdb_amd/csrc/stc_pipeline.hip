@@ -2485,15 +2485,18 @@ struct DBuf {
     void release() { if (p) hipFree(p); p = nullptr; cap = 0; }
 };
 
-/* a step's meetings */
+/* a step's meetings: the three arrays in one allocation, as long as its capacity each (with an allocation each, to be
+ * grown and freed in the first steps, 16 contexts took 353 ms to a steady state together, and 185 with one) */
 struct MeetBuf {
-    DBuf<unsigned long long> keys;
-    DBuf<uint32_t> starts;
-    DBuf<uint4> mbrs;
-    int ensure(size_t n) { return keys.ensure(n) || starts.ensure(n) || mbrs.ensure(n) ? -1 : 0; }
-    void release() { keys.release(); starts.release(); mbrs.release(); }
-    Meets view() const { return Meets{keys.p, starts.p, mbrs.p}; }
+    DBuf<Bucket> mem;
+    int ensure(size_t n) { return mem.ensure(n); }
+    void release() { mem.release(); }
+    uint4 *mbrs() const { return (uint4 *)mem.p; }
+    unsigned long long *keys() const { return (unsigned long long *)(mbrs() + mem.cap); }
+    uint32_t *starts() const { return (uint32_t *)(keys() + mem.cap); }
+    Meets view() const { return Meets{keys(), starts(), mbrs()}; }
 };
+static_assert(sizeof(Bucket) == sizeof(uint4) + sizeof(unsigned long long) + sizeof(uint32_t), "a bucket of each array");
 
 /* A flushed run: metadata on the host, payload in a pinned block that the
  * copy stream fills while later steps run. */
@@ -2865,7 +2868,7 @@ static int export_live(StcCtx *c, uint64_t cap, Take take) {
     if (c->last_live != c->mlen) { /* dead buckets: the tiles' outputs by a scan */
         if (c->xtiles.ensure(tiles + stc_radix_temp_words((uint32_t)tiles))) return fail(c, STC_E_CAPACITY, "export tiles");
         hipLaunchKernelGGL(k_live_tiles, dim3((uint32_t)tiles), dim3(256), 0, c->s,
-                           (const unsigned long long *)c->meet[c->cur].keys.p, c->mlen, c->xtiles.p);
+                           (const unsigned long long *)c->meet[c->cur].keys(), c->mlen, c->xtiles.p);
         CK(hipGetLastError());
         CKRC(stc_exclusive_scan_u32(c->xtiles.p, c->xtiles.p, (uint32_t)tiles, nullptr, c->xtiles.p + tiles, c->s));
         base.resize(tiles);
@@ -3567,14 +3570,14 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     if (c->tbounds.ensure(n_tiles + 1ull) || c->towner.ensure(n_tiles)) return fail(c, STC_E_CAPACITY, "merge tile bounds");
     if (c->pairs_boxed) {
         hipLaunchKernelGGL(k_tile_bounds<PairHit>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairHit *)c->pbox.p, c->plen, (const unsigned long long *)c->meet[cu].keys.p,
+                           (const PairHit *)c->pbox.p, c->plen, (const unsigned long long *)c->meet[cu].keys(),
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)nullptr, c->tbounds.p);
     } else {
         hipLaunchKernelGGL(k_tile_owner, dim3(blocks_for(c->n, 256)), dim3(256), 0, s, (const uint32_t *)c->moff[nx].p,
                            c->n, c->towner.p);
         hipLaunchKernelGGL(k_tile_bounds<PairSlot>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairSlot *)c->pnew.p, c->plen, (const unsigned long long *)c->meet[cu].keys.p,
+                           (const PairSlot *)c->pnew.p, c->plen, (const unsigned long long *)c->meet[cu].keys(),
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)c->towner.p, c->tbounds.p);
     }
@@ -3602,12 +3605,12 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         if (c->pairs_boxed)
             hipLaunchKernelGGL(k_meet_merge<PairHit>, dim3(mgrid), dim3(256), 0, s, (const PairHit *)c->pbox.p,
                                c->plen, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].keys.p, c->meet[nx].starts.p, c->meet[nx].mbrs.p, ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
+                               c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
                                (const uint32_t *)nullptr, c->n, cnt);
         else
             hipLaunchKernelGGL(k_meet_merge<PairSlot>, dim3(mgrid), dim3(256), 0, s, (const PairSlot *)c->pnew.p,
                                c->plen, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].keys.p, c->meet[nx].starts.p, c->meet[nx].mbrs.p, ma, mt, (const float2 *)c->posf.p, (const uint32_t *)c->moff[nx].p,
+                               c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)c->posf.p, (const uint32_t *)c->moff[nx].p,
                                (const uint32_t *)c->towner.p, c->n, cnt);
         CK(hipGetLastError());
         CK(hipEventRecord(c->ev[9], s));
