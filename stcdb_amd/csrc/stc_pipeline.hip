@@ -42,13 +42,13 @@
 #include "stc_flush.h"
 #include "stc_table.h"
 #include "stc_schema.h"
+#include "stc_serve.h"
 #include "stc_query.h"
 #include "../../include/stcdb.h"
 
 #include <algorithm>
 #include <type_traits>
 #include <cmath>
-#include <condition_variable>
 #include <mutex>
 #include <thread>
 #include <atomic>
@@ -2489,6 +2489,7 @@ struct DBuf {
  * grown and freed in the first steps, 16 contexts took 353 ms to a steady state together, and 185 with one) */
 struct MeetBuf {
     DBuf<Bucket> mem;
+    bool holds(size_t n) const { return mem.p && n <= mem.cap; }
     int ensure(size_t n) { return mem.ensure(n); }
     void release() { mem.release(); }
     uint4 *mbrs() const { return (uint4 *)mem.p; }
@@ -2671,22 +2672,15 @@ struct StcCtx {
     SchemaState sch;
     /* Serving: query batches run on their own stream against the state the
      * last completed step published, while the next step runs. A batch holds
-     * a lease on the meeting array and the memtable epoch it reads; a step
-     * waits for the leases on what it overwrites (the other meeting array,
-     * and the memtable from index 0 once a flush emptied it). */
+     * a lease on the state it reads; what a step overwrites (the other meeting
+     * array, and the memtable from index 0 once a flush emptied it) or frees
+     * leaves the published state first and waits for the leases then
+     * (stc_serve.h). */
     hipStream_t qs = nullptr;
     std::mutex q_mu;                     /* one query batch at a time: its buffers and stream */
-    std::mutex pub_mu;                   /* pub_*, readers_* */
     std::mutex err_mu;                   /* err: a query thread and the stepping thread can both fail */
-    std::condition_variable pub_cv;
-    QueryState pub;                      /* the state queries read */
-    bool pub_valid = false;
-    int pub_meet = 0;                    /* meeting array of pub */
+    Published<QueryState> pub;           /* the state queries read */
     uint32_t epoch = 0;                  /* memtable epoch: +1 at every flush */
-    uint32_t pub_epoch = 0;
-    uint32_t readers_meet[2] = {0, 0};
-    uint32_t readers_epoch[2] = {0, 0};
-    uint32_t readers_total = 0;
 };
 
 /* publish the state after a step (or a change of the runs) to queries */
@@ -2713,25 +2707,7 @@ static void publish(StcCtx *c) {
         st.run_ctfs.push_back(c->runs[r].ctfs.data());
         st.run_stats.push_back(c->runs[r].stats.data());
     }
-    std::lock_guard<std::mutex> lk(c->pub_mu);
-    c->pub = std::move(st);
-    c->pub_meet = c->cur;
-    c->pub_epoch = c->epoch;
-    c->pub_valid = c->stepped;
-}
-
-/* wait until no query batch reads meeting array mi (and, with old_memtable,
- * the memtable of an earlier epoch) */
-static void wait_readers(StcCtx *c, int mi, bool old_memtable) {
-    std::unique_lock<std::mutex> lk(c->pub_mu);
-    c->pub_cv.wait(lk, [&] {
-        return c->readers_meet[mi] == 0 && (!old_memtable || c->readers_epoch[(c->epoch + 1) & 1] == 0);
-    });
-}
-/* wait until no query batch is in flight */
-static void wait_all_readers(StcCtx *c) {
-    std::unique_lock<std::mutex> lk(c->pub_mu);
-    c->pub_cv.wait(lk, [&] { return c->readers_total == 0; });
+    c->pub.publish(std::move(st), c->cur, c->epoch, c->stepped);
 }
 
 /* the QTree the step's kernels descend */
@@ -2785,10 +2761,9 @@ static int sync_counters(StcCtx *c) {
     return 0;
 }
 
-static void wait_all_readers(StcCtx *c);
 static int ensure_records(StcCtx *c, uint64_t need) {
     if (need <= c->rec_cap) return 0;
-    wait_all_readers(c); /* the old buffers are freed below */
+    const uint64_t held = std::max<uint64_t>(c->kv_count, c->pub.state().n_rec); /* also what queries still read */
     uint64_t nc = std::max<uint64_t>(need + need / 2, 1 << 16);
     uint64_t *k = nullptr;
     float4 *b = nullptr;
@@ -2796,15 +2771,23 @@ static int ensure_records(StcCtx *c, uint64_t need) {
     CK(hipMalloc((void **)&k, nc * 16));
     CK(hipMalloc((void **)&b, nc * 16));
     CK(hipMalloc((void **)&o, nc * 4));
-    if (c->kv_count) {
-        CK(hipMemcpyAsync(k, c->rec_keys, c->kv_count * 16, hipMemcpyDeviceToDevice, c->s));
-        CK(hipMemcpyAsync(b, c->rec_boxes, c->kv_count * 16, hipMemcpyDeviceToDevice, c->s));
-        CK(hipMemcpyAsync(o, c->rec_ord, c->kv_count * 4, hipMemcpyDeviceToDevice, c->s));
+    if (held) {
+        CK(hipMemcpyAsync(k, c->rec_keys, held * 16, hipMemcpyDeviceToDevice, c->s));
+        CK(hipMemcpyAsync(b, c->rec_boxes, held * 16, hipMemcpyDeviceToDevice, c->s));
+        CK(hipMemcpyAsync(o, c->rec_ord, held * 4, hipMemcpyDeviceToDevice, c->s));
     }
     CK(hipStreamSynchronize(c->s));
-    if (c->rec_keys) hipFree(c->rec_keys);
-    if (c->rec_boxes) hipFree(c->rec_boxes);
-    if (c->rec_ord) hipFree(c->rec_ord);
+    /* the published state names the new buffers before the old ones go: a batch may come at any time */
+    c->pub.replace(
+        [&](QueryState &st) {
+            st.rec_keys = k;
+            st.rec_boxes = b;
+        },
+        [&] {
+            if (c->rec_keys) hipFree(c->rec_keys);
+            if (c->rec_boxes) hipFree(c->rec_boxes);
+            if (c->rec_ord) hipFree(c->rec_ord);
+        });
     c->rec_keys = k;
     c->rec_boxes = b;
     c->rec_ord = o;
@@ -2976,17 +2959,17 @@ static int keep_run_on_device(StcCtx *c, RunHost &run) {
 
 /* release every run's host block (a queued copy still completes) and HBM block */
 static void drop_all_runs(StcCtx *c) {
-    wait_all_readers(c); /* the runs' device blocks are freed below */
-    for (auto &r : c->runs) {
+    std::vector<RunHost> gone;
+    gone.swap(c->runs);
+    publish(c); /* without them, before their device blocks go */
+    c->pub.wait_earlier();
+    for (auto &r : gone) {
         release_block(c, r.blk, true);
         if (r.dev) {
             (void)hipStreamSynchronize(c->s);
             (void)hipFree(r.dev);
-            r.dev = nullptr;
         }
     }
-    c->runs.clear();
-    publish(c);
 }
 
 /* Wait for an asynchronous flush and take its run: the main stream waits for
@@ -3024,6 +3007,18 @@ static int join_flush(StcCtx *c) {
         publish(c);
     }
     return STC_OK;
+}
+
+/* Room for n meetings of the step in the array that it writes. An array that
+ * has to grow is freed, and while a flush is pending the published state is
+ * still the one before its step's, which reads that very array: the flush is
+ * joined first (which publishes), and nothing reads the array any more. */
+static int ensure_meetings(StcCtx *c, uint64_t n) {
+    MeetBuf &m = c->meet[c->cur ^ 1];
+    if (m.holds(n)) return STC_OK;
+    JOIN_FLUSH(c);
+    c->pub.clear(c->cur ^ 1, false, c->epoch);
+    return m.ensure(n) ? fail(c, STC_E_CAPACITY, "meeting arrays") : STC_OK;
 }
 
 extern "C" {
@@ -3156,7 +3151,7 @@ int stc_destroy(void *vc) {
     StcCtx *c = (StcCtx *)vc;
     if (!c) return STC_OK;
     (void)join_flush(c);
-    wait_all_readers(c);
+    c->pub.wait_all();
     if (c->s) hipStreamSynchronize(c->s);
     c->xy_in.release(); c->codes.release(); c->idx.release(); c->codes_alt.release(); c->idx_alt.release();
     c->temp.release(); c->dlon.release(); c->posf.release(); c->lxy.release(); c->ld.release(); c->nodes.release();
@@ -3471,9 +3466,11 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
         CK(hipMemcpy(c->acc.p, accepted.data(), accepted.size() * sizeof(unsigned long long), hipMemcpyHostToDevice));
     const int nx = c->cur ^ 1;
     CKRC(stc_exclusive_scan_u32(c->pcount.p, c->moff[nx].p, n, c->moff[nx].p + n, c->temp.p, s));
-    wait_readers(c, nx, false); /* queries of an earlier state may still read meet[nx] */
-    if (c->pnew.ensure(total + 1) || c->meet[nx].ensure(total + 1))
-        return fail(c, STC_E_CAPACITY, "pair and meeting arrays");
+    {
+        const int rc = ensure_meetings(c, total + 1);
+        if (rc) return rc;
+    }
+    if (c->pnew.ensure(total + 1)) return fail(c, STC_E_CAPACITY, "pair array");
     CK(hipEventRecord(c->ev[6], s));
     /* the place passes' owners a wave reads at once and workgroups at most. Short segments: 8 owners below
      * 256k objects (200k: 29 us, 16: 39), 16 above (1M: 144 us, 8: 150, 32: 159), 4k workgroups (1M: 144, 16k:
@@ -3588,7 +3585,7 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     const uint32_t mgrid = std::max<uint32_t>(
         std::min<uint32_t>((n_tiles + 3) / 4, std::min<uint32_t>(std::max<uint32_t>(n_tiles / 40, 2048), 65536)), 1);
     /* the merge writes meet[nx] and, after a flush emptied the memtable, records from index 0 */
-    wait_readers(c, nx, kv_before == 0);
+    c->pub.clear(nx, kv_before == 0, c->epoch);
     const bool schema_step = c->dyn && g.nodes;
     int schema_rc = STC_OK;
     for (int attempt = 0;; attempt++) {
@@ -3861,9 +3858,12 @@ int stc_step_meetings(void *vc, const stc_meeting_unit *units, uint64_t nu64, ui
     CK(hipEventRecord(c->ev[2], s));
     if (c->units_in.ensure(nu + 1ull) || c->ukeys.ensure(nu + 1ull) || c->ukeys_alt.ensure(nu + 1ull) ||
         c->uidx.ensure(nu + 1ull) || c->uidx_alt.ensure(nu + 1ull) ||
-        c->utemp.ensure(stc_radix_temp_words(std::max<uint32_t>(nu + 1, c->n)) + 64) || c->pbox.ensure(nu + 1ull) ||
-        (wait_readers(c, c->cur ^ 1, false), c->meet[c->cur ^ 1].ensure(nu + 1ull)))
+        c->utemp.ensure(stc_radix_temp_words(std::max<uint32_t>(nu + 1, c->n)) + 64) || c->pbox.ensure(nu + 1ull))
         return fail(c, STC_E_CAPACITY, "meeting unit buffers");
+    {
+        const int rc = ensure_meetings(c, nu + 1ull);
+        if (rc) return rc;
+    }
     if (nu) {
         CK(hipMemcpyAsync(c->units_in.p, units, (size_t)nu * sizeof(stc_meeting_unit), hipMemcpyHostToDevice, s));
         hipLaunchKernelGGL(k_units_decode, dim3(blocks_for(nu, 256)), dim3(256), 0, s, c->units_in.p, nu, c->n,
@@ -4112,19 +4112,9 @@ static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *
     if (need && hipMemGetInfo(&free_b, &total_b) == hipSuccess && need + STC_QUERY_RESERVE > free_b)
         return fail(c, STC_E_CAPACITY, "admission: the batch needs " + std::to_string(need) + " bytes of device memory, " +
                                            std::to_string(free_b) + " free");
-    QueryState st;
-    int mi;
-    uint32_t ep;
-    {
-        std::lock_guard<std::mutex> lk(c->pub_mu);
-        if (!c->pub_valid) return fail(c, STC_E_STATE, "no step processed");
-        st = c->pub;
-        mi = c->pub_meet;
-        ep = c->pub_epoch;
-        c->readers_meet[mi]++;
-        c->readers_epoch[ep & 1]++;
-        c->readers_total++;
-    }
+    Published<QueryState>::Lease lease;
+    if (!c->pub.take(&lease)) return fail(c, STC_E_STATE, "no step processed, or the last one failed");
+    const QueryState &st = lease.state;
     std::vector<stc_query> built;
     bool run = true;
     if constexpr (!std::is_same<Make, std::nullptr_t>::value) {
@@ -4138,13 +4128,7 @@ static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *
     } else {
         *n_hits = 0;
     }
-    {
-        std::lock_guard<std::mutex> lk(c->pub_mu);
-        c->readers_meet[mi]--;
-        c->readers_epoch[ep & 1]--;
-        c->readers_total--;
-    }
-    c->pub_cv.notify_all();
+    c->pub.give_back(lease);
     if (rc) return fail(c, rc, std::string("query: ") + g_last_fail);
     if (state_step) *state_step = st.last_t;
     return STC_OK;
@@ -4345,7 +4329,6 @@ int stc_compact_runs(void *vc, uint32_t first, uint32_t count) {
     StcCtx *c = (StcCtx *)vc;
     if (!c || count == 0) return STC_E_ARG;
     JOIN_FLUSH(c);
-    wait_all_readers(c); /* the merged runs' blocks are freed and the memtable buffers reused */
     if ((uint64_t)first + count > c->runs.size()) return fail(c, STC_E_ARG, "run range out of bounds");
     if (count == 1) return STC_OK;
     const uint32_t n = c->n;
@@ -4441,13 +4424,16 @@ int stc_compact_runs(void *vc, uint32_t first, uint32_t count) {
         return rc;
     }
     CK(hipStreamSynchronize(s));
-    for (uint32_t r = first; r < first + count; r++) {
-        release_block(c, c->runs[r].blk);
-        (void)hipFree(c->runs[r].dev);
-    }
+    std::vector<RunHost> gone;
+    for (uint32_t r = first; r < first + count; r++) gone.push_back(std::move(c->runs[r]));
     c->runs.erase(c->runs.begin() + first, c->runs.begin() + first + count);
     c->runs.insert(c->runs.begin() + first, std::move(run));
-    publish(c);
+    publish(c); /* without the merged runs, before their blocks go */
+    c->pub.wait_earlier();
+    for (RunHost &r : gone) {
+        release_block(c, r.blk);
+        (void)hipFree(r.dev);
+    }
     return STC_OK;
 }
 
