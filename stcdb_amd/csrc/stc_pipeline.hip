@@ -2586,7 +2586,8 @@ struct StcCtx {
     DBuf<double2> xy_in;
     DBuf<uint32_t> codes, idx, codes_alt, idx_alt, temp;
     DBuf<double> dlon, ld;
-    DBuf<float2> posf;                   /* positions by id as floats: the owners' side of the pair slots */
+    DBuf<float2> posf, posf_new;         /* positions by id as floats (the owners' side of the pair slots), of the last
+                                            completed position step and of the one under way */
     DBuf<double2> lxy;
     DBuf<Node> nodes;
     DBuf<FrontierItem> frontier_a, frontier_b;
@@ -2608,7 +2609,7 @@ struct StcCtx {
      * segments (offsets [n + 1], live buckets per segment [n]) used in turn */
     DBuf<uint32_t> pcount;
     DBuf<PairSlot> ptmp, pnew;           /* the long segments' pair slots as found, and all slots sorted by key */
-    DBuf<PairHit> pbox;                  /* a replayed step's pairs (key and MBR), sorted by key */
+    DBuf<PairHit> pbox, pbox_new;        /* a replayed step's pairs (key and MBR), sorted by key, likewise */
     bool pairs_boxed = false;            /* the last step's pairs are in pbox (replayed units), not pnew */
     DBuf<uint32_t> psrc;                 /* collected pair sources, a run per owner */
     DBuf<uint2> pkrun;                   /* per owner in leaf order: its run of psrc (start, length) */
@@ -2618,7 +2619,7 @@ struct StcCtx {
     DBuf<uint32_t> towner;               /* merge tiles' first owners (the slots carry no owner) */
     int cur = 0;                         /* meet[cur] holds the meetings of the last step */
     uint64_t mlen = 0;                   /* buckets of meet[cur] (live and tombstones) */
-    uint64_t plen = 0;                   /* entries of pnew (the last step's pair slots) */
+    uint64_t plen = 0;                   /* the last step's pair slots */
     DBuf<unsigned long long> acc;        /* band pairs the host accepted, sorted */
     DBuf<uint32_t> spill_big, spill_huge, spill_giant;
     DBuf<unsigned long long> gsrt;       /* global sort keys of very large segments */
@@ -3112,7 +3113,7 @@ int stc_create(const stc_config *cfg, const stc_box *mbr, void **out) {
     }
     size_t front_cap = n / (c->cap + 1) + 2;
     if (c->xy_in.ensure(n) || c->codes.ensure(n) || c->idx.ensure(n) || c->codes_alt.ensure(n) ||
-        c->idx_alt.ensure(n) || c->dlon.ensure(n) || c->posf.ensure(n) || c->lxy.ensure(n) || c->ld.ensure(n) ||
+        c->idx_alt.ensure(n) || c->dlon.ensure(n) || c->posf.ensure(n) || c->posf_new.ensure(n) || c->lxy.ensure(n) || c->ld.ensure(n) ||
         c->nodes.ensure(node_cap) || c->frontier_a.ensure(front_cap) || c->frontier_b.ensure(front_cap) ||
         c->pt_leaf.ensure(n) || c->pt_lv.ensure(n) || c->lp.ensure(n) ||
         c->lunits.ensure(n) || c->prange.ensure(n) ||
@@ -3154,7 +3155,7 @@ int stc_destroy(void *vc) {
     c->pub.wait_all();
     if (c->s) hipStreamSynchronize(c->s);
     c->xy_in.release(); c->codes.release(); c->idx.release(); c->codes_alt.release(); c->idx_alt.release();
-    c->temp.release(); c->dlon.release(); c->posf.release(); c->lxy.release(); c->ld.release(); c->nodes.release();
+    c->temp.release(); c->dlon.release(); c->posf.release(); c->posf_new.release(); c->lxy.release(); c->ld.release(); c->nodes.release();
     c->frontier_a.release(); c->frontier_b.release(); c->leaf_count.release(); c->leaf_start.release();
     c->leaf_node.release(); c->pt_leaf.release(); c->pt_lv.release(); c->lp.release();
     c->lunits.release(); c->urange.release(); c->prange.release();
@@ -3163,7 +3164,7 @@ int stc_destroy(void *vc) {
     c->rev_leaf.release(); c->rev_pid.release(); c->rev_leaf_alt.release(); c->rev_pid_alt.release();
     c->rev_start.release();
     c->rev.release(); c->rev_dl.release();
-    c->pcount.release(); c->pnew.release(); c->acc.release();
+    c->pcount.release(); c->pnew.release(); c->pbox.release(); c->pbox_new.release(); c->acc.release();
     for (int i = 0; i < 2; i++) { c->meet[i].release(); c->moff[i].release(); }
     c->ptmp.release(); c->tbounds.release(); c->towner.release(); c->psrc.release(); c->pkrun.release();
     c->spill_big.release(); c->spill_huge.release(); c->spill_giant.release(); c->gsrt.release();
@@ -3224,6 +3225,8 @@ struct StepGeom {
     uint64_t units, pairs, ambiguous;
     uint32_t rebuilt;
     uint64_t candidates = 0;
+    uint64_t slots = 0;                  /* pair slots of the step: in pbox_new when replayed, else in pnew */
+    bool boxed = false;
 };
 static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out);
 
@@ -3272,7 +3275,7 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
 
     /* 1-2: cells, Morton codes, dpm_lon; sort codes */
     hipLaunchKernelGGL(k_prep, dim3(blocks_for(n, 256)), dim3(256), 0, s, xy, n, c->map, c->codes.p, c->idx.p,
-                       c->dlon.p, c->posf.p, cnt);
+                       c->dlon.p, c->posf_new.p, cnt);
     CK(hipGetLastError());
     /* the order the partition walks the points in: Morton order, or with a kept schema the previous
      * step's leaf order (objects move a few metres a step, so it is as coherent, without the sort) */
@@ -3533,10 +3536,8 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
         CKRC(sync_counters(c));
     }
     if (c->hcnt->table_fail) return fail(c, STC_E_HIP, "a pair segment was longer than its sort's scratch");
-    c->plen = total;
-    c->pairs_boxed = false;
     CK(hipEventRecord(c->ev[3], s));
-    StepGeom g{n_nodes, n_leaves, n_units, 0, n_amb, 0, n_cand};
+    StepGeom g{n_nodes, n_leaves, n_units, 0, n_amb, 0, n_cand, total, false};
     return step_tail(c, t, g, out);
 }
 
@@ -3563,18 +3564,18 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     const Counters before = *c->hcnt; /* as read last: nothing since has changed them */
     Counters h;
     /* tiles of the step's pairs and their ranges in the previous meetings */
-    const uint32_t n_tiles = (uint32_t)std::max<uint64_t>((c->plen + MTILE - 1) / MTILE, 1);
+    const uint32_t n_tiles = (uint32_t)std::max<uint64_t>((g.slots + MTILE - 1) / MTILE, 1);
     if (c->tbounds.ensure(n_tiles + 1ull) || c->towner.ensure(n_tiles)) return fail(c, STC_E_CAPACITY, "merge tile bounds");
-    if (c->pairs_boxed) {
+    if (g.boxed) {
         hipLaunchKernelGGL(k_tile_bounds<PairHit>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairHit *)c->pbox.p, c->plen, (const unsigned long long *)c->meet[cu].keys(),
+                           (const PairHit *)c->pbox_new.p, g.slots, (const unsigned long long *)c->meet[cu].keys(),
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)nullptr, c->tbounds.p);
     } else {
         hipLaunchKernelGGL(k_tile_owner, dim3(blocks_for(c->n, 256)), dim3(256), 0, s, (const uint32_t *)c->moff[nx].p,
                            c->n, c->towner.p);
         hipLaunchKernelGGL(k_tile_bounds<PairSlot>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairSlot *)c->pnew.p, c->plen, (const unsigned long long *)c->meet[cu].keys(),
+                           (const PairSlot *)c->pnew.p, g.slots, (const unsigned long long *)c->meet[cu].keys(),
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)c->towner.p, c->tbounds.p);
     }
@@ -3599,15 +3600,15 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         const MemtableDev mt{c->rec_keys, c->rec_boxes, c->rec_cap, c->rec_ord, c->same_pid_count, c->sids};
         const Meets mo = c->meet[cu].view();
         CK(hipEventRecord(c->ev[8], s));
-        if (c->pairs_boxed)
-            hipLaunchKernelGGL(k_meet_merge<PairHit>, dim3(mgrid), dim3(256), 0, s, (const PairHit *)c->pbox.p,
-                               c->plen, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
+        if (g.boxed)
+            hipLaunchKernelGGL(k_meet_merge<PairHit>, dim3(mgrid), dim3(256), 0, s, (const PairHit *)c->pbox_new.p,
+                               g.slots, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
                                c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
                                (const uint32_t *)nullptr, c->n, cnt);
         else
             hipLaunchKernelGGL(k_meet_merge<PairSlot>, dim3(mgrid), dim3(256), 0, s, (const PairSlot *)c->pnew.p,
-                               c->plen, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)c->posf.p, (const uint32_t *)c->moff[nx].p,
+                               g.slots, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
+                               c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)c->posf_new.p, (const uint32_t *)c->moff[nx].p,
                                (const uint32_t *)c->towner.p, c->n, cnt);
         CK(hipGetLastError());
         CK(hipEventRecord(c->ev[9], s));
@@ -3642,7 +3643,11 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     c->last_live = met.live;
     c->last_expired = met.expired;
     c->cur = nx;
-    c->mlen = c->plen;
+    /* what the exports read, with the meetings: a step that fails before this leaves the last one's */
+    c->mlen = c->plen = g.slots;
+    c->pairs_boxed = g.boxed;
+    if (g.boxed) std::swap(c->pbox, c->pbox_new);
+    else std::swap(c->posf, c->posf_new);
     g.pairs = met.live;
     if (schema_rc) return fail(c, schema_rc, std::string("schema update: ") + g_last_fail);
 
@@ -3858,7 +3863,7 @@ int stc_step_meetings(void *vc, const stc_meeting_unit *units, uint64_t nu64, ui
     CK(hipEventRecord(c->ev[2], s));
     if (c->units_in.ensure(nu + 1ull) || c->ukeys.ensure(nu + 1ull) || c->ukeys_alt.ensure(nu + 1ull) ||
         c->uidx.ensure(nu + 1ull) || c->uidx_alt.ensure(nu + 1ull) ||
-        c->utemp.ensure(stc_radix_temp_words(std::max<uint32_t>(nu + 1, c->n)) + 64) || c->pbox.ensure(nu + 1ull))
+        c->utemp.ensure(stc_radix_temp_words(std::max<uint32_t>(nu + 1, c->n)) + 64) || c->pbox_new.ensure(nu + 1ull))
         return fail(c, STC_E_CAPACITY, "meeting unit buffers");
     {
         const int rc = ensure_meetings(c, nu + 1ull);
@@ -3872,7 +3877,7 @@ int stc_step_meetings(void *vc, const stc_meeting_unit *units, uint64_t nu64, ui
         CKRC(sort_pairs((const uint64_t *)c->ukeys.p, (const uint32_t *)c->uidx.p, c->ukeys, c->uidx, c->ukeys_alt, c->uidx_alt, nu,
                         32 + std::max(1, ilog2_ceil(c->n)), c->utemp.p, s));
         hipLaunchKernelGGL(k_units_gather, dim3(blocks_for(nu, 256)), dim3(256), 0, s, c->ukeys.p, c->uidx.p,
-                           c->units_in.p, nu, c->pbox.p, cnt);
+                           c->units_in.p, nu, c->pbox_new.p, cnt);
         CK(hipGetLastError());
     }
     CKRC(sync_counters(c));
@@ -3884,16 +3889,14 @@ int stc_step_meetings(void *vc, const stc_meeting_unit *units, uint64_t nu64, ui
     CK(hipEventRecord(c->ev[6], s));
     CK(hipMemsetAsync(c->pcount.p, 0, 4ull * c->n, s));
     if (nu) {
-        hipLaunchKernelGGL(k_owner_hist, dim3(blocks_for(nu, 256)), dim3(256), 0, s, (const PairHit *)c->pbox.p, nu,
+        hipLaunchKernelGGL(k_owner_hist, dim3(blocks_for(nu, 256)), dim3(256), 0, s, (const PairHit *)c->pbox_new.p, nu,
                            c->pcount.p);
         CK(hipGetLastError());
     }
     CKRC(stc_exclusive_scan_u32(c->pcount.p, c->moff[nx].p, c->n, c->moff[nx].p + c->n, c->utemp.p, s));
     CK(hipEventRecord(c->ev[7], s));
-    c->plen = nu;
-    c->pairs_boxed = true;
     CK(hipEventRecord(c->ev[3], s));
-    StepGeom g{0, 0, 0, 0, 0, 0};
+    StepGeom g{0, 0, 0, 0, 0, 0, 0, nu, true};
     int rc = step_tail(c, t, g, out);
     if (rc == STC_OK && out) out->new_records = out->kv_count - kv_before;
     return rc;
@@ -4007,7 +4010,7 @@ int stc_build_schema(void *vc, const double *xy, int32_t xy_on_device) {
     }
     /* the points' Morton order keeps each wave of the build's counting on few nodes */
     hipLaunchKernelGGL(k_prep, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->s, src, c->n, c->map, c->codes.p,
-                       c->idx.p, c->dlon.p, (float2 *)nullptr, c->dcnt); /* posf keeps the last step's positions */
+                       c->idx.p, c->dlon.p, (float2 *)nullptr, c->dcnt); /* no step's positions */
     CK(hipGetLastError());
     CKRC(sort_pairs((const uint32_t *)c->codes.p, (const uint32_t *)c->idx.p, c->codes, c->idx, c->codes_alt, c->idx_alt, c->n, 28,
                     c->temp.p, c->s));
