@@ -2485,19 +2485,33 @@ struct DBuf {
     void release() { if (p) hipFree(p); p = nullptr; cap = 0; }
 };
 
-/* a step's meetings: the three arrays in one allocation, as long as its capacity each (with an allocation each, to be
+/* a step's meetings: the three arrays (MeetLayout) in one allocation (with an allocation each, to be
  * grown and freed in the first steps, 16 contexts took 353 ms to a steady state together, and 185 with one) */
 struct MeetBuf {
-    DBuf<Bucket> mem;
-    bool holds(size_t n) const { return mem.p && n <= mem.cap; }
-    int ensure(size_t n) { return mem.ensure(n); }
-    void release() { mem.release(); }
-    uint4 *mbrs() const { return (uint4 *)mem.p; }
-    unsigned long long *keys() const { return (unsigned long long *)(mbrs() + mem.cap); }
-    uint32_t *starts() const { return (uint32_t *)(keys() + mem.cap); }
+    uint8_t *mem = nullptr;
+    MeetLayout lay{0};
+    bool holds(size_t n) const { return mem && n <= lay.cap; }
+    int ensure(size_t n) {
+        if (holds(n)) return 0;
+        release();
+        const MeetLayout l(std::max<size_t>(n + n / 2, 1024));
+        if (hipMalloc((void **)&mem, l.bytes) != hipSuccess) {
+            mem = nullptr;
+            return -1;
+        }
+        lay = l;
+        return 0;
+    }
+    void release() {
+        if (mem) hipFree(mem);
+        mem = nullptr;
+        lay = MeetLayout(0);
+    }
+    uint4 *mbrs() const { return (uint4 *)mem; }
+    unsigned long long *keys() const { return (unsigned long long *)(mem + lay.keys); }
+    uint32_t *starts() const { return (uint32_t *)(mem + lay.starts); }
     Meets view() const { return Meets{keys(), starts(), mbrs()}; }
 };
-static_assert(sizeof(Bucket) == sizeof(uint4) + sizeof(unsigned long long) + sizeof(uint32_t), "a bucket of each array");
 
 /* A flushed run: metadata on the host, payload in a pinned block that the
  * copy stream fills while later steps run. */
