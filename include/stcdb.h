@@ -363,8 +363,9 @@ int stc_query_batch_room(void *ctx, const stc_query *q, uint32_t nq, stc_hit *hi
  * step on the device; that step waits only where it overwrites what an
  * earlier batch still reads (the other meeting array; the memtable from its
  * start after a flush). Batches are admitted by free device memory: one whose
- * query list and hit buffer would leave less than 1 GiB free returns
- * STC_E_CAPACITY (split it and retry). stc_query_batch_at also reports the
+ * tables (its queries, ids and the cells of its boxes), candidates and hit
+ * buffer would leave less than 1 GiB free returns STC_E_CAPACITY (split it and
+ * retry). stc_query_batch_at also reports the
  * timestep of the state it answered. Only stc_query_batch, stc_query_batch_room,
  * stc_query_batch_at and stc_live_search may run concurrently with stc_step on one context;
  * stc_drop_runs and stc_compact_runs wait for batches in flight. The

@@ -4114,38 +4114,38 @@ int stc_sync(void *vc) {
     return STC_OK;
 }
 
-/* One query batch over the state the last completed step published: admission by free device
- * memory, a lease on that state's meeting array and memtable epoch for the batch's duration, the
- * batch on the query stream. `make` (when given) builds the batch from the published step instead
+/* One query batch over the state the last completed step published: a lease on that state for the
+ * batch's duration, admission by free device memory, the batch on the query stream. `make` (when given) builds the batch from the published step instead
  * of `q`; returning false answers with no hits. */
 extern "C++" {
 template <class Make>
 static int query_published(StcCtx *c, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap, uint64_t *n_hits,
                            uint64_t *counts, uint32_t *state_step, Make make, QueryRoom *more = nullptr) {
     std::lock_guard<std::mutex> ql(c->q_mu);
-    /* admission: what the batch's query list, counters and hit buffer add to the query buffers */
-    const uint64_t need = stc_query_bufs_growth(c->qb, nq, hits ? cap : 0);
-    size_t free_b = 0, total_b = 0;
-    if (need && hipMemGetInfo(&free_b, &total_b) == hipSuccess && need + STC_QUERY_RESERVE > free_b)
-        return fail(c, STC_E_CAPACITY, "admission: the batch needs " + std::to_string(need) + " bytes of device memory, " +
-                                           std::to_string(free_b) + " free");
     Published<QueryState>::Lease lease;
     if (!c->pub.take(&lease)) return fail(c, STC_E_STATE, "no step processed, or the last one failed");
     const QueryState &st = lease.state;
-    std::vector<stc_query> built;
-    bool run = true;
-    if constexpr (!std::is_same<Make, std::nullptr_t>::value) {
-        run = make(st.last_t, built);
-        q = built.data();
-        nq = (uint32_t)built.size();
-    }
+    QueryAdmission adm{STC_QUERY_RESERVE};
     int rc = 0;
-    if (run) {
-        rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, STC_QUERY_RESERVE, more, c->qs);
-    } else {
-        *n_hits = 0;
+    try {
+        std::vector<stc_query> built;
+        bool run = true;
+        if constexpr (!std::is_same<Make, std::nullptr_t>::value) {
+            run = make(st.last_t, built);
+            q = built.data();
+            nq = (uint32_t)built.size();
+        }
+        if (run) rc = stc_query_run(c->qb, st, q, nq, hits, cap, n_hits, counts, adm, more, c->qs);
+        else *n_hits = 0;
+    } catch (const std::bad_alloc &) { /* of the batch's host tables, before its first launch or with nothing left to launch */
+        (void)hipStreamSynchronize(c->qs);
+        rc = STC_E_CAPACITY;
+        g_last_fail = "host memory of the batch's tables";
     }
     c->pub.give_back(lease);
+    if (adm.refused)
+        return fail(c, rc, "admission: the batch needs " + std::to_string(adm.need) + " bytes of device memory, " +
+                               std::to_string(adm.free) + " free");
     if (rc) return fail(c, rc, std::string("query: ") + g_last_fail);
     if (state_step) *state_step = st.last_t;
     return STC_OK;

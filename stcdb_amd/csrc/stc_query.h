@@ -53,17 +53,26 @@ struct QueryState {
 struct QueryBufs;                    /* device scratch of the query path, grown on demand */
 QueryBufs *stc_query_bufs_new();
 void stc_query_bufs_free(QueryBufs *b);
-/* device bytes a batch of nq queries storing up to cap hits would add to b */
-uint64_t stc_query_bufs_growth(const QueryBufs *b, uint32_t nq, uint64_t cap);
+/* device bytes of a batch's tables (its queries and counters, the id hash, the range queries' cell lists, the filters) */
+uint64_t stc_query_table_bytes(const stc_query *q, uint32_t nq, const double *map);
+/* A batch is admitted when the device memory that it would add leaves `reserve` bytes free; else nothing is allocated
+ * and STC_E_CAPACITY is returned with `refused` set. */
+struct QueryAdmission {
+    uint64_t reserve;
+    uint64_t need = 0, free = 0;
+    bool refused = false;
+    bool fits(uint64_t more);
+    int refuse(uint64_t more);
+};
 /* stc_query_batch_room's further arguments */
 struct QueryRoom {
     stc_room room;
     void *arg;
     bool all;                        /* every hit is stored */
 };
-/* reserve: device memory that scratch not counted there leaves free; more: null but for stc_query_batch_room */
+/* more: null but for stc_query_batch_room */
 int stc_query_run(QueryBufs *b, const QueryState &st, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap,
-                  uint64_t *n_hits, uint64_t *counts, uint64_t reserve, QueryRoom *more, hipStream_t s);
+                  uint64_t *n_hits, uint64_t *counts, QueryAdmission &adm, QueryRoom *more, hipStream_t s);
 /* Compaction input: every record of run R (the kv_count records of its CTFs,
  * kv_count = the sum of their kv_capacity, then the oversize buffer) in
  * memtable form at keys/boxes[out0 ..], ends re-based on `base`, boxes decoded

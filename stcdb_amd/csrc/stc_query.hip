@@ -51,40 +51,76 @@ struct QDev {
     float fx[2], fy[2], fix, fiy;    /* range filter: the map's low corner in two parts, cells per degree */
 };
 
-/* host tables on their way to the device: built in pinned memory, sent with one copy */
+#define QPIECE (8ull << 20) /* pinned bytes an upload goes through at a time */
+
+/* host tables on their way to the device, as long as the batch makes them: built in pinned memory and sent with one copy
+ * up to QPIECE, in pieces of that beyond (their sources stay as they are until then) */
 struct QueryUpload {
     uint8_t *host = nullptr, *dev = nullptr;
-    uint64_t cap = 0, used = 0;
+    uint64_t host_cap = 0, cap = 0, used = 0;
+    bool pieces = false;
+    struct Table { const uint8_t *src; uint64_t at, bytes; }; /* src null: zeros */
+    std::vector<Table> tables;
+    /* device bytes that begin(bytes) would add */
+    uint64_t growth(uint64_t bytes) const { return bytes <= cap ? 0 : room_for(bytes); }
     /* room for `bytes`, and nothing in it */
     int begin(uint64_t bytes) {
         used = 0;
-        if (bytes <= cap) return 0;
-        release();
-        const uint64_t nc = bytes + bytes / 2 + 4096;
-        if (hipHostMalloc((void **)&host, nc, hipHostMallocDefault) != hipSuccess || hipMalloc((void **)&dev, nc) != hipSuccess) {
-            release();
-            return -1;
+        tables.clear();
+        pieces = bytes > QPIECE;
+        const uint64_t hc = std::min<uint64_t>(room_for(bytes), QPIECE);
+        if (bytes > cap) {
+            if (dev) (void)hipFree(dev);
+            dev = nullptr;
+            cap = 0;
+            if (hipMalloc((void **)&dev, room_for(bytes)) != hipSuccess) {
+                dev = nullptr;
+                return -1;
+            }
+            cap = room_for(bytes);
         }
-        cap = nc;
+        if (std::min<uint64_t>(bytes, QPIECE) > host_cap) {
+            if (host) (void)hipHostFree(host);
+            host = nullptr;
+            host_cap = 0;
+            if (hipHostMalloc((void **)&host, hc, hipHostMallocDefault) != hipSuccess) {
+                host = nullptr;
+                return -1;
+            }
+            host_cap = hc;
+        }
         return 0;
     }
     static uint64_t room(uint64_t bytes) { return (bytes + 15) & ~15ull; }
+    static uint64_t room_for(uint64_t bytes) { return bytes + bytes / 2 + 4096; }
     /* a table of n (from src, or zeros), and where it will be on the device */
     template <typename T>
     T *put(const T *src, uint64_t n) {
-        uint8_t *at = host + used;
         T *d = (T *)(dev + used);
-        if (src) memcpy(at, src, n * sizeof(T));
-        else memset(at, 0, n * sizeof(T));
+        if (pieces) tables.push_back(Table{(const uint8_t *)src, used, n * sizeof(T)});
+        else if (src) memcpy(host + used, src, n * sizeof(T));
+        else memset(host + used, 0, n * sizeof(T));
         used += room(n * sizeof(T));
         return d;
     }
-    hipError_t send(hipStream_t s) { return hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, s); }
+    hipError_t send(hipStream_t s) {
+        if (!pieces) return hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, s);
+        for (const Table &t : tables)
+            for (uint64_t o = 0; o < t.bytes; o += host_cap) {
+                const uint64_t n = std::min<uint64_t>(host_cap, t.bytes - o);
+                if (t.src) memcpy(host, t.src + o, n);
+                else memset(host, 0, n);
+                hipError_t e = hipMemcpyAsync(dev + t.at + o, host, n, hipMemcpyHostToDevice, s);
+                if (e == hipSuccess) e = hipStreamSynchronize(s);
+                if (e != hipSuccess) return e;
+            }
+        return hipSuccess;
+    }
     void release() {
         if (host) (void)hipHostFree(host);
         if (dev) (void)hipFree(dev);
         host = dev = nullptr;
-        cap = 0;
+        host_cap = cap = 0;
     }
 };
 
@@ -106,14 +142,6 @@ struct QueryBufs {
                          * costs a wait more (some 30 us; the host takes about 80 at 1,000 hits) */
 #define QRANK 16384u    /* and up to this many are ranked by comparing all with all */
 
-
-uint64_t stc_query_bufs_growth(const QueryBufs *b, uint32_t nq, uint64_t cap) {
-    uint64_t need = 0;
-    const uint64_t h_cap = b ? b->hits_cap : 0, list = nq * (sizeof(stc_query) + 8ull) + 8;
-    if (list > (b ? b->batch.cap : 0)) need += list * 3 / 2;
-    if (cap > h_cap) need += cap * sizeof(stc_hit) * 3 / 2;
-    return need;
-}
 
 void stc_query_bufs_free(QueryBufs *b) {
     if (!b) return;
@@ -1041,94 +1069,128 @@ static bool ctf_may_intersect(const stc_ctf_meta &c, const double *box) {
     return box[0] <= hi0 && box[2] >= lo0 && box[1] <= hi1 && box[3] >= lo1;
 }
 
+/* The tables of a batch that its kernels look into, and their bytes on the device (from the counts alone, before the
+ * longest of them, the cells' lists, is made). */
+struct QueryTables {
+    std::vector<uint32_t> oq, rq;            /* object and pair queries, range queries */
+    uint32_t bits = 0, f_bits = 5;           /* of the id hash; of the scans' id filter */
+    std::vector<uint32_t> key;               /* hash of the queried ids */
+    std::vector<int32_t> head, next;
+    std::vector<uint32_t> start, list;       /* range queries by grid cell */
+    std::vector<uint32_t> filter;
+    uint64_t listed = 0, bytes = 0;
+
+    template <class F>
+    static void cells(const stc_query &q, const double *map, F f) {
+        const double ix = QGRID / (map[2] - map[0]), iy = QGRID / (map[3] - map[1]);
+        const double *b = q.box;
+        const int cx0 = grid_cell(b[0], map[0], ix), cx1 = grid_cell(b[2], map[0], ix);
+        const int cy0 = grid_cell(b[1], map[1], iy), cy1 = grid_cell(b[3], map[1], iy);
+        for (int cy = cy0; cy <= cy1; cy++)
+            for (int cx = cx0; cx <= cx1; cx++) f(cy * QGRID + cx);
+    }
+
+    void plan(const stc_query *q, uint32_t nq, const double *map) {
+        for (uint32_t i = 0; i < nq; i++) (q[i].kind == STC_Q_RANGE ? rq : oq).push_back(i);
+        if (!oq.empty()) {
+            bits = 6;
+            while ((1ull << bits) < 2ull * oq.size()) bits++;
+            const uint32_t size = 1u << bits, mask = size - 1;
+            key.assign(size, 0xFFFFFFFFu);
+            head.assign(size, -1);
+            next.assign(nq, -1);
+            for (size_t j = oq.size(); j-- > 0;) { /* insert in reverse: lists keep query order */
+                uint32_t qi = oq[j], id = q[qi].oid, h = oid_slot(id, bits);
+                while (key[h] != 0xFFFFFFFFu && key[h] != id) h = (h + 1) & mask;
+                key[h] = id;
+                next[qi] = head[h];
+                head[h] = (int32_t)qi;
+            }
+            /* the scans' filter: 64 bits or more per queried id, 2^16 (8 KB of LDS) at most */
+            f_bits = std::min(bits + 5, 16u);
+        }
+        filter.assign((1u << f_bits) / 32 + QGRID * QGRID / 32 + (rq.empty() ? 0 : QFINE * QFINE / 32), 0u);
+        for (uint32_t i : oq) {
+            const uint32_t h = oid_slot(q[i].oid, f_bits);
+            filter[h >> 5] |= 1u << (h & 31);
+        }
+        if (!rq.empty()) { /* counted per cell; listed in query order by list_cells */
+            uint32_t *cell_bits = filter.data() + (1u << f_bits) / 32;
+            start.assign(QGRID * QGRID + 1, 0);
+            for (uint32_t qi : rq) cells(q[qi], map, [&](int c) { start[c + 1]++; });
+            for (int c = 0; c < QGRID * QGRID; c++) {
+                listed += start[c + 1];
+                if (start[c + 1]) cell_bits[c >> 5] |= 1u << (c & 31);
+                start[c + 1] = (uint32_t)listed;
+            }
+            /* the fine grid's cells at and around the boxes; all of them where the map is too small for 32 bits */
+            const double x0 = map[0], y0 = map[1], ix = QGRID / (map[2] - map[0]), iy = QGRID / (map[3] - map[1]);
+            uint32_t *fine = cell_bits + QGRID * QGRID / 32;
+            const double fine_per = (double)QFINE / QGRID;
+            auto fine_of = [&](double v, double v0, double inv, int off) {
+                const double f = (v - v0) * inv * fine_per;
+                return std::min(std::max((!(f >= 0.0) ? 0 : f >= (double)QFINE ? QFINE - 1 : (int)f) + off, 0), QFINE - 1);
+            };
+            if (!(ix < 1e30 && iy < 1e30)) std::fill(fine, fine + QFINE * QFINE / 32, ~0u);
+            else
+                for (uint32_t qi : rq) {
+                    const double *b = q[qi].box;
+                    const int x0c = fine_of(b[0], x0, ix, -1), x1c = fine_of(b[2], x0, ix, 1);
+                    for (int y = fine_of(b[1], y0, iy, -1); y <= fine_of(b[3], y0, iy, 1); y++)
+                        for (int w = x0c >> 5; w <= x1c >> 5; w++)
+                            fine[y * (QFINE / 32) + w] |= (w == x0c >> 5 ? ~0u << (x0c & 31) : ~0u) & (w == x1c >> 5 ? ~0u >> (31 - (x1c & 31)) : ~0u);
+                }
+        }
+        for (uint64_t b : std::initializer_list<uint64_t>{(nq + 1ull) * 8, nq * sizeof(stc_query), key.size() * 4ull, head.size() * 4ull,
+                                                          next.size() * 4ull, oq.size() * 4ull, start.size() * 4ull, listed * 4, filter.size() * 4ull})
+            bytes += QueryUpload::room(b);
+    }
+
+    void list_cells(const stc_query *q, const double *map) {
+        if (rq.empty()) return;
+        list.resize(listed);
+        std::vector<uint32_t> at(start.begin(), start.end() - 1);
+        for (uint32_t qi : rq) cells(q[qi], map, [&](int c) { list[at[c]++] = qi; });
+    }
+};
+
+uint64_t stc_query_table_bytes(const stc_query *q, uint32_t nq, const double *map) {
+    QueryTables t;
+    t.plan(q, nq, map);
+    return t.bytes;
+}
+
+/* device memory for `need` bytes more, with the reserve left? */
+bool QueryAdmission::fits(uint64_t more) {
+    size_t total_b = 0, free_b = 0;
+    if (!more || hipMemGetInfo(&free_b, &total_b) != hipSuccess) return true;
+    free = free_b;
+    return more + reserve <= free_b;
+}
+int QueryAdmission::refuse(uint64_t more) {
+    need = more;
+    refused = true;
+    return STC_E_CAPACITY;
+}
+
 int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32_t nq, stc_hit *hits, uint64_t cap,
-                  uint64_t *n_hits, uint64_t *counts, uint64_t reserve, QueryRoom *more, hipStream_t s) {
+                  uint64_t *n_hits, uint64_t *counts, QueryAdmission &adm, QueryRoom *more, hipStream_t s) {
     if (nq == 0) {
         *n_hits = 0;
         if (more) more->all = true;
         return STC_OK;
     }
-    /* hash of the queried ids (object and pair queries) */
-    std::vector<uint32_t> oq;
-    for (uint32_t i = 0; i < nq; i++)
-        if (q[i].kind == STC_Q_OID || q[i].kind == STC_Q_PAIR) oq.push_back(i);
-    uint32_t bits = 0;
-    std::vector<uint32_t> key;
-    std::vector<int32_t> head, next;
-    if (!oq.empty()) {
-        bits = 6;
-        while ((1ull << bits) < 2ull * oq.size()) bits++;
-        const uint32_t size = 1u << bits, mask = size - 1;
-        key.assign(size, 0xFFFFFFFFu);
-        head.assign(size, -1);
-        next.assign(nq, -1);
-        for (size_t j = oq.size(); j-- > 0;) { /* insert in reverse: lists keep query order */
-            uint32_t qi = oq[j], id = q[qi].oid, h = oid_slot(id, bits);
-            while (key[h] != 0xFFFFFFFFu && key[h] != id) h = (h + 1) & mask;
-            key[h] = id;
-            next[qi] = head[h];
-            head[h] = (int32_t)qi;
-        }
-    }
-
-    /* grid of the range queries */
-    const double x0 = st.map[0], y0 = st.map[1];
-    const double ix = QGRID / (st.map[2] - st.map[0]), iy = QGRID / (st.map[3] - st.map[1]);
-    /* the scans' filter: 64 bits or more per queried id, 2^16 (8 KB of LDS) at most */
-    uint32_t f_bits = 5;
-    if (!oq.empty()) f_bits = std::min(bits + 5, 16u);
-    std::vector<uint32_t> rq;
-    for (uint32_t i = 0; i < nq; i++)
-        if (q[i].kind == STC_Q_RANGE) rq.push_back(i);
-    std::vector<uint32_t> filter((1u << f_bits) / 32 + QGRID * QGRID / 32 + (rq.empty() ? 0 : QFINE * QFINE / 32), 0u);
-    for (uint32_t i : oq) {
-        const uint32_t h = oid_slot(q[i].oid, f_bits);
-        filter[h >> 5] |= 1u << (h & 31);
-    }
-    uint32_t *cell_bits = filter.data() + (1u << f_bits) / 32;
-    std::vector<uint32_t> start, list;
-    if (!rq.empty()) { /* counted per cell, then listed in query order */
-        start.assign(QGRID * QGRID + 1, 0);
-        auto cells = [&](uint32_t qi, auto &&f) {
-            const double *b = q[qi].box;
-            const int cx0 = grid_cell(b[0], x0, ix), cx1 = grid_cell(b[2], x0, ix);
-            const int cy0 = grid_cell(b[1], y0, iy), cy1 = grid_cell(b[3], y0, iy);
-            for (int cy = cy0; cy <= cy1; cy++)
-                for (int cx = cx0; cx <= cx1; cx++) f(cy * QGRID + cx);
-        };
-        for (uint32_t qi : rq) cells(qi, [&](int c) { start[c + 1]++; });
-        for (int c = 0; c < QGRID * QGRID; c++) {
-            if (start[c + 1]) cell_bits[c >> 5] |= 1u << (c & 31);
-            start[c + 1] += start[c];
-        }
-        list.resize(start.back());
-        std::vector<uint32_t> at(start.begin(), start.end() - 1);
-        for (uint32_t qi : rq) cells(qi, [&](int c) { list[at[c]++] = qi; });
-        /* the fine grid's cells at and around the boxes; all of them where the map is too small for 32 bits */
-        uint32_t *fine = cell_bits + QGRID * QGRID / 32;
-        const double fine_per = (double)QFINE / QGRID;
-        auto fine_of = [&](double v, double v0, double inv, int off) {
-            const double f = (v - v0) * inv * fine_per;
-            return std::min(std::max((!(f >= 0.0) ? 0 : f >= (double)QFINE ? QFINE - 1 : (int)f) + off, 0), QFINE - 1);
-        };
-        if (!(ix < 1e30 && iy < 1e30)) std::fill(fine, fine + QFINE * QFINE / 32, ~0u);
-        else
-            for (uint32_t qi : rq) {
-                const double *b = q[qi].box;
-                const int x0c = fine_of(b[0], x0, ix, -1), x1c = fine_of(b[2], x0, ix, 1);
-                for (int y = fine_of(b[1], y0, iy, -1); y <= fine_of(b[3], y0, iy, 1); y++)
-                    for (int w = x0c >> 5; w <= x1c >> 5; w++)
-                        fine[y * (QFINE / 32) + w] |= (w == x0c >> 5 ? ~0u << (x0c & 31) : ~0u) & (w == x1c >> 5 ? ~0u >> (31 - (x1c & 31)) : ~0u);
-            }
-    }
-
-    /* one copy for all of it (each table was a copy of its own, waited for: 10 us and more a piece) */
-    uint64_t bytes = 0;
-    for (uint64_t b : std::initializer_list<uint64_t>{(nq + 1ull) * 8, nq * sizeof(stc_query), key.size() * 4, head.size() * 4,
-                                                      next.size() * 4, oq.size() * 4, start.size() * 4, list.size() * 4, filter.size() * 4})
-        bytes += QueryUpload::room(b);
+    QueryTables T;
+    T.plan(q, nq, st.map);
+    const std::vector<uint32_t> &oq = T.oq, &rq = T.rq;
+    const uint32_t nruns = (uint32_t)st.runs.size();
+    const uint64_t hits_need = std::max<uint64_t>(hits ? cap : 0, 1);
+    const uint64_t need = B->batch.growth(T.bytes) + (hits_need > B->hits_cap ? hits_need * sizeof(stc_hit) * 3 / 2 : 0);
+    if (T.listed > 0xFFFFFFFFull || !adm.fits(need)) return adm.refuse(need);
+    T.list_cells(q, st.map);
+    const uint64_t bytes = T.bytes;
     const uint64_t most = hits ? std::min<uint64_t>(cap, QSORT_HOST) : 0, res_words = nq + 1ull + most * 7;
-    if (B->batch.begin(bytes) || grow(&B->hits, &B->hits_cap, std::max<uint64_t>(cap, 1)))
+    if (B->batch.begin(bytes) || grow(&B->hits, &B->hits_cap, hits_need))
         return stc_hip_fail(hipErrorOutOfMemory, "query buffers", __FILE__, __LINE__);
     if (B->res_cap < res_words) {
         if (B->res) (void)hipHostFree(B->res);
@@ -1141,16 +1203,18 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     QDev Q;
     unsigned long long *counters = U.put((const unsigned long long *)nullptr, nq + 1ull); /* total hits, then per query */
     Q.q = U.put(q, nq);
-    Q.oh_key = U.put(key.data(), key.size());
-    Q.oh_head = U.put(head.data(), head.size());
-    Q.q_next = U.put(next.data(), next.size());
+    Q.oh_key = U.put(T.key.data(), T.key.size());
+    Q.oh_head = U.put(T.head.data(), T.head.size());
+    Q.q_next = U.put(T.next.data(), T.next.size());
     const uint32_t *oq_dev = U.put(oq.data(), oq.size());
-    Q.g_start = U.put(start.data(), start.size());
-    Q.g_list = U.put(list.data(), list.size());
-    Q.filter = U.put(filter.data(), filter.size());
-    Q.f_bits = f_bits;
-    Q.oh_bits = bits;
+    Q.g_start = U.put(T.start.data(), T.start.size());
+    Q.g_list = U.put(T.list.data(), T.list.size());
+    Q.filter = U.put(T.filter.data(), T.filter.size());
+    Q.f_bits = T.f_bits;
+    Q.oh_bits = T.bits;
     Q.n_range = (uint32_t)rq.size();
+    const double x0 = st.map[0], y0 = st.map[1];
+    const double ix = QGRID / (st.map[2] - st.map[0]), iy = QGRID / (st.map[3] - st.map[1]);
     Q.x0 = x0;
     Q.y0 = y0;
     Q.ix = ix;
@@ -1167,7 +1231,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     Q.counts = counters + 1;
     Q.nq = nq;
     Q.lds = nq <= QLDS;
-    const size_t q_scan_lds = ((Q.lds ? nq : 0) + filter.size()) * sizeof(uint32_t);
+    const size_t q_scan_lds = ((Q.lds ? nq : 0) + T.filter.size()) * sizeof(uint32_t);
     QCK(U.send(s));
     /* counts a planner adds without a kernel (CTFs wholly inside a range query) */
     std::vector<unsigned long long> planned(nq, 0);
@@ -1175,9 +1239,9 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     /* live meetings and memtable */
     if (st.stepped && st.meets.keys && st.nb) {
         const dim3 g((uint32_t)std::min<uint64_t>(blocks(st.nb, 256), 4096));
-        if (Q.n_range && bits) hipLaunchKernelGGL((k_q_live<true, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
+        if (Q.n_range && T.bits) hipLaunchKernelGGL((k_q_live<true, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
         else if (Q.n_range) hipLaunchKernelGGL((k_q_live<false, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
-        else if (bits) hipLaunchKernelGGL((k_q_live<true, false>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
+        else if (T.bits) hipLaunchKernelGGL((k_q_live<true, false>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
         QCK(hipGetLastError());
     }
     if (st.n_rec) {
@@ -1186,7 +1250,6 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         QCK(hipGetLastError());
     }
     /* runs */
-    const uint32_t nruns = (uint32_t)st.runs.size();
     if (nruns) {
         std::vector<uint4> cand;
         if (!rq.empty()) { /* while the scans run */
@@ -1220,8 +1283,17 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
             }
         }
         if (!oq.empty() || !cand.empty()) {
-            if (B->runs.begin(QueryUpload::room(nruns * sizeof(QueryRunDev)) + QueryUpload::room(cand.size() * sizeof(uint4))))
+            /* their number is known while the scans run: planned ahead of them, a batch of 2,000 would wait for the plan */
+            const uint64_t rb = QueryUpload::room(nruns * sizeof(QueryRunDev)) + QueryUpload::room(cand.size() * sizeof(uint4)),
+                           growth = B->runs.growth(rb);
+            if (!adm.fits(growth)) {
+                QCK(hipStreamSynchronize(s)); /* the scans, which read the batch's tables */
+                return adm.refuse(growth);
+            }
+            if (B->runs.begin(rb)) {
+                (void)hipStreamSynchronize(s);
                 return stc_hip_fail(hipErrorOutOfMemory, "query runs", __FILE__, __LINE__);
+            }
             const QueryRunDev *runs = B->runs.put(st.runs.data(), nruns);
             const uint4 *cand_dev = B->runs.put(cand.data(), cand.size());
             QCK(B->runs.send(s));
@@ -1261,7 +1333,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     uint64_t stored = Q.cap ? std::min<uint64_t>(cnt[0], cap) : 0;
     bool sorted = false;
     if (stored > QSORT_HOST && hits) {
-        const int rc = fetch_sorted(B, st, nq, stored, hits, reserve, &sorted, s);
+        const int rc = fetch_sorted(B, st, nq, stored, hits, adm.reserve, &sorted, s);
         if (rc) return rc;
     }
     if (stored && hits && !sorted) {
