@@ -2676,6 +2676,7 @@ struct StcCtx {
     bool drop_pending = false;           /* stc_drop_runs came while a flush thread ran */
     bool lp_valid = false;               /* lp holds a position step's leaf order (a permutation of the points) */
     uint8_t *xout = nullptr;             /* pinned: two chunks of an export on its way to the caller */
+    DBuf<uint8_t> xdev;                  /* one, where no pinned memory was to be had */
     hipEvent_t xev[2] = {nullptr, nullptr};
     DBuf<uint32_t> xtiles;               /* first output of each export tile, and the scan's scratch */
     PinnedPool pinned;
@@ -2832,11 +2833,25 @@ static int sort_pairs(const K *kin, const uint32_t *vin, DBuf<K> &k, DBuf<uint32
 }
 
 /* Chunks of an export: launch(k, buffer) fills chunk k of the pinned buffer on the context's stream,
- * take(k, buffer) copies it to the caller while the next one is filled. */
+ * take(k, buffer) copies it to the caller while the next one is filled. Without pinned memory a chunk
+ * at a time comes through device memory. */
 template <class Launch, class Take>
 static int export_chunks(StcCtx *c, uint64_t chunks, Launch launch, Take take) {
     constexpr size_t size = (size_t)LCHUNK * LTILE * 32;
-    if (!c->xout) CK(hipHostMalloc((void **)&c->xout, 2 * size, hipHostMallocDefault));
+    if (!c->xout && hipHostMalloc((void **)&c->xout, 2 * size, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->xout = nullptr;
+        if (c->xdev.ensure(size)) return fail(c, STC_E_CAPACITY, "export chunk");
+        std::vector<uint8_t> chunk(size);
+        for (uint64_t k = 0; k < chunks; k++) {
+            launch(k, c->xdev.p);
+            CK(hipGetLastError());
+            CK(hipMemcpyAsync(chunk.data(), c->xdev.p, size, hipMemcpyDeviceToHost, c->s));
+            CK(hipStreamSynchronize(c->s));
+            take(k, chunk.data());
+        }
+        return 0;
+    }
     for (int i = 0; i < 2; i++)
         if (!c->xev[i]) CK(hipEventCreateWithFlags(&c->xev[i], hipEventDisableTiming));
     auto start = [&](uint64_t k) {
@@ -3208,6 +3223,7 @@ int stc_destroy(void *vc) {
     for (int i = 0; i < 2; i++)
         if (c->xev[i]) (void)hipEventDestroy(c->xev[i]);
     c->xtiles.release();
+    c->xdev.release();
     for (int i = 0; i < 14; i++) if (c->ev[i]) hipEventDestroy(c->ev[i]);
     stc_schema_free(&c->sch);
     if (c->s) hipStreamDestroy(c->s);

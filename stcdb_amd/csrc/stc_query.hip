@@ -54,7 +54,8 @@ struct QDev {
 #define QPIECE (8ull << 20) /* pinned bytes an upload goes through at a time */
 
 /* host tables on their way to the device, as long as the batch makes them: built in pinned memory and sent with one copy
- * up to QPIECE, in pieces of that beyond (their sources stay as they are until then) */
+ * up to QPIECE, in pieces of that beyond (their sources stay as they are until then). Where no pinned memory is to be had
+ * they go as they are. */
 struct QueryUpload {
     uint8_t *host = nullptr, *dev = nullptr;
     uint64_t host_cap = 0, cap = 0, used = 0;
@@ -83,11 +84,13 @@ struct QueryUpload {
             if (host) (void)hipHostFree(host);
             host = nullptr;
             host_cap = 0;
-            if (hipHostMalloc((void **)&host, hc, hipHostMallocDefault) != hipSuccess) {
+            if (hipHostMalloc((void **)&host, hc, hipHostMallocDefault) == hipSuccess) {
+                host_cap = hc;
+            } else {
                 host = nullptr;
-                return -1;
+                pieces = true;
+                (void)hipGetLastError();
             }
-            host_cap = hc;
         }
         return 0;
     }
@@ -106,11 +109,12 @@ struct QueryUpload {
     hipError_t send(hipStream_t s) {
         if (!pieces) return hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, s);
         for (const Table &t : tables)
-            for (uint64_t o = 0; o < t.bytes; o += host_cap) {
-                const uint64_t n = std::min<uint64_t>(host_cap, t.bytes - o);
-                if (t.src) memcpy(host, t.src + o, n);
-                else memset(host, 0, n);
-                hipError_t e = hipMemcpyAsync(dev + t.at + o, host, n, hipMemcpyHostToDevice, s);
+            for (uint64_t o = 0, n; o < t.bytes; o += n) {
+                n = std::min<uint64_t>(host ? host_cap : t.bytes, t.bytes - o);
+                if (host && t.src) memcpy(host, t.src + o, n);
+                else if (host) memset(host, 0, n);
+                hipError_t e = host || t.src ? hipMemcpyAsync(dev + t.at + o, host ? host : t.src + o, n, hipMemcpyHostToDevice, s)
+                                             : hipMemsetAsync(dev + t.at, 0, n, s);
                 if (e == hipSuccess) e = hipStreamSynchronize(s);
                 if (e != hipSuccess) return e;
             }
@@ -977,8 +981,8 @@ __global__ void k_hit_place(const uint64_t *__restrict__ hits, const uint32_t *_
  * target, start, end): up to QRANK of them ranked, more by a radix sort of the packed fields on the device, then
  * chunks gathered in order into pinned memory and copied out while the next is
  * gathered. *done stays false when the fields do not pack, a value does not fit
- * its bits, or the scratch would leave less than `reserve` bytes of device
- * memory: the caller then sorts on the host. (330,000 hits: one host thread
+ * its bits, the scratch would leave less than `reserve` bytes of device memory,
+ * or no pinned memory is to be had: the caller then sorts on the host. (330,000 hits: one host thread
  * sorted them in 17 ms; the sort takes 0.25 ms, the fetch is bound by the link and
  * the copy into the caller's memory.) */
 static int fetch_sorted(QueryBufs *B, const QueryState &st, uint32_t nq, uint64_t n64, stc_hit *hits, uint64_t reserve,
@@ -1001,10 +1005,14 @@ static int fetch_sorted(QueryBufs *B, const QueryState &st, uint32_t nq, uint64_
             return STC_OK;
         }
     }
-    if (!B->wide) QCK(hipHostMalloc((void **)&B->wide, sizeof(uint32_t), hipHostMallocDefault));
-    for (int i = 0; i < 2; i++) {
-        if (!B->out[i]) QCK(hipHostMalloc((void **)&B->out[i], QFETCH * sizeof(stc_hit), hipHostMallocDefault));
+    bool pinned = B->wide || hipHostMalloc((void **)&B->wide, sizeof(uint32_t), hipHostMallocDefault) == hipSuccess;
+    for (int i = 0; i < 2 && pinned; i++) {
+        pinned = B->out[i] || hipHostMalloc((void **)&B->out[i], QFETCH * sizeof(stc_hit), hipHostMallocDefault) == hipSuccess;
         if (!B->out_ev[i]) QCK(hipEventCreateWithFlags(&B->out_ev[i], hipEventDisableTiming));
+    }
+    if (!pinned) {
+        (void)hipGetLastError(); /* the host sorts */
+        return STC_OK;
     }
     if (ranked) {
         uint32_t *rank = (uint32_t *)B->sort;
@@ -1196,8 +1204,12 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         if (B->res) (void)hipHostFree(B->res);
         B->res = nullptr;
         B->res_cap = 0;
-        QCK(hipHostMalloc((void **)&B->res, (res_words + res_words / 2) * 8, hipHostMallocDefault));
-        B->res_cap = res_words + res_words / 2;
+        if (hipHostMalloc((void **)&B->res, (res_words + res_words / 2) * 8, hipHostMallocDefault) == hipSuccess) {
+            B->res_cap = res_words + res_words / 2;
+        } else { /* the counters are copied instead, and the hits with them */
+            B->res = nullptr;
+            (void)hipGetLastError();
+        }
     }
     QueryUpload &U = B->batch;
     QDev Q;
@@ -1308,11 +1320,17 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     }
 
     /* results */
-    hipLaunchKernelGGL(k_q_finish, dim3(std::min<uint32_t>(blocks(res_words, 256), 256)), dim3(256), 0, s, counters, nq,
-                       (const uint64_t *)B->hits, most, B->res);
-    QCK(hipGetLastError());
+    std::vector<uint64_t> copied;
+    if (B->res) {
+        hipLaunchKernelGGL(k_q_finish, dim3(std::min<uint32_t>(blocks(res_words, 256), 256)), dim3(256), 0, s, counters, nq,
+                           (const uint64_t *)B->hits, most, B->res);
+        QCK(hipGetLastError());
+    } else {
+        copied.resize(nq + 1ull);
+        QCK(hipMemcpyAsync(copied.data(), counters, (nq + 1ull) * 8, hipMemcpyDeviceToHost, s));
+    }
     QCK(hipStreamSynchronize(s));
-    const uint64_t *cnt = B->res;
+    const uint64_t *cnt = B->res ? B->res : copied.data();
     uint64_t total = 0; /* the hits of the queries that store theirs */
     for (uint32_t i = 0; i < nq; i++) {
         const uint64_t ci = cnt[i + 1] + planned[i];
@@ -1337,7 +1355,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
         if (rc) return rc;
     }
     if (stored && hits && !sorted) {
-        if (stored <= most) memcpy(hits, cnt + nq + 1, stored * sizeof(stc_hit));
+        if (B->res && stored <= most) memcpy(hits, cnt + nq + 1, stored * sizeof(stc_hit));
         else QCK(hipMemcpy(hits, B->hits, stored * sizeof(stc_hit), hipMemcpyDeviceToHost));
         std::sort(hits, hits + stored, [](const stc_hit &a, const stc_hit &b) {
             if (a.query != b.query) return a.query < b.query;
