@@ -111,6 +111,7 @@ uint32_t stc_flush_raster_capped(const void *counters);
 
 int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count);
 void stc_flush_free(FlushWork *w);
+/* not 0: no run, and the memtable is as it was (flushed again, it gives the same run) */
 int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s);
 /* queue the last flush's copies to its pinned block behind the work queued on s so far (no-op when none wait) */
 int stc_flush_release(FlushWork *w, hipStream_t s);

@@ -688,6 +688,14 @@ __global__ __launch_bounds__(256) void k_bitmap_keys(const uint64_t *__restrict_
         if (bm[i]) atomicOr(&gw[i], bm[i]);
 }
 
+/* the oversize marks as they were before the STR sort overwrote them: a flush that does not finish, or starts over,
+ * leaves the memtable to be flushed again. The marks by area come out the same then; those by duration have no other
+ * record. */
+__global__ void k_restore_sids(uint32_t n, const uint8_t *__restrict__ part_tail, uint16_t *__restrict__ sids) {
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) sids[i] = part_tail[i];
+}
+
 /* the memtable's per-object state, empty (geometry.cu:2111-2131) */
 __global__ void k_reset_objects(uint32_t n, uint32_t *same_pid_count, uint16_t *sids) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -790,16 +798,20 @@ static int ensure_rec(FlushWork *w, uint64_t K) {
     void *ptrs[] = {w->keys_out, w->boxes_out, w->tkeys, w->tboxes, w->key_bytes};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    w->rec_cap = 0; /* until all of them are there again */
     w->keys_out = nullptr; w->boxes_out = nullptr; w->tkeys = nullptr; w->tboxes = nullptr; w->key_bytes = nullptr;
     if (hipMalloc((void **)&w->keys_out, nc * 16) || hipMalloc((void **)&w->boxes_out, nc * 16) ||
         hipMalloc((void **)&w->tkeys, nc * 16) || hipMalloc((void **)&w->tboxes, nc * 16) ||
-        hipMalloc((void **)&w->key_bytes, nc * 16))
-        return STC_E_HIP;
+        hipMalloc((void **)&w->key_bytes, nc * 16)) {
+        (void)hipGetLastError();
+        return stc_hip_fail(hipErrorOutOfMemory, "flush scratch", __FILE__, __LINE__);
+    }
     w->rec_cap = nc;
     return 0;
 }
 
-int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s) {
+/* *marked: the sids hold CTFs, no longer only the marks */
+static int flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, bool *marked, bool *again, hipStream_t s) {
     const uint32_t n = a->n, C = a->ctf_count;
     const uint32_t split = (uint32_t)std::sqrt((double)C);
     const uint64_t K = a->kv_count;
@@ -857,6 +869,7 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     hipLaunchKernelGGL(k_strip_keys, dim3(blocks_for(n, B)), dim3(B), 0, s, w->mid, n, sc, split, fc);
     FRC(sort_mid(w->oids, sc.on ? (int)sc.strip_bits : 40));
     /* and F3 */
+    *marked = true;
     hipLaunchKernelGGL(k_make_sid, dim3(blocks_for(n, B * CAP_ITEMS)), dim3(B), 0, s, w->oids, n, split, a->sids,
                        a->same_pid_count, w->capacity, C, fc);
     FCK(hipGetLastError());
@@ -905,7 +918,8 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     const FlushCounters &hfc = head.fc;
     if (hfc.str_wide && sc.on) { /* cannot happen for records inside the map; redone over the full keys */
         w->str_full = true;
-        return stc_flush_run(w, a, out, s);
+        *again = true;
+        return 0;
     }
     const stc_ctf_meta *hctfs = (const stc_ctf_meta *)((const FlushHead *)w->head + 1);
     std::vector<stc_ctf_meta> ctfs(hctfs, hctfs + C);
@@ -935,7 +949,10 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     L.counters = place(sizeof(FlushCounters));
     L.total = off;
     out->blk = out->acquire(out->acquire_ctx, L.total);
-    if (!out->blk.p) return stc_hip_fail(hipErrorOutOfMemory, "pinned run buffer", __FILE__, __LINE__);
+    if (!out->blk.p) {
+        (void)hipGetLastError();
+        return stc_hip_fail(hipErrorOutOfMemory, "pinned run buffer", __FILE__, __LINE__);
+    }
     if (a->reset_memtable) {
         hipLaunchKernelGGL(k_reset_objects, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a->same_pid_count, a->sids);
         FCK(hipGetLastError());
@@ -970,6 +987,23 @@ int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s
     info.oversize_oid_count = hfc.oversize_oid_count;
     info.key_bytes = head.key_bytes;
     return 0;
+}
+
+int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s) {
+    for (;;) {
+        bool marked = false, again = false;
+        const int rc = flush_run(w, a, out, &marked, &again, s);
+        if (!rc && !again) return 0;
+        if (marked) {
+            hipLaunchKernelGGL(k_restore_sids, dim3(blocks_for(a->n, 256)), dim3(256), 0, s, a->n, w->part_tail, a->sids);
+            const hipError_t e = hipGetLastError();
+            if (!rc && e != hipSuccess) return stc_hip_fail(e, "restoring the marks", __FILE__, __LINE__);
+        }
+        if (rc) {
+            (void)hipStreamSynchronize(s);
+            return rc;
+        }
+    }
 }
 
 uint32_t stc_flush_raster_capped(const void *counters) {

@@ -2670,6 +2670,8 @@ struct StcCtx {
     int frc = 0;                         /* its status and message */
     std::string ferr;
     FlushOut fout;
+    uint64_t f_kv_count = 0;             /* the memtable that it flushes */
+    uint32_t f_oversize = 0, f_end_time_min = 0;
     bool flush_fresh = false;            /* the joined run's copies wait for the next collect pass */
     bool fms_pending = false;            /* a joined flush whose device time is not reported yet */
     float flush_done_ms = 0;
@@ -2949,7 +2951,7 @@ static int queue_run_copies(StcCtx *c, bool now = true) {
 
 /* Copy a just-flushed run out of the flush buffers into its own HBM block
  * (packed keys, CTF metadata and bases, sids, oversize buffer) for queries. */
-static int keep_run_on_device(StcCtx *c, RunHost &run) {
+static int fill_device_run(StcCtx *c, RunHost &run) {
     const FlushWork &w = c->flushw;
     const uint32_t C = run.info.ctf_count, n = run.info.num_objects, nt = run.info.oversize_count;
     const uint64_t nf = run.info.kv_count;
@@ -2987,6 +2989,18 @@ static int keep_run_on_device(StcCtx *c, RunHost &run) {
     return stc_query_ctf_stats(q, run.ctfs.data(), run.stats, s) ? fail(c, STC_E_HIP, std::string("run statistics: ") + g_last_fail) : 0;
 }
 
+/* not 0: the run has no device block */
+static int keep_run_on_device(StcCtx *c, RunHost &run) {
+    const int rc = fill_device_run(c, run);
+    if (rc && run.dev) {
+        (void)hipStreamSynchronize(c->s);
+        (void)hipFree(run.dev);
+        run.dev = nullptr;
+    }
+    if (rc) (void)hipGetLastError();
+    return rc;
+}
+
 /* release every run's host block (a queued copy still completes) and HBM block */
 static void drop_all_runs(StcCtx *c) {
     std::vector<RunHost> gone;
@@ -3011,9 +3025,12 @@ static int join_flush(StcCtx *c) {
     c->fthr.join();
     c->frun = false;
     settle_deferred(c);
-    if (c->frc) {
+    if (c->frc) { /* its records are still the memtable's: the next step flushes them */
         release_block(c, c->fout.blk);
         c->fout = FlushOut();
+        c->kv_count = c->f_kv_count;
+        c->oversize_oid_count = c->f_oversize;
+        c->end_time_min = c->f_end_time_min;
         return fail(c, c->frc, "flush: " + c->ferr);
     }
     CK(hipStreamWaitEvent(c->s, c->fev[2], 0));
@@ -3027,8 +3044,8 @@ static int join_flush(StcCtx *c) {
     run.has_sorted = c->fout.has_sorted;
     run.blk = c->fout.blk;
     c->fout = FlushOut();
-    if (c->cfg.device_runs) CKRC(keep_run_on_device(c, run));
-    c->runs.push_back(std::move(run));
+    const int rc = c->cfg.device_runs ? keep_run_on_device(c, run) : 0;
+    c->runs.push_back(std::move(run)); /* without its device block, it can still be read */
     c->flush_fresh = true;
     if (c->drop_pending) { /* stc_drop_runs came while the flush ran */
         c->drop_pending = false;
@@ -3036,7 +3053,7 @@ static int join_flush(StcCtx *c) {
     } else {
         publish(c);
     }
-    return STC_OK;
+    return rc;
 }
 
 /* Room for n meetings of the step in the array that it writes. An array that
@@ -3684,6 +3701,7 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     /* 10: flush */
     uint32_t flushed = 0;
     if (c->kv_count > c->cfg.kv_restriction) {
+        int kept = 0;
         CK(hipEventRecord(c->ev[4], s));
         FlushArgs fa{};
         fa.n = n;
@@ -3712,6 +3730,9 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
             c->fout = FlushOut();
             c->fout.acquire = pool_acquire;
             c->fout.acquire_ctx = &c->pinned;
+            c->f_kv_count = fa.kv_count;
+            c->f_oversize = fa.oversize_oid_count;
+            c->f_end_time_min = fa.end_time_min;
             c->frun = true;
             c->fthr = std::thread([c, fa]() {
                 if (hipSetDevice(c->device) != hipSuccess || hipStreamWaitEvent(c->fs, c->fev[0], 0) != hipSuccess ||
@@ -3744,8 +3765,8 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
             run.lay = fo.lay;
             run.has_sorted = fo.has_sorted;
             run.blk = fo.blk;
-            if (c->cfg.device_runs) CKRC(keep_run_on_device(c, run));
-            c->runs.push_back(std::move(run));
+            kept = c->cfg.device_runs ? keep_run_on_device(c, run) : 0;
+            c->runs.push_back(std::move(run)); /* without its device block, it can still be read */
         }
         /* the memtable's per-object state was reset inside the flush (reset_memtable) */
         c->kv_count = 0;
@@ -3753,6 +3774,7 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
         c->end_time_min = t; /* process.cpp:271 with end_time_max = cur_time */
         c->epoch++;
         flushed = 1;
+        if (kept) return kept;
     }
     if (flushed) CK(hipEventRecord(c->ev[5], s));
     CK(hipEventSynchronize(c->ev[5])); /* without a flush reached already: the counters were written after it */
@@ -4453,7 +4475,6 @@ int stc_compact_runs(void *vc, uint32_t first, uint32_t count) {
     release();
     if (rc) {
         release_block(c, run.blk);
-        if (run.dev) (void)hipFree(run.dev);
         return rc;
     }
     CK(hipStreamSynchronize(s));

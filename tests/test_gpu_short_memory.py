@@ -99,3 +99,115 @@ assert np.array_equal(gpu.active()[0], ok)
 gpu.close()
 print("done")
 """)
+
+
+FLUSHES = r"""
+import test_gpu_compact as T
+w = workload("c1", num_objects=3000, kv_restriction=600, min_meet_time=2, max_meet_time=%d, ctf_count=16, reach_distance=15.0,
+             keep_pairs=3, device_runs=%d, async_flush=%d)
+w["gen"].update(n_hotspots=2, hotspot_frac=0.5, hotspot_sigma=300.0)
+gpu, orc = Pipeline(w["cfg"], w["box"]), O.Oracle(dict(w["cfg"], async_flush=0), w["box"])
+
+class Valid:
+    # the packed keys that a run has: none of a CTF flagged as wider than a key can be, and those of records in CTFs alone
+    # (an object that is oversize by the duration of a meeting is counted in its CTF too, as in the reference)
+    def __init__(self, p):
+        self.p, self.num_runs = p, p.num_runs
+    def run(self, i):
+        r = self.p.run(i)
+        m, at, left, out = r["ctfs"], 0, r["info"]["kv_count"], []
+        for cap, bits in zip(m["kv_capacity"].astype(int), m["key_bit"].astype(int)):
+            if bits <= 128:
+                out.append(r["key_bytes"][at:at + min(cap, left) * (bits // 8)])
+            at += cap * (bits // 8)
+            left = max(left - cap, 0)
+        return dict(r, key_bytes=np.concatenate(out))
+
+def same_runs(tag):
+    T.same_runs(Valid(gpu), Valid(orc), tag)
+frames = [xy.copy() for _, xy in HostTrace(w["gen"]).steps(30)]
+flushes = 0
+
+def refused(f, what):
+    try:
+        f()
+    except L.StcError as e:
+        assert what in str(e), e
+        return True
+    raise SystemExit("not refused")
+
+def history():
+    q = np.zeros(3000, dtype=QUERY_DTYPE)
+    q["kind"], q["t1"], q["oid"] = Q_OID, 1000, np.arange(3000)
+    out = []
+    for p in (gpu, orc):
+        h = p.query(q)[0]
+        out.append(np.sort(np.rec.fromarrays([h[k] for k in ("pid", "target", "start", "end")])))
+    return out
+"""
+
+
+def test_a_flush_without_pinned_memory_is_made_again(tmp_path):
+    """the same run as if nothing had failed, with objects that are oversize by the duration of a meeting"""
+    child(tmp_path, FLUSHES % (5, 0, 0) + r"""
+for t, xy in enumerate(frames):
+    o = orc.step(xy, t)
+    flushes += o["flushed"]
+    if o["flushed"] and flushes in (2, 5):
+        host.value = 1 << 20
+        assert refused(lambda: gpu.step(xy, t), "pinned run buffer")
+        host.value = NONE
+    g = gpu.step(xy, t)
+    assert g["flushed"] == o["flushed"], t
+assert failed.value >= 2 and flushes > 6
+same_runs("pinned")
+assert sum(orc.run(i)["info"]["oversize_count"] for i in range(flushes)) > 0
+gpu.close()
+print("done")
+""")
+
+
+def test_a_flush_beside_the_steps_that_fails_keeps_its_records(tmp_path):
+    child(tmp_path, FLUSHES % (64, 1, 1) + r"""
+for t, xy in enumerate(frames):
+    o = orc.step(xy, t)
+    flushes += o["flushed"]
+    if o["flushed"] and flushes == 2:
+        gpu.num_runs()
+        host.value = 1 << 20
+        gpu.step(xy, t)
+        assert refused(gpu.num_runs, "pinned run buffer")
+        host.value = NONE
+    else:
+        gpu.step(xy, t)
+n = gpu.num_runs()
+assert failed.value == 1 and n >= flushes - 2
+a, b = history()
+assert len(a) > 1000 and np.array_equal(a, b)
+gpu.close()
+print("done")
+""")
+
+
+def test_a_run_without_device_memory_is_still_read(tmp_path):
+    child(tmp_path, FLUSHES % (64, 1, 0) + r"""
+for t, xy in enumerate(frames):
+    o = orc.step(xy, t)
+    flushes += o["flushed"]
+    if o["flushed"] and flushes == 6:
+        dev.value = 1
+        assert refused(lambda: gpu.step(xy, t), "run.dev")
+        dev.value = NONE
+    else:
+        g = gpu.step(xy, t)
+        assert g["flushed"] == o["flushed"], t
+    if flushes == 6 and t + 1 < len(frames) and o["flushed"]:
+        break
+assert flushes == 6 and failed.value >= 1
+same_runs("device block")
+for u in range(t + 1, len(frames)):
+    gpu.step(frames[u], u)
+assert gpu.num_runs() > 7
+gpu.close()
+print("done")
+""")
