@@ -260,11 +260,12 @@ struct QStage {
     uint32_t *n;
 };
 
+template <bool STORE = true>
 __device__ inline void q_emit(const QDev &Q, const QStage &st, uint32_t qi, uint32_t pid, uint32_t target, uint32_t start,
                               uint32_t end, uint32_t source, const double *m) {
     if (Q.lds) atomicAdd(&q_lds[qi], 1u);
     else atomicAdd(&Q.counts[qi], 1ull);
-    if (!Q.cap || (Q.q[qi].flags & STC_QF_COUNT)) return;
+    if (!STORE || !Q.cap || (Q.q[qi].flags & STC_QF_COUNT)) return;
     const uint32_t at = atomicAdd(st.n, 1u);
     if (at < QSTAGE) st.h[at] = stc_hit{qi, pid, target, start, end, source, {m[0], m[1], m[2], m[3]}};
     else q_store(Q, qi, pid, target, start, end, source, m);
@@ -313,11 +314,12 @@ __device__ inline void q_stage_end(const QDev &Q, const QStage &st, const uint32
     q_stage_out(Q, st, min(n[wv], (uint32_t)QSTAGE), b);
 }
 
-#define Q_STAGE(st)                                                   \
-    __shared__ stc_hit st##_h[256 / STC_WAVE][QSTAGE];                \
-    __shared__ uint32_t st##_n[256 / STC_WAVE];                       \
-    const QStage st{st##_h[threadIdx.x / STC_WAVE], st##_n + threadIdx.x / STC_WAVE}; \
-    if ((threadIdx.x & (STC_WAVE - 1)) == 0) *st.n = 0;               \
+/* the workgroup's stages; without `on` (no hit is stored) only their shape */
+#define Q_STAGE(st, on)                                                       \
+    __shared__ stc_hit st##_h[(on) ? 256 / STC_WAVE : 1][(on) ? QSTAGE : 1];  \
+    __shared__ uint32_t st##_n[256 / STC_WAVE];                               \
+    const QStage st{st##_h[(on) ? threadIdx.x / STC_WAVE : 0], st##_n + threadIdx.x / STC_WAVE}; \
+    if ((threadIdx.x & (STC_WAVE - 1)) == 0) *st.n = 0;                       \
     __syncthreads()
 
 __device__ inline bool q_time(const stc_query &q, uint32_t s, uint32_t e) { return s <= q.t1 && e >= q.t0; }
@@ -360,17 +362,19 @@ __device__ inline int32_t oid_queries(const QDev &Q, uint32_t pid) {
 }
 
 /* the queries of that list for one meeting seen from pid */
+template <bool STORE = true>
 __device__ inline void match_oid(const QDev &Q, const QStage &st, int32_t qi, uint32_t pid, uint32_t target, uint32_t s,
                                  uint32_t e, uint32_t src, const double *m) {
     for (; qi >= 0; qi = Q.q_next[qi]) {
         const stc_query &q = Q.q[qi];
         if (!q_time(q, s, e)) continue;
         if (q.kind == STC_Q_OID || (q.kind == STC_Q_PAIR && q.oid2 == target))
-            q_emit(Q, st, (uint32_t)qi, pid, target, s, e, src, m);
+            q_emit<STORE>(Q, st, (uint32_t)qi, pid, target, s, e, src, m);
     }
 }
 
 /* range queries of one meeting (called once per meeting) */
+template <bool STORE = true>
 __device__ inline void match_range(const QDev &Q, const QStage &st, const uint32_t *flt, uint32_t pid, uint32_t target, uint32_t s,
                                    uint32_t e, uint32_t src, const double *m) {
     const uint32_t *cells = flt + (1u << Q.f_bits) / 32;
@@ -387,7 +391,7 @@ __device__ inline void match_range(const QDev &Q, const QStage &st, const uint32
                 if (!q_time(q, s, e) || !q_box(q, m)) continue;
                 if (!one && (grid_cell(fmax(m[0], q.box[0]), Q.x0, Q.ix) != cx || grid_cell(fmax(m[1], q.box[1]), Q.y0, Q.iy) != cy))
                     continue; /* counted in the cell of the intersection's low corner */
-                q_emit(Q, st, qi, pid, target, s, e, src, m);
+                q_emit<STORE>(Q, st, qi, pid, target, s, e, src, m);
             }
         }
 }
@@ -465,15 +469,29 @@ __device__ inline void decode_tail(const uint64_t *o_keys, const float4 *o_boxes
  * meetings read whole or looked up one by one: 1,000 objects among 256M
  * meetings 2.10 -> 0.83 ms (8 bytes each at 2.5 TB/s; the id filter and the
  * table now bound it), one among 10M 52 -> 25 us, 48 crowded boxes with 446,000
- * hits 465 -> 257 us (with the hits' reservations, at q_emit); 128 mixed
- * queries, bound by the lookups, 408 -> 429. */
-template <bool OIDS, bool RANGES>
+ * hits 465 -> 257 us (with the hits' reservations, at q_emit).
+ * Where ranges are counted, or asked among ids, most of the time goes to the
+ * lookups, whose reads the waves in flight have to hide. The round's meetings
+ * all go to the list before any is looked up (AFTER), so that the lookup is in
+ * the code once and runs with their boxes out of the registers, and a batch
+ * that stores no hit (STORE) has no stage for them: 82 to 86 registers, five
+ * waves a SIMD and 15 KB of LDS a workgroup become 61 and 16, or 48 (eight
+ * waves) and 3. 8.6M meetings: 100 counted boxes of 50 to 500 m where people
+ * are 362 -> 316 us, 20,000 of them 26.1 -> 23.1 ms, 256 of the whole map
+ * 19.9 -> 17.6 (28-byte meetings looked up as they came: 351 us, 23.9 and
+ * 17.4 ms), 128 mixed queries 576 -> 540 us. Counting batches read two
+ * meetings a lane at a time (one small box: 166 us; four 171, eight 190).
+ * The lookup stays inside the round with ids alone, where few meetings pass and
+ * it is short (1,000 ids: 167 us, 176 after it), and for stored ranges alone,
+ * bound by their hits (1,000 boxes, a thousand hits kept: 5.30 ms, 5.41). */
+template <bool OIDS, bool RANGES, bool STORE>
 __global__ __launch_bounds__(256) void k_q_live(Meets t, uint64_t nb, uint32_t last_t, QDev Q) {
-    constexpr int U = RANGES ? 4 : 8;
-    __shared__ uint64_t wait[256 / STC_WAVE][2 * STC_WAVE];
+    constexpr int U = RANGES ? (STORE ? 4 : 2) : 8;
+    constexpr bool AFTER = RANGES && (OIDS || !STORE); /* lookups after the round */
+    __shared__ uint32_t wait[256 / STC_WAVE][(AFTER ? U + 1 : 2) * STC_WAVE];
     const uint32_t *flt = q_scan_begin(Q);
-    Q_STAGE(st);
-    uint64_t *wq = wait[threadIdx.x / STC_WAVE];
+    Q_STAGE(st, STORE);
+    uint32_t *wq = wait[threadIdx.x / STC_WAVE];
     uint32_t waiting = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(STC_WAVE - 1u));
@@ -484,55 +502,62 @@ __global__ __launch_bounds__(256) void k_q_live(Meets t, uint64_t nb, uint32_t l
         __builtin_amdgcn_wave_barrier();
         waiting -= n;
         if (lane < n) {
-            const uint64_t i = wq[waiting + lane];
+            const uint64_t i = wq[waiting + lane]; /* a step has fewer than 2^32 meetings */
             const Bucket b = t.at(i);
             const uint32_t a = (uint32_t)(b.key >> 32), c = (uint32_t)b.key;
             if (c != DEAD_B) {
                 const double m[4] = {o2f(b.mbr[0]), o2f(b.mbr[1]), o2f(b.mbr[2]), o2f(b.mbr[3])};
                 /* a live meeting ends at the step that built the arrays */
                 if constexpr (OIDS) {
-                    match_oid(Q, st, oid_queries(Q, a), a, c, b.start, last_t, 0, m);
-                    match_oid(Q, st, oid_queries(Q, c), c, a, b.start, last_t, 0, m);
+                    match_oid<STORE>(Q, st, oid_queries(Q, a), a, c, b.start, last_t, 0, m);
+                    match_oid<STORE>(Q, st, oid_queries(Q, c), c, a, b.start, last_t, 0, m);
                 }
-                if constexpr (RANGES) match_range(Q, st, flt, a, c, b.start, last_t, 0, m);
+                if constexpr (RANGES) match_range<STORE>(Q, st, flt, a, c, b.start, last_t, 0, m);
             }
         }
-        q_stage_drain(Q, st);
+        if constexpr (STORE) q_stage_drain(Q, st);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); /* the list's places are written again */
+        __builtin_amdgcn_wave_barrier();
     };
-    for (uint64_t i0 = first; i0 < nb; i0 += stride * U) {
-        unsigned long long key[U];
-        uint4 mbr[U];
+    for (uint64_t i0 = first;; i0 += stride * U) {
+        const bool end = i0 >= nb;
+        if (!end) {
+            unsigned long long key[U];
+            uint4 mbr[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const uint64_t i = min(i0 + lane + u * stride, nb - 1);
-            if constexpr (OIDS) key[u] = t.keys[i];
-            if constexpr (RANGES) mbr[u] = t.mbrs[i];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const uint64_t i = i0 + lane + u * stride;
-            bool pass = false;
-            if constexpr (RANGES) pass = q_may_box(Q, flt, o2f(mbr[u].x), o2f(mbr[u].y), o2f(mbr[u].z), o2f(mbr[u].w));
-            if constexpr (OIDS) {
-                pass = pass || q_may_oid(Q, flt, (uint32_t)(key[u] >> 32)) || q_may_oid(Q, flt, (uint32_t)key[u]);
-                pass = pass && (uint32_t)key[u] != DEAD_B;
+            for (int u = 0; u < U; u++) {
+                const uint64_t i = min(i0 + lane + u * stride, nb - 1);
+                if constexpr (OIDS) key[u] = t.keys[i];
+                if constexpr (RANGES) mbr[u] = t.mbrs[i];
             }
-            pass = pass && i < nb;
-            const uint64_t passing = __ballot(pass);
-            if (pass) wq[waiting + (uint32_t)__popcll(passing & lt)] = i;
-            waiting += (uint32_t)__popcll(passing);
-            if (waiting >= STC_WAVE) look_up(STC_WAVE);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint64_t i = i0 + lane + u * stride;
+                bool pass = false;
+                if constexpr (RANGES) pass = q_may_box(Q, flt, o2f(mbr[u].x), o2f(mbr[u].y), o2f(mbr[u].z), o2f(mbr[u].w));
+                if constexpr (OIDS) {
+                    pass = pass || q_may_oid(Q, flt, (uint32_t)(key[u] >> 32)) || q_may_oid(Q, flt, (uint32_t)key[u]);
+                    pass = pass && (uint32_t)key[u] != DEAD_B;
+                }
+                pass = pass && i < nb;
+                const uint64_t passing = __ballot(pass);
+                if (pass) wq[waiting + (uint32_t)__popcll(passing & lt)] = (uint32_t)i;
+                waiting += (uint32_t)__popcll(passing);
+                if constexpr (!AFTER)
+                    if (waiting >= STC_WAVE) look_up(STC_WAVE);
+            }
         }
+        while (waiting >= (end ? 1u : (uint32_t)STC_WAVE)) look_up(min(waiting, (uint32_t)STC_WAVE));
+        if (end) break;
     }
-    look_up(waiting);
-    q_stage_end(Q, st, st_n);
+    if constexpr (STORE) q_stage_end(Q, st, st_n);
     q_scan_end(Q);
 }
 
 __global__ __launch_bounds__(256) void k_q_mem(const uint64_t *__restrict__ keys, const float4 *__restrict__ boxes,
                                                uint64_t n, uint32_t base, QDev Q) {
     const uint32_t *flt = q_scan_begin(Q);
-    Q_STAGE(st);
+    Q_STAGE(st, true);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(STC_WAVE - 1u)), lane = threadIdx.x & (STC_WAVE - 1);
     for (uint64_t i0 = first; i0 < n; i0 += stride) {
@@ -646,7 +671,7 @@ __global__ __launch_bounds__(256) void k_q_run_range(const QueryRunDev *__restri
     const QueryRunDev R = runs[cd.y];
     uint32_t pid, target, start, end, found = 0;
     double m[4];
-    Q_STAGE(st);
+    Q_STAGE(st, true);
     const bool store = Q.cap && !(q.flags & STC_QF_COUNT);
     auto hit = [&]() {
         found++;
@@ -1251,9 +1276,17 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     /* live meetings and memtable */
     if (st.stepped && st.meets.keys && st.nb) {
         const dim3 g((uint32_t)std::min<uint64_t>(blocks(st.nb, 256), 4096));
-        if (Q.n_range && T.bits) hipLaunchKernelGGL((k_q_live<true, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
-        else if (Q.n_range) hipLaunchKernelGGL((k_q_live<false, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
-        else if (T.bits) hipLaunchKernelGGL((k_q_live<true, false>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);
+        bool stores = false;
+        for (uint32_t i = 0; i < nq && Q.cap && !stores; i++) stores = !(q[i].flags & STC_QF_COUNT);
+#define Q_LIVE(OIDS, RANGES)                                                                                                        \
+    do {                                                                                                                            \
+        if (stores) hipLaunchKernelGGL((k_q_live<OIDS, RANGES, true>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q); \
+        else hipLaunchKernelGGL((k_q_live<OIDS, RANGES, false>), g, dim3(256), q_scan_lds, s, st.meets, st.nb, st.last_t, Q);       \
+    } while (0)
+        if (Q.n_range && T.bits) Q_LIVE(true, true);
+        else if (Q.n_range) Q_LIVE(false, true);
+        else if (T.bits) Q_LIVE(true, false);
+#undef Q_LIVE
         QCK(hipGetLastError());
     }
     if (st.n_rec) {
