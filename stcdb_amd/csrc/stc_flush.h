@@ -109,7 +109,9 @@ struct FlushOut {
 /* FlushCounters::raster_capped of the copied counters (flag 8 of every CTF) */
 uint32_t stc_flush_raster_capped(const void *counters);
 
-int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count);
+/* head: stc_flush_head_bytes of pinned memory, which stays the caller's */
+size_t stc_flush_head_bytes(uint32_t ctf_count);
+int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count, void *head);
 void stc_flush_free(FlushWork *w);
 /* not 0: no run, and the memtable is as it was (flushed again, it gives the same run) */
 int stc_flush_run(FlushWork *w, const FlushArgs *a, FlushOut *out, hipStream_t s);

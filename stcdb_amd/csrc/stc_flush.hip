@@ -719,7 +719,10 @@ __global__ void k_reset_objects(uint32_t n, uint32_t *same_pid_count, uint16_t *
         if (rc_) return rc_;                                                       \
     } while (0)
 
-int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count) {
+size_t stc_flush_head_bytes(uint32_t ctf_count) { return sizeof(FlushHead) + ctf_count * sizeof(stc_ctf_meta); }
+
+int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count, void *head) {
+    w->head = head;
     w->n = n;
     w->ctf_count = ctf_count;
     size_t N = n;
@@ -737,8 +740,7 @@ int stc_flush_init(FlushWork *w, uint32_t n, uint32_t ctf_count) {
     if (hipStreamCreateWithFlags(&w->cs, hipStreamNonBlocking) ||
         hipEventCreateWithFlags(&w->ready, hipEventDisableTiming) ||
         hipEventCreateWithFlags(&w->copied, hipEventDisableTiming) ||
-        hipEventCreateWithFlags(&w->planned, hipEventDisableTiming) ||
-        hipHostMalloc((void **)&w->head, sizeof(FlushHead) + ctf_count * sizeof(stc_ctf_meta), hipHostMallocDefault))
+        hipEventCreateWithFlags(&w->planned, hipEventDisableTiming))
         return STC_E_HIP;
     w->scan_temp_words = stc_radix_temp_words(n) + 64;
     if (hipMalloc((void **)&w->scan_temp, w->scan_temp_words * 4)) return STC_E_HIP;
@@ -752,7 +754,6 @@ void stc_flush_free(FlushWork *w) {
     if (w->ready) (void)hipEventDestroy(w->ready);
     if (w->copied) (void)hipEventDestroy(w->copied);
     if (w->planned) (void)hipEventDestroy(w->planned);
-    if (w->head) (void)hipHostFree(w->head);
     void *ptrs[] = {w->chunks, w->sids_out, w->o_bitmap_dev, w->mid, w->mid_alt, w->oids, w->oids_alt, w->slots, w->obj_first, w->group, w->capacity, w->ctf_base,
                     w->ctf_byte_base, w->ctfs, w->bitmaps, w->flags, w->part_tail, w->obj_key, w->obj_id, w->obj_cnt,
                     w->scan_temp, w->keys_out, w->boxes_out, w->tkeys, w->tboxes, w->key_bytes};

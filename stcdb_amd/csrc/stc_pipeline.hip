@@ -2645,10 +2645,11 @@ struct StcCtx {
     uint32_t *same_pid_count = nullptr;
     uint16_t *sids = nullptr;
     Counters *dcnt = nullptr;
-    Counters *hcnt = nullptr;  /* pinned */
-    uint32_t *hseq = nullptr;  /* pinned: the last wait whose counters are in hcnt */
+    uint8_t *hctl = nullptr;   /* pinned: hcnt, hinit, hseq and the flush's head in one block (each of its own is 250 us to free) */
+    Counters *hcnt = nullptr;
+    uint32_t *hseq = nullptr;  /* the last wait whose counters are in hcnt */
     uint32_t seq = 0;
-    Counters *hinit = nullptr; /* pinned: initial counter values of a step */
+    Counters *hinit = nullptr; /* initial counter values of a step */
     uint32_t oversize_oid_count = 0;
     uint32_t end_time_min = 0;
     uint64_t kv_count = 0;
@@ -3171,10 +3172,11 @@ int stc_create(const stc_config *cfg, const stc_box *mbr, void **out) {
         c->temp.ensure(stc_radix_temp_words((uint32_t)std::max<size_t>(n, node_cap)) + 64))
         return bad("device allocation failed");
     if (hipMalloc((void **)&c->dcnt, sizeof(Counters)) != hipSuccess) return bad("counters");
-    if (hipHostMalloc((void **)&c->hcnt, sizeof(Counters), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&c->hseq, 64, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&c->hinit, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
-        return bad("pinned");
+    const size_t part = (sizeof(Counters) + 255) & ~(size_t)255;
+    if (hipHostMalloc((void **)&c->hctl, 2 * part + 256 + stc_flush_head_bytes(C), hipHostMallocDefault) != hipSuccess) return bad("pinned");
+    c->hcnt = (Counters *)c->hctl;
+    c->hinit = (Counters *)(c->hctl + part);
+    c->hseq = (uint32_t *)(c->hctl + 2 * part);
     *c->hseq = 0;
     /* no meetings yet: every segment of the current array is empty */
     uint64_t nb = cfg->num_meeting_buckets ? cfg->num_meeting_buckets : 2ull * n;
@@ -3187,7 +3189,7 @@ int stc_create(const stc_config *cfg, const stc_box *mbr, void **out) {
     hipMemsetAsync(c->same_pid_count, 0, 4ull * n, c->s);
     hipMemsetAsync(c->sids, 0, 2ull * n, c->s);
     if (ensure_records(c, std::max<uint64_t>(1 << 16, (uint64_t)cfg->kv_restriction + 2))) return bad("records");
-    if (stc_flush_init(&c->flushw, n, C)) return bad("flush buffers");
+    if (stc_flush_init(&c->flushw, n, C, c->hctl + 2 * part + 256)) return bad("flush buffers");
     c->qb = stc_query_bufs_new();
     if (hipStreamSynchronize(c->s) != hipSuccess) return bad("init sync");
     *out = c;
@@ -3222,10 +3224,8 @@ int stc_destroy(void *vc) {
     if (c->same_pid_count) hipFree(c->same_pid_count);
     if (c->sids) hipFree(c->sids);
     if (c->dcnt) hipFree(c->dcnt);
-    if (c->hcnt) hipHostFree(c->hcnt);
-    if (c->hseq) hipHostFree(c->hseq);
-    if (c->hinit) hipHostFree(c->hinit);
     stc_flush_free(&c->flushw);
+    if (c->hctl) hipHostFree(c->hctl);
     for (auto &r : c->runs) {
         release_block(c, r.blk);
         if (r.dev) (void)hipFree(r.dev);

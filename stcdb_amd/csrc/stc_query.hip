@@ -59,7 +59,7 @@ struct QDev {
 struct QueryUpload {
     uint8_t *host = nullptr, *dev = nullptr;
     uint64_t host_cap = 0, cap = 0, used = 0;
-    bool pieces = false;
+    bool pieces = false, lent = false; /* lent: host is part of QueryBufs::first */
     struct Table { const uint8_t *src; uint64_t at, bytes; }; /* src null: zeros */
     std::vector<Table> tables;
     /* device bytes that begin(bytes) would add */
@@ -81,9 +81,7 @@ struct QueryUpload {
             cap = room_for(bytes);
         }
         if (std::min<uint64_t>(bytes, QPIECE) > host_cap) {
-            if (host) (void)hipHostFree(host);
-            host = nullptr;
-            host_cap = 0;
+            free_host();
             if (hipHostMalloc((void **)&host, hc, hipHostMallocDefault) == hipSuccess) {
                 host_cap = hc;
             } else {
@@ -120,11 +118,17 @@ struct QueryUpload {
             }
         return hipSuccess;
     }
+    void free_host() {
+        if (host && !lent) (void)hipHostFree(host);
+        host = nullptr;
+        host_cap = 0;
+        lent = false;
+    }
     void release() {
-        if (host) (void)hipHostFree(host);
+        free_host();
         if (dev) (void)hipFree(dev);
-        host = dev = nullptr;
-        host_cap = cap = 0;
+        dev = nullptr;
+        cap = 0;
     }
 };
 
@@ -132,6 +136,14 @@ struct QueryBufs {
     QueryUpload batch, runs;         /* the batch's tables and zeroed counters; the runs and their candidates */
     uint64_t *res = nullptr;         /* pinned: the counters, then the first hits */
     uint64_t res_cap = 0;
+    uint8_t *first = nullptr;        /* pinned: the two uploads' and res's first room in one (a block each is 250 us to free) */
+    bool res_lent = false;
+    void free_res() {
+        if (res && !res_lent) (void)hipHostFree(res);
+        res = nullptr;
+        res_cap = 0;
+        res_lent = false;
+    }
     stc_hit *hits = nullptr;
     uint64_t hits_cap = 0;
     uint8_t *sort = nullptr;         /* keys and places of the hits, and the sort's scratch */
@@ -151,7 +163,8 @@ void stc_query_bufs_free(QueryBufs *b) {
     if (!b) return;
     b->batch.release();
     b->runs.release();
-    if (b->res) (void)hipHostFree(b->res);
+    b->free_res();
+    if (b->first) (void)hipHostFree(b->first);
     if (b->hits) (void)hipFree(b->hits);
     if (b->sort) (void)hipFree(b->sort);
     for (int i = 0; i < 2; i++) {
@@ -179,9 +192,20 @@ static int grow(T **p, uint64_t *cap, uint64_t need) {
 /* with room for an ordinary batch, so that a context's first one allocates nothing */
 QueryBufs *stc_query_bufs_new() {
     QueryBufs *b = new QueryBufs();
-    (void)b->batch.begin(64u << 10);
-    (void)b->runs.begin(32u << 10);
-    if (hipHostMalloc((void **)&b->res, (QSORT_HOST * 7 + 4096) * 8, hipHostMallocDefault) == hipSuccess) b->res_cap = QSORT_HOST * 7 + 4096;
+    const uint64_t batch = 100u << 10, runs = 50u << 10, res = (QSORT_HOST * 7 + 4096) * 8;
+    if (hipHostMalloc((void **)&b->first, batch + runs + res, hipHostMallocDefault) == hipSuccess) {
+        b->batch.host = b->first;
+        b->batch.host_cap = batch;
+        b->runs.host = b->first + batch;
+        b->runs.host_cap = runs;
+        b->res = (uint64_t *)(b->first + batch + runs);
+        b->res_cap = res / 8;
+        b->batch.lent = b->runs.lent = b->res_lent = true;
+    } else {
+        b->first = nullptr;
+    }
+    if (hipMalloc((void **)&b->batch.dev, batch) == hipSuccess) b->batch.cap = batch;
+    if (hipMalloc((void **)&b->runs.dev, runs) == hipSuccess) b->runs.cap = runs;
     (void)grow(&b->hits, &b->hits_cap, 12u << 10);
     (void)hipGetLastError(); /* what could not be had now is asked for by the batch that needs it */
     return b;
@@ -1226,9 +1250,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     if (B->batch.begin(bytes) || grow(&B->hits, &B->hits_cap, hits_need))
         return stc_hip_fail(hipErrorOutOfMemory, "query buffers", __FILE__, __LINE__);
     if (B->res_cap < res_words) {
-        if (B->res) (void)hipHostFree(B->res);
-        B->res = nullptr;
-        B->res_cap = 0;
+        B->free_res();
         if (hipHostMalloc((void **)&B->res, (res_words + res_words / 2) * 8, hipHostMallocDefault) == hipSuccess) {
             B->res_cap = res_words + res_words / 2;
         } else { /* the counters are copied instead, and the hits with them */

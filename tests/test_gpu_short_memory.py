@@ -16,7 +16,7 @@ SHIM = r"""
 #include <stddef.h>
 static int (*real_host)(void **, size_t, unsigned), (*real_dev)(void **, size_t);
 size_t fail_host_from = (size_t)-1, fail_dev_from = (size_t)-1; /* allocations of at least so many bytes fail */
-int failed = 0;
+int failed = 0, host_calls = 0;
 int shim_init(const char *hip) {
     void *h = dlopen(hip, RTLD_LAZY);
     real_host = (int (*)(void **, size_t, unsigned))dlsym(h, "hipHostMalloc");
@@ -24,6 +24,7 @@ int shim_init(const char *hip) {
     return real_host && real_dev;
 }
 int hipHostMalloc(void **p, size_t n, unsigned f) {
+    host_calls++;
     if (n >= fail_host_from) { failed++; return 2; }
     return real_host(p, n, f);
 }
@@ -208,6 +209,28 @@ same_runs("device block")
 for u in range(t + 1, len(frames)):
     gpu.step(frames[u], u)
 assert gpu.num_runs() > 7
+gpu.close()
+print("done")
+""")
+
+
+def test_a_context_makes_few_pinned_blocks(tmp_path):
+    """each is a quarter of a millisecond to free: one of a context's own and one of its queries', and no more for its first
+    step, query and flush than the run's"""
+    child(tmp_path, r"""
+calls = C.c_int.in_dll(shim, "host_calls")
+w = workload("c1", num_objects=3000, kv_restriction=100, min_meet_time=1, reach_distance=15.0)
+w["gen"].update(n_hotspots=2, hotspot_frac=0.5, hotspot_sigma=300.0)
+gpu = Pipeline(w["cfg"], w["box"])
+assert calls.value <= 2, calls.value
+before = calls.value
+q = np.zeros(5, dtype=QUERY_DTYPE)
+q["kind"], q["t1"], q["oid"] = Q_OID, 100, np.arange(5)
+flushed = 0
+for t, xy in HostTrace(w["gen"]).steps(6):
+    flushed += gpu.step(xy, t)["flushed"]
+    gpu.query(q)
+assert flushed and calls.value - before <= flushed, (calls.value, flushed)
 gpu.close()
 print("done")
 """)
