@@ -39,6 +39,7 @@ HIT_DTYPE = np.dtype([("query", "<u4"), ("pid", "<u4"), ("target", "<u4"), ("sta
 Q_OID, Q_RANGE, Q_PAIR = 1, 2, 3
 QF_COUNT = 1  # STC_QF_COUNT: count the query's hits, store none
 FETCH_ROWS = 1 << 14  # hits a query without a capacity has room for at first
+GUESS_ROWS = 1 << 17  # and a live search at most (eight an object would be 3.4 GB of device memory for 5M objects)
 # stc_meeting_unit: the reference's 32-byte meeting_unit (src/tracing/workbench.h:62-83)
 MEETING_UNIT_DTYPE = np.dtype([("key", "<u8"), ("start", "<u4"), ("end", "<u4"), ("mbr", "<f4", (4,))])
 assert MEETING_UNIT_DTYPE.itemsize == 32
@@ -281,14 +282,18 @@ class Pipeline:
         _check(self.lib.stc_query_batch(self.ctx, _ptr(q), len(q), _ptr(hits), len(hits), C.byref(n), _ptr(counts)), self.ctx)
         return hits[:min(n.value, len(hits))]
 
-    def _fetch(self, rows, into, call):
-        """all hits of call(buffer, n): one call where they fit in `into`, or
-        in a first guess of `rows`, else a second with room for all"""
+    def _fetch(self, rows, call):
+        """all hits of call(buffer, n): one call where they fit in a first guess of `rows`, else a second with room for
+        all. A guess that is not admitted (STC_E_CAPACITY: it is larger than what there is to store) is asked without"""
         n = C.c_uint64()
-        hits = into if into is not None and len(into) else np.empty(rows, dtype=HIT_DTYPE)
-        _check(call(hits, n), self.ctx)
+        hits = np.empty(rows, dtype=HIT_DTYPE)
+        rc = call(hits, n)
+        if rc == L.STC_E_CAPACITY:
+            hits = hits[:0]
+            rc = call(None, n)
+        _check(rc, self.ctx)
         if n.value <= len(hits):
-            return hits[:n.value] if hits is into else hits[:n.value].copy()
+            return hits[:n.value].copy()
         hits = np.empty(n.value, dtype=HIT_DTYPE)
         _check(call(hits, n), self.ctx)
         return hits[:min(n.value, len(hits))]
@@ -309,8 +314,8 @@ class Pipeline:
         """established live contacts of the given objects (stc_live_search);
         hits as HIT_DTYPE with `query` the index into pids"""
         pids = np.ascontiguousarray(pids, dtype=np.uint32)
-        return self._fetch(1024 + 8 * len(pids), None, lambda h, n: self.lib.stc_live_search(
-            self.ctx, _ptr(pids), len(pids), _ptr(h), len(h), C.byref(n)))
+        return self._fetch(min(1024 + 8 * len(pids), GUESS_ROWS), lambda h, n: self.lib.stc_live_search(
+            self.ctx, _ptr(pids), len(pids), _ptr(h), 0 if h is None else len(h), C.byref(n)))
 
     def dump_run(self, i, directory, prefix, ctb):
         """write run i in the reference's file layout (stc_dump_run)"""
