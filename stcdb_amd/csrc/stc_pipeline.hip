@@ -43,6 +43,7 @@
 #include "stc_table.h"
 #include "stc_schema.h"
 #include "stc_serve.h"
+#include "stc_wait.h"
 #include "stc_query.h"
 #include "../../include/stcdb.h"
 
@@ -2769,13 +2770,7 @@ static int sync_counters(StcCtx *c) {
     hipLaunchKernelGGL(k_counters_out, dim3(1), dim3(256), 0, c->s, (const Counters *)c->dcnt, c->hcnt,
                        (const uint32_t *)c->sch.dcount, c->sch.hcount, c->hseq, seq);
     CK(hipGetLastError());
-    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(300);
-    do {
-        for (int k = 0; k < 32; k++) {
-            if (__atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) == seq) return 0;
-            __builtin_ia32_pause();
-        }
-    } while (std::chrono::steady_clock::now() < until);
+    if (look_for([&] { return __atomic_load_n(c->hseq, __ATOMIC_ACQUIRE) == seq; }, std::chrono::microseconds(300))) return 0;
     CK(hipStreamSynchronize(c->s));
     return 0;
 }
