@@ -26,8 +26,10 @@
  *               emitting pass, so no global atomics and a deterministic order.
  *  7. refine    the combinations of the check units (cuda_refinement,
  *               geometry.cu:424-497) regrouped by the owner of their pair (its
- *               smaller id): one wavefront per owner counts its pairs, a prefix
- *               sum gives each owner a segment, and a second pass writes them.
+ *               smaller id): each is decided once, a wave taking the owners of
+ *               a stretch together (collect); a prefix sum of the counts gives
+ *               each owner a segment, and a second pass sorts its pairs into
+ *               it (place).
  *  8. meetings  the live meetings are key-sorted segments, one per owner; a
  *  9. identify  merge per owner joins the step's pairs with the previous
  *               step's segment (insert/extend, geometry.cu:469-494) and turns
@@ -464,9 +466,8 @@ __global__ void k_amb_gather(const double2 *__restrict__ xy, const uint2 *__rest
     out[i] = make_double4(p.x, p.y, q.x, q.y);
 }
 
-/* leaf-ordered SoA and each point's rank within its leaf; and, a thread per leaf, the points beyond its buffer */
-/* Positions and scales in leaf order; the points' leaves in that order are the
- * sort's keys. Bound by the two reads at the points' ids, a line each (with the
+/* Positions and scales in leaf order (the points' leaves in that order are the
+ * sort's keys) and, a thread per leaf, the points beyond its buffer. Bound by the two reads at the points' ids, a line each (with the
  * leaf read there too and each point's rank written there, 5M objects 350 us;
  * 197 so). */
 __global__ void k_gather(const double2 *__restrict__ xy, const double *__restrict__ dlon,
@@ -689,7 +690,6 @@ __device__ inline unsigned long long wave_sum_u64(unsigned long long v) {
     return v;
 }
 
-/* geometry of the step that the pair passes read */
 /* a border point of the reverse lists in one 32-byte read: position, 1/dpm_lon
  * and id (its dpm_lon, needed only inside the guard band, is kept apart) */
 struct __align__(32) RevPt {
@@ -697,9 +697,8 @@ struct __align__(32) RevPt {
     uint32_t pid, pad;
 };
 
+/* geometry of the step that the pair passes read */
 struct PairGeo {
-    const double2 *xy;
-    const double *dlon;
     const double2 *lxy;                  /* positions in leaf order (one 16-byte read per candidate) */
     const uint32_t *pt_leaf, *leaf_start, *leaf_count, *lp;
     const double *ld;                    /* dpm_lon in leaf order */
@@ -709,7 +708,6 @@ struct PairGeo {
     const uint4 *prange;                 /* per point in leaf order: its later leaf members and the border
                                             points above it with a unit to its leaf (first, count, first, count) */
     const uint32_t *units;               /* the cross units' leaves, point after point */
-    const uint32_t *uoffset, *ucount;    /* a point's cross units: units[uoffset[p] ..] */
     const uint32_t *rev_start, *rev_pid; /* per leaf, by pid: the border points with a cross unit to it */
     const RevPt *rev;                    /* their positions, 1/dpm_lon and ids, in rev_pid order */
     const double *rev_dl;                /* their dpm_lon */
@@ -741,19 +739,6 @@ __device__ inline float4 pair_mbr(float ax, float ay, float bx, float by) {
 
 #define SRC_REV 0x80000000u /* source index tag: an index into the reverse lists, not the leaf-ordered arrays */
 
-/* Every (unit, member) combination of the step whose pair is owned by a,
- * visited by the 64 lanes of a wave, at most one per lane per call of
- * f(valid, decision, source) (source: the other point's index in the
- * leaf-ordered arrays, or SRC_REV | its index in the reverse lists):
- *   (i)   a against the later (larger-id) kept members of its own leaf (the
- *         inside unit of geometry.cu:258; probe a);
- *   (ii)  a against the kept members above a of the leaves of a's cross units
- *         (geometry.cu:295-392; probe a);
- *   (iii) the border points above a that have a cross unit to a's leaf, when a
- *         is a kept member of it (probe: the border point).
- * Each combination of the reference's refinement (geometry.cu:424-497) is
- * visited exactly once, by the owner of its pair. Wave-uniform. The collect
- * pass takes this form only for an owner with more sources than it lists. */
 /* first index i in [0, n) with arr[i] > v (n when none) for ascending arr: the
  * wave's lanes probe 64 evenly spaced entries per round, so a search takes one
  * or two dependent loads where a binary search takes log2(n). Wave-uniform. */
@@ -785,6 +770,19 @@ __device__ inline uint32_t place_of(const PairGeo &g, uint32_t a, int lane) {
     return st + wave_upper_bound(g.lp + st, g.leaf_count[L], a, lane) - 1;
 }
 
+/* Every (unit, member) combination of the step whose pair is owned by a,
+ * visited by the 64 lanes of a wave, at most one per lane per call of
+ * f(valid, decision, source) (source: the other point's index in the
+ * leaf-ordered arrays, or SRC_REV | its index in the reverse lists):
+ *   (i)   a against the later (larger-id) kept members of its own leaf (the
+ *         inside unit of geometry.cu:258; probe a);
+ *   (ii)  a against the kept members above a of the leaves of a's cross units
+ *         (geometry.cu:295-392; probe a);
+ *   (iii) the border points above a that have a cross unit to a's leaf, when a
+ *         is a kept member of it (probe: the border point).
+ * Each combination of the reference's refinement (geometry.cu:424-497) is
+ * visited exactly once, by the owner of its pair. Wave-uniform. The collect
+ * pass takes this form only for an owner with more sources than it lists. */
 template <class F>
 __device__ inline void owner_combos_by_source(uint32_t w, uint32_t a, const PairGeo &g, int lane, F &f) {
     const uint32_t L = g.lleaf[w];
@@ -2024,14 +2022,14 @@ __device__ inline uint32_t lower_bound_bucket(const M &s, uint32_t n, unsigned l
 }
 
 /* Merge of the step's pairs (pn, sorted by key, dead slots behind each owner's
- * live pairs) with the previous step's meetings (mold, sorted the same way),
+ * live pairs) with the previous step's meetings (okey, ostart, ombr, sorted the same way),
  * tile by tile, one wave per tile: the tile's range of previous meetings (tb)
  * is staged whole in the wave's LDS, then each new slot is read once and
  * joined with it. A live pair continues the previous meeting of its key
  * (start kept, MBR widened) or opens one (insert/extend, geometry.cu:469-494);
  * a dead slot becomes a tombstone; a previous meeting whose key has no pair
  * expires and, when it lasted long enough inside the map, becomes two records
- * (identify, geometry.cu:595-737). mnew[i] is built from pn[i]. A range
+ * (identify, geometry.cu:595-737). Entry i of the new arrays is built from pn[i]. A range
  * longer than OCAP is searched in global memory. */
 #define OPF (OCAP / STC_WAVE)   /* previous meetings per lane loaded at a tile's start */
 #define SPF (MTILE / STC_WAVE)  /* pair slots per lane loaded at a tile's start */
@@ -3420,10 +3418,9 @@ static int step_impl(StcCtx *c, const double2 *xy, uint32_t t, stc_step_out *out
                        (const uint32_t *)c->leaf_count.p, (const uint32_t *)c->rev_start.p,
                        (const uint32_t *)c->rev_pid.p, c->buf, c->prange.p);
     CK(hipGetLastError());
-    const PairGeo pg{xy, c->dlon.p, c->lxy.p, c->pt_leaf.p, c->leaf_start.p,
+    const PairGeo pg{c->lxy.p, c->pt_leaf.p, c->leaf_start.p,
                      c->leaf_count.p, c->lp.p, c->ld.p, c->lkeys.p, c->lunits.p, c->urange.p, c->prange.p,
-                     c->units.p, c->uoffset.p,
-                     c->ucount.p, c->rev_start.p, c->rev_pid.p,
+                     c->units.p, c->rev_start.p, c->rev_pid.p,
                      c->rev.p, c->rev_dl.p, n, c->buf, r, c->band, r * r * (1.0 - 1e-12),
                      r * r * (1.0 + 1e-12)};
     /* the collect pass: owners a wave takes on at a time, and a multiple of 8 workgroups for the XCD-aware
@@ -4396,38 +4393,37 @@ int stc_compact_runs(void *vc, uint32_t first, uint32_t count) {
     hipStream_t s = c->s;
     uint64_t *keys = nullptr;
     float4 *boxes = nullptr;
-    uint32_t *spc = nullptr, *dcount = nullptr, *ord = nullptr;
+    uint32_t *spc = nullptr, *dbad = nullptr, *ord = nullptr;
     uint16_t *sids = nullptr;
     auto release = [&]() {
         (void)hipStreamSynchronize(s);
-        for (void *p : {(void *)keys, (void *)boxes, (void *)spc, (void *)dcount, (void *)ord, (void *)sids})
+        for (void *p : {(void *)keys, (void *)boxes, (void *)spc, (void *)dbad, (void *)ord, (void *)sids})
             if (p) (void)hipFree(p);
     };
     if (hipMalloc((void **)&keys, std::max<uint64_t>(total, 1) * 16) ||
         hipMalloc((void **)&boxes, std::max<uint64_t>(total, 1) * 16) || hipMalloc((void **)&spc, 4ull * n) ||
-        hipMalloc((void **)&dcount, 8) || hipMalloc((void **)&ord, std::max<uint64_t>(total, 1) * 4) || hipMalloc((void **)&sids, 2ull * n)) {
+        hipMalloc((void **)&dbad, 4) || hipMalloc((void **)&ord, std::max<uint64_t>(total, 1) * 4) || hipMalloc((void **)&sids, 2ull * n)) {
         release();
         return fail(c, STC_E_CAPACITY, "compaction buffers");
     }
     int rc = STC_OK;
-    uint32_t h_count[2] = {0, 0}; /* objects with records, bad ids */
+    uint32_t bad = 0; /* a record's ids are not below num_objects */
     if (hipMemsetAsync(spc, 0, 4ull * n, s) || hipMemsetAsync(sids, 0, 2ull * n, s) ||
-        hipMemsetAsync(dcount, 0, 8, s))
+        hipMemsetAsync(dbad, 0, 4, s))
         rc = STC_E_HIP;
     uint64_t out0 = 0;
     for (uint32_t r = first; r < first + count && !rc; r++) {
         const RunHost &R = c->runs[r];
-        rc = stc_compact_decode(R.qdev, in_ctf[r - first], n, base, out0, keys, boxes, spc, ord, sids, dcount + 1,
-                                s);
+        rc = stc_compact_decode(R.qdev, in_ctf[r - first], n, base, out0, keys, boxes, spc, ord, sids, dbad, s);
         out0 += in_ctf[r - first] + R.info.oversize_count;
     }
-    if (!rc && (hipMemcpyAsync(h_count, dcount, 8, hipMemcpyDeviceToHost, s) || hipStreamSynchronize(s)))
+    if (!rc && (hipMemcpyAsync(&bad, dbad, 4, hipMemcpyDeviceToHost, s) || hipStreamSynchronize(s)))
         rc = STC_E_HIP;
     if (rc) {
         release();
         return fail(c, rc, std::string("compaction decode: ") + g_last_fail);
     }
-    if (h_count[1]) {
+    if (bad) {
         release();
         return fail(c, STC_E_STATE, "an input run holds a record whose object id is not below num_objects");
     }
