@@ -1933,7 +1933,7 @@ __global__ void k_tile_owner(const uint32_t *__restrict__ poff, uint32_t n, uint
  * two segments mostly hold the same partners) and widens by doubling steps
  * until it brackets the key, so a few dependent reads usually suffice. */
 template <class S>
-__global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const unsigned long long *__restrict__ mold,
+__global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, Meets mold,
                               const uint32_t *__restrict__ ooff, const uint32_t *__restrict__ poff, uint64_t n_o,
                               uint32_t n_tiles, const uint32_t *__restrict__ towner, uint32_t *__restrict__ tb) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1952,11 +1952,11 @@ __global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const unsi
     if (hi > lo && np_a) {
         /* bracket [lo, hi) around the scaled guess g: keys below lo are < key, keys from hi on are >= key */
         const uint32_t g = lo + (uint32_t)(((uint64_t)(first - p0) * (hi - lo)) / np_a);
-        if (g < hi && mold[g] < key) {
+        if (g < hi && mold.key(g) < key) {
             uint32_t step = 1, l = g + 1;
             while (l < hi) {
                 const uint32_t probe = min(l + step - 1, hi - 1);
-                if (mold[probe] < key) {
+                if (mold.key(probe) < key) {
                     l = probe + 1;
                     step <<= 1;
                 } else {
@@ -1966,10 +1966,10 @@ __global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const unsi
             }
             lo = l;
         } else {
-            uint32_t step = 1, r = g; /* mold[r] >= key or r == hi */
+            uint32_t step = 1, r = g; /* mold.key(r) >= key or r == hi */
             while (r > lo) {
                 const uint32_t probe = r - min(step, r - lo);
-                if (mold[probe] < key) {
+                if (mold.key(probe) < key) {
                     lo = probe + 1;
                     break;
                 }
@@ -1981,7 +1981,7 @@ __global__ void k_tile_bounds(const S *__restrict__ pn, uint64_t n_p, const unsi
     }
     while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (mold[mid] < key) lo = mid + 1;
+        if (mold.key(mid) < key) lo = mid + 1;
         else hi = mid;
     }
     tb[t] = lo;
@@ -2022,25 +2022,23 @@ __device__ inline uint32_t lower_bound_bucket(const M &s, uint32_t n, unsigned l
 }
 
 /* Merge of the step's pairs (pn, sorted by key, dead slots behind each owner's
- * live pairs) with the previous step's meetings (okey, ostart, ombr, sorted the same way),
+ * live pairs) with the previous step's meetings (old, sorted the same way),
  * tile by tile, one wave per tile: the tile's range of previous meetings (tb)
  * is staged whole in the wave's LDS, then each new slot is read once and
  * joined with it. A live pair continues the previous meeting of its key
  * (start kept, MBR widened) or opens one (insert/extend, geometry.cu:469-494);
  * a dead slot becomes a tombstone; a previous meeting whose key has no pair
  * expires and, when it lasted long enough inside the map, becomes two records
- * (identify, geometry.cu:595-737). Entry i of the new arrays is built from pn[i]. A range
+ * (identify, geometry.cu:595-737). New meeting i is built from pn[i]. A range
  * longer than OCAP is searched in global memory. */
 #define OPF (OCAP / STC_WAVE)   /* previous meetings per lane loaded at a tile's start */
 #define SPF (MTILE / STC_WAVE)  /* pair slots per lane loaded at a tile's start */
 
 template <class S>
 __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, uint64_t n_p,
-                                                    const unsigned long long *__restrict__ okey,
-                                                    const uint32_t *__restrict__ ostart, const uint4 *__restrict__ ombr,
+                                                    const uint8_t *__restrict__ old,
                                                     const uint32_t *__restrict__ tb, uint32_t n_tiles,
-                                                    unsigned long long *__restrict__ nkey, uint32_t *__restrict__ nstart,
-                                                    uint4 *__restrict__ nmbr, MergeArgs ma,
+                                                    uint8_t *__restrict__ mnew, MergeArgs ma,
                                                     MemtableDev mt, const float2 *__restrict__ posf,
                                                     const uint32_t *__restrict__ poff, const uint32_t *__restrict__ towner,
                                                     uint32_t n_obj, Counters *cnt) {
@@ -2083,6 +2081,7 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
         }
         const uint64_t i0 = (uint64_t)t * MTILE;
         const uint32_t np = i0 < n_p ? (uint32_t)min<uint64_t>(MTILE, n_p - i0) : 0u;
+        uint8_t *block = mnew + (uint64_t)t * MEET_BLOCK_BYTES; /* the tile's new meetings */
         /* all loads of the tile are issued before the first wait; indices are clamped into the
          * arrays (each holds at least one entry) and lanes past the tile's ends ignore theirs */
         S ps[SPF];
@@ -2093,8 +2092,7 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
 #pragma unroll
         for (int k = 0; k < OPF; k++) {
             const uint32_t i = min(o0 + lane + k * STC_WAVE, olast);
-            const uint4 m = ombr[i];
-            po[k] = Bucket{okey[i], ostart[i], {m.x, m.y, m.z, m.w}};
+            po[k] = Meets{old}.at(i);
         }
         /* the starts of the 64 owners after a0 (a0 owns the tile's first slot), read with the rest */
         uint32_t bst = 0;
@@ -2198,9 +2196,9 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
                     /* streamed out past the caches: the arrays are read again only by the next step */
                     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
                     const u32x4 mb = {nb.mbr[0], nb.mbr[1], nb.mbr[2], nb.mbr[3]};
-                    __builtin_nontemporal_store(nb.key, nkey + i0 + i);
-                    __builtin_nontemporal_store(nb.start, nstart + i0 + i);
-                    __builtin_nontemporal_store(mb, (u32x4 *)(nmbr + i0 + i));
+                    __builtin_nontemporal_store(nb.key, (unsigned long long *)(block + MEET_KEYS_AT) + i);
+                    __builtin_nontemporal_store(nb.start, (uint32_t *)(block + MEET_STARTS_AT) + i);
+                    __builtin_nontemporal_store(mb, (u32x4 *)block + i);
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -2243,7 +2241,7 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
             }
         };
         if (oin) join(StagedMeets{ob_l});
-        else join(MeetsFrom{Meets{okey, ostart, ombr}, o0});
+        else join(MeetsFrom{Meets{old}, o0});
         __builtin_amdgcn_wave_barrier(); /* the wave's LDS is reused by its next tile */
     }
     /* the waves' last staged meetings with one reservation, and one update of each counter, per
@@ -2292,13 +2290,13 @@ __global__ __launch_bounds__(256) void k_meet_merge(const S *__restrict__ pn, ui
 #define LCHUNK 16u     /* export tiles of a chunk */
 
 /* live buckets of each export tile */
-__global__ __launch_bounds__(256) void k_live_tiles(const unsigned long long *__restrict__ keys, uint64_t n, uint32_t *__restrict__ tiles) {
+__global__ __launch_bounds__(256) void k_live_tiles(Meets m, uint64_t n, uint32_t *__restrict__ tiles) {
     __shared__ uint32_t wsum[256 / STC_WAVE];
     const int lane = threadIdx.x & (STC_WAVE - 1), wv = threadIdx.x / STC_WAVE;
     uint32_t c = 0;
     for (uint32_t r = 0; r < LTILE / 256; r++) {
         const uint64_t i = (uint64_t)blockIdx.x * LTILE + r * 256 + threadIdx.x;
-        c += (uint32_t)__popcll(__ballot(i < n && (uint32_t)keys[i] != DEAD_B));
+        c += (uint32_t)__popcll(__ballot(i < n && (uint32_t)m.key(i) != DEAD_B));
     }
     if (lane == 0) wsum[wv] = c;
     __syncthreads();
@@ -2484,33 +2482,30 @@ struct DBuf {
     void release() { if (p) hipFree(p); p = nullptr; cap = 0; }
 };
 
-/* a step's meetings: the three arrays (MeetLayout) in one allocation (with an allocation each, to be
- * grown and freed in the first steps, 16 contexts took 353 ms to a steady state together, and 185 with one) */
+/* a step's meetings: whole blocks of them */
 struct MeetBuf {
     uint8_t *mem = nullptr;
-    MeetLayout lay{0};
-    bool holds(size_t n) const { return mem && n <= lay.cap; }
+    size_t cap = 0;
+    bool holds(size_t n) const { return mem && n <= cap; }
     int ensure(size_t n) {
         if (holds(n)) return 0;
         release();
-        const MeetLayout l(std::max<size_t>(n + n / 2, 1024));
-        if (hipMalloc((void **)&mem, l.bytes) != hipSuccess) {
+        const size_t blocks = (n + n / 2) / MEET_BLOCK + 1;
+        if (hipMalloc((void **)&mem, blocks * MEET_BLOCK_BYTES) != hipSuccess) {
             mem = nullptr;
             return -1;
         }
-        lay = l;
+        cap = blocks * MEET_BLOCK;
         return 0;
     }
     void release() {
         if (mem) hipFree(mem);
         mem = nullptr;
-        lay = MeetLayout(0);
+        cap = 0;
     }
-    uint4 *mbrs() const { return (uint4 *)mem; }
-    unsigned long long *keys() const { return (unsigned long long *)(mem + lay.keys); }
-    uint32_t *starts() const { return (uint32_t *)(mem + lay.starts); }
-    Meets view() const { return Meets{keys(), starts(), mbrs()}; }
+    Meets view() const { return Meets{mem}; }
 };
+static_assert(MEET_BLOCK == MTILE && MEET_BLOCK_BYTES == MEET_BLOCK * sizeof(Bucket), "a merge tile is a block, a bucket an entry of each row");
 
 /* A flushed run: metadata on the host, payload in a pinned block that the
  * copy stream fills while later steps run. */
@@ -2877,7 +2872,7 @@ static int export_live(StcCtx *c, uint64_t cap, Take take) {
     if (c->last_live != c->mlen) { /* dead buckets: the tiles' outputs by a scan */
         if (c->xtiles.ensure(tiles + stc_radix_temp_words((uint32_t)tiles))) return fail(c, STC_E_CAPACITY, "export tiles");
         hipLaunchKernelGGL(k_live_tiles, dim3((uint32_t)tiles), dim3(256), 0, c->s,
-                           (const unsigned long long *)c->meet[c->cur].keys(), c->mlen, c->xtiles.p);
+                           c->meet[c->cur].view(), c->mlen, c->xtiles.p);
         CK(hipGetLastError());
         CKRC(stc_exclusive_scan_u32(c->xtiles.p, c->xtiles.p, (uint32_t)tiles, nullptr, c->xtiles.p + tiles, c->s));
         base.resize(tiles);
@@ -3607,14 +3602,14 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
     if (c->tbounds.ensure(n_tiles + 1ull) || c->towner.ensure(n_tiles)) return fail(c, STC_E_CAPACITY, "merge tile bounds");
     if (g.boxed) {
         hipLaunchKernelGGL(k_tile_bounds<PairHit>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairHit *)c->pbox_new.p, g.slots, (const unsigned long long *)c->meet[cu].keys(),
+                           (const PairHit *)c->pbox_new.p, g.slots, c->meet[cu].view(),
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)nullptr, c->tbounds.p);
     } else {
         hipLaunchKernelGGL(k_tile_owner, dim3(blocks_for(c->n, 256)), dim3(256), 0, s, (const uint32_t *)c->moff[nx].p,
                            c->n, c->towner.p);
         hipLaunchKernelGGL(k_tile_bounds<PairSlot>, dim3(blocks_for(n_tiles + 1ull, 256)), dim3(256), 0, s,
-                           (const PairSlot *)c->pnew.p, g.slots, (const unsigned long long *)c->meet[cu].keys(),
+                           (const PairSlot *)c->pnew.p, g.slots, c->meet[cu].view(),
                            (const uint32_t *)c->moff[cu].p, (const uint32_t *)c->moff[nx].p, c->mlen, n_tiles,
                            (const uint32_t *)c->towner.p, c->tbounds.p);
     }
@@ -3637,17 +3632,16 @@ static int step_tail(StcCtx *c, uint32_t t, StepGeom &g, stc_step_out *out) {
             CK(hipMemcpyAsync(cnt, c->hinit, sizeof(Counters), hipMemcpyHostToDevice, s));
         }
         const MemtableDev mt{c->rec_keys, c->rec_boxes, c->rec_cap, c->rec_ord, c->same_pid_count, c->sids};
-        const Meets mo = c->meet[cu].view();
         CK(hipEventRecord(c->ev[8], s));
         if (g.boxed)
             hipLaunchKernelGGL(k_meet_merge<PairHit>, dim3(mgrid), dim3(256), 0, s, (const PairHit *)c->pbox_new.p,
-                               g.slots, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
+                               g.slots, (const uint8_t *)c->meet[cu].mem, (const uint32_t *)c->tbounds.p, n_tiles,
+                               c->meet[nx].mem, ma, mt, (const float2 *)nullptr, (const uint32_t *)nullptr,
                                (const uint32_t *)nullptr, c->n, cnt);
         else
             hipLaunchKernelGGL(k_meet_merge<PairSlot>, dim3(mgrid), dim3(256), 0, s, (const PairSlot *)c->pnew.p,
-                               g.slots, mo.keys, mo.starts, mo.mbrs, (const uint32_t *)c->tbounds.p, n_tiles,
-                               c->meet[nx].keys(), c->meet[nx].starts(), c->meet[nx].mbrs(), ma, mt, (const float2 *)c->posf_new.p, (const uint32_t *)c->moff[nx].p,
+                               g.slots, (const uint8_t *)c->meet[cu].mem, (const uint32_t *)c->tbounds.p, n_tiles,
+                               c->meet[nx].mem, ma, mt, (const float2 *)c->posf_new.p, (const uint32_t *)c->moff[nx].p,
                                (const uint32_t *)c->towner.p, c->n, cnt);
         CK(hipGetLastError());
         CK(hipEventRecord(c->ev[9], s));

@@ -551,8 +551,8 @@ __global__ __launch_bounds__(256) void k_q_live(Meets t, uint64_t nb, uint32_t l
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const uint64_t i = min(i0 + lane + u * stride, nb - 1);
-                if constexpr (OIDS) key[u] = t.keys[i];
-                if constexpr (RANGES) mbr[u] = t.mbrs[i];
+                if constexpr (OIDS) key[u] = t.key(i);
+                if constexpr (RANGES) mbr[u] = t.mbr(i);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -1296,7 +1296,7 @@ int stc_query_run(QueryBufs *B, const QueryState &st, const stc_query *q, uint32
     std::vector<unsigned long long> planned(nq, 0);
 
     /* live meetings and memtable */
-    if (st.stepped && st.meets.keys && st.nb) {
+    if (st.stepped && st.meets.base && st.nb) {
         const dim3 g((uint32_t)std::min<uint64_t>(blocks(st.nb, 256), 4096));
         bool stores = false;
         for (uint32_t i = 0; i < nq && Q.cap && !stores; i++) stores = !(q[i].flags & STC_QF_COUNT);
