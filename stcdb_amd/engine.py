@@ -39,7 +39,7 @@ HIT_DTYPE = np.dtype([("query", "<u4"), ("pid", "<u4"), ("target", "<u4"), ("sta
 Q_OID, Q_RANGE, Q_PAIR = 1, 2, 3
 QF_COUNT = 1  # STC_QF_COUNT: count the query's hits, store none
 FETCH_ROWS = 1 << 14  # hits a query without a capacity has room for at first
-GUESS_ROWS = 1 << 17  # and a live search at most (eight an object would be 3.4 GB of device memory for 5M objects)
+GUESS_ROWS = 1 << 21  # and a live search at most (eight an object would be 3.4 GB of device memory for 5M objects)
 # stc_meeting_unit: the reference's 32-byte meeting_unit (src/tracing/workbench.h:62-83)
 MEETING_UNIT_DTYPE = np.dtype([("key", "<u8"), ("start", "<u4"), ("end", "<u4"), ("mbr", "<f4", (4,))])
 assert MEETING_UNIT_DTYPE.itemsize == 32

@@ -19,16 +19,18 @@ class SearchStub:
         if cap > self.room:
             return L.STC_E_CAPACITY
         n._obj.value = self.found
-        for i in range(min(cap, self.found)):
-            ctypes.cast(hits, ctypes.POINTER(ctypes.c_uint32))[i * 14] = i
+        if cap:
+            out = np.ctypeslib.as_array(ctypes.cast(hits, ctypes.POINTER(ctypes.c_uint32)), shape=(cap * 14,))
+            out[: min(cap, self.found) * 14 : 14] = np.arange(min(cap, self.found))
         return 0
 
 
 @pytest.mark.parametrize("pids,found,room,asked", [
     (1, 5, 1 << 40, [1032]),                          # fits the guess
     (1, 5000, 1 << 40, [1032, 5000]),                 # does not
-    (5_000_000, 7, 1 << 40, [1 << 17]),               # the guess does not grow with the list without bound
-    (5_000_000, 200_000, 1 << 40, [1 << 17, 200_000]),
+    (5_000_000, 7, 1 << 40, [1 << 21]),               # the guess does not grow with the list without bound
+    (1_000_000, 200_000, 1 << 40, [1 << 21]),
+    (5_000_000, 2_100_000, 1 << 40, [1 << 21, 2_100_000]),
     (100, 20, 100, [1824, 0, 20]),                    # a guess that is refused where the hits are not
     (100, 0, 100, [1824, 0]),
 ])
