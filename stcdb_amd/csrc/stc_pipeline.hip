@@ -467,9 +467,9 @@ __global__ void k_amb_gather(const double2 *__restrict__ xy, const uint2 *__rest
 }
 
 /* Positions and scales in leaf order (the points' leaves in that order are the
- * sort's keys) and, a thread per leaf, the points beyond its buffer. Bound by the two reads at the points' ids, a line each (with the
- * leaf read there too and each point's rank written there, 5M objects 350 us;
- * 197 so). */
+ * sort's keys) and, a thread per leaf, the points beyond its buffer. Bound by
+ * the two reads at the points' ids, a line each (with the leaf read there too
+ * and each point's rank written there, 5M objects 350 us; 197 so). */
 __global__ void k_gather(const double2 *__restrict__ xy, const double *__restrict__ dlon,
                          const uint32_t *__restrict__ lp, uint32_t n, double2 *__restrict__ lxy, double *__restrict__ ld,
                          const uint32_t *__restrict__ leaf_count, uint32_t nl, uint32_t buf, Counters *cnt) {
@@ -955,8 +955,9 @@ struct CollectLds {          /* one wave's: the source ranges of the owners at h
  * round's 64 combinations form a 64-bit mask, and the set bits up to a lane
  * tell its range. Takes are compacted in that order, so each owner's run is
  * contiguous; the takes ahead of an owner's first combination are counted by
- * its lane. What bounds it: the issue of some hundred instructions a round,
- * the positions coming from cache. With an owner per wave instead, the set-up
+ * its lane. What bounds it: the issue of some hundred instructions a round
+ * (0.6 of the VALU's slots at 10M objects) and, at that size, the positions
+ * that the L2s do not hold (14.7 GB). With an owner per wave instead, the set-up
  * of an owner and the unfilled lanes of its last round took most of the time
  * where owners have few combinations (50k objects, 26 each: 137 us, now 22;
  * 1M, 97 each: 529 us, now 333; 5M, 145 each: 3.76 ms, now 2.42; 10M, 220 each:
